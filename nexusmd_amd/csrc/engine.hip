@@ -137,6 +137,20 @@ static int grid_rule(double L) {
     return p;
 }
 
+// Pair-list entries per chunk of the pair kernel, by the system's own size (not
+// the batch's: a request's arithmetic is the same alone and in any batch).  A
+// chunk costs its wavefront a claim, the i data and a force flush besides its
+// entries, so large systems take the longest; a small system's list in chunks of
+// 32 leaves most of the chip idle while a few wavefronts work through theirs.
+// FP64, whose pairs are dear: us per 100 steps of the 1,500-bead chain with 8,
+// 16, 32 entries: 7980, 9330, 13170; per 25 of 100,000 atoms: 19680, 18010,
+// 17560.  Mixed, where the kernels beside the pair kernel end after it on small
+// systems and its extra flushes delay them: 7950, 7840, 7730 on the chain.
+static int chunk_entries_for(int n_atoms, bool mixed) {
+    if (mixed) return kChunkEntries;
+    return n_atoms < 6000 ? 8 : kChunkEntries;
+}
+
 // ----------------------------------------------------------- tuning cache
 //
 // Launch shapes chosen by autotune, by key, for the process; with
@@ -324,7 +338,8 @@ class Engine : public EngineBase {
             d.list_off = (int)list_off;
             d.list_cap = (int)std::min<double>(2.0e9, per_super * d.super_cap + 64);
             d.chunk_off = (int)chunk_off;
-            d.chunk_cap = d.list_cap / kChunkEntries + d.super_cap;
+            d.chunk_entries = chunk_entries_for(n, P::mixed);
+            d.chunk_cap = d.list_cap / d.chunk_entries + d.super_cap;
             d.emask_off = (int)emask_off;
             d.emask_cap = (int)(std::max<long long>(256, (long long)h.excl_idx.size() / 2 + 64) * h.list_scale);
             // PME grid
@@ -443,15 +458,11 @@ class Engine : public EngineBase {
         dalloc(&B.cl_half, S / 8 + 1, o, B.stream);
         dalloc(&B.super_sys, B.n_super_cap, o, B.stream);
         dalloc(&B.super_item, B.n_super_cap, o, B.stream);
-        dalloc(&B.chunk_sys, B.n_chunk_cap, o, B.stream);
         dalloc(&B.slot_zkey, S, o, B.stream);
         dalloc(&B.slot_wpos, S, o, B.stream);
         dalloc(&B.chunks, B.n_chunk_cap, o, B.stream);
         dalloc(&B.chunk_prefix, B.nsys + 1, o, B.stream);
-        dalloc(&B.chunk_cost, B.n_chunk_cap, o, B.stream);
         B.pair_blocks = pair_grid_blocks<P>(B.n_cu, B.n_chunk_cap, tuning_.pair_per_cu);
-        B.pair_waves = B.pair_blocks * kPairWaves;
-        dalloc(&B.wave_start, (size_t)B.pair_waves + 1, o, B.stream);
         dalloc(&B.pair_pool, (size_t)kPoolInts, o, B.stream);
         if (B.nsys == 1 && lite_mode_) {
             // the update's report to the host, for the choice of step graph
@@ -486,7 +497,7 @@ class Engine : public EngineBase {
         hipStream_t st = B.stream;
         const int ns = B.nsys;
         std::vector<double> mass, invm, q, sig, eps;
-        std::vector<int> atom_sys, slot_sys, col_sys, super_sys, chunk_sys, eoff(1, 0), eidx;
+        std::vector<int> atom_sys, slot_sys, col_sys, super_sys, eoff(1, 0), eidx;
         std::vector<int2> epairs, bidx;
         std::vector<double2> bpar, apar;
         std::vector<int4> aidx, tidx;
@@ -542,7 +553,6 @@ class Engine : public EngineBase {
             for (int i = 0; i < d.slot_cap; ++i) slot_sys.push_back(s);
             for (int i = 0; i < d.ncx * d.ncy; ++i) col_sys.push_back(s);
             for (int i = 0; i < d.super_cap; ++i) super_sys.push_back(s);
-            for (int i = 0; i < d.chunk_cap; ++i) chunk_sys.push_back(s);
             for (auto& b : h.bonds) { bidx.push_back(make_int2(a0 + b.p1, a0 + b.p2)); bpar.push_back(make_double2(b.d, b.k)); }
             for (auto& a : h.angles) {
                 aidx.push_back(make_int4(a0 + a.p1, a0 + a.p2, a0 + a.p3, 0));
@@ -669,7 +679,6 @@ class Engine : public EngineBase {
         upload(B.slot_sys, slot_sys, st);
         upload(B.col_sys, col_sys, st);
         upload(B.super_sys, super_sys, st);
-        upload(B.chunk_sys, chunk_sys, st);
         upload(B.excl_off, eoff, st);
         upload(B.excl_idx, eidx, st);
         upload(B.excl_pairs, epairs, st);

@@ -25,8 +25,8 @@
 //
 // Every kernel first checks the system's rebuild flag, which the integrator
 // raises when an atom has moved more than skin/2 since the last build; the
-// last kernel (nl_waves) cuts the chunk ranges of the pair kernel's
-// wavefronts, and the kernel launched before the pair kernel clears the flag
+// last kernel (nl_waves) lines the systems' chunks up for the pair kernel, and
+// the kernel launched before the pair kernel clears the flag
 // (nl_clear_flag when no pair kernel follows).  Between builds the integrator
 // keeps the slot-order positions current.
 #include "nx_device.h"
@@ -400,7 +400,7 @@ __global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysC
                                                           const float4* cl_half, const float4* slot_wpos,
                                                           const int* atom_of_slot, const int* slot_of_atom,
                                                           const int* excl_off, const int* excl_idx, uint2* list,
-                                                          unsigned long long* emask, int4* chunks, int* chunk_cost,
+                                                          unsigned long long* emask, int4* chunks,
                                                           int n_items_total) {
     const int item = xcd_remap(blockIdx.x, gridDim.x);
     if (item >= n_items_total) return;
@@ -639,7 +639,7 @@ __global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysC
             atomicOr(&emask[(size_t)g * 8 + k], 1ull << (x_rec[t] & 63u));
         }
     }
-    const int nch = (ne + kChunkEntries - 1) / kChunkEntries;
+    const int ce = d.chunk_entries, nch = (ne + ce - 1) / ce;
     if (tid == 0) {
         const int b = atomicAdd(&sc[s].list_count, ne);
         lbase = (b + ne > d.list_cap) ? -1 : b;
@@ -665,24 +665,19 @@ __global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysC
         super_item[item] = it;
     }
     for (int c = tid; c < nch; c += kPlThreads) {
-        const int e0 = d.list_off + lbase + c * kChunkEntries;
-        const int e1 = d.list_off + lbase + min(ne, (c + 1) * kChunkEntries);
+        const int e0 = d.list_off + lbase + c * ce;
+        const int e1 = d.list_off + lbase + min(ne, (c + 1) * ce);
         chunks[d.chunk_off + cbase + c] = make_int4(fc, ncl, e0, e1);
-        int cost = kCostChunk;
-        for (int e = c * kChunkEntries; e < min(ne, (c + 1) * kChunkEntries); ++e)
-            cost += kCostEntry + kCostTile * __popc(l_ent[e] >> 24);
-        chunk_cost[d.chunk_off + cbase + c] = cost;
     }
 }
 
 // Last kernel of the list work, one block.  After a build in any system of the
-// batch: the batch's chunk order (system by system, prefix[]) and, for the NW
-// wavefronts of the pair kernel, contiguous chunk ranges of near-equal cost:
-// chunk g goes to wavefront floor(NW * (midpoint of g's cost interval) / total
-// cost), so wave_start[w] is the first chunk whose midpoint reaches w / NW of
-// the total.
-constexpr int kWavesLdsSys = 1024;     // systems whose chunk prefix nl_waves keeps in LDS
-
+// batch: the batch's chunk order, system by system (prefix[], its last element
+// the batch's chunk count).  The pair kernel cuts its ranges from the count
+// alone; cutting them here by each chunk's estimated work took this one block
+// 19 us a step in a 24-request batch, 40 us a build at 100k atoms and 420 us at
+// a million, and a prefix over the systems takes 3.
+//
 // With `pool` non-null it also does what the pair kernel's set-up launch does
 // (after every read of the flags): clears the rebuild flags, counts the
 // builds and resets the pair kernel's claim counters.  In a step without the
@@ -695,10 +690,9 @@ constexpr int kWavesLdsSys = 1024;     // systems whose chunk prefix nl_waves ke
 // steps done, and the report count, in one 16-byte store.  The report is a
 // forecast aid only: the device freezes a step whose list is due whatever
 // the host chose.
-__device__ __forceinline__ void waves_pair_begin(SysCount* sc, int nsys, int* pool, int lite, unsigned* step_seq,
-                                                 StepInfo* info, float dmax2) {
+__device__ __forceinline__ void waves_pair_begin(SysCount* sc, int nsys, int lite, unsigned* step_seq, StepInfo* info,
+                                                 float dmax2) {
     const int tid = threadIdx.x;
-    if (tid < 8) pool[tid * kPoolStride] = 0;
     for (int s = tid; s < nsys; s += blockDim.x) {
         const int due = sc[s].rebuild;
         if (due) {
@@ -719,106 +713,42 @@ __device__ __forceinline__ void waves_pair_begin(SysCount* sc, int nsys, int* po
     }
 }
 
-__global__ __launch_bounds__(1024) void nl_waves(const SysDev* sd, SysCount* sc, int nsys, const int* chunk_cost,
-                                                 int* prefix, int* wave_start, int NW, int* pool, int lite,
-                                                 unsigned* step_seq, StepInfo* info, unsigned* step_max) {
-    __shared__ int any, total;
-    __shared__ long long wsum[16];
-    __shared__ float dmax_s[1];
-    __shared__ int pre_s[kWavesLdsSys + 1], off_s[kWavesLdsSys];
+__global__ __launch_bounds__(kPlThreads) void nl_waves(const SysDev* sd, SysCount* sc, int nsys, int* prefix,
+                                                       int pair_blocks, int* pool, int lite, unsigned* step_seq,
+                                                       StepInfo* info, unsigned* step_max) {
+    __shared__ int wsum[kPlThreads / 64];
     const int tid = threadIdx.x;
+    float dmax2 = 0.0f;
     if (info && tid < 64) {     // the largest of the update's slots (wave 0), which it clears
-        float m = 0.0f;
         if (tid < kStepMaxSlots) {
-            m = __uint_as_float(step_max[tid]);
+            dmax2 = __uint_as_float(step_max[tid]);
             step_max[tid] = 0u;
         }
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-        if (tid == 0) dmax_s[0] = m;
+        for (int o = 32; o > 0; o >>= 1) dmax2 = fmaxf(dmax2, __shfl_xor(dmax2, o, 64));
     }
-    if (tid == 0) {
-        int a = 0;
-        if (!lite)      // no list was built: the ranges of the last build stand
-            for (int s = 0; s < nsys; ++s) a |= sc[s].rebuild;
-        if (a) {
-            int t = 0;
-            for (int s = 0; s < nsys; ++s) {
-                prefix[s] = t;
-                if (s < kWavesLdsSys) { pre_s[s] = t; off_s[s] = sd[s].chunk_off; }
-                // a system whose build overflowed has an incomplete list (a block that
-                // overflowed reserved chunk slots it did not write): no pair work
-                if (!sc[s].overflow) t += min(sc[s].n_chunks, sd[s].chunk_cap);
-            }
-            prefix[nsys] = t;
-            if (nsys <= kWavesLdsSys) pre_s[nsys] = t;
-            total = t;
-        }
-        any = a;
+    int due = 0;
+    if (!lite)      // without the list kernels no list was built: the last build's order stands
+        for (int s = tid; s < nsys; s += kPlThreads) due |= sc[s].rebuild;
+    const int any = __syncthreads_or(due);      // the flags are read before they are cleared
+    if (pool) waves_pair_begin(sc, nsys, lite, step_seq, info, dmax2);
+    if (!any) {
+        if (pool) pool_begin(tid, prefix[nsys], pool, pair_blocks);
+        return;
     }
-    __syncthreads();
-    const float dmax2 = (info && tid == 0) ? dmax_s[0] : 0.0f;
-    if (pool) waves_pair_begin(sc, nsys, pool, lite, step_seq, info, dmax2);       // the flags were read above
-    if (!any) return;
-    const int T = total;
-    const bool lds = nsys <= kWavesLdsSys;
-    auto pre = [&](int s) { return lds ? pre_s[s] : prefix[s]; };
-    auto sys_of = [&](int g) {          // largest s with prefix[s] <= g
-        int lo = 0, hi = nsys - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (pre(mid) <= g) lo = mid; else hi = mid - 1;
-        }
-        return lo;
-    };
-    auto cost_of = [&](int g, int& s) {
-        while (g >= pre(s + 1)) ++s;
-        return (long long)chunk_cost[(lds ? off_s[s] : sd[s].chunk_off) + g - pre(s)];
-    };
-    const int per = (T + (int)blockDim.x - 1) / (int)blockDim.x;
-    const int g_begin = min(T, tid * per), g_end = min(T, g_begin + per);
-    long long mine = 0;
-    int s = (g_begin < g_end) ? sys_of(g_begin) : 0;
-    for (int g = g_begin; g < g_end; ++g) mine += cost_of(g, s);
-    // block exclusive scan of the per-thread sums
-    long long incl = mine;
-    const int lane = tid & 63, wv = tid >> 6;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const long long t = __shfl_up(incl, o);
-        if (lane >= o) incl += t;
+    int carry = 0;
+    for (int base = 0; base < nsys; base += kPlThreads) {
+        const int s = base + tid;
+        // a system whose build overflowed has an incomplete list (a block that
+        // overflowed reserved chunk slots it did not write): no pair work
+        const int n = (s < nsys && !sc[s].overflow) ? min(sc[s].n_chunks, sd[s].chunk_cap) : 0;
+        int total;
+        const int pre = block_excl_scan(n, wsum, total);
+        if (s < nsys) prefix[s] = carry + pre;
+        carry += total;
     }
-    if (lane == 63) wsum[wv] = incl;
-    __syncthreads();
-    long long base = incl - mine, ctot = 0;
-    for (int w2 = 0; w2 < (int)(blockDim.x >> 6); ++w2) {
-        if (w2 < wv) base += wsum[w2];
-        ctot += wsum[w2];
-    }
-    if (T == 0) {
-        for (int w = tid; w <= NW; w += blockDim.x) wave_start[w] = 0;
-    } else if (g_begin < g_end) {
-        // doubled units: M_g = 2 * (cost before g) + cost of g; wave of g = M_g * NW / (2 * ctot)
-        auto wave_of = [&](long long M) { return (int)min((long long)NW - 1, M * NW / (2 * ctot)); };
-        int a_prev = -1;
-        if (g_begin > 0) {
-            int sp = sys_of(g_begin - 1);
-            const long long cp = cost_of(g_begin - 1, sp);
-            a_prev = wave_of(2 * (base - cp) + cp);
-        }
-        long long cum = base;
-        s = sys_of(g_begin);
-        int a = a_prev;
-        for (int g = g_begin; g < g_end; ++g) {
-            const long long c = cost_of(g, s);
-            a = wave_of(2 * cum + c);
-            for (int w = a_prev + 1; w <= a; ++w) wave_start[w] = g;
-            a_prev = a;
-            cum += c;
-        }
-        if (g_end == T)
-            for (int w = a + 1; w <= NW; ++w) wave_start[w] = T;
-    }
+    if (tid == 0) prefix[nsys] = carry;
+    if (pool) pool_begin(tid, carry, pool, pair_blocks);
 }
 
 // Clears the rebuild flags when no pair kernel follows (its first launch does
@@ -839,8 +769,8 @@ void launch_nlist(Batch<P>& B, bool clear_flags, int part) {
     auto nb = [](long n, int t) { return (unsigned)((n + t - 1) / t); };
     if (part == 2 || part == 3) {   // the last kernel alone, doing the pair kernel's set-up too
         // (part 3: in a step without the other list kernels)
-        nl_waves<<<1, 1024, 0, st>>>(B.d_sys, B.d_cnt, B.nsys, B.chunk_cost, B.chunk_prefix, B.wave_start, B.pair_waves,
-                                     B.pair_pool, part == 3 ? 1 : 0, B.step_seq, B.step_info, B.step_max);
+        nl_waves<<<1, kPlThreads, 0, st>>>(B.d_sys, B.d_cnt, B.nsys, B.chunk_prefix, B.pair_blocks, B.pair_pool,
+                                           part == 3 ? 1 : 0, B.step_seq, B.step_info, B.step_max);
         return;
     }
     nl_bin<<<nb(B.n_atoms, T), T, 0, st>>>(B.d_sys, B.d_cnt, B.atom_sys, B.X, B.Y, B.Z, B.atom_col, B.col_tmp,
@@ -854,10 +784,10 @@ void launch_nlist(Batch<P>& B, bool clear_flags, int part) {
                                             B.slot_zkey, B.slot_wpos, B.pos, B.lj, B.XB, B.YB, B.ZB);
     nl_pairlist<<<B.n_super_cap, kPlThreads, 0, st>>>(B.d_sys, B.d_cnt, B.super_sys, B.super_item, B.col_count, B.col_slot,
                                               B.cl_ctr, B.cl_half, B.slot_wpos, B.atom_of_slot, B.slot_of_atom, B.excl_off,
-                                              B.excl_idx, B.list, B.emask, B.chunks, B.chunk_cost, B.n_super_cap);
+                                              B.excl_idx, B.list, B.emask, B.chunks, B.n_super_cap);
     if (part == 1) return;  // all but the last kernel
-    nl_waves<<<1, 1024, 0, st>>>(B.d_sys, B.d_cnt, B.nsys, B.chunk_cost, B.chunk_prefix, B.wave_start, B.pair_waves,
-                                 nullptr, 0, nullptr, nullptr, nullptr);
+    nl_waves<<<1, kPlThreads, 0, st>>>(B.d_sys, B.d_cnt, B.nsys, B.chunk_prefix, B.pair_blocks, nullptr, 0, nullptr,
+                                       nullptr, nullptr);
     if (clear_flags) nl_clear_flag<<<nb(B.nsys, 64), 64, 0, st>>>(B.d_cnt, B.nsys);
 }
 

@@ -8,8 +8,8 @@
 // eps'_i = 2 sqrt(eps_i), so E_LJ = eps'_i eps'_j (s^6 - 1) s^6.
 //
 // Work decomposition: the list is cut into chunks of up to kChunkEntries
-// entries of one super-cluster (up to 8 clusters of 8 atoms); the wavefronts
-// of each XCD claim that XCD's chunks one at a time from a counter.  Lane
+// entries of one super-cluster (up to 8 clusters of 8 atoms); wavefronts claim
+// chunks one at a time, their XCD's first.  Lane
 // l = 8*ia + ja holds i-atom ia of the current i-cluster and j-atom ja of the
 // current j-cluster, so one (i-cluster, j-cluster) tile is 64 pairs in one
 // VALU pass.  i-forces stay in registers over the chunk; j-forces are reduced
@@ -141,8 +141,7 @@ constexpr unsigned long long kLowerTriangle = lower_triangle_mask();
 
 template <class P, bool ENERGY>
 __device__ __forceinline__ void pair_body(const SysDev* __restrict__ sd, const int* __restrict__ prefix,
-                                                   int nsys, const int* __restrict__ wave_start,
-                                                   const int4* __restrict__ chunks,
+                                                   int nsys, const int4* __restrict__ chunks,
                                                    const uint2* __restrict__ list,
                                                    const unsigned long long* __restrict__ emask,
                                                    const typename P::real4* __restrict__ pos,
@@ -166,28 +165,25 @@ __device__ __forceinline__ void pair_body(const SysDev* __restrict__ sd, const i
     real* jf = jf_s[w];
     uint2* jw = jw_s[w];
 
-    // The list build cuts the batch's chunks into one contiguous range of equal
-    // estimated work per wavefront.  The wavefronts of one XCD (blocks b with
-    // b % 8 equal, as the hardware hands them out) pool their ranges and claim
-    // chunks one at a time from an XCD counter until the pool is empty.  A fixed
+    // Each XCD's wavefronts (blocks b with b % 8 equal, as the hardware hands
+    // them out) share a contiguous range of the batch's chunks, in proportion to
+    // their number, and claim chunks one at a time from an XCD counter.  A fixed
     // range per wavefront finished 1.3x apart on one CU: the sequencer issues
     // for its oldest wavefront first, so the first block placed on a CU ran
     // ahead of the third.  Adjacent chunks are spatial neighbours, so an XCD's
-    // L2 sees one region.  Every chunk is done whole by one wavefront: its
-    // arithmetic does not depend on who does it or when.
-    const int nb = gridDim.x, xcd = blockIdx.x & 7;
-    const int per = (nb + 7) >> 3, full = (nb & 7) ? (nb & 7) : 8;     // blocks per XCD, as in xcd_remap
-    const int xb = (xcd < full) ? xcd * per : full * per + (xcd - full) * (per - 1);
-    const int xn = (xcd < full) ? per : per - 1;
-    const int lo = wave_start[xb * kPairWaves], hi = wave_start[(xb + xn) * kPairWaves];
-    int* counter = pool + xcd * kPoolStride;
+    // L2 sees one region.  A wavefront's first chunk is fixed (the counters start
+    // past those), which keeps the first claims' round trip out of the small
+    // systems' time.  Every chunk is done whole by one wavefront: its arithmetic
+    // does not depend on who does it or when.
+    int* counter = pool + (blockIdx.x & 7) * kPoolStride;
+    const int hi = __builtin_amdgcn_readfirstlane(counter[kPoolEnd]);
     // lane 0 claims the next chunk; the result is read (and waited for) later
     auto claim = [&]() {
         int t = 0;
         if (lane == 0) t = atomicAdd(counter, 1);
         return t;
     };
-    auto claimed = [&](int t) { return lo + __builtin_amdgcn_readfirstlane(t); };
+    auto claimed = [&](int t) { return __builtin_amdgcn_readfirstlane(t); };
     const real ke = (real)kOne4PiEps0;
 
     // Everything a chunk needs from memory before its first pair: the chunk
@@ -237,7 +233,7 @@ __device__ __forceinline__ void pair_body(const SysDev* __restrict__ sd, const i
 
     // The mixed path prefetches the next chunk across the flush below; the FP64
     // kernel is register-bound and fetches at the top of each chunk.
-    int g = claimed(claim());
+    int g = __builtin_amdgcn_readfirstlane(counter[kPoolFirst]) + (int)(blockIdx.x >> 3) * kPairWaves + w;
     Pre cur;
     if (P::mixed && g < hi) cur = fetch(g);
     while (g < hi) {
@@ -459,11 +455,10 @@ __device__ __forceinline__ void pair_body(const SysDev* __restrict__ sd, const i
 }
 
 #define NX_PAIR_PARAMS(P)                                                                                      \
-    const SysDev *__restrict__ sd, const int *__restrict__ prefix, int nsys, const int *__restrict__ wave_start,  \
-        const int4 *__restrict__ chunks, const uint2 *__restrict__ list, const unsigned long long *__restrict__ emask, \
+    const SysDev *__restrict__ sd, const int *__restrict__ prefix, int nsys, const int4 *__restrict__ chunks, const uint2 *__restrict__ list, const unsigned long long *__restrict__ emask, \
         const typename P::real4 *__restrict__ pos, const typename P::real2 *__restrict__ lj, typename P::facc *FX,    \
         typename P::facc *FY, typename P::facc *FZ, long long *energy, int *__restrict__ pool
-#define NX_PAIR_ARGS sd, prefix, nsys, wave_start, chunks, list, emask, pos, lj, FX, FY, FZ, energy, pool
+#define NX_PAIR_ARGS sd, prefix, nsys, chunks, list, emask, pos, lj, FX, FY, FZ, energy, pool
 
 // The pair kernels.  The mixed one without energies must stay within
 // PrecMixed::pair_max_vgpr VGPRs (the compiler offers no cap short of a higher
@@ -543,7 +538,7 @@ static int pair_blocks_per_cu() {
 // three per CU: the rest of a CU's wave slots go to the bonded and PME kernels
 // running beside it.  Measured on the 100k-atom step (mixed, five resident
 // blocks possible): 3 per CU 261 us, 4 per CU 303 us, 2 per CU 268 us.
-// Fixed per batch layout: the list build cuts the chunk ranges for it.
+// Fixed per batch layout: the claim counters are set for it.
 template <class P>
 int pair_grid_blocks(int n_cu, int n_chunk_cap, int per_cu_request) {
     // a requested count (the autotuner's) is capped by what a CU can hold at once
@@ -557,9 +552,9 @@ int pair_grid_blocks(int n_cu, int n_chunk_cap, int per_cu_request) {
 // separate launch it also gives the kernels forked to the side stream (bonded
 // terms, PME) a head start on the CUs before the pair kernel's persistent grid
 // takes its slots; without it the step measured about 10% slower.
-__global__ void pair_begin_kernel(SysCount* sc, int nsys, int* pool) {
+__global__ void pair_begin_kernel(SysCount* sc, int nsys, const int* prefix, int* pool, int pair_blocks) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < 8) pool[s * kPoolStride] = 0;     // no chunk of the pair kernel claimed yet
+    pool_begin(s, prefix[nsys], pool, pair_blocks);
     if (s >= nsys) return;
     if (sc[s].rebuild) {
         sc[s].rebuild = 0;
@@ -569,7 +564,8 @@ __global__ void pair_begin_kernel(SysCount* sc, int nsys, int* pool) {
 
 template <class P>
 void launch_pair_begin(Batch<P>& B) {
-    pair_begin_kernel<<<(B.nsys + 63) / 64, 64, 0, B.stream>>>(B.d_cnt, B.nsys, B.pair_pool);
+    pair_begin_kernel<<<(B.nsys + 63) / 64, 64, 0, B.stream>>>(B.d_cnt, B.nsys, B.chunk_prefix, B.pair_pool,
+                                                               B.pair_blocks);
 }
 
 template <class P>
@@ -577,11 +573,11 @@ void launch_pair_kernel(Batch<P>& B, bool energy) {
     if (B.n_chunk_cap == 0) return;
     const unsigned blocks = (unsigned)B.pair_blocks;
     if (energy)
-        pair_kernel_of<P, true>()<<<blocks, 256, 0, B.stream>>>(B.d_sys, B.chunk_prefix, B.nsys, B.wave_start, B.chunks, B.list,
+        pair_kernel_of<P, true>()<<<blocks, 256, 0, B.stream>>>(B.d_sys, B.chunk_prefix, B.nsys, B.chunks, B.list,
                                                            B.emask, B.pos, B.lj, B.FSx, B.FSy, B.FSz, B.energy,
                                                            B.pair_pool);
     else
-        pair_kernel_of<P, false>()<<<blocks, 256, 0, B.stream>>>(B.d_sys, B.chunk_prefix, B.nsys, B.wave_start, B.chunks, B.list,
+        pair_kernel_of<P, false>()<<<blocks, 256, 0, B.stream>>>(B.d_sys, B.chunk_prefix, B.nsys, B.chunks, B.list,
                                                             B.emask, B.pos, B.lj, B.FSx, B.FSy, B.FSz, B.energy,
                                                             B.pair_pool);
 }

@@ -47,6 +47,7 @@ struct SysDev {
     int col_off, ncx, ncy, col_cap;   // columns: ncx*ncy
     int super_off, super_cap;
     int chunk_off, chunk_cap;    // pair-kernel work items (list chunks)
+    int chunk_entries;           // pair-list entries per chunk (chunk_entries_for)
     int list_off, list_cap;
     int emask_off, emask_cap;
     double colw[2];              // column widths
@@ -85,22 +86,17 @@ struct __align__(16) StepInfo {
 // slots of the update's largest squared displacement (block b adds to slot b % 64)
 constexpr int kStepMaxSlots = 64;
 
-constexpr int kChunkEntries = 32;       // pair-list entries per chunk, the pair kernel's unit of work
+constexpr int kChunkEntries = 32;       // most pair-list entries per chunk, the pair kernel's unit of work
 // Pair-list entries one super-cluster may hold (the list build keeps them in
 // LDS).  A super-cluster is 64 atoms of one column, about 3.5 nm tall at water
 // density, with ~700-950 j clusters within rlist = 1.1 nm: 1024 was exceeded
 // by a few super-clusters of a 1M-atom water box.
 constexpr int kSuperListCap = 2048;
 constexpr int kPairWaves = 4;           // independent wavefronts per 256-thread pair-kernel block
-// Estimated pair-kernel work in quarter tiles: per tile, per list entry (the
-// j loads, the j-force reduction and its LDS staging) and per chunk (i staging
-// and the force flush).  Fitted to per-wavefront times of the 100k-atom step:
-// 0.16 us per tile and 0.46 us per entry.  The list build writes the sum per
-// chunk and cuts the chunks into contiguous ranges of equal sums, one per
-// wavefront; the pair kernel pools the ranges of each XCD.
-constexpr int kCostTile = 4, kCostEntry = 11, kCostChunk = 24;
-// The pair kernel's chunk counters, one per XCD, 128 bytes apart.
+// The pair kernel's chunk ranges, one per XCD, 128 bytes apart: the next chunk
+// to hand out, and the range's first and end chunk.
 constexpr int kPoolStride = 32, kPoolInts = 8 * kPoolStride;
+constexpr int kPoolFirst = 1, kPoolEnd = 2;
 
 // Second word of a pair-list entry: the exclusion-mask id in the low 26 bits
 // (kNoMask: the tile has no listed exclusion) and the j-cluster's periodic
@@ -348,6 +344,21 @@ __device__ __forceinline__ double sum_group8(double v) {
     v += __hiloint2double(dpp_xor2(__double2hiint(v)), dpp_xor2(__double2loint(v)));
     v += __hiloint2double(dpp_hmirror(__double2hiint(v)), dpp_hmirror(__double2loint(v)));
     return v;
+}
+
+// Before a pair kernel of nb blocks, threads x < 8: XCD x's range of the n
+// chunks, in proportion to its blocks (b % 8 == x), and its counter past the
+// first chunk of each of its wavefronts.
+__device__ __forceinline__ void pool_begin(int x, int n, int* pool, int nb) {
+    if (x >= 8) return;
+    auto first = [&](int y) {
+        const int b = y * (nb >> 3) + min(y, nb & 7);      // blocks of the XCDs below y
+        return (n / nb) * b + (n % nb) * b / nb;
+    };
+    int* p = pool + x * kPoolStride;
+    p[kPoolFirst] = first(x);
+    p[kPoolEnd] = first(x + 1);
+    p[0] = first(x) + ((nb >> 3) + (x < (nb & 7) ? 1 : 0)) * kPairWaves;
 }
 
 // XCD-aware block order: consecutive work items land on one XCD (8 XCDs,

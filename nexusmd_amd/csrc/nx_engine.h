@@ -82,19 +82,16 @@ struct Batch {
     float4* slot_wpos = nullptr;    // build-time wrapped position of each slot, w = 1 (atom) or 0 (padding)
     int* super_sys = nullptr;
     int4* super_item = nullptr;
-    int* chunk_sys = nullptr;
     int4* chunks = nullptr;         // (first cluster, n clusters, first entry, end entry)
     int* chunk_prefix = nullptr;    // [nsys + 1] running total of chunks over systems
-    int* chunk_cost = nullptr;      // per chunk: estimated pair-kernel work (list build)
-    int* wave_start = nullptr;      // [pair_waves + 1] chunk ranges of equal estimated work (per XCD: its waves' union)
-    int* pair_pool = nullptr;       // [kPoolInts] per XCD: chunks claimed so far by the running pair kernel
+    int* pair_pool = nullptr;       // [kPoolInts] per XCD: chunks handed out so far by the running pair kernel
     // one-system batches: nl_waves' report to the host (host memory, mapped),
     // the report count (device) and the update's largest squared displacement
     // (device, kStepMaxSlots float bit patterns)
     StepInfo* step_info = nullptr;
     unsigned* step_seq = nullptr;
     unsigned* step_max = nullptr;
-    int pair_blocks = 0, pair_waves = 0;
+    int pair_blocks = 0;
     int n_cu = 0;                   // compute units of the device
     int n_chunk_cap = 0;
     uint2* list = nullptr;

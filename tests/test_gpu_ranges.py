@@ -1,0 +1,49 @@
+"""Kernels at the edges of the ranges their launch rules choose between.
+
+Forces of both paths against the FP64 oracle, relative RMS: FP64 <= 1e-9, mixed
+<= 5e-4 (the bounds of the other parity tests).
+"""
+import numpy as np
+import pytest
+
+from nexusmd_amd import _lib as L
+from nexusmd_amd import engine as E
+from nexusmd_amd import systems as S
+from oracle import pyoracle as O
+
+from _util import bare_system, rel_rms
+
+pytestmark = pytest.mark.gpu
+
+TOL = {L.FP64: 1e-9, L.MIXED: 5e-4}
+
+
+def _gas(n, box, seed, grid=(0, 0, 0), cutoff=0.9):
+    """n charged LJ particles on a jittered lattice in an oblong box."""
+    rng = np.random.default_rng(seed)
+    box = np.asarray(box, float)
+    k = np.ceil(box * (n / box.prod()) ** (1 / 3)).astype(int)
+    while k.prod() < n:
+        k[np.argmin(k / box)] += 1
+    g = np.stack(np.meshgrid(*[np.arange(m) + 0.5 for m in k], indexing="ij"), -1).reshape(-1, 3) * (box / k)
+    g = g[rng.permutation(len(g))[:n]] + rng.normal(0.0, 0.01, (n, 3))
+    q = rng.normal(0.0, 0.5, n)
+    return bare_system(g % box, np.zeros(3), box, q=q - q.mean(), sig=rng.uniform(0.15, 0.2, n),
+                       eps=rng.uniform(0.1, 0.6, n), cutoff=cutoff, grid=grid)
+
+
+def _check(sys, prec, what, **kw):
+    print("[gpu] %s n=%d precision=%d" % (what, sys.n, prec), flush=True)
+    ctx = E.Context(sys, precision=prec, **kw)
+    f, _ = ctx.compute_forces()
+    ctx.close()
+    ref, _ = O.compute_forces(O.Prepared(sys))
+    assert rel_rms(f, ref) <= TOL[prec]
+
+
+@pytest.mark.parametrize("prec", [L.FP64, L.MIXED])
+@pytest.mark.parametrize("n", [5, 5999, 6000])
+def test_chunk_sizes(n, prec):
+    """Either side of the size where the FP64 pair kernel takes shorter chunks,
+    and a system with far fewer chunks than wavefronts."""
+    _check(_gas(n, (2.1, 4.3, 5.9), n, grid=(20, 40, 60)), prec, "chunk sizes")
