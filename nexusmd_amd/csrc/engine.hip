@@ -299,6 +299,7 @@ class Engine : public EngineBase {
             d.rlist = rc + skin;
             d.skin_half2 = skin > 0 ? 0.25 * skin * skin : -1.0;
             d.alpha = (1.0 / rc) * sqrt(-log(2.0 * h.nb.ewald_tolerance));
+            if (!(d.alpha * d.alpha * d.rc2 <= kErfSeriesMax)) B.all_series = false;
             if (h.nb.use_switch && h.nb.switch_distance < rc) {
                 d.sw_on = h.nb.switch_distance;
                 d.sw_inv = 1.0 / (rc - h.nb.switch_distance);

@@ -91,6 +91,42 @@ __device__ __forceinline__ float pair_mixed(float r2, float qq, float sig, float
     return fmaf(qq, cy, dl) * inv_r2;
 }
 
+// FP64 path inside the range of the series: 1/r^3 - alpha^3 B(alpha^2 r^2) in
+// place of (erfc + 2 alpha r exp / sqrt(pi)) / r^3, and 1/r from the hardware's
+// reciprocal square root with one third-order step (its first error, 2^-26 or
+// less, goes to the third power).  The kernel is bound by its vector
+// instructions (82% of its time issuing them, 111 a tile): with library erfc,
+// exp, sqrt and division the 100,000-atom system's launch took 512 us, with the
+// series 328.  The forces' error against 64 bits stays what it was (6e-14 of
+// their norm, from the fixed-point sums).
+template <bool ENERGY>
+__device__ __forceinline__ double pair_fp64_series(double r2, double qq, double sig, double epsij, double alpha,
+                                                   double sw_on, double sw_inv, double& ecoul, double& elj) {
+#pragma clang fp contract(off)      // the same operations in both kernels below
+    double y = __builtin_amdgcn_rsq(r2);
+    const double err = fma(-(r2 * y), y, 1.0);
+    y = fma(y * err, fma(0.375, err, 0.5), y);
+    const double y2 = y * y, s = alpha * alpha * r2;
+    const double cf = qq * fma(-(alpha * alpha * alpha), erf_series(kErfB, s), y2 * y);
+    double s2 = sig * y;
+    s2 *= s2;
+    const double s6 = s2 * s2 * s2;
+    const double es = epsij * s6;
+    double lf = es * fma(12.0, s6, -6.0) * y2;
+    double le = es * (s6 - 1.0);
+    if (sw_on >= 0.0) {
+        const double r = r2 * y;
+        const double t = r > sw_on ? (r - sw_on) * sw_inv : 0.0;
+        const double sv = fma(t * t * t, fma(t, fma(-6.0, t, 15.0), -10.0), 1.0);
+        const double sd = t * t * fma(t, fma(-30.0, t, 60.0), -30.0) * sw_inv;
+        lf = fma(sv, lf, -(le * sd * y));
+        le *= sv;
+    }
+    if constexpr (ENERGY) ecoul = qq * fma(-alpha, erf_series(kErfA, s), y);
+    elj = le;
+    return cf + lf;
+}
+
 // FP64 path: the reference's formulas with library erfc/exp.
 __device__ __forceinline__ double pair_fp64(double r2, double qq, double sig, double epsij, double alpha,
                                             double sw_on, double sw_inv, double& ecoul, double& elj) {
@@ -139,7 +175,7 @@ constexpr unsigned long long lower_triangle_mask() {
 }
 constexpr unsigned long long kLowerTriangle = lower_triangle_mask();
 
-template <class P, bool ENERGY>
+template <class P, bool ENERGY, bool ALL_SERIES>
 __device__ __forceinline__ void pair_body(const SysDev* __restrict__ sd, const int* __restrict__ prefix,
                                                    int nsys, const int4* __restrict__ chunks,
                                                    const uint2* __restrict__ list,
@@ -251,6 +287,7 @@ __device__ __forceinline__ void pair_body(const SysDev* __restrict__ sd, const i
         const real rc2 = (real)sd[s].rc2;
         const real alpha = (real)sd[s].alpha;
         const real sw_on = (real)sd[s].sw_on, sw_inv = (real)sd[s].sw_inv;
+        const bool series = (double)alpha * (double)alpha * (double)rc2 <= kErfSeriesMax;   // FP64 path only
         const MixedPair mpc = mixed_pair_const(sd[s]);   // mixed path only
         {
             real4 p = cur.p;
@@ -375,9 +412,11 @@ __device__ __forceinline__ void pair_body(const SysDev* __restrict__ sd, const i
                     } else {
                         dEdR = 0;
                         ecv = elv = 0;
-                        if (on)
-                            dEdR = pair_fp64(r2, pi.w * pjs.w, li.x + lj_j.x, li.y * lj_j.y, alpha, sw_on,
-                                             sw_inv, ecv, elv);
+                        if (on) {
+                            const real qq = pi.w * pjs.w, sg = li.x + lj_j.x, ep = li.y * lj_j.y;
+                            if (ALL_SERIES || series) dEdR = pair_fp64_series<ENERGY>(r2, qq, sg, ep, alpha, sw_on, sw_inv, ecv, elv);
+                            else dEdR = pair_fp64(r2, qq, sg, ep, alpha, sw_on, sw_inv, ecv, elv);
+                        }
                     }
                     // every displacement is finite (padding slots included), so the
                     // zero of an off lane gives zero force
@@ -467,20 +506,23 @@ __device__ __forceinline__ void pair_body(const SysDev* __restrict__ sd, const i
 template <bool ENERGY>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PrecMixed::pair_waves_per_simd))) void
 pair_kernel_mixed(NX_PAIR_PARAMS(PrecMixed)) {
-    pair_body<PrecMixed, ENERGY>(NX_PAIR_ARGS);
+    pair_body<PrecMixed, ENERGY, true>(NX_PAIR_ARGS);
 }
-template <bool ENERGY>
+// The FP64 kernel with the series alone, for batches whose every system is in
+// its range, needs 147 VGPRs; with the library functions beside it (chosen per
+// system) 219.
+template <bool ENERGY, bool ALL_SERIES>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PrecFP64::pair_waves_per_simd))) void
 pair_kernel_fp64(NX_PAIR_PARAMS(PrecFP64)) {
-    pair_body<PrecFP64, ENERGY>(NX_PAIR_ARGS);
+    pair_body<PrecFP64, ENERGY, ALL_SERIES>(NX_PAIR_ARGS);
 }
 #undef NX_PAIR_ARGS
 #undef NX_PAIR_PARAMS
 
 template <class P, bool ENERGY>
-constexpr auto pair_kernel_of() {
+static auto pair_kernel_of(bool all_series) {
     if constexpr (P::mixed) return pair_kernel_mixed<ENERGY>;
-    else return pair_kernel_fp64<ENERGY>;
+    else return all_series ? pair_kernel_fp64<ENERGY, true> : pair_kernel_fp64<ENERGY, false>;
 }
 
 // Explicit pair set (atom ids, first > second) with the FP64 test of the pair kernel.
@@ -527,7 +569,7 @@ template <class P>
 static int pair_blocks_per_cu() {
     static const int v = [] {
         int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, pair_kernel_of<P, false>(), 256, 0) != hipSuccess || n <= 0)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, pair_kernel_of<P, false>(true), 256, 0) != hipSuccess || n <= 0)
             n = 2;
         return n;
     }();
@@ -535,15 +577,17 @@ static int pair_blocks_per_cu() {
 }
 
 // Persistent grid of the pair kernel, all blocks resident at once, at most
-// three per CU: the rest of a CU's wave slots go to the bonded and PME kernels
-// running beside it.  Measured on the 100k-atom step (mixed, five resident
-// blocks possible): 3 per CU 261 us, 4 per CU 303 us, 2 per CU 268 us.
+// three per CU (FP64: two): the rest of a CU's wave slots go to the bonded and
+// PME kernels running beside it.  Measured on the 100k-atom step (mixed, five
+// resident blocks possible): 3 per CU 261 us, 4 per CU 303 us, 2 per CU 268 us.
+// FP64 (three possible): 2 per CU 459 us, 3 per CU 461, 1 per CU 636; the
+// 24,000-atom water box 164, 177, 198.
 // Fixed per batch layout: the claim counters are set for it.
 template <class P>
 int pair_grid_blocks(int n_cu, int n_chunk_cap, int per_cu_request) {
     // a requested count (the autotuner's) is capped by what a CU can hold at once
     const int occ = pair_blocks_per_cu<P>();
-    const int per_cu = per_cu_request > 0 ? std::min(per_cu_request, occ) : std::min(occ, 3);
+    const int per_cu = per_cu_request > 0 ? std::min(per_cu_request, occ) : std::min(occ, P::mixed ? 3 : 2);
     return std::max(1, std::min((n_chunk_cap + kPairWaves - 1) / kPairWaves, per_cu * std::max(1, n_cu)));
 }
 
@@ -573,11 +617,11 @@ void launch_pair_kernel(Batch<P>& B, bool energy) {
     if (B.n_chunk_cap == 0) return;
     const unsigned blocks = (unsigned)B.pair_blocks;
     if (energy)
-        pair_kernel_of<P, true>()<<<blocks, 256, 0, B.stream>>>(B.d_sys, B.chunk_prefix, B.nsys, B.chunks, B.list,
+        pair_kernel_of<P, true>(B.all_series)<<<blocks, 256, 0, B.stream>>>(B.d_sys, B.chunk_prefix, B.nsys, B.chunks, B.list,
                                                            B.emask, B.pos, B.lj, B.FSx, B.FSy, B.FSz, B.energy,
                                                            B.pair_pool);
     else
-        pair_kernel_of<P, false>()<<<blocks, 256, 0, B.stream>>>(B.d_sys, B.chunk_prefix, B.nsys, B.chunks, B.list,
+        pair_kernel_of<P, false>(B.all_series)<<<blocks, 256, 0, B.stream>>>(B.d_sys, B.chunk_prefix, B.nsys, B.chunks, B.list,
                                                             B.emask, B.pos, B.lj, B.FSx, B.FSy, B.FSz, B.energy,
                                                             B.pair_pool);
 }

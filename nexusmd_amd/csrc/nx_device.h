@@ -276,9 +276,9 @@ __device__ __forceinline__ void wave_energy_add(long long* energy, int s, int te
 // Reference minimum image: one +-L correction (PeriodicBoundaryCondition.cpp:93-104),
 // written with selects so that it compiles without branches.
 __device__ __forceinline__ double min_image1(double d, double L) {
-    const double h = 0.5 * L;
-    const double up = d - L, dn = d + L;
-    return d > h ? up : (d < -h ? dn : d);
+    // d - L, d + L or d, as one subtraction of +-L or 0
+    const double n = fabs(d) > 0.5 * L ? copysign(L, d) : 0.0;
+    return d - n;
 }
 __device__ __forceinline__ float min_image1(float d, float L) {
     const float h = 0.5f * L;
@@ -297,6 +297,50 @@ __device__ __forceinline__ void continuous_position(const SysDev& d, double x, d
     p[0] = xb + min_image1(x - xb, d.L[0]);
     p[1] = yb + min_image1(y - yb, d.L[1]);
     p[2] = zb + min_image1(z - zb, d.L[2]);
+}
+
+// erf(x) / x and (erf(x) - 2 x exp(-x^2) / sqrt(pi)) / x^3 as functions of
+// s = x^2.  Both are entire, so a polynomial over a bounded range converges like
+// a Taylor series: Chebyshev interpolants over s in [0, 8] (computed with 60
+// digits), written in powers of u = s / 4 - 1.  Truncation < 2e-17 of 1/x and
+// 1/x^3, evaluation error < 1e-16.  With them the Ewald direct-space term is
+// 1/r - alpha A and 1/r^3 - alpha^3 B, and its exclusion correction alpha A and
+// alpha^3 B, without an exponential, an error function or a division.
+constexpr double kErfSeriesMax = 8.0;
+constexpr double kErfA[22] = {
+    4.97661132509476356e-01, -2.38497073577692176e-01, 1.58205819829175892e-01, -1.04282202718857353e-01,
+    6.36909469069244089e-02, -3.52770678385127892e-02, 1.76407892660984562e-02, -7.98271979410423126e-03,
+    3.28479326482311422e-03, -1.23607961382126200e-03, 4.27785551802345595e-04, -1.36889844490136983e-04,
+    4.07025421452981889e-05, -1.12958817428514669e-05, 2.93769052661021184e-06, -7.18648852211750148e-07,
+    1.66084339812328716e-07, -3.62878189045594433e-08, 7.39320016599416468e-09, -1.46104235443290689e-09,
+    3.30946272093021783e-10, -5.91195428737397584e-11,
+};
+constexpr double kErfB[23] = {
+    1.19248536788846074e-01, -1.58205819829177086e-01, 1.56423304078287251e-01, -1.27381893813754754e-01,
+    8.81926695962295254e-02, -5.29223678004963477e-02, 2.79395192802459787e-02, -1.31391730358153547e-02,
+    5.56235825464281540e-03, -2.13892789596149347e-03, 7.52894182292228559e-04, -2.44214774792607923e-04,
+    7.34231151212477582e-05, -2.05648756537177909e-05, 5.39009625215538716e-06, -1.32724573457226400e-06,
+    3.08155303970224502e-07, -6.77366262557539614e-08, 1.41082605777249840e-08, -2.74907686745350267e-09,
+    5.19796833377220498e-10, -1.12077170695342987e-10, 1.92301651041994177e-11,
+};
+// a b + c with the constant c in scalar registers.  Written out because the
+// compiler otherwise picks the two-address form, whose addend is its result: a
+// copy of the constant, kept in vector registers, before every step.
+__device__ __forceinline__ double fma_const(double a, double b, double c) {
+    double r;
+    asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "s"(c));
+    return r;
+}
+template <int N>
+__device__ __forceinline__ double erf_series(const double (&c)[N], double s) {
+    // even and odd powers as two chains: half the depth
+    const double u = fma(s, 0.25, -1.0), u2 = u * u;
+    double e = c[(N - 1) & ~1], o = c[(N - 2) | 1];
+#pragma unroll
+    for (int k = ((N - 1) & ~1) - 2; k >= 0; k -= 2) e = fma_const(e, u2, c[k]);
+#pragma unroll
+    for (int k = ((N - 2) | 1) - 2; k >= 1; k -= 2) o = fma_const(o, u2, c[k]);
+    return fma(o, u, e);
 }
 
 // r^2 without contraction, left-to-right as Coords3D::dot (Coords3D.h:116-124).

@@ -92,6 +92,7 @@ struct Batch {
     unsigned* step_seq = nullptr;
     unsigned* step_max = nullptr;
     int pair_blocks = 0;
+    bool all_series = true;         // every system's alpha^2 rc^2 is within kErfSeriesMax
     int n_cu = 0;                   // compute units of the device
     int n_chunk_cap = 0;
     uint2* list = nullptr;

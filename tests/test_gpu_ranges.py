@@ -47,3 +47,14 @@ def test_chunk_sizes(n, prec):
     """Either side of the size where the FP64 pair kernel takes shorter chunks,
     and a system with far fewer chunks than wavefronts."""
     _check(_gas(n, (2.1, 4.3, 5.9), n, grid=(20, 40, 60)), prec, "chunk sizes")
+
+
+@pytest.mark.parametrize("tol", [1.7e-4, 1.6e-4, 1e-7])
+def test_fp64_direct_space_either_side_of_the_series(tol):
+    """alpha^2 rc^2 just inside and outside the range of the FP64 pair kernel's
+    series (8), and far outside."""
+    s = _gas(900, (2.2, 2.0, 2.4), 3, grid=(24, 24, 24))
+    s.ewald_tol = tol
+    s.pos[1] = (s.pos[0] + [0.03, 0.02, 0.01]) % s.L       # a close contact
+    assert (-np.log(2 * tol) <= 8.0) == (tol == 1.7e-4)
+    _check(s, L.FP64, "series range")
