@@ -358,38 +358,7 @@ class Engine : public EngineBase {
                 tw_off += g[k];
                 fft_maxK_ = std::max(fft_maxK_, g[k]);
             }
-            // spread tiling: column blocks b x b and nz slabs whose LDS region fits kSpreadLdsPoints
-            {
-                d.sp_margin = 0.5 * skin + 0.002;
-                long long best = -1;
-                int bb = 0, bnz = 0;
-                const int bmax = std::min(12, std::max(ncx, ncy));
-                // a tuned block size is taken when it fits; otherwise the cost model chooses
-                const int want = tuning_.spread_block > 0 ? std::min(tuning_.spread_block, bmax) : 0;
-                for (int pass = want > 0 ? 0 : 1; pass < 2 && best < 0; ++pass)
-                for (int b = pass == 0 ? want : 1; b <= (pass == 0 ? want : bmax); ++b) {
-                    for (int nz = 1; nz <= g[2]; ++nz) {
-                        auto ext = [&](double w, int K, double Lk, bool full) {
-                            if (full) return K;
-                            const double hh = Lk / K;
-                            int n = (int)ceil((w + 2 * d.sp_margin) / hh) + 6;
-                            return n >= K ? K : n;
-                        };
-                        const int nx = ext(b * d.colw[0], g[0], d.L[0], b >= ncx);
-                        const int ny = ext(b * d.colw[1], g[1], d.L[1], b >= ncy);
-                        const int nzp = ext(d.L[2] / nz, g[2], d.L[2], nz == 1);
-                        const long long pts = (long long)nx * spread_plane(ny, nzp);
-                        if (pts > kSpreadLdsPoints) continue;
-                        const long long tiles = (long long)((ncx + b - 1) / b) * ((ncy + b - 1) / b) * nz;
-                        const long long cost = pts * tiles + 2000 * (tiles < 128 ? 128 - tiles : 0);
-                        if (best < 0 || cost < best) { best = cost; bb = b; bnz = nz; }
-                        break;   // the smallest fitting nz for this b
-                    }
-                }
-                d.sp_block[0] = bb;
-                d.sp_block[1] = bb;
-                d.sp_block[2] = bnz;
-            }
+            d.sp_margin = 0.5 * skin + 0.002;
             rg_off += (long long)g[0] * g[1] * g[2];
             cg_off += (long long)g[0] * g[1] * (g[2] / 2 + 1);
             d.bond_off = bond_off;
@@ -459,7 +428,6 @@ class Engine : public EngineBase {
         dalloc(&B.cl_half, S / 8 + 1, o, B.stream);
         dalloc(&B.super_sys, B.n_super_cap, o, B.stream);
         dalloc(&B.super_item, B.n_super_cap, o, B.stream);
-        dalloc(&B.slot_zkey, S, o, B.stream);
         dalloc(&B.slot_wpos, S, o, B.stream);
         dalloc(&B.chunks, B.n_chunk_cap, o, B.stream);
         dalloc(&B.chunk_prefix, B.nsys + 1, o, B.stream);
@@ -481,7 +449,6 @@ class Engine : public EngineBase {
         force_full_ = true;
         dalloc(&B.list, (size_t)B.n_list_cap, o, B.stream);
         dalloc(&B.emask, (size_t)B.n_emask_cap * 8, o, B.stream);
-        dalloc(&B.rgrid, (size_t)B.rgrid_total, o, B.stream);
         dalloc(&B.cgrid, (size_t)B.cgrid_total, o, B.stream);
         dalloc(&B.phi, (size_t)B.rgrid_total, o, B.stream);
         dalloc(&B.eta, (size_t)B.cgrid_total, o, B.stream);
@@ -505,8 +472,7 @@ class Engine : public EngineBase {
         std::vector<double4> tpar;
         std::vector<real> eta;
         std::vector<real2> tw;
-        std::vector<int4> zi, yi, xi, sp_tiles;
-        int direct_slots = 0;
+        std::vector<int4> zi, pi, li, yi, xi;
         const int maxK = fft_maxK_;
         // LDS per FFT block: two buffers of T lines plus the twiddles, within 60 KiB
         const int Tfit = std::max(1, std::min(8, (int)((61440 / (int)sizeof(real2) - maxK) / (2 * maxK))));
@@ -516,18 +482,32 @@ class Engine : public EngineBase {
         B.fft_maxK = maxK;
         // plane passes when every system's planes fit one workgroup's LDS; the x
         // pass splits the kz range so that the batch has about 512 x blocks
-        bool plane = fft_plane_enabled();
+        bool plane = fft_plane_enabled(), plane_spread = true;
         int sum_ky = 0;
+        long long rows = 0;
         for (int s = 0; s < ns; ++s) {
             const SysDev& d = B.sys[s];
             if (plane_lds_bytes<real2>(d.grid[1], d.grid[2]) > kMaxBlockLds ||
                 xpass_lds_bytes<real2>(d.grid[0], 1) > kMaxBlockLds)
                 plane = false;
+            if (plane_spread_lds_bytes<real2>(d.grid[1], d.grid[2]) > kPlaneSpreadLds) plane_spread = false;
             sum_ky += d.grid[1];
+            rows += (long long)d.grid[0] * d.grid[1];
         }
         const int xtarget = tuning_.fft_xblocks > 0 ? tuning_.fft_xblocks : 512;
         const int xsplit = std::max(1, (xtarget + sum_ky - 1) / std::max(1, sum_ky));
         B.fft_plane = plane ? 1 : 0;
+        // The spread goes into the plane pass where the plane's workgroup finds room
+        // beside the pair kernel's on a CU: one launch and one trip of the spectrum
+        // less (us a step, together against apart: 100,000 atoms at 96^3 mixed 214,
+        // 220; the 1,500-bead chain 71, 72).  A larger one would wait for the pair
+        // kernel to end, and the spread then goes over rows (100,000 atoms FP64, 155
+        // KB a plane: 463 together, 412 apart).
+        B.fft_split = !plane || !plane_spread;
+        // rows per workgroup of the spread: three workgroups per CU, at least 8 rows
+        // (each sees the atoms of four more)
+        const int want_rows = (int)std::max<long long>(8, rows / (3 * B.n_cu));
+        B.fft_spread_lds = 0;
         B.fft_plane_lds = 0;
         B.fft_x_lds = 0;
         for (int s = 0; s < ns; ++s) {
@@ -600,16 +580,23 @@ class Engine : public EngineBase {
                     v.y = (real)sin(ang);
                     tw.push_back(v);
                 }
-            if (d.sp_block[0] > 0) {
-                const int b = d.sp_block[0], nz = d.sp_block[2];
-                for (int bx = 0; bx < (d.ncx + b - 1) / b; ++bx)
-                    for (int by = 0; by < (d.ncy + b - 1) / b; ++by)
-                        for (int bz = 0; bz < nz; ++bz) sp_tiles.push_back(make_int4(s, bx, by, bz));
+            // the spread: whole planes, or rows of them, an even count as equal as they come
+            if (B.fft_split) {
+                const int most = std::max(2, std::min(kSpreadZPoints / Kz * 2, want_rows)), blocks = (Ky + most - 1) / most;
+                const int ny = std::min(Ky, ((Ky + blocks - 1) / blocks + 1) & ~1);
+                for (int x = 0; x < Kx; ++x)
+                    for (int y = 0; y < Ky; y += ny) zi.push_back(make_int4(s, x, y, std::min(ny, Ky - y)));
+                B.fft_spread_lds =
+                    std::max(B.fft_spread_lds, (size_t)(Kz + spread_points<real2>((ny + 1) / 2 * Kz, ny, Kz)) * sizeof(real2) +
+                                                   spread_lds_bytes(kSpreadZThreads));
+                for (int x = 0; x < Kx; ++x)
+                    for (int k = 0; k < Kzh; k += T) yi.push_back(make_int4(s, x, k, 0));
             } else {
-                direct_slots += d.slot_cap;
+                for (int x = 0; x < Kx; ++x) zi.push_back(make_int4(s, x, 0, 0));
+                B.fft_spread_lds = std::max(B.fft_spread_lds, plane_spread_lds_bytes<real2>(Ky, Kz));
             }
             if (B.fft_plane) {
-                for (int x = 0; x < Kx; ++x) zi.push_back(make_int4(s, x, 0, 0));
+                for (int x = 0; x < Kx; ++x) pi.push_back(make_int4(s, x, 0, 0));
                 int nk = (Kzh + xsplit - 1) / xsplit;
                 while (nk > 1 && xpass_lds_bytes<real2>(Kx, nk) > kMaxBlockLds) nk = (nk + 1) / 2;
                 for (int y = 0; y < Ky; ++y)
@@ -617,9 +604,7 @@ class Engine : public EngineBase {
                 B.fft_plane_lds = std::max(B.fft_plane_lds, plane_lds_bytes<real2>(Ky, Kz));
                 B.fft_x_lds = std::max(B.fft_x_lds, xpass_lds_bytes<real2>(Kx, nk));
             } else {
-                for (int l = 0; l < Kx * Ky; l += T) zi.push_back(make_int4(s, l, std::min(T, Kx * Ky - l), 0));
-                for (int x = 0; x < Kx; ++x)
-                    for (int k = 0; k < Kzh; k += T) yi.push_back(make_int4(s, x, k, 0));
+                for (int l = 0; l < Kx * Ky; l += T) li.push_back(make_int4(s, l, std::min(T, Kx * Ky - l), 0));
                 for (int y = 0; y < Ky; ++y)
                     for (int k = 0; k < Kzh; k += T) xi.push_back(make_int4(s, y, k, 0));
             }
@@ -659,14 +644,14 @@ class Engine : public EngineBase {
         dalloc(&B.excl_off, eoff.size(), owned_, B.stream);
         dalloc(&B.excl_idx, std::max<size_t>(1, eidx.size()), owned_, B.stream);
         if (B.n_excl_pairs) dalloc(&B.excl_pairs, epairs.size(), owned_, B.stream);
-        B.n_spread_tiles = (int)sp_tiles.size();
-        B.n_spread_direct_slots = direct_slots;
-        dalloc(&B.spread_tiles, std::max<size_t>(1, sp_tiles.size()), owned_, B.stream);
-        upload(B.spread_tiles, sp_tiles, st);
         dalloc(&B.fftz_items, zi.size(), owned_, B.stream);
+        dalloc(&B.fftp_items, pi.size(), owned_, B.stream);
+        dalloc(&B.fftl_items, li.size(), owned_, B.stream);
         dalloc(&B.ffty_items, yi.size(), owned_, B.stream);
         dalloc(&B.fftx_items, xi.size(), owned_, B.stream);
         B.n_fftz = (int)zi.size();
+        B.n_fftp = (int)pi.size();
+        B.n_fftl = (int)li.size();
         B.n_ffty = (int)yi.size();
         B.n_fftx = (int)xi.size();
         HIPCHK(prepare_fft<P>(B));
@@ -692,6 +677,8 @@ class Engine : public EngineBase {
         upload(B.eta, eta, st);
         upload(B.twiddle, tw, st);
         upload(B.fftz_items, zi, st);
+        upload(B.fftp_items, pi, st);
+        upload(B.fftl_items, li, st);
         upload(B.ffty_items, yi, st);
         upload(B.fftx_items, xi, st);
         HIPCHK(hipMemsetAsync(B.d_cnt, 0, sizeof(SysCount) * B.nsys, st));
@@ -1560,12 +1547,6 @@ class Engine : public EngineBase {
             for (int c = 1; c <= occ; ++c) { Tuning t = base; t.pair_per_cu = c; consider(t); }
         }
         {
-            int bmax = 1;
-            for (const SysDev& d : B.sys) bmax = std::max(bmax, std::min(12, std::max(d.ncx, d.ncy)));
-            const Tuning base = best;
-            for (int b = 1; b <= bmax; ++b) { Tuning t = base; t.spread_block = b; consider(t); }
-        }
-        {
             const Tuning base = best;
             if (B.fft_plane) {
                 for (int x : {128, 256, 1024, 2048}) { Tuning t = base; t.fft_xblocks = x; consider(t); }
@@ -1622,7 +1603,7 @@ class Engine : public EngineBase {
     static size_t footprint_bytes(const Batch<P>& b) {
         size_t A = b.n_atoms, S = b.n_slots_cap;
         return A * (14 * 8 + 3 * 4 + 3 * sizeof(facc)) + S * (3 * 4 + sizeof(real4) + sizeof(real2) + 3 * sizeof(facc)) +
-               (size_t)b.n_list_cap * 8 + (size_t)b.n_emask_cap * 64 + (size_t)b.rgrid_total * (sizeof(typename P::gacc) + sizeof(real)) +
+               (size_t)b.n_list_cap * 8 + (size_t)b.n_emask_cap * 64 + (size_t)b.rgrid_total * sizeof(real) +
                (size_t)b.cgrid_total * (sizeof(real2) + sizeof(real));
     }
 

@@ -177,7 +177,7 @@ __global__ __launch_bounds__(256) void nl_columns(const SysDev* sd, SysCount* sc
                                                   const double* Y, const double* Z, const double* Q,
                                                   const double* sig, const double* eps, int* atom_of_slot,
                                                   int* slot_of_atom, float4* cl_ctr, float4* cl_half,
-                                                  int4* super_item, float* slot_zkey, float4* slot_wpos,
+                                                  int4* super_item, float4* slot_wpos,
                                                   typename P::real4* pos, typename P::real2* lj, double* XB,
                                                   double* YB, double* ZB) {
     using real = typename P::real;
@@ -233,10 +233,6 @@ __global__ __launch_bounds__(256) void nl_columns(const SysDev* sd, SysCount* sc
             const int a = ids[i];
             atom_of_slot[slot] = a;
             slot_of_atom[a] = slot;
-            // round down so that a key never exceeds the true z (slab binning stays monotone)
-            float zk = (float)key[i];
-            if ((double)zk > key[i]) zk = nextafterf(zk, -1.0f);
-            slot_zkey[slot] = zk;
             double w[3];
             wrapped(d, X[a], Y[a], Z[a], w);
             slot_wpos[slot] = make_float4((float)w[0], (float)w[1], (float)w[2], 1.0f);
@@ -781,7 +777,7 @@ void launch_nlist(Batch<P>& B, bool clear_flags, int part) {
     nl_columns<P><<<B.n_cols, 256, 0, st>>>(B.d_sys, B.d_cnt, B.col_sys, B.col_count, B.col_fill, B.col_slot,
                                             B.col_super, B.slot_tmp, B.X, B.Y, B.Z, B.q, B.sig, B.eps,
                                             B.atom_of_slot, B.slot_of_atom, B.cl_ctr, B.cl_half, B.super_item,
-                                            B.slot_zkey, B.slot_wpos, B.pos, B.lj, B.XB, B.YB, B.ZB);
+                                            B.slot_wpos, B.pos, B.lj, B.XB, B.YB, B.ZB);
     nl_pairlist<<<B.n_super_cap, kPlThreads, 0, st>>>(B.d_sys, B.d_cnt, B.super_sys, B.super_item, B.col_count, B.col_slot,
                                               B.cl_ctr, B.cl_half, B.slot_wpos, B.atom_of_slot, B.slot_of_atom, B.excl_off,
                                               B.excl_idx, B.list, B.emask, B.chunks, B.n_super_cap);

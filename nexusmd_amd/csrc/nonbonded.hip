@@ -156,15 +156,6 @@ __device__ __forceinline__ double pair_fp64(double r2, double qq, double sig, do
     return dEdR;
 }
 
-// Wave-local ordering of LDS traffic (lanes of one wavefront exchanging data
-// through LDS; the other wavefronts of the block run independently).
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-
 // Lanes l = 8 * ia + ja with ja <= ia: on a diagonal tile (i and j the same
 // cluster) these are the self pairs and the half counted from the other side.
 constexpr unsigned long long lower_triangle_mask() {

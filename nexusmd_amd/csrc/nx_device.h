@@ -57,7 +57,6 @@ struct SysDev {
     int excl_off, n_excl;        // excluded pair list
     int bond_off, n_bonds, angle_off, n_angles, tors_off, n_tors;
     int tw_off[3];               // twiddle-table offsets per axis
-    int sp_block[3];             // spread tiling: columns per block in x, y; z slabs (0 = direct atomics)
     double sp_margin;            // distance an atom may move between rebuilds
 };
 
@@ -271,6 +270,14 @@ __device__ __forceinline__ void wave_energy_add(long long* energy, int s, int te
     } else if (valid) {
         energy_add_fixed(&energy[s * E_NTERMS + term], q);
     }
+}
+
+// Wave-local ordering of LDS traffic (lanes of one wavefront exchanging data
+// through LDS; the other wavefronts of the block run independently).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Reference minimum image: one +-L correction (PeriodicBoundaryCondition.cpp:93-104),

@@ -21,15 +21,28 @@ struct HostSystem;   // engine.hip
 
 // Plane FFT passes: threads per block, LDS available to one workgroup on gfx950.
 constexpr int kPlaneThreads = 1024;
+constexpr int kSpreadPlaneThreads = 768;     // with the spread: three waves per SIMD of at most 56 VGPRs
+// Most LDS of a plane pass with the spread: what the pair kernel's blocks leave of a CU's 160 KB.
+constexpr size_t kPlaneSpreadLds = 100 * 1024;
 constexpr int kXPassThreads = 512;
 constexpr size_t kMaxBlockLds = 160 * 1024 - 1024;   // less the kernels' static LDS
 
-// LDS-tiled spreading: the tile region holds at most kSpreadLdsPoints grid
-// points; its x planes are spread_plane(ny, nz) points apart, an odd count, so
-// that the five lanes of one atom (one x plane each) fall on five different
-// LDS banks (with an even stride they could all land on one).
-constexpr int kSpreadLdsPoints = 7680;   // 60 KB of int64 / double
-__host__ __device__ constexpr int spread_plane(int ny, int nz) { return (ny * nz) | 1; }
+// LDS bytes of the spread in a block of `threads`: its table of slot segments
+// and 128 queued slots per wavefront.
+constexpr int kSpreadSegs = 64;
+constexpr size_t spread_lds_bytes(int threads) { return (size_t)(3 * kSpreadSegs + 2 + threads / 64 * 128) * sizeof(int); }
+// Complex points that two line buffers of cap points, or ny rows of the spread's
+// sums (Kz + 4 long, 8 bytes each) in their place, take.
+template <typename R2>
+__host__ __device__ constexpr int spread_points(int cap, int ny, int Kz) {
+    const int sums = (int)(((size_t)ny * (Kz + 4) * 8 + sizeof(R2) - 1) / sizeof(R2));
+    return 2 * cap > sums ? 2 * cap : sums;
+}
+// Spread and z pass of the line FFT: threads per block, and the complex points
+// one of them moves (two rows of the grid make one complex line).
+constexpr int kSpreadZThreads = 512;
+constexpr int kSpreadZPerThread = 6;
+constexpr int kSpreadZPoints = kSpreadZThreads * kSpreadZPerThread;
 
 // LDS bytes of a plane pass (two buffers, the y and z twiddles).
 template <typename R2>
@@ -37,6 +50,14 @@ inline size_t plane_lds_bytes(int Ky, int Kz) {
     const int np = (Ky + 1) / 2, Kzh = Kz / 2 + 1;
     const int cap = np * Kz > Ky * Kzh ? np * Kz : Ky * Kzh;
     return (size_t)(Ky + Kz + 2 * cap) * sizeof(R2);
+}
+
+// The same with the spread in it.
+template <typename R2>
+inline size_t plane_spread_lds_bytes(int Ky, int Kz) {
+    const int np = (Ky + 1) / 2, Kzh = Kz / 2 + 1;
+    const int cap = np * Kz > Ky * Kzh ? np * Kz : Ky * Kzh;
+    return (size_t)(Ky + Kz + spread_points<R2>(cap, Ky, Kz)) * sizeof(R2) + spread_lds_bytes(kSpreadPlaneThreads);
 }
 
 // LDS bytes of an x pass over nk wave numbers kz (two buffers, the twiddles).
@@ -118,22 +139,21 @@ struct Batch {
 
     // PME
     using gacc = typename P::gacc;
-    gacc* rgrid = nullptr;          // spread charges [sum Kx*Ky*Kz], fixed point (P::grid_scale)
     real2* cgrid = nullptr;         // half spectrum [sum Kx*Ky*(Kz/2+1)]
     real* phi = nullptr;            // potential grid [sum Kx*Ky*Kz]
     real* eta = nullptr;            // influence function on the half spectrum
     real2* twiddle = nullptr;       // per system, per axis exp(-2 pi i t / K)
     long long rgrid_total = 0, cgrid_total = 0, tw_total = 0;
-    int4* spread_tiles = nullptr;   // (sys, column block x, column block y, z slab)
-    int n_spread_tiles = 0, n_spread_direct_slots = 0;
-    float* slot_zkey = nullptr;     // build-time z of each slot (sorted within a column)
-    int4* fftz_items = nullptr;     // (sys, first line, n lines, 0)
+    int4* fftz_items = nullptr;     // spread: (sys, x, y0, ny), or whole planes (sys, x)
+    int4* fftp_items = nullptr;     // inverse plane pass: (sys, x)
+    int4* fftl_items = nullptr;     // inverse z pass: (sys, first line, n lines, 0)
     int4* ffty_items = nullptr;     // (sys, x, kz0, 0)
     int4* fftx_items = nullptr;     // (sys, y, kz0, 0)
-    int n_fftz = 0, n_ffty = 0, n_fftx = 0;
+    int n_fftz = 0, n_fftp = 0, n_fftl = 0, n_ffty = 0, n_fftx = 0;
     int fft_lines = 1, fft_tile = 1, fft_maxK = 0;
-    int fft_plane = 0;              // 1: plane passes (fftz_items = planes, fftx_items = x blocks)
-    size_t fft_plane_lds = 0, fft_x_lds = 0;
+    int fft_plane = 0;              // 1: plane passes (fftp_items, fftx_items = x blocks); 0: line passes
+    int fft_split = 0;              // 1: spread and z pass over rows, then a y pass; 0: spread in the plane pass
+    size_t fft_spread_lds = 0, fft_plane_lds = 0, fft_x_lds = 0;
     int pme_any = 0;
 
     // energies [nsys][E_NTERMS] in 2^30 fixed point

@@ -82,60 +82,19 @@ __device__ __forceinline__ long long grid_fixed(double v) {
     s = fmin(fmax(s, -9.2e18), 9.2e18);
     return (long long)rint(s);
 }
-template <typename R>
-__device__ __forceinline__ void grid_add(long long* g, R v) {
-    atomicAdd(reinterpret_cast<unsigned long long*>(g), static_cast<unsigned long long>(grid_fixed(v)));
-}
 // LDS accumulation (a ds_add_u64)
-template <typename R>
-__device__ __forceinline__ void grid_add_lds(long long* g, R v) {
-    atomicAdd(reinterpret_cast<unsigned long long*>(g), static_cast<unsigned long long>(grid_fixed(v)));
-}
-// adding an already accumulated value
-__device__ __forceinline__ void grid_add_acc(long long* g, long long v) {
+__device__ __forceinline__ void lds_add(long long* g, long long v) {
     atomicAdd(reinterpret_cast<unsigned long long*>(g), static_cast<unsigned long long>(v));
 }
-
-// One thread per (slot, ix): 25 grid updates each.
+// grid_fixed(v) for |v| below grid_fixed_small: v scaled and added to 1.5 2^52 in
+// FP64 is rounded to an integer in the low bits of the sum, three instructions
+// where the 64-bit conversion takes about 18.  The same integer: both round to
+// nearest, ties to even.
 template <class P>
-__global__ void pme_spread_kernel(const SysDev* __restrict__ sd, const SysCount* __restrict__ sc,
-                                  const int* __restrict__ slot_sys, const int* __restrict__ atom_of_slot,
-                                  const typename P::real4* __restrict__ pos, typename P::gacc* rgrid,
-                                  int n_slots_total) {
-    side_priority();
-    using real = typename P::real;
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int slot = (int)(t / 5), ix = (int)(t % 5);
-    if (slot >= n_slots_total) return;
-    const int s = slot_sys[slot];
-    const SysDev& d = sd[s];
-    if (slot - d.slot_off >= sc[s].n_slots || sc[s].overflow) return;
-    if (atom_of_slot[slot] < 0) return;
-    if (d.grid[0] == 0 || d.sp_block[0] > 0) return;
-    const typename P::real4 p = pos[slot];
-    const int Kx = d.grid[0], Ky = d.grid[1], Kz = d.grid[2];
-    int i0, i1, i2;
-    real f0, f1, f2;
-    grid_index<real>(p.x, d.invL[0], Kx, i0, f0);
-    grid_index<real>(p.y, d.invL[1], Ky, i1, f1);
-    grid_index<real>(p.z, d.invL[2], Kz, i2, f2);
-    real tx[5], dtx[5], ty[5], dty[5], tz[5], dtz[5];
-    bspline5<real>(f0, tx, dtx);
-    bspline5<real>(f1, ty, dty);
-    bspline5<real>(f2, tz, dtz);
-    const real qx = p.w * tx[ix];
-    const int xi = (i0 + ix) % Kx;
-    typename P::gacc* g = rgrid + d.rgrid_off + (long long)xi * Ky * Kz;
-#pragma unroll
-    for (int iy = 0; iy < 5; ++iy) {
-        const int yi = (i1 + iy) % Ky;
-        const real qxy = qx * ty[iy];
-#pragma unroll
-        for (int iz = 0; iz < 5; ++iz) {
-            const int zi = (i2 + iz) % Kz;
-            grid_add(&g[(long long)yi * Kz + zi], qxy * tz[iz]);
-        }
-    }
+constexpr double grid_fixed_small = 2251799813685248.0 / P::grid_scale;     // 2^51 units
+template <class P>
+__device__ __forceinline__ long long grid_fixed_fast(typename P::real v) {
+    return __double_as_longlong(fma((double)v, P::grid_scale, 6755399441055744.0)) - 0x4338000000000000ll;
 }
 
 // Quotient of non-negative integers n, d with n + d < 2^22 through a float
@@ -144,175 +103,176 @@ __global__ void pme_spread_kernel(const SysDev* __restrict__ sd, const SysCount*
 // (n / d + 1) 2^-23, which is less.
 __device__ __forceinline__ int qdiv(int n, float inv_d) { return (int)(((float)n + 0.5f) * inv_d); }
 
-// LDS-tiled spreading.  One workgroup per (system, column block, z slab):
-// the atoms binned into those columns at the last neighbour-list build whose
-// build-time z lies in the slab.  Their stencils are accumulated in an LDS copy
-// of the grid region they can reach (block + slab, widened by the distance an
-// atom may move between rebuilds, + 4 points for the order-5 stencil), then
-// the region is added to the global grid once, z-contiguous.  An atom outside
-// the region (never, while the rebuild criterion holds) adds directly.
-constexpr int kSpreadTileCols = 144;    // columns per block: at most 12 x 12 (the host's choice)
+// Charge spreading by ownership.  A workgroup owns ny rows (y0, y0 + 1, ..) of
+// one x plane of the grid, every z: it finds the atoms whose stencils touch
+// them, adds their points in LDS (fixed point: exact, whatever the order) and
+// goes on to the z transform with the sums in place.  No charge grid in global
+// memory: nothing is cleared, added atomically or read back.  Each atom is
+// visited by the five planes of its stencil, 25 points in each.  (Tiles that
+// owned atoms, with every tile's halo added to a global grid, took 35 us alone
+// on 100,000 atoms at 96^3 and 565 us at 128^3, where the halos made 20 million
+// global atomics; the transform then read and cleared the grid.)
+//
+// The candidates are the slots of the neighbour-list columns the rows' atoms
+// were binned into at the last build, widened by the distance an atom may have
+// moved since: column cx of x is a contiguous range of slots, and so is a range
+// of columns cy in it.  A wavefront takes 64 candidates at a time, keeps those
+// that touch its rows in a queue of its own, and spreads 64 of them at once.
+struct SpreadArgs {
+    const SysCount* sc;     // by system
+    const int* col_count;
+    const int* col_slot;
+};
 
 template <class P>
-__global__ __launch_bounds__(256) void pme_spread_tiled(const SysDev* __restrict__ sd,
-                                                        const SysCount* __restrict__ sc,
-                                                        const int4* __restrict__ tiles,
-                                                        const int* __restrict__ col_count,
-                                                        const int* __restrict__ col_slot,
-                                                        const float* __restrict__ slot_zkey,
-                                                        const typename P::real4* __restrict__ pos,
-                                                        typename P::gacc* rgrid) {
-    side_priority();
+__device__ __forceinline__ void spread_rows(const SysDev& d, const SpreadArgs& a,
+                                            const typename P::real4* __restrict__ pos, int x, int y0, int ny, int* lds,
+                                            long long* g) {
     using real = typename P::real;
-    using acc = typename P::gacc;
-    __shared__ acc g[kSpreadLdsPoints];
-    __shared__ int c_first[kSpreadTileCols], c_cnt[kSpreadTileCols], c_a[kSpreadTileCols], c_e[kSpreadTileCols];
-    __shared__ int c_pre[kSpreadTileCols + 1];
-    const int4 t = tiles[blockIdx.x];          // (sys, bx, by, bz)
-    const int s = t.x;
-    const SysDev& d = sd[s];
-    if (sc[s].n_slots == 0 || sc[s].overflow) return;     // overflowed build: the system is frozen
     const int Kx = d.grid[0], Ky = d.grid[1], Kz = d.grid[2];
-    const int BX = d.sp_block[0], BY = d.sp_block[1], NZ = d.sp_block[2];
-    const int cx0 = t.y * BX, cx1 = min(d.ncx, cx0 + BX);
-    const int cy0 = t.z * BY, cy1 = min(d.ncy, cy0 + BY);
-    const double zs = d.L[2] / NZ;
-    const double z0 = t.w * zs, z1 = (t.w + 1 == NZ) ? d.L[2] + 1.0 : (t.w + 1) * zs;
-    const double zlo = t.w * zs;
-    const double m = d.sp_margin;
-    // region origin and extent per axis (full axis when the block spans it)
-    int lo[3], n[3];
-    {
-        const double a0[3] = {cx0 * d.colw[0], cy0 * d.colw[1], zlo};
-        const double a1[3] = {cx1 * d.colw[0], cy1 * d.colw[1], (t.w + 1) * zs};
-        const bool full[3] = {cx0 == 0 && cx1 == d.ncx, cy0 == 0 && cy1 == d.ncy, NZ == 1};
-        const int K[3] = {Kx, Ky, Kz};
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const double h = d.L[k] / K[k];
-            int l = (int)floor((a0[k] - m) / h);
-            int u = (int)floor((a1[k] + m) / h) + 4;
-            if (full[k] || u - l + 1 >= K[k]) { l = 0; u = K[k] - 1; }
-            lo[k] = l;
-            n[k] = u - l + 1;
-        }
-    }
-    const bool fx = (n[0] == Kx && lo[0] == 0), fy = (n[1] == Ky && lo[1] == 0), fz = (n[2] == Kz && lo[2] == 0);
-    const int pl = spread_plane(n[1], n[2]), nyz = n[1] * n[2];     // x-plane stride in LDS, points per plane
-    const int npts = n[0] * pl;
-    if (npts > kSpreadLdsPoints) return;       // host guarantees the fit
-    for (int i = threadIdx.x; i < npts; i += blockDim.x) g[i] = acc(0);
-    __syncthreads();
-    // The block's columns (at most kSpreadTileCols) and, per column, the slots
-    // whose build-time z lies in the slab: the slab bounds are found where the
-    // column's sorted keys step across them, by all threads at once
-    // (independent loads, no per-column search chain).
-    const int ncy_t = cy1 - cy0, ncol = (cx1 - cx0) * ncy_t;
-    for (int q = threadIdx.x; q < ncol; q += blockDim.x) {
-        const int col = d.col_off + (cx0 + q / ncy_t) * d.ncy + cy0 + q % ncy_t;
-        c_first[q] = col_slot[col];
-        c_cnt[q] = col_count[col];
-        c_a[q] = 0;
-        c_e[q] = 0;
-    }
-    __syncthreads();
-    {
-        const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
-        for (int q = wv; q < ncol; q += nw) {
-            const int first = c_first[q], cnt = c_cnt[q];
-            for (int i = lane; i < cnt; i += 64) {
-                const double k1 = (double)slot_zkey[first + i];
-                const double k0 = (i > 0) ? (double)slot_zkey[first + i - 1] : -1.0e300;
-                if (k0 < z0 && z0 <= k1) c_a[q] = i;
-                if (k0 < z1 && z1 <= k1) c_e[q] = i;
-                if (i == cnt - 1) {
-                    if (k1 < z0) c_a[q] = cnt;
-                    if (k1 < z1) c_e[q] = cnt;
-                }
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    int* seg_slot = lds;                          // first slot of each segment
+    int* seg_end = lds + kSpreadSegs;             // past its last slot
+    int* seg_chunk = lds + 2 * kSpreadSegs;       // its first chunk of 64 slots; the total at [n_seg]
+    int* n_seg = lds + 3 * kSpreadSegs + 1;
+    int* queue = lds + 3 * kSpreadSegs + 2 + wv * 128;
+    // rows are Kz + 4 long: a stencil runs past the end, and the reader folds the
+    // last four points onto the first (no wrapped index in the inner loop)
+    const int ls = Kz + 4;
+    for (int i = threadIdx.x; i < ny * ls; i += blockDim.x) g[i] = 0ll;
+    if (wv == 0) {
+        // columns of x (and y) that can hold an atom of these rows: stencils start
+        // at most four points before a row
+        const double hx = d.L[0] / Kx, hy = d.L[1] / Ky, m = d.sp_margin;
+        int xa = (int)floor(((x - 4) * hx - m) / d.colw[0]), nx = (int)floor(((x + 1) * hx + m) / d.colw[0]) - xa + 1;
+        int ya = (int)floor(((y0 - 4) * hy - m) / d.colw[1]), nyc = (int)floor(((y0 + ny) * hy + m) / d.colw[1]) - ya + 1;
+        if (nx >= d.ncx) { xa = 0; nx = d.ncx; }
+        // whole columns of x when the rows need them (or there are too many for the table)
+        const bool whole = nyc >= d.ncy || nx * 2 > kSpreadSegs;
+        if (xa < 0) xa += d.ncx;
+        if (ya < 0) ya += d.ncy;
+        int slot = 0, len = 0, n;
+        if (whole) {
+            // lane 0: columns xa .. of x, lane 1: those past the last, wrapped
+            n = xa + nx > d.ncx ? 2 : 1;
+            const int c0 = lane == 0 ? xa : 0, c1 = lane == 0 ? min(xa + nx, d.ncx) : xa + nx - d.ncx;
+            if (lane < n) {
+                const int last = d.col_off + c1 * d.ncy - 1;
+                slot = a.col_slot[d.col_off + c0 * d.ncy];
+                len = a.col_slot[last] + ((a.col_count[last] + 7) & ~7) - slot;
+            }
+        } else {
+            const int parts = ya + nyc > d.ncy ? 2 : 1;
+            n = nx * parts;
+            if (lane < n) {
+                int cx = xa + lane / parts;
+                if (cx >= d.ncx) cx -= d.ncx;
+                const int c0 = lane % parts == 0 ? ya : 0;
+                const int c1 = lane % parts == 0 ? min(ya + nyc, d.ncy) : ya + nyc - d.ncy;
+                const int first = d.col_off + cx * d.ncy + c0, last = d.col_off + cx * d.ncy + c1 - 1;
+                slot = a.col_slot[first];
+                len = a.col_slot[last] + ((a.col_count[last] + 7) & ~7) - slot;
             }
         }
+        const int chunks = (len + 63) >> 6;
+        int incl = chunks;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int t = __shfl_up(incl, o);
+            if (lane >= o) incl += t;
+        }
+        if (lane < n) {
+            seg_slot[lane] = slot;
+            seg_end[lane] = slot + len;
+            seg_chunk[lane] = incl - chunks;
+        }
+        if (lane == n - 1) {
+            seg_chunk[n] = incl;
+            *n_seg = n;
+        }
     }
     __syncthreads();
-    if (threadIdx.x == 0) {     // running count of the columns' slab atoms
-        int t = 0;
-        for (int q = 0; q < ncol; ++q) {
-            c_pre[q] = t;
-            t += c_e[q] - c_a[q];
-        }
-        c_pre[ncol] = t;
-    }
-    __syncthreads();
-    const int nat = c_pre[ncol];
-    // 5 threads per atom (one per x plane), over all the block's columns
-    for (int w = threadIdx.x; w < nat * 5; w += blockDim.x) {
-        const int at = w / 5, ix = w - at * 5;
-        int lo_q = 0, hi_q = ncol - 1;          // column q with c_pre[q] <= at < c_pre[q + 1]
-        while (lo_q < hi_q) {
-            const int mid = (lo_q + hi_q + 1) >> 1;
-            if (c_pre[mid] <= at) lo_q = mid; else hi_q = mid - 1;
-        }
-        const int slot = c_first[lo_q] + c_a[lo_q] + (at - c_pre[lo_q]);
+    const int ns = *n_seg, total = seg_chunk[ns];
+    auto spread = [&](int slot) {
         const typename P::real4 p = pos[slot];
+        // every weight is below 1, so a charge below the bound keeps its products so
+        const bool small = fabs(p.w) < (real)grid_fixed_small<P>;
         int i0, i1, i2;
         real f0, f1, f2;
         grid_index<real>(p.x, d.invL[0], Kx, i0, f0);
         grid_index<real>(p.y, d.invL[1], Ky, i1, f1);
         grid_index<real>(p.z, d.invL[2], Kz, i2, f2);
-        real tx[5], dtx[5], ty[5], dty[5], tz[5], dtz[5];
-        bspline5<real>(f0, tx, dtx);
-        bspline5<real>(f1, ty, dty);
-        bspline5<real>(f2, tz, dtz);
-        int u0 = fx ? i0 : i0 - lo[0];
-        int u1 = fy ? i1 : i1 - lo[1];
-        int u2 = fz ? i2 : i2 - lo[2];
-        if (!fx) { if (u0 < 0) u0 += Kx; else if (u0 >= Kx) u0 -= Kx; }
-        if (!fy) { if (u1 < 0) u1 += Ky; else if (u1 >= Ky) u1 -= Ky; }
-        if (!fz) { if (u2 < 0) u2 += Kz; else if (u2 >= Kz) u2 -= Kz; }
-        const bool inside = (fx || (u0 >= 0 && u0 + 4 < n[0])) && (fy || (u1 >= 0 && u1 + 4 < n[1])) &&
-                            (fz || (u2 >= 0 && u2 + 4 < n[2]));
-        const real qx = p.w * tx[ix];
-        if (inside) {
-            int x = u0 + ix;
-            if (fx && x >= Kx) x -= Kx;
+        real tx[5], ty[5], tz[5], dt[5];
+        bspline5<real>(f0, tx, dt);
+        bspline5<real>(f1, ty, dt);
+        bspline5<real>(f2, tz, dt);
+        int ix = x - i0;
+        if (ix < 0) ix += Kx;
+        real qx = p.w * tx[0];
 #pragma unroll
-            for (int iy = 0; iy < 5; ++iy) {
-                int y = u1 + iy;
-                if (fy && y >= Ky) y -= Ky;
+        for (int k = 1; k < 5; ++k)
+            if (ix == k) qx = p.w * tx[k];
+        int y = i1 - y0;
+        if (y < 0) y += Ky;
+        long long* row = g + y * ls + i2;
+#pragma unroll
+        for (int iy = 0; iy < 5; ++iy) {
+            if (y < ny) {
                 const real qxy = qx * ty[iy];
+                if (small) {
 #pragma unroll
-                for (int iz = 0; iz < 5; ++iz) {
-                    int z = u2 + iz;
-                    if (fz && z >= Kz) z -= Kz;
-                    grid_add_lds(&g[x * pl + y * n[2] + z], qxy * tz[iz]);
+                    for (int iz = 0; iz < 5; ++iz) lds_add(row + iz, grid_fixed_fast<P>(qxy * tz[iz]));
+                } else {
+                    for (int iz = 0; iz < 5; ++iz) lds_add(row + iz, grid_fixed(qxy * tz[iz]));
                 }
             }
-        } else {
-            const int xi = (i0 + ix) % Kx;
-            acc* gg = rgrid + d.rgrid_off + (long long)xi * Ky * Kz;
-#pragma unroll
-            for (int iy = 0; iy < 5; ++iy) {
-                const int yi = (i1 + iy) % Ky;
-                const real qxy = qx * ty[iy];
-#pragma unroll
-                for (int iz = 0; iz < 5; ++iz) grid_add(&gg[(long long)yi * Kz + (i2 + iz) % Kz], qxy * tz[iz]);
-            }
+            const bool last = y + 1 == Ky;
+            y = last ? 0 : y + 1;
+            row += last ? (1 - Ky) * ls : ls;
+        }
+    };
+    int nq = 0;
+    // the slot of this lane's candidate in chunk c (-1: none) and, loaded while the
+    // chunk before it is worked on, its position
+    auto candidate = [&](int c) {
+        if (c >= total) return -1;
+        int s = 0;
+        while (s + 1 < ns && seg_chunk[s + 1] <= c) ++s;
+        const int slot = seg_slot[s] + (c - seg_chunk[s]) * 64 + lane;
+        return slot < seg_end[s] ? slot : -1;
+    };
+    int slot_n = candidate(wv);
+    typename P::real4 p_n;
+    if (slot_n >= 0) p_n = pos[slot_n];
+    for (int c = wv; c < total; c += nw) {
+        const int slot = slot_n;
+        const typename P::real4 p = p_n;
+        slot_n = candidate(c + nw);
+        if (slot_n >= 0) p_n = pos[slot_n];
+        bool hit = false;
+        if (slot >= 0) {
+            int i0, i1;
+            real f;
+            grid_index<real>(p.x, d.invL[0], Kx, i0, f);
+            grid_index<real>(p.y, d.invL[1], Ky, i1, f);
+            int ix = x - i0, y = i1 - y0;
+            if (ix < 0) ix += Kx;
+            if (y < 0) y += Ky;
+            hit = p.x < (real)(0.5 * kPadPos) && ix < 5 && (y < ny || y + 4 >= Ky);
+        }
+        const unsigned long long m = __ballot(hit);
+        if (hit) queue[nq + __popcll(m & ((1ull << lane) - 1ull))] = slot;
+        nq += __popcll(m);
+        wave_lds_sync();
+        if (nq >= 64) {
+            spread(queue[lane]);
+            nq -= 64;
+            if (lane < nq) queue[lane] = queue[64 + lane];
+            wave_lds_sync();
         }
     }
+    if (lane < nq) spread(queue[lane]);
     __syncthreads();
-    // flush the region (z fastest: contiguous global addresses)
-    const float inv_pl = 1.0f / (float)pl, inv_nz = 1.0f / (float)n[2];
-    for (int i = threadIdx.x; i < npts; i += blockDim.x) {
-        const acc v = g[i];
-        if (v == acc(0)) continue;             // also the plane padding, never written
-        const int x = qdiv(i, inv_pl), r = i - x * pl;     // i, pl <= kSpreadLdsPoints
-        if (r >= nyz) continue;
-        const int y = qdiv(r, inv_nz), z = r - y * n[2];
-        int gx = lo[0] + x, gy = lo[1] + y, gz = lo[2] + z;
-        gx = gx < 0 ? gx + Kx : (gx >= Kx ? gx - Kx : gx);
-        gy = gy < 0 ? gy + Ky : (gy >= Ky ? gy - Ky : gy);
-        gz = gz < 0 ? gz + Kz : (gz >= Kz ? gz - Kz : gz);
-        grid_add_acc(&rgrid[d.rgrid_off + ((long long)gx * Ky + gy) * Kz + gz], v);
-    }
 }
 
 // Force from the potential grid (NonbondedForce.cpp:407-461).  A block of
@@ -525,10 +485,80 @@ __device__ R2* fft_lines_lds(R2* a, R2* b, int N, int lines, int ls, int es, con
 __device__ __forceinline__ float fixed_to_real(long long v, float) { return (float)((double)v * (1.0 / PrecMixed::grid_scale)); }
 __device__ __forceinline__ double fixed_to_real(long long v, double) { return (double)v * (1.0 / PrecFP64::grid_scale); }
 
+// Point (row y, z) of a grid plane: rows of Kz points in memory, of Kz + 4 as the
+// spread leaves them in LDS.
+template <bool SPREAD>
+__device__ __forceinline__ long long grid_value(const long long* g, int y, int z, int Kz) {
+    if constexpr (!SPREAD) return g[y * Kz + z];
+    const long long* row = g + y * (Kz + 4);
+    return z < 4 ? row[z] + row[z + Kz] : row[z];
+}
+
+// Z pass forward with the spread: rows y0 .. y0 + ny - 1 of plane x, two rows as
+// one complex line (see fft_plane_fwd).  item = (sys, x, y0, ny)
+template <class P>
+__global__ __launch_bounds__(kSpreadZThreads) void fft_z_spread(const SysDev* __restrict__ sd,
+                                                               const int4* __restrict__ items, SpreadArgs sp,
+                                                               const typename P::real4* __restrict__ pos,
+                                                               typename P::real2* cgrid,
+                                                               const typename P::real2* __restrict__ tw) {
+    side_priority();
+    using real = typename P::real;
+    using R2 = typename P::real2;
+    extern __shared__ unsigned char smem_raw[];
+    const int4 it = items[blockIdx.x];
+    const SysDev& d = sd[it.x];
+    const SysCount& sc = sp.sc[it.x];
+    if (sc.n_slots == 0 || sc.overflow) return;      // overflowed build: the system is frozen
+    const int x = it.y, y0 = it.z, ny = it.w;
+    const int Ky = d.grid[1], Kz = d.grid[2], Kzh = Kz / 2 + 1, np = (ny + 1) >> 1, cap = np * Kz;
+    R2* TW = reinterpret_cast<R2*>(smem_raw);
+    R2* A = TW + Kz;
+    R2* B = A + cap;
+    load_twiddles(TW, tw + d.tw_off[2], Kz);
+    typename P::gacc* g = reinterpret_cast<typename P::gacc*>(A);
+    spread_rows<P>(d, sp, pos, x, y0, ny, reinterpret_cast<int*>(A + spread_points<R2>(cap, ny, Kz)), g);
+    // through registers into place, as in fft_plane_fwd
+    const float inv_kz = 1.0f / (float)Kz;
+    R2 v[kSpreadZPerThread];
+#pragma unroll
+    for (int u = 0; u < kSpreadZPerThread; ++u) {
+        const int i = threadIdx.x + u * kSpreadZThreads;
+        if (i < cap) {
+            const int p = qdiv(i, inv_kz), z = i - p * Kz;
+            v[u].x = fixed_to_real(grid_value<true>(g, 2 * p, z, Kz), (real)0);
+            v[u].y = (2 * p + 1 < ny) ? fixed_to_real(grid_value<true>(g, 2 * p + 1, z, Kz), (real)0) : (real)0;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kSpreadZPerThread; ++u) {
+        const int i = threadIdx.x + u * kSpreadZThreads;
+        if (i < cap) A[i] = v[u];
+    }
+    __syncthreads();
+    R2* Z = fft_lines_lds<real, R2>(A, B, Kz, np, Kz, 1, TW, -1);
+    R2* c = cgrid + d.cgrid_off + ((long long)x * Ky + y0) * Kzh;
+    const float inv_kzh = 1.0f / (float)Kzh;
+    for (int i = threadIdx.x; i < ny * Kzh; i += kSpreadZThreads) {
+        const int y = qdiv(i, inv_kzh), k = i - y * Kzh;
+        const R2 zk = Z[(y >> 1) * Kz + k], zn = Z[(y >> 1) * Kz + (k == 0 ? 0 : Kz - k)];
+        R2 r;
+        if (y & 1) {
+            r.x = (real)0.5 * (zk.y + zn.y);
+            r.y = (real)0.5 * (zn.x - zk.x);
+        } else {
+            r.x = (real)0.5 * (zk.x + zn.x);
+            r.y = (real)0.5 * (zk.y - zn.y);
+        }
+        c[i] = r;
+    }
+}
+
 // Z pass forward: R2C.  item = (sys, first line, n lines)
 template <class P>
 __global__ __launch_bounds__(256) void fft_z_fwd(const SysDev* __restrict__ sd, const int4* __restrict__ items,
-                                                 typename P::gacc* __restrict__ rgrid,
+                                                 const typename P::gacc* __restrict__ rgrid,
                                                  typename P::real2* cgrid, const typename P::real2* __restrict__ tw) {
     side_priority();
     using real = typename P::real;
@@ -543,13 +573,11 @@ __global__ __launch_bounds__(256) void fft_z_fwd(const SysDev* __restrict__ sd, 
     R2* B = smem + nl * Kz;
     R2* TW = B + nl * Kz;
     load_twiddles(TW, tw + d.tw_off[2], Kz);
-    // the spread grid is cleared as it is read: the next spread adds into it
-    typename P::gacc* g = rgrid + d.rgrid_off + (long long)line0 * Kz;
+    const typename P::gacc* g = rgrid + d.rgrid_off + (long long)line0 * Kz;
     for (int i = threadIdx.x; i < nl * Kz; i += blockDim.x) {
         R2 v;
         v.x = fixed_to_real(g[i], (real)0);
         v.y = 0;
-        g[i] = typename P::gacc(0);
         A[i] = v;
     }
     __syncthreads();
@@ -729,12 +757,14 @@ __global__ __launch_bounds__(256) void fft_x_plain(const SysDev* __restrict__ sd
 // The complex-to-real inverse packs them the same way: Z_k = A_k + i B_k over
 // the Hermitian extension, then a = Re, b = Im of the inverse transform.
 
-// Forward: plane x of the spread grid -> plane x of the half spectrum (z then y).
+// Forward: plane x of the charge grid -> plane x of the half spectrum (z then y).
+// The grid's plane is spread here (SPREAD) or read from `rgrid`.
 // item = (sys, x)
-template <class P>
-__global__ __launch_bounds__(kPlaneThreads) void fft_plane_fwd(const SysDev* __restrict__ sd,
+template <class P, bool SPREAD>
+__global__ __launch_bounds__(SPREAD ? kSpreadPlaneThreads : kPlaneThreads) void fft_plane_fwd(const SysDev* __restrict__ sd,
                                                               const int4* __restrict__ items,
-                                                              typename P::gacc* __restrict__ rgrid,
+                                                              const typename P::gacc* __restrict__ rgrid, SpreadArgs sp,
+                                                              const typename P::real4* __restrict__ pos,
                                                               typename P::real2* cgrid,
                                                               const typename P::real2* __restrict__ tw) {
     side_priority();
@@ -753,20 +783,49 @@ __global__ __launch_bounds__(kPlaneThreads) void fft_plane_fwd(const SysDev* __r
     R2* Bf = A + cap;
     load_twiddles(TWy, tw + d.tw_off[1], Ky);
     load_twiddles(TWz, tw + d.tw_off[2], Kz);
-    // the spread grid is cleared as it is read: the next spread adds into it
-    typename P::gacc* g = rgrid + d.rgrid_off + (long long)x * Ky * Kz;
     const float inv_kz = 1.0f / (float)Kz;
-    for (int i = threadIdx.x; i < np * Kz; i += blockDim.x) {
+    // rows 2p and 2p + 1 as one complex line
+    auto line_pair = [&](const typename P::gacc* g, int i) {
         const int p = qdiv(i, inv_kz), z = i - p * Kz;
         R2 v;
-        v.x = fixed_to_real(g[(2 * p) * Kz + z], (real)0);
-        g[(2 * p) * Kz + z] = typename P::gacc(0);
-        v.y = (real)0;
-        if (2 * p + 1 < Ky) {
-            v.y = fixed_to_real(g[(2 * p + 1) * Kz + z], (real)0);
-            g[(2 * p + 1) * Kz + z] = typename P::gacc(0);
+        v.x = fixed_to_real(grid_value<SPREAD>(g, 2 * p, z, Kz), (real)0);
+        v.y = (2 * p + 1 < Ky) ? fixed_to_real(grid_value<SPREAD>(g, 2 * p + 1, z, Kz), (real)0) : (real)0;
+        return v;
+    };
+    if constexpr (SPREAD) {
+        // the sums take the room of the two line buffers: through registers into place
+        const SysCount& sc = sp.sc[it.x];
+        if (sc.n_slots == 0 || sc.overflow) return;      // overflowed build: the system is frozen
+        typename P::gacc* g = reinterpret_cast<typename P::gacc*>(A);
+        spread_rows<P>(d, sp, pos, x, 0, Ky, reinterpret_cast<int*>(A + spread_points<R2>(cap, Ky, Kz)), g);
+        if constexpr (P::mixed) {
+            // a point of the line takes the room of the sum at its own index, and
+            // reads the sums at that index or past it
+            for (int b = 0; b < np * Kz; b += kSpreadPlaneThreads) {
+                const int i = b + threadIdx.x;
+                R2 v;
+                if (i < np * Kz) v = line_pair(g, i);
+                __syncthreads();
+                if (i < np * Kz) A[i] = v;
+            }
+        } else {
+            constexpr int kMax = (int)(kMaxBlockLds / (2 * sizeof(R2)) + kSpreadPlaneThreads - 1) / kSpreadPlaneThreads;
+            R2 v[kMax];
+#pragma unroll
+            for (int u = 0; u < kMax; ++u) {
+                const int i = threadIdx.x + u * kSpreadPlaneThreads;
+                if (i < np * Kz) v[u] = line_pair(g, i);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < kMax; ++u) {
+                const int i = threadIdx.x + u * kSpreadPlaneThreads;
+                if (i < np * Kz) A[i] = v[u];
+            }
         }
-        A[i] = v;
+    } else {
+        const typename P::gacc* g = rgrid + d.rgrid_off + (long long)x * Ky * Kz;
+        for (int i = threadIdx.x; i < np * Kz; i += blockDim.x) A[i] = line_pair(g, i);
     }
     __syncthreads();
     R2* Z = fft_lines_lds<real, R2>(A, Bf, Kz, np, Kz, 1, TWz, -1);
@@ -903,24 +962,6 @@ __global__ __launch_bounds__(kPlaneThreads) void fft_x_block(const SysDev* __res
 }
 
 template <class P>
-void launch_pme_spread(Batch<P>& B) {
-    if (!B.pme_any) return;
-    const int T = 256;
-    // the grid starts cleared (allocation) and the forward transform clears it
-    // again as it reads it, so every spread adds into zeros
-    if (B.n_spread_tiles > 0)
-        pme_spread_tiled<P><<<B.n_spread_tiles, 256, 0, B.stream>>>(B.d_sys, B.d_cnt, B.spread_tiles, B.col_count,
-                                                                    B.col_slot, B.slot_zkey, B.pos, B.rgrid);
-    if (B.n_spread_direct_slots > 0) {
-        // systems whose region does not fit the LDS tile: per-atom global atomics
-        const long long nthr = (long long)B.n_slots_cap * 5;
-        pme_spread_kernel<P><<<(unsigned)((nthr + T - 1) / T), T, 0, B.stream>>>(B.d_sys, B.d_cnt, B.slot_sys,
-                                                                                 B.atom_of_slot, B.pos, B.rgrid,
-                                                                                 B.n_slots_cap);
-    }
-}
-
-template <class P>
 static size_t fft_smem(const Batch<P>& B, int lines, int N) {
     return (size_t)(2 * lines + 1) * N * sizeof(typename P::real2);   // two line buffers + twiddles
 }
@@ -934,10 +975,11 @@ bool fft_plane_enabled() {
 // Raises the dynamic-LDS limit of the plane kernels to what the batch needs.
 template <class P>
 hipError_t prepare_fft(Batch<P>& B) {
-    if (!B.fft_plane) return hipSuccess;
-    const int pl = (int)B.fft_plane_lds, xl = (int)B.fft_x_lds;
+    const int sl = (int)B.fft_spread_lds, pl = (int)B.fft_plane_lds, xl = (int)B.fft_x_lds;
     const hipFuncAttribute a = hipFuncAttributeMaxDynamicSharedMemorySize;
-    hipError_t e = hipFuncSetAttribute((const void*)fft_plane_fwd<P>, a, pl);
+    hipError_t e = hipFuncSetAttribute(
+        B.fft_split ? (const void*)fft_z_spread<P> : (const void*)fft_plane_fwd<P, true>, a, sl);
+    if (!B.fft_plane) return e;
     if (e == hipSuccess) e = hipFuncSetAttribute((const void*)fft_plane_inv<P>, a, pl);
     if (e == hipSuccess) e = hipFuncSetAttribute((const void*)fft_x_block<P, 2>, a, xl);
     if (e == hipSuccess) e = hipFuncSetAttribute((const void*)fft_x_block<P, 3>, a, xl);
@@ -945,15 +987,20 @@ hipError_t prepare_fft(Batch<P>& B) {
 }
 
 template <class P>
-void launch_fft_forward(Batch<P>& B) {
+void launch_pme_spread(Batch<P>& B) {
     if (!B.pme_any) return;
-    if (B.fft_plane) {
-        fft_plane_fwd<P><<<B.n_fftz, kPlaneThreads, B.fft_plane_lds, B.stream>>>(B.d_sys, B.fftz_items, B.rgrid,
-                                                                               B.cgrid, B.twiddle);
-        return;
-    }
-    fft_z_fwd<P><<<B.n_fftz, 256, fft_smem(B, B.fft_lines, B.fft_maxK), B.stream>>>(B.d_sys, B.fftz_items, B.rgrid,
-                                                                                   B.cgrid, B.twiddle);
+    const SpreadArgs sp{B.d_cnt, B.col_count, B.col_slot};
+    if (!B.fft_split)
+        fft_plane_fwd<P, true><<<B.n_fftz, kSpreadPlaneThreads, B.fft_spread_lds, B.stream>>>(
+            B.d_sys, B.fftz_items, nullptr, sp, B.pos, B.cgrid, B.twiddle);
+    else
+        fft_z_spread<P><<<B.n_fftz, kSpreadZThreads, B.fft_spread_lds, B.stream>>>(B.d_sys, B.fftz_items, sp, B.pos,
+                                                                                 B.cgrid, B.twiddle);
+}
+
+template <class P>
+void launch_fft_forward(Batch<P>& B) {
+    if (!B.pme_any || !B.fft_split) return;      // the spread's launch ran the plane pass
     fft_y<P><<<B.n_ffty, 256, fft_smem(B, B.fft_tile, B.fft_maxK), B.stream>>>(B.d_sys, B.ffty_items, B.cgrid,
                                                                               B.twiddle, B.fft_tile, -1);
 }
@@ -982,13 +1029,13 @@ template <class P>
 void launch_fft_inverse(Batch<P>& B) {
     if (!B.pme_any) return;
     if (B.fft_plane) {
-        fft_plane_inv<P><<<B.n_fftz, kPlaneThreads, B.fft_plane_lds, B.stream>>>(B.d_sys, B.fftz_items, B.cgrid,
+        fft_plane_inv<P><<<B.n_fftp, kPlaneThreads, B.fft_plane_lds, B.stream>>>(B.d_sys, B.fftp_items, B.cgrid,
                                                                                B.phi, B.twiddle);
         return;
     }
     fft_y<P><<<B.n_ffty, 256, fft_smem(B, B.fft_tile, B.fft_maxK), B.stream>>>(B.d_sys, B.ffty_items, B.cgrid,
                                                                               B.twiddle, B.fft_tile, +1);
-    fft_z_inv<P><<<B.n_fftz, 256, fft_smem(B, B.fft_lines, B.fft_maxK), B.stream>>>(B.d_sys, B.fftz_items, B.cgrid,
+    fft_z_inv<P><<<B.n_fftl, 256, fft_smem(B, B.fft_lines, B.fft_maxK), B.stream>>>(B.d_sys, B.fftl_items, B.cgrid,
                                                                                    B.phi, B.twiddle);
 }
 
@@ -1068,7 +1115,7 @@ void fft3d_roundtrip(int nx, int ny, int nz, const double* in, double* out, bool
         hipMalloc(&db, bi.size() * sizeof(int4));
         hipMemcpyAsync(dp, pi.data(), pi.size() * sizeof(int4), hipMemcpyHostToDevice, st);
         hipMemcpyAsync(db, bi.data(), bi.size() * sizeof(int4), hipMemcpyHostToDevice, st);
-        hipFuncSetAttribute((const void*)fft_plane_fwd<P>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl);
+        hipFuncSetAttribute((const void*)fft_plane_fwd<P, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl);
         hipFuncSetAttribute((const void*)fft_plane_inv<P>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl);
         hipFuncSetAttribute((const void*)fft_x_block<P, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)xl);
         hipFuncSetAttribute((const void*)fft_x_block<P, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)xl);
@@ -1080,7 +1127,7 @@ void fft3d_roundtrip(int nx, int ny, int nz, const double* in, double* out, bool
         }
         hipMemcpyAsync(rg, h.data(), G * sizeof(typename P::gacc), hipMemcpyHostToDevice, st);
         if (plane) {
-            fft_plane_fwd<P><<<(unsigned)pi.size(), kPlaneThreads, pl, st>>>(dd, dp, rg, cg, dtw);
+            fft_plane_fwd<P, false><<<(unsigned)pi.size(), kPlaneThreads, pl, st>>>(dd, dp, rg, {}, nullptr, cg, dtw);
             fft_x_block<P, 0><<<(unsigned)bi.size(), kXPassThreads, xl, st>>>(dd, db, cg, nullptr, dtw, nullptr);
         } else {
             fft_z_fwd<P><<<(unsigned)zi.size(), 256, sm, st>>>(dd, dz, rg, cg, dtw);
@@ -1253,12 +1300,12 @@ nx_status fft3d_r2c_noalloc(int device, int nx, int ny, int nz, const double* in
     noalloc_to_fixed_kernel<<<(unsigned)((G + 255) / 256), 256, 0, st>>>(rg, G, P::grid_scale);
     if (plane) {
         const size_t pl = plane_lds_bytes<R2>(ny, nz), xl = xpass_lds_bytes<R2>(nx, nzh);
-        if ((e = hipFuncSetAttribute((const void*)fft_plane_fwd<P>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        if ((e = hipFuncSetAttribute((const void*)fft_plane_fwd<P, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int)pl)) != hipSuccess ||
             (e = hipFuncSetAttribute((const void*)fft_x_block<P, 0>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int)xl)) != hipSuccess)
             return fail(e, "hipFuncSetAttribute");
-        fft_plane_fwd<P><<<(unsigned)n0, kPlaneThreads, pl, st>>>(dd, items, rg, cg, dtw);
+        fft_plane_fwd<P, false><<<(unsigned)n0, kPlaneThreads, pl, st>>>(dd, items, rg, {}, nullptr, cg, dtw);
         fft_x_block<P, 0><<<(unsigned)n1, kXPassThreads, xl, st>>>(dd, items + n0, cg, nullptr, dtw, nullptr);
     } else {
         const size_t sm = (size_t)(2 * T + 1) * maxK * sizeof(R2);

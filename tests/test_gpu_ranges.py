@@ -58,3 +58,40 @@ def test_fp64_direct_space_either_side_of_the_series(tol):
     s.pos[1] = (s.pos[0] + [0.03, 0.02, 0.01]) % s.L       # a close contact
     assert (-np.log(2 * tol) <= 8.0) == (tol == 1.7e-4)
     _check(s, L.FP64, "series range")
+
+
+@pytest.mark.parametrize("prec", [L.FP64, L.MIXED])
+@pytest.mark.parametrize("grid,skin", [((20, 24, 30), 0.1),      # whole planes
+                                       ((27, 45, 25), 0.0),      # odd rows, no buffer
+                                       ((6, 10, 9), 0.3),        # stencils of most of the box
+                                       ((24, 150, 100), 0.1),    # rows of planes (FP64), a y pass
+                                       ((15, 135, 160), 0.1),    # rows of planes (both)
+                                       ((8, 9, 1000), 0.1)])     # two rows at a time
+def test_spread_shapes(grid, skin, prec):
+    """Charge spreading over whole planes and over rows, forces on every atom."""
+    s = _gas(1203, (2.0, 2.9, 2.3), 17, grid=grid)
+    s.pos = (s.pos - s.pos[5] - 1e-9) % s.L       # one atom just inside the far corner
+    s.pos = s.pos[np.random.default_rng(1).permutation(s.n)]
+    _check(s, prec, "spread %s" % (grid,), skin=skin)
+
+
+def test_spread_of_large_charges():
+    """Charges past the bound of the short conversion to fixed point (8 e in FP64)."""
+    s = _gas(700, (2.0, 2.0, 2.0), 4, grid=(24, 24, 24))
+    s.q *= 30.0
+    assert (np.abs(s.q) > 8).sum() > 100 and (np.abs(s.q) < 8).sum() > 100
+    _check(s, L.FP64, "large charges")
+
+
+@pytest.mark.parametrize("prec", [L.FP64, L.MIXED])
+def test_line_and_plane_passes_agree(prec, monkeypatch):
+    s = _gas(1500, (2.4, 2.6, 2.2), 8, grid=(30, 36, 25))
+    out = []
+    for plane in ("1", "0"):
+        monkeypatch.setenv("NEXUSMD_FFT_PLANE", plane)
+        ctx = E.Context(s, precision=prec)
+        out.append(ctx.compute_forces()[0])
+        ctx.close()
+    # the inverse transforms differ (one or two real lines at a time), the spread and
+    # the forward ones do not: rounding only
+    assert rel_rms(out[0], out[1]) <= (1e-13 if prec == L.FP64 else 1e-6)
