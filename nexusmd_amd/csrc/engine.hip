@@ -140,15 +140,16 @@ static int grid_rule(double L) {
 // Pair-list entries per chunk of the pair kernel, by the system's own size (not
 // the batch's: a request's arithmetic is the same alone and in any batch).  A
 // chunk costs its wavefront a claim, the i data and a force flush besides its
-// entries, so large systems take the longest; a small system's list in chunks of
-// 32 leaves most of the chip idle while a few wavefronts work through theirs.
-// FP64, whose pairs are dear: us per 100 steps of the 1,500-bead chain with 8,
-// 16, 32 entries: 7980, 9330, 13170; per 25 of 100,000 atoms: 19680, 18010,
-// 17560.  Mixed, where the kernels beside the pair kernel end after it on small
-// systems and its extra flushes delay them: 7950, 7840, 7730 on the chain.
+// entries, so large systems take the longest; with fewer chunks than a few per
+// wavefront the last ones to end leave the chip idle.  us a step with 8, 12, 16,
+// 24, 32 entries (mixed): 1,500-bead chain 66.8 66.0 66.3 68.2 73.5; water of
+// 24,000 atoms 87.6 86.9 87.2 93.6 97.5, of 36,000 95.5 96.2 98.6 101 109, of a
+// million 1598 1524 1470 1439 1426; solvated chains of 100,000 196 190 188 190
+// 193.  FP64: chain 69.0 69.2 75.6 90.4 100; 24,000 171 158 155 155 157; 100,000
+// 454 389 376 375 377.
 static int chunk_entries_for(int n_atoms, bool mixed) {
-    if (mixed) return kChunkEntries;
-    return n_atoms < 6000 ? 8 : kChunkEntries;
+    if (n_atoms >= 300000) return kChunkEntries;
+    return mixed ? (n_atoms < 60000 ? 12 : 16) : (n_atoms < 6000 ? 8 : 16);
 }
 
 // ----------------------------------------------------------- tuning cache
@@ -310,13 +311,14 @@ class Engine : public EngineBase {
             d.n_atoms = n;
             d.atom_off = (int)atom_off;
             d.pair_image = pair_image_ ? 1 : 0;
-            // columns of ~8/rho^(1/3) nm so that a cluster of 8 is roughly cubic
+            // columns as wide as 64 atoms are tall, so that a super-cluster is about a
+            // cube; their quarters hold at most 2048 atoms, 700 on average
             const double V = d.L[0] * d.L[1] * d.L[2];
             const double rho = std::max(1e-3, n / V);
-            double cw = cbrt(8.0 / rho);
+            double cw = 2.0 * cbrt(8.0 / rho);
             int ncx = std::max(1, (int)floor(d.L[0] / cw));
             int ncy = std::max(1, (int)floor(d.L[1] / cw));
-            while ((double)n / ((double)ncx * ncy) > 700.0) { ncx += 1; ncy += 1; }
+            while ((double)n / (4.0 * ncx * ncy) > 700.0) { ncx += 1; ncy += 1; }
             d.ncx = ncx;
             d.ncy = ncy;
             d.colw[0] = d.L[0] / ncx;
@@ -331,8 +333,7 @@ class Engine : public EngineBase {
             const double w = std::max(d.colw[0], d.colw[1]);
             const double hz = std::min(d.L[2], 64.0 / (rho * d.colw[0] * d.colw[1]));
             const double r = d.rlist;
-            double ext = (std::min(d.L[0], w + 2 * r + 2 * w)) * (std::min(d.L[1], w + 2 * r + 2 * w)) *
-                         std::min(d.L[2], hz + 2 * r + 0.5);
+            double ext = std::min(d.L[0], w + 2 * r) * std::min(d.L[1], w + 2 * r) * std::min(d.L[2], hz + 2 * r);
             double per_super = 1.5 * (rho / 8.0) * ext * h.list_scale;
             per_super = std::min(per_super, (double)kSuperListCap);
             per_super = std::max(per_super, 16.0);
@@ -422,12 +423,15 @@ class Engine : public EngineBase {
         dalloc(&B.FSx, S, o, B.stream);
         dalloc(&B.FSy, S, o, B.stream);
         dalloc(&B.FSz, S, o, B.stream);
-        for (int** p : {&B.col_sys, &B.col_count, &B.col_fill, &B.col_slot, &B.col_super, &B.col_tmp})
+        for (int** p : {&B.col_sys, &B.col_count, &B.col_fill, &B.col_slot, &B.col_super})
             dalloc(p, B.n_cols, o, B.stream);
+        dalloc(&B.col_tmp, (size_t)4 * B.n_cols, o, B.stream);
         dalloc(&B.cl_ctr, S / 8 + 1, o, B.stream);
         dalloc(&B.cl_half, S / 8 + 1, o, B.stream);
         dalloc(&B.super_sys, B.n_super_cap, o, B.stream);
         dalloc(&B.super_item, B.n_super_cap, o, B.stream);
+        dalloc(&B.sup_ctr, B.n_super_cap, o, B.stream);
+        dalloc(&B.sup_half, B.n_super_cap, o, B.stream);
         dalloc(&B.slot_wpos, S, o, B.stream);
         dalloc(&B.chunks, B.n_chunk_cap, o, B.stream);
         dalloc(&B.chunk_prefix, B.nsys + 1, o, B.stream);

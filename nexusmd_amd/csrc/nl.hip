@@ -4,22 +4,28 @@
 // NeighborList.cpp:12-154), which rebuilds a std::map voxel hash every step.
 // Here, per rebuild:
 //   1. nl_bin      : counting sort of atoms into xy columns (one atomic per
-//                    distinct column in a wavefront);
+//                    distinct quarter column in a wavefront);
 //   2. nl_scan     : per-system exclusive scan -> slot ranges (columns padded
 //                    to 8-atom clusters) and super-cluster ranges; clears the
 //                    bin counters for the next build;
 //   3. nl_scatter  : atoms into their column's slot range;
-//   4. nl_columns  : per column, sort by (z, atom id) in LDS -> deterministic
-//                    slot order; cluster bounding boxes; build positions in
+//   4. nl_columns  : per column, sort by z -> super-clusters of 64 consecutive
+//                    atoms, each split by x, y and z medians into 8 clusters of
+//                    8 (ties by the order before, the first by atom id:
+//                    deterministic); bounding boxes of both; build positions in
 //                    slot order; the slot-order positions, charges and LJ
 //                    parameters the force kernels read, and each atom's build
 //                    position for the displacement test;
-//   5. nl_pairlist : one block per super-cluster (8 clusters of 8 atoms):
-//                    j-clusters of nearby columns whose bounding box is within
+//   5. nl_pairlist : one block per super-cluster: the super-clusters of nearby
+//                    columns, then their clusters, whose bounding box is within
 //                    rlist of an i-cluster (half list: j >= i), then per tile
 //                    the 64 atom pairs, keeping only tiles with a pair within
 //                    rlist; an 8-bit mask of interacting i-clusters per entry,
 //                    and 64-bit exclusion masks for tiles holding excluded pairs.
+// Columns are about as wide as 64 atoms are tall, so a super-cluster is about a
+// cube and a j cluster near it meets most of its clusters: 5 tiles an entry on
+// liquids, where super-clusters of one 8-atom-wide column (3.5 nm tall) had 2.9.
+// The pair kernel pays ~45 instructions per entry besides its tiles.
 // The pair kernel applies r^2 < rc^2 exactly per pair, so the evaluated pair
 // set is the reference's set whatever the buffer (skin) is.
 //
@@ -34,7 +40,9 @@
 
 namespace nx {
 
-constexpr int kColSortCap = 2048;     // atoms per column sorted in LDS
+constexpr int kQuarterCap = 2048;     // most atoms in a quarter of a column (2 x 2 in xy)
+constexpr int kColSortCap = 4 * kQuarterCap;     // atoms per column sorted in LDS
+constexpr int kColThreads = 512;      // threads per column in nl_columns
 constexpr int kListCap = kSuperListCap;   // pair-list entries per super-cluster (LDS)
 constexpr int kExclCap = 2048;        // exclusion triples per super-cluster (LDS)
 
@@ -77,7 +85,8 @@ __device__ __forceinline__ int wave_keyed_increment(int* counter, int key) {
     return res;
 }
 
-// Column of every atom and the column counts (into col_tmp, zero between builds).
+// Column of every atom and the counts of the columns' quarters (into col_tmp, zero
+// between builds).
 __global__ void nl_bin(const SysDev* sd, SysCount* sc, const int* atom_sys, const double* X, const double* Y,
                        const double* Z, int* atom_col, int* col_tmp, int n_atoms_total) {
     int a = blockIdx.x * blockDim.x + threadIdx.x;
@@ -87,18 +96,16 @@ __global__ void nl_bin(const SysDev* sd, SysCount* sc, const int* atom_sys, cons
     const SysDev& d = sd[s];
     double w[3];
     wrapped(d, X[a], Y[a], Z[a], w);
-    int cx = (int)(w[0] / d.colw[0]);
-    int cy = (int)(w[1] / d.colw[1]);
-    cx = cx < 0 ? 0 : (cx >= d.ncx ? d.ncx - 1 : cx);
-    cy = cy < 0 ? 0 : (cy >= d.ncy ? d.ncy - 1 : cy);
-    int col = d.col_off + cx * d.ncy + cy;
+    const int qx = min(max((int)(w[0] / (0.5 * d.colw[0])), 0), 2 * d.ncx - 1);
+    const int qy = min(max((int)(w[1] / (0.5 * d.colw[1])), 0), 2 * d.ncy - 1);
+    const int col = d.col_off + (qx >> 1) * d.ncy + (qy >> 1);
     atom_col[a] = col;
-    wave_keyed_increment(col_tmp, col);
+    wave_keyed_increment(col_tmp, 4 * col + 2 * (qx & 1) + (qy & 1));
 }
 
 // One block per system: scan padded column counts; col_tmp -> col_count and
 // back to zero.
-__global__ void nl_scan(const SysDev* sd, SysCount* sc, int* col_tmp, int* col_count, int* col_slot,
+__global__ void nl_scan(const SysDev* sd, SysCount* sc, int4* col_tmp, int* col_count, int* col_slot,
                         int* col_super) {
     int s = blockIdx.x;
     if (!sc[s].rebuild) return;
@@ -108,6 +115,7 @@ __global__ void nl_scan(const SysDev* sd, SysCount* sc, int* col_tmp, int* col_c
     // list kernels is cleared before the kernels after this one read the flags
     if (threadIdx.x == 0 && (sc[s].overflow & kStaleList)) sc[s].overflow &= ~kStaleList;
     __shared__ int tot_slot, tot_sup, carry_slot, carry_sup;
+    int crowded = 0;
     __shared__ int ws[1024], wsup[1024];
     if (threadIdx.x == 0) { carry_slot = 0; carry_sup = 0; }
     __syncthreads();
@@ -115,9 +123,11 @@ __global__ void nl_scan(const SysDev* sd, SysCount* sc, int* col_tmp, int* col_c
         int c = base + threadIdx.x;
         int cnt = 0;
         if (c < nc) {
-            cnt = col_tmp[d.col_off + c];
+            const int4 q = col_tmp[d.col_off + c];
+            cnt = q.x + q.y + q.z + q.w;
+            crowded |= max(max(q.x, q.y), max(q.z, q.w)) > kQuarterCap;
             col_count[d.col_off + c] = cnt;
-            col_tmp[d.col_off + c] = 0;
+            col_tmp[d.col_off + c] = make_int4(0, 0, 0, 0);
         }
         int ps = (cnt + 7) & ~7;
         int pu = (cnt + 63) >> 6;
@@ -141,17 +151,18 @@ __global__ void nl_scan(const SysDev* sd, SysCount* sc, int* col_tmp, int* col_c
         if (threadIdx.x == blockDim.x - 1) { carry_slot += ws[threadIdx.x]; carry_sup += wsup[threadIdx.x]; }
         __syncthreads();
     }
+    crowded = __syncthreads_or(crowded);
     if (threadIdx.x == 0) {
         tot_slot = carry_slot;
         tot_sup = carry_sup;
-        int ovf = (tot_slot > d.slot_cap) || (tot_sup > d.super_cap);
+        int ovf = (tot_slot > d.slot_cap) || (tot_sup > d.super_cap) || crowded;
         sc[s].n_slots = ovf ? 0 : tot_slot;
         sc[s].n_clusters = ovf ? 0 : tot_slot / 8;
         sc[s].n_super = ovf ? 0 : tot_sup;
         sc[s].list_count = 0;
         sc[s].emask_count = 0;
         sc[s].n_chunks = 0;
-        if (ovf) sc[s].overflow |= 1;
+        if (ovf) sc[s].overflow |= crowded ? 2 : 1;
     }
 }
 
@@ -160,81 +171,119 @@ __global__ void nl_scatter(const SysDev* sd, SysCount* sc, const int* atom_sys, 
     int a = blockIdx.x * blockDim.x + threadIdx.x;
     if (a >= n_atoms_total) return;
     int s = atom_sys[a];
-    if (!sc[s].rebuild || (sc[s].overflow & 1)) return;
+    if (!sc[s].rebuild || (sc[s].overflow & 3)) return;
     int col = atom_col[a];
     int k = wave_keyed_increment(col_fill, col);
     int slot = col_slot[col] + k;
     if (slot < sd[s].slot_off + sd[s].slot_cap) slot_atom_tmp[slot] = a;
 }
 
-// One block (256 threads) per column: deterministic z order, cluster boxes,
+// Compare-exchange steps j, j / 2, .. 1 of a bitonic merge of one key per lane;
+// `up`: the lane's run ascends.
+__device__ __forceinline__ unsigned long long wave_merge(unsigned long long key, int j, bool up) {
+    const int lane = threadIdx.x & 63;
+    for (; j > 0; j >>= 1) {
+        const unsigned long long o = __shfl_xor(key, j, 64);
+        const bool low = (lane & j) == 0;
+        key = ((key < o) == (low == up)) ? key : o;
+    }
+    return key;
+}
+// Ascending sort of the keys of each group of n lanes (a power of two).
+__device__ __forceinline__ unsigned long long wave_sort(unsigned long long key, int n) {
+    const int lane = threadIdx.x & 63;
+    for (int k = 2; k <= n; k <<= 1) key = wave_merge(key, k >> 1, k == n || (lane & k) == 0);
+    return key;
+}
+// A sort key of a non-negative coordinate (its float bits order like it) and a
+// tie-breaker.
+__device__ __forceinline__ unsigned long long sort_key(double v, unsigned tie) {
+    return ((unsigned long long)__float_as_uint((float)v) << 32) | tie;
+}
+constexpr unsigned long long kSortLast = 0xffffffffull << 32;
+
+// One block per column: deterministic order, cluster and super-cluster boxes,
 // super items, and the slot-order data of the force kernels (pos: x, y, z, q;
 // kPadPos coordinates and q = 0 on padding slots; lj: sigma/2, 2 sqrt(eps)).
+// The z sort runs in LDS down to distance 64 and on the lanes of a wavefront
+// below; the splits of a super-cluster are sorts on its wavefront's lanes.
 template <class P>
-__global__ __launch_bounds__(256) void nl_columns(const SysDev* sd, SysCount* sc, const int* col_sys,
-                                                  const int* col_count, int* col_fill, const int* col_slot,
-                                                  const int* col_super, const int* slot_atom_tmp, const double* X,
-                                                  const double* Y, const double* Z, const double* Q,
-                                                  const double* sig, const double* eps, int* atom_of_slot,
-                                                  int* slot_of_atom, float4* cl_ctr, float4* cl_half,
-                                                  int4* super_item, float4* slot_wpos,
-                                                  typename P::real4* pos, typename P::real2* lj, double* XB,
-                                                  double* YB, double* ZB) {
+__global__ __launch_bounds__(kColThreads) void nl_columns(const SysDev* sd, SysCount* sc, const int* col_sys,
+                                                          const int* col_count, int* col_fill, const int* col_slot,
+                                                          const int* col_super, const int* slot_atom_tmp,
+                                                          const double* X, const double* Y, const double* Z,
+                                                          const double* Q, const double* sig, const double* eps,
+                                                          int* atom_of_slot, int* slot_of_atom, float4* cl_ctr,
+                                                          float4* cl_half, float4* sup_ctr, float4* sup_half,
+                                                          int4* super_item, float4* slot_wpos,
+                                                          typename P::real4* pos, typename P::real2* lj, double* XB,
+                                                          double* YB, double* ZB) {
     using real = typename P::real;
     const int col = blockIdx.x;
     const int s = col_sys[col];
-    if (!sc[s].rebuild || (sc[s].overflow & 1)) return;
+    if (!sc[s].rebuild) return;
     if (threadIdx.x == 0) col_fill[col] = 0;          // the scatter is done: zero for the next build
+    if (sc[s].overflow & 3) return;
     const SysDev& d = sd[s];
     const int cnt = col_count[col];
     const int first = col_slot[col];
-    __shared__ double key[kColSortCap];
-    __shared__ int ids[kColSortCap];
-    if (cnt > kColSortCap) {
-        if (threadIdx.x == 0) atomicOr(&sc[s].overflow, 2);
-        return;
-    }
-    int np2 = 1;
-    while (np2 < cnt) np2 <<= 1;
-    for (int i = threadIdx.x; i < np2; i += blockDim.x) {
-        if (i < cnt) {
-            int a = slot_atom_tmp[first + i];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    extern __shared__ unsigned long long key[];       // kColSortCap
+    int n = 64;
+    while (n < cnt) n <<= 1;
+    // runs of 64, alternating in direction
+    for (int b = wv * 64; b < n; b += kColThreads) {
+        unsigned long long k = kSortLast | 0xffffffffull;
+        if (b + lane < cnt) {
+            const int a = slot_atom_tmp[first + b + lane];
             double w[3];
             wrapped(d, X[a], Y[a], Z[a], w);
-            key[i] = w[2];
-            ids[i] = a;
-        } else {
-            key[i] = 1e300;
-            ids[i] = 0x7fffffff;
+            k = sort_key(w[2], (unsigned)a);
         }
+        for (int m = 2; m < 64; m <<= 1) k = wave_merge(k, m >> 1, (lane & m) == 0);
+        key[b + lane] = wave_merge(k, 32, (b & 64) == 0);
     }
     __syncthreads();
-    // bitonic sort by (z, atom id)
-    for (int k = 2; k <= np2; k <<= 1) {
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int i = threadIdx.x; i < np2; i += blockDim.x) {
-                int l = i ^ j;
-                if (l > i) {
-                    bool up = (i & k) == 0;
-                    bool gt = (key[i] > key[l]) || (key[i] == key[l] && ids[i] > ids[l]);
-                    if (gt == up) {
-                        double tk = key[i]; key[i] = key[l]; key[l] = tk;
-                        int ti = ids[i]; ids[i] = ids[l]; ids[l] = ti;
-                    }
+    for (int k = 128; k <= n; k <<= 1) {
+        for (int j = k >> 1; j >= 64; j >>= 1) {
+            for (int t = tid; t < n / 2; t += kColThreads) {
+                const int i = 2 * t - (t & (j - 1));      // the t-th index with bit j clear
+                const unsigned long long x = key[i], y = key[i + j];
+                if ((x > y) == ((i & k) == 0)) {
+                    key[i] = y;
+                    key[i + j] = x;
                 }
             }
             __syncthreads();
         }
+        for (int b = wv * 64; b < n; b += kColThreads) key[b + lane] = wave_merge(key[b + lane], 32, (b & k) == 0);
+        __syncthreads();
     }
-    const int padded = (cnt + 7) & ~7;
-    for (int i = threadIdx.x; i < padded; i += blockDim.x) {
-        int slot = first + i;
-        if (i < cnt) {
-            const int a = ids[i];
+    // super-clusters: 64 consecutive atoms, one wavefront each
+    const int ncl = (cnt + 7) >> 3, nsup = (cnt + 63) >> 6;
+    for (int u = wv; u < nsup; u += kColThreads / 64) {
+        const int m = min(64, cnt - u * 64);              // its atoms
+        int a = -1;
+        double w[3] = {0, 0, 0};
+        if (lane < m) {
+            a = (int)(unsigned)key[u * 64 + lane];
+            wrapped(d, X[a], Y[a], Z[a], w);
+        }
+        // halves by x, quarters by y, eighths by z; `from`: the lane an atom was on
+        const unsigned long long last = kSortLast | (unsigned)lane;
+        int from = (int)(wave_sort(lane < m ? sort_key(w[0], (unsigned)lane) : last, 64) & 63u);
+        double v = __shfl(w[1], from, 64);
+        from = (int)(wave_sort(from < m ? sort_key(v, (unsigned)from) : kSortLast | (unsigned)from, 32) & 63u);
+        v = __shfl(w[2], from, 64);
+        from = (int)(wave_sort(from < m ? sort_key(v, (unsigned)from) : kSortLast | (unsigned)from, 16) & 63u);
+        a = __shfl(a, from, 64);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) w[k] = __shfl(w[k], from, 64);
+        const int slot = first + u * 64 + lane;
+        // padding sorts last at every level, so the m atoms are on the first m lanes
+        if (lane < m) {
             atom_of_slot[slot] = a;
             slot_of_atom[a] = slot;
-            double w[3];
-            wrapped(d, X[a], Y[a], Z[a], w);
             slot_wpos[slot] = make_float4((float)w[0], (float)w[1], (float)w[2], 1.0f);
             // the build position is the wrapped one; the mixed path's slot
             // positions continue from it until the next build, the FP64 path's
@@ -252,7 +301,7 @@ __global__ __launch_bounds__(256) void nl_columns(const SysDev* sd, SysCount* sc
             XB[a] = w[0];
             YB[a] = w[1];
             ZB[a] = w[2];
-        } else {
+        } else if (lane < ((m + 7) & ~7)) {
             atom_of_slot[slot] = -1;
             const float nan = __int_as_float(0x7fc00000);     // compares false in every distance test
             slot_wpos[slot] = make_float4(nan, nan, nan, 0.f);
@@ -265,42 +314,41 @@ __global__ __launch_bounds__(256) void nl_columns(const SysDev* sd, SysCount* sc
             l.y = 0;
             lj[slot] = l;
         }
-    }
-    // cluster bounding boxes in wrapped coordinates
-    const int ncl = padded >> 3;
-    for (int c = threadIdx.x; c < ncl; c += blockDim.x) {
-        double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-        for (int t = 0; t < 8; ++t) {
-            int i = c * 8 + t;
-            if (i >= cnt) break;
-            int a = ids[i];
-            double w[3];
-            wrapped(d, X[a], Y[a], Z[a], w);
-            for (int k = 0; k < 3; ++k) { lo[k] = fmin(lo[k], w[k]); hi[k] = fmax(hi[k], w[k]); }
+        // bounding boxes in wrapped coordinates
+        float lo[3], hi[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            lo[k] = lane < m ? (float)w[k] : 1e30f;
+            hi[k] = lane < m ? (float)w[k] : -1e30f;
         }
-        int gcl = (first >> 3) + c;
-        float4 ctr, half;
-        ctr.x = (float)(0.5 * (lo[0] + hi[0]));
-        ctr.y = (float)(0.5 * (lo[1] + hi[1]));
-        ctr.z = (float)(0.5 * (lo[2] + hi[2]));
-        ctr.w = 0.f;
-        half.x = (float)(0.5 * (hi[0] - lo[0])) + 1e-5f;
-        half.y = (float)(0.5 * (hi[1] - lo[1])) + 1e-5f;
-        half.z = (float)(0.5 * (hi[2] - lo[2])) + 1e-5f;
-        half.w = 0.f;
-        cl_ctr[gcl] = ctr;
-        cl_half[gcl] = half;
-    }
-    // super-cluster items of this column
-    const int nsup = (cnt + 63) >> 6;
-    const int sup0 = col_super[col];
-    for (int u = threadIdx.x; u < nsup; u += blockDim.x) {
-        int4 it;
-        it.x = (first >> 3) + u * 8;                 // first global cluster
-        it.y = min(8, ncl - u * 8);                  // clusters in the item
-        it.z = 0;
-        it.w = 0;
-        super_item[sup0 + u] = it;
+        for (int o = 1; o < 64; o <<= 1) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                lo[k] = fminf(lo[k], __shfl_xor(lo[k], o, 64));
+                hi[k] = fmaxf(hi[k], __shfl_xor(hi[k], o, 64));
+            }
+            if (o == 4 || o == 32) {
+                float4 ctr, half;
+                ctr.x = 0.5f * (lo[0] + hi[0]);
+                ctr.y = 0.5f * (lo[1] + hi[1]);
+                ctr.z = 0.5f * (lo[2] + hi[2]);
+                ctr.w = 0.f;
+                half.x = 0.5f * (hi[0] - lo[0]) + 1e-5f;
+                half.y = 0.5f * (hi[1] - lo[1]) + 1e-5f;
+                half.z = 0.5f * (hi[2] - lo[2]) + 1e-5f;
+                half.w = 0.f;
+                if (o == 4 && (lane & 7) == 0 && lane < m) {
+                    cl_ctr[slot >> 3] = ctr;
+                    cl_half[slot >> 3] = half;
+                }
+                if (o == 32 && lane == 0) {
+                    sup_ctr[col_super[col] + u] = ctr;
+                    sup_half[col_super[col] + u] = half;
+                }
+            }
+        }
+        if (lane == 0)      // first global cluster, clusters in the item
+            super_item[col_super[col] + u] = make_int4((first >> 3) + u * 8, min(8, ncl - u * 8), 0, 0);
     }
 }
 
@@ -380,11 +428,12 @@ __device__ __forceinline__ int block_excl_scan(int v, int* wsum, int& total) {
 
 // One block of kPlThreads per super-cluster item:
 //   1. the columns of the xy window whose rectangle comes within rlist of the
-//      super-cluster's box, in increasing column order;
-//   2. their clusters as one flat candidate range, one thread per candidate:
-//      cluster box against each i-cluster box, ordered compaction; the
-//      entry's periodic image (tile_image), when one image holds for all of
-//      its tiles, else the per-pair marker;
+//      super-cluster's box, in increasing column order; of their super-clusters,
+//      those whose box does (one thread each, ordered compaction);
+//   2. their clusters, one thread per candidate: cluster box against each
+//      i-cluster box, ordered compaction; the entry's periodic image
+//      (tile_image), when one image holds for all of its tiles, else the
+//      per-pair marker;
 //   3. per entry and i-cluster, the 64 atom pairs at build positions, one
 //      wavefront per entry: a tile is kept only if one of its pairs is within
 //      rlist (both atoms move at most skin/2 before the next build, so every
@@ -392,9 +441,10 @@ __device__ __forceinline__ int block_excl_scan(int v, int* wsum, int& total) {
 //   4. exclusion masks for the kept tiles.
 __global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysCount* sc, const int* super_sys,
                                                           int4* super_item, const int* col_count,
-                                                          const int* col_slot, const float4* cl_ctr,
-                                                          const float4* cl_half, const float4* slot_wpos,
-                                                          const int* atom_of_slot, const int* slot_of_atom,
+                                                          const float4* cl_ctr,
+                                                          const float4* cl_half, const float4* sup_ctr,
+                                                          const float4* sup_half, const int* col_super,
+                                                          const float4* slot_wpos, const int* atom_of_slot, const int* slot_of_atom,
                                                           const int* excl_off, const int* excl_idx, uint2* list,
                                                           unsigned long long* emask, int4* chunks,
                                                           int n_items_total) {
@@ -418,7 +468,7 @@ __global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysC
     __shared__ int n_x, id_base, lbase, cbase;
     __shared__ float4 ic[8], ih[8];
     __shared__ float4 ip[64];                     // i-atom build positions (NaN for padding)
-    __shared__ int w_first[kPlThreads], w_pre[kPlThreads];
+    __shared__ int w_first[kPlThreads], w_pre[kPlThreads], near_s[kPlThreads];
     __shared__ int wsum[kPlThreads / 64];
     if (tid == 0) n_x = 0;
     if (tid < 8) {
@@ -437,14 +487,8 @@ __global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysC
     // atoms until the next build (skin/2 each) and 1e-3 nm for float round-off
     const float img_slack = (float)(d.rlist - d.rc) + 1e-3f;
 
-    // xy box of the super-cluster
-    float xlo = 1e30f, xhi = -1e30f, ylo = 1e30f, yhi = -1e30f;
-    for (int k = 0; k < ncl; ++k) {
-        xlo = fminf(xlo, ic[k].x - ih[k].x); xhi = fmaxf(xhi, ic[k].x + ih[k].x);
-        ylo = fminf(ylo, ic[k].y - ih[k].y); yhi = fmaxf(yhi, ic[k].y + ih[k].y);
-    }
-    const float scx = 0.5f * (xlo + xhi), scy = 0.5f * (ylo + yhi);
-    const float shx = 0.5f * (xhi - xlo), shy = 0.5f * (yhi - ylo);
+    const float4 scc = sup_ctr[item], sch = sup_half[item];
+    const float scx = scc.x, scy = scc.y, shx = sch.x, shy = sch.y;
     const float cwx = (float)d.colw[0], cwy = (float)d.colw[1];
 
     // window of columns around the super-cluster's own column
@@ -461,7 +505,7 @@ __global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysC
     int ne = 0;                                   // entries so far (the same in every thread)
     for (int w0 = 0; w0 < nwin; w0 += kPlThreads) {
         const int w = w0 + tid;
-        int ccl = 0, cfirst = 0;
+        int nsu = 0, sfirst = 0;
         if (w < nwin) {
             const int cx = window_col(w / ny_c, cx0, Dx, d.ncx, nx_c);
             const int cy = window_col(w % ny_c, cy0, Dy, d.ncy, ny_c);
@@ -472,44 +516,61 @@ __global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysC
             gy = fmaxf(0.f, fminf(gy, Ly - gy) - 0.5f * cwy - 1e-3f - shy);
             if (gx * gx + gy * gy < rl2) {
                 const int col = d.col_off + cx * d.ncy + cy;
-                ccl = (col_count[col] + 7) >> 3;
-                cfirst = col_slot[col] >> 3;
+                nsu = (col_count[col] + 63) >> 6;
+                sfirst = col_super[col];
             }
         }
         int total;
-        const int pre = block_excl_scan(ccl, wsum, total);
+        const int pre = block_excl_scan(nsu, wsum, total);
         w_pre[tid] = pre;
-        w_first[tid] = cfirst;
+        w_first[tid] = sfirst;
         __syncthreads();
         for (int b = 0; b < total; b += kPlThreads) {
+            // a super-cluster each, from its own index on (the half list)
             const int t = b + tid;
-            unsigned int im = 0, img = kImgPerPair;
-            int cj = 0;
+            int sj = 0;
+            bool near = false;
             if (t < total) {
                 int lo = 0, hi = kPlThreads - 1;      // last column whose range starts at or before t
                 while (lo < hi) {
                     const int m = (lo + hi + 1) >> 1;
                     if (w_pre[m] <= t) lo = m; else hi = m - 1;
                 }
-                cj = w_first[lo] + (t - w_pre[lo]);
-                const float4 jc = cl_ctr[cj], jh = cl_half[cj];
-                int code = -1;
+                sj = w_first[lo] + (t - w_pre[lo]);
+                near = sj >= item && bbox_gap2(scc, sch, sup_ctr[sj], sup_half[sj], Lx, Ly, Lz) < rl2;
+            }
+            int nnear;
+            const int at = block_excl_scan(near, wsum, nnear);
+            if (near) near_s[at] = sj;
+            __syncthreads();
+            for (int c = 0; c < nnear * 8; c += kPlThreads) {
+                const int u = c + tid;
+                unsigned int im = 0, img = kImgPerPair;
+                int cj = 0;
+                if (u < nnear * 8) {
+                    const int4 js = super_item[near_s[u >> 3]];
+                    cj = js.x + (u & 7);
+                    if ((u & 7) < js.y) {
+                        const float4 jc = cl_ctr[cj], jh = cl_half[cj];
+                        int code = -1;
 #pragma unroll
-                for (int k = 0; k < 8; ++k)
-                    if (k < ncl && cj >= fc + k && bbox_gap2(ic[k], ih[k], jc, jh, Lx, Ly, Lz) < rl2) {
-                        im |= 1u << k;
-                        const int ck = tile_image(ic[k], ih[k], jc, jh, Lx, Ly, Lz, iLx, iLy, iLz, img_slack);
-                        code = (ck < 0 || (code >= 0 && ck != code) || code == kImgMixed) ? kImgMixed : ck;
+                        for (int k = 0; k < 8; ++k)
+                            if (k < ncl && cj >= fc + k && bbox_gap2(ic[k], ih[k], jc, jh, Lx, Ly, Lz) < rl2) {
+                                im |= 1u << k;
+                                const int ck = tile_image(ic[k], ih[k], jc, jh, Lx, Ly, Lz, iLx, iLy, iLz, img_slack);
+                                code = (ck < 0 || (code >= 0 && ck != code) || code == kImgMixed) ? kImgMixed : ck;
+                            }
+                        img = (d.pair_image && code >= 0 && code != kImgMixed) ? image_bits(code) : kImgPerPair;
                     }
-                img = (d.pair_image && code >= 0 && code != kImgMixed) ? image_bits(code) : kImgPerPair;
+                }
+                int cnt;
+                const int pos = ne + block_excl_scan(im != 0, wsum, cnt);
+                if (im && pos < kListCap) {
+                    l_ent[pos] = (unsigned)cj | (im << 24);
+                    l_img[pos] = (unsigned char)img;
+                }
+                ne += cnt;
             }
-            int cnt;
-            const int pos = ne + block_excl_scan(im != 0, wsum, cnt);
-            if (im && pos < kListCap) {
-                l_ent[pos] = (unsigned)cj | (im << 24);
-                l_img[pos] = (unsigned char)img;
-            }
-            ne += cnt;
         }
         __syncthreads();
     }
@@ -635,7 +696,8 @@ __global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysC
             atomicOr(&emask[(size_t)g * 8 + k], 1ull << (x_rec[t] & 63u));
         }
     }
-    const int ce = d.chunk_entries, nch = (ne + ce - 1) / ce;
+    // chunks of at most chunk_entries entries, as equal as they come
+    const int nch = (ne + d.chunk_entries - 1) / d.chunk_entries, ce = nch > 0 ? (ne + nch - 1) / nch : 1;
     if (tid == 0) {
         const int b = atomicAdd(&sc[s].list_count, ne);
         lbase = (b + ne > d.list_cap) ? -1 : b;
@@ -771,15 +833,16 @@ void launch_nlist(Batch<P>& B, bool clear_flags, int part) {
     }
     nl_bin<<<nb(B.n_atoms, T), T, 0, st>>>(B.d_sys, B.d_cnt, B.atom_sys, B.X, B.Y, B.Z, B.atom_col, B.col_tmp,
                                           B.n_atoms);
-    nl_scan<<<B.nsys, 1024, 0, st>>>(B.d_sys, B.d_cnt, B.col_tmp, B.col_count, B.col_slot, B.col_super);
+    nl_scan<<<B.nsys, 1024, 0, st>>>(B.d_sys, B.d_cnt, reinterpret_cast<int4*>(B.col_tmp), B.col_count, B.col_slot, B.col_super);
     nl_scatter<<<nb(B.n_atoms, T), T, 0, st>>>(B.d_sys, B.d_cnt, B.atom_sys, B.atom_col, B.col_slot, B.col_fill,
                                               B.slot_tmp, B.n_atoms);
-    nl_columns<P><<<B.n_cols, 256, 0, st>>>(B.d_sys, B.d_cnt, B.col_sys, B.col_count, B.col_fill, B.col_slot,
+    nl_columns<P><<<B.n_cols, kColThreads, kColSortCap * sizeof(unsigned long long), st>>>(
+                                            B.d_sys, B.d_cnt, B.col_sys, B.col_count, B.col_fill, B.col_slot,
                                             B.col_super, B.slot_tmp, B.X, B.Y, B.Z, B.q, B.sig, B.eps,
-                                            B.atom_of_slot, B.slot_of_atom, B.cl_ctr, B.cl_half, B.super_item,
-                                            B.slot_wpos, B.pos, B.lj, B.XB, B.YB, B.ZB);
-    nl_pairlist<<<B.n_super_cap, kPlThreads, 0, st>>>(B.d_sys, B.d_cnt, B.super_sys, B.super_item, B.col_count, B.col_slot,
-                                              B.cl_ctr, B.cl_half, B.slot_wpos, B.atom_of_slot, B.slot_of_atom, B.excl_off,
+                                            B.atom_of_slot, B.slot_of_atom, B.cl_ctr, B.cl_half, B.sup_ctr, B.sup_half,
+                                            B.super_item, B.slot_wpos, B.pos, B.lj, B.XB, B.YB, B.ZB);
+    nl_pairlist<<<B.n_super_cap, kPlThreads, 0, st>>>(B.d_sys, B.d_cnt, B.super_sys, B.super_item, B.col_count,
+                                              B.cl_ctr, B.cl_half, B.sup_ctr, B.sup_half, B.col_super, B.slot_wpos, B.atom_of_slot, B.slot_of_atom, B.excl_off,
                                               B.excl_idx, B.list, B.emask, B.chunks, B.n_super_cap);
     if (part == 1) return;  // all but the last kernel
     nl_waves<<<1, kPlThreads, 0, st>>>(B.d_sys, B.d_cnt, B.nsys, B.chunk_prefix, B.pair_blocks, nullptr, 0, nullptr,

@@ -44,7 +44,7 @@ struct SysDev {
     double sw_on, sw_inv;        // switching: r_switch, 1/(rc - r_switch); sw_on < 0 = off
     int n_atoms, atom_off;
     int slot_off, slot_cap;
-    int col_off, ncx, ncy, col_cap;   // columns: ncx*ncy
+    int col_off, ncx, ncy, col_cap;   // columns: ncx*ncy, each of 2 x 2 quarters
     int super_off, super_cap;
     int chunk_off, chunk_cap;    // pair-kernel work items (list chunks)
     int chunk_entries;           // pair-list entries per chunk (chunk_entries_for)
@@ -87,9 +87,8 @@ constexpr int kStepMaxSlots = 64;
 
 constexpr int kChunkEntries = 32;       // most pair-list entries per chunk, the pair kernel's unit of work
 // Pair-list entries one super-cluster may hold (the list build keeps them in
-// LDS).  A super-cluster is 64 atoms of one column, about 3.5 nm tall at water
-// density, with ~700-950 j clusters within rlist = 1.1 nm: 1024 was exceeded
-// by a few super-clusters of a 1M-atom water box.
+// LDS).  A super-cluster is 64 atoms, about a 0.9 nm cube at water density, with
+// ~150 j clusters of higher index within rlist = 1.1 nm.
 constexpr int kSuperListCap = 2048;
 constexpr int kPairWaves = 4;           // independent wavefronts per 256-thread pair-kernel block
 // The pair kernel's chunk ranges, one per XCD, 128 bytes apart: the next chunk

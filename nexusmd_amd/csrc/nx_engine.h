@@ -98,8 +98,9 @@ struct Batch {
 
     // columns / clusters / pair list
     int *col_sys = nullptr, *col_count = nullptr, *col_fill = nullptr, *col_slot = nullptr, *col_super = nullptr;
-    int* col_tmp = nullptr;         // bin counts during a build (zero between builds)
-    float4 *cl_ctr = nullptr, *cl_half = nullptr;
+    int* col_tmp = nullptr;         // counts of the columns' quarters during a build (zero between builds)
+    float4 *cl_ctr = nullptr, *cl_half = nullptr;     // cluster boxes at the last build
+    float4 *sup_ctr = nullptr, *sup_half = nullptr;   // super-cluster boxes
     float4* slot_wpos = nullptr;    // build-time wrapped position of each slot, w = 1 (atom) or 0 (padding)
     int* super_sys = nullptr;
     int4* super_item = nullptr;

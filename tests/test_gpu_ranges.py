@@ -95,3 +95,40 @@ def test_line_and_plane_passes_agree(prec, monkeypatch):
     # the inverse transforms differ (one or two real lines at a time), the spread and
     # the forward ones do not: rounding only
     assert rel_rms(out[0], out[1]) <= (1e-13 if prec == L.FP64 else 1e-6)
+
+
+@pytest.mark.parametrize("prec", [L.FP64, L.MIXED])
+@pytest.mark.parametrize("n,box", [(63, (2.0, 2.0, 2.0)), (64, (2.0, 2.0, 2.0)), (65, (2.0, 2.0, 2.0)),
+                                   (777, (2.0, 2.1, 9.0)),      # tall columns
+                                   (777, (9.0, 2.1, 2.0)),      # one column across
+                                   (2500, (2.3, 2.3, 2.3))])    # a dense box: many super-clusters a column
+def test_super_cluster_shapes(n, box, prec):
+    """Columns with no, one, a part of one and many super-clusters; the pair set
+    bit for bit in FP64."""
+    s = _gas(n, box, n + 1, grid=(24, 24, 48))
+    _check(s, prec, "super-clusters", skin=0.1)
+    if prec == L.FP64:
+        ctx = E.Context(s, precision=prec, skin=0.1)
+        got = ctx.neighbor_pairs()
+        ctx.close()
+        want = O.pairs(s, O.exclusions(s), method="brute")
+        assert len(got) == len(want) and set(map(tuple, got.tolist())) == set(map(tuple, want.tolist()))
+
+
+def test_coincident_columns_sort_by_atom():
+    """Atoms with equal coordinates on every axis in turn (ties in every sort of
+    the super-cluster splits) keep a deterministic list: two contexts, one set of bits."""
+    s = _gas(600, (2.2, 2.2, 2.2), 9, grid=(24, 24, 24))
+    s.pos[:200, 0] = 0.7
+    s.pos[150:400, 1] = 1.1
+    s.pos[300:, 2] = 0.4 + 1.4 * (np.arange(300) % 2)
+    s.pos[:, 2] += 1e-3 * np.arange(600)       # no two atoms on one point
+    s.pos %= s.L
+    s.eps[:] = 0.0                              # close contacts: charges alone
+    _check(s, L.FP64, "ties")
+    f = []
+    for _ in range(2):
+        ctx = E.Context(s, precision=L.MIXED)
+        f.append(ctx.compute_forces()[0])
+        ctx.close()
+    np.testing.assert_array_equal(f[0], f[1])
