@@ -457,7 +457,8 @@ class Engine : public EngineBase {
         dalloc(&B.phi, (size_t)B.rgrid_total, o, B.stream);
         dalloc(&B.eta, (size_t)B.cgrid_total, o, B.stream);
         dalloc(&B.twiddle, (size_t)B.tw_total, o, B.stream);
-        dalloc(&B.energy, (size_t)B.nsys * E_NTERMS, o, B.stream);
+        dalloc(&B.energy, (size_t)B.nsys * kEnergySlots * E_NTERMS, o, B.stream);
+        dalloc(&B.energy_total, (size_t)B.nsys * E_NTERMS, o, B.stream);
         dalloc(&d_count_, 1, o, B.stream);
         if (B.n_bonds) { dalloc(&B.bond_idx, B.n_bonds, o, B.stream); dalloc(&B.bond_par, B.n_bonds, o, B.stream); }
         if (B.n_angles) { dalloc(&B.angle_idx, B.n_angles, o, B.stream); dalloc(&B.angle_par, B.n_angles, o, B.stream); }
@@ -903,7 +904,9 @@ class Engine : public EngineBase {
         HIPCHK(hipStreamWaitEvent(B.stream, join_, 0));
     }
 
-    void zero_energy() { HIPCHK(hipMemsetAsync(B.energy, 0, sizeof(long long) * B.nsys * E_NTERMS, B.stream)); }
+    void zero_energy() {
+        HIPCHK(hipMemsetAsync(B.energy, 0, sizeof(long long) * B.nsys * kEnergySlots * E_NTERMS, B.stream));
+    }
 
     void begin_call() {
         evs_.clear();
@@ -1212,7 +1215,7 @@ class Engine : public EngineBase {
 
     void energies_out(int s, int mask, nx_energies* e) {
         std::vector<long long> h(E_NTERMS);
-        copy_sync(h.data(), B.energy + (size_t)s * E_NTERMS, sizeof(long long) * E_NTERMS, hipMemcpyDeviceToHost);
+        copy_sync(h.data(), B.energy_total + (size_t)s * E_NTERMS, sizeof(long long) * E_NTERMS, hipMemcpyDeviceToHost);
         energies_from(h.data(), s, mask, e);
     }
 
@@ -1245,6 +1248,7 @@ class Engine : public EngineBase {
         zero_energy();
         forces(mask, true);
         if (kinetic) launch_kinetic<P>(B, dt);
+        launch_energy_sum<P>(B);
         HIPCHK(hipStreamSynchronize(B.stream));
         if (F) gather_forces(*F);
         if (pos || vel) get_state(pos, vel);
@@ -1299,8 +1303,9 @@ class Engine : public EngineBase {
         zero_energy();
         forces(mask, true);
         launch_kinetic<P>(B, dt);
+        launch_energy_sum<P>(B);
         launch_report_snapshot<P>(B, r.d_stage);
-        HIPCHK(hipMemcpyAsync(r.d_energy, B.energy, ebytes, hipMemcpyDeviceToDevice, B.stream));
+        HIPCHK(hipMemcpyAsync(r.d_energy, B.energy_total, ebytes, hipMemcpyDeviceToDevice, B.stream));
         HIPCHK(hipMemcpyAsync(r.d_cnt, B.d_cnt, cbytes, hipMemcpyDeviceToDevice, B.stream));
         HIPCHK(hipEventRecord(packed_, B.stream));
         HIPCHK(hipStreamWaitEvent(copy_, packed_, 0));

@@ -99,6 +99,23 @@ __global__ void kinetic_kernel(const int* __restrict__ atom_sys, const int* __re
     wave_energy_add(energy, s < 0 ? 0 : s, E_KIN, ke, s >= 0);
 }
 
+// A block per system: thread = (part of the slots, term).
+__global__ __launch_bounds__(64) void energy_sum_kernel(const long long* __restrict__ energy, long long* total) {
+    const int s = blockIdx.x, term = threadIdx.x & (E_NTERMS - 1), part = threadIdx.x / E_NTERMS;
+    static_assert(E_NTERMS == 8, "a wavefront holds 8 parts of 8 terms");
+    long long t = 0;
+    for (int k = part; k < kEnergySlots; k += 64 / E_NTERMS) t += energy[((size_t)s * kEnergySlots + k) * E_NTERMS + term];
+    for (int o = E_NTERMS; o < 64; o <<= 1) t += __shfl_xor(t, o, 64);
+    if (part == 0) total[s * E_NTERMS + term] = t;
+}
+
+template <class P>
+void launch_energy_sum(Batch<P>& B) {
+    energy_sum_kernel<<<B.nsys, 64, 0, B.stream>>>(B.energy, B.energy_total);
+}
+template void launch_energy_sum<PrecFP64>(Batch<PrecFP64>&);
+template void launch_energy_sum<PrecMixed>(Batch<PrecMixed>&);
+
 // The largest squared displacement of the block's atoms, into slot
 // blockIdx % kStepMaxSlots of step_max (one atomic per block, few blocks per
 // slot; every thread calls it).  The next nl_waves launch reads and clears

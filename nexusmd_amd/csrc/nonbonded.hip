@@ -258,6 +258,18 @@ __device__ __forceinline__ void pair_body(const SysDev* __restrict__ sd, const i
         return q;
     };
 
+    int e_sys = -1;
+    long long ec_sum = 0, el_sum = 0;
+    auto flush_energy = [&]() {
+        if (e_sys < 0) return;
+        ec_sum = wave_sum(ec_sum);
+        el_sum = wave_sum(el_sum);
+        if (lane == 0) {
+            energy_add_fixed(energy, e_sys, E_COUL, ec_sum);
+            energy_add_fixed(energy, e_sys, E_LJ, el_sum);
+        }
+        ec_sum = el_sum = 0;
+    };
     // The mixed path prefetches the next chunk across the flush below; the FP64
     // kernel is register-bound and fetches at the top of each chunk.
     int g = __builtin_amdgcn_readfirstlane(counter[kPoolFirst]) + (int)(blockIdx.x >> 3) * kPairWaves + w;
@@ -472,16 +484,17 @@ __device__ __forceinline__ void pair_body(const SysDev* __restrict__ sd, const i
             facc_add(&FZ[slot], jf[2 * 64 + lane]);
         }
         if constexpr (ENERGY) {
-            const long long ec = wave_sum(energy_fixed(ec_acc));
-            const long long el = wave_sum(energy_fixed(el_acc));
-            if (lane == 0) {
-                energy_add_fixed(&energy[s * E_NTERMS + E_COUL], ec);
-                energy_add_fixed(&energy[s * E_NTERMS + E_LJ], el);
-            }
+            // each lane's share of the chunk is rounded; the integers add up over the
+            // wavefront's chunks of one system before they leave it
+            if (s != e_sys) flush_energy();
+            e_sys = s;
+            ec_sum += energy_fixed(ec_acc);
+            el_sum += energy_fixed(el_acc);
         }
         wave_lds_sync();   // LDS of this wave is reused by its next chunk
         g = gn;
     }
+    if constexpr (ENERGY) flush_energy();
 }
 
 #define NX_PAIR_PARAMS(P)                                                                                      \

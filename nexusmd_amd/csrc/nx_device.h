@@ -217,7 +217,12 @@ __device__ __forceinline__ long long energy_fixed(double v) {
     s = fmin(fmax(s, -9.2e18), 9.2e18);
     return __double2ll_rn(s);
 }
-__device__ __forceinline__ void energy_add_fixed(long long* e, long long v) {
+// A system's sums are spread over kEnergySlots copies, by block: a million
+// atoms' terms are 16,000 wavefronts, and that many atomics on one address took
+// 1.8 ms where the kernel needs 30 us.  energy_sum_kernel adds the copies up.
+constexpr int kEnergySlots = 64;
+__device__ __forceinline__ void energy_add_fixed(long long* energy, int s, int term, long long v) {
+    long long* e = energy + ((size_t)s * kEnergySlots + blockIdx.x % kEnergySlots) * E_NTERMS + term;
     atomicAdd(reinterpret_cast<unsigned long long*>(e), static_cast<unsigned long long>(v));
 }
 
@@ -239,8 +244,8 @@ __device__ __forceinline__ long long wave_sum(long long v) {
     return v;
 }
 
-// Block-wide (<=1024 threads) sum of fixed-point energies into slot e (one atomic per block).
-__device__ __forceinline__ void block_energy_add(long long* e, long long v) {
+// Block-wide (<=1024 threads) sum of fixed-point energies into system s's term (one atomic per block).
+__device__ __forceinline__ void block_energy_add(long long* energy, int s, int term, long long v) {
     __shared__ long long part[16];
     v = wave_sum(v);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -250,12 +255,12 @@ __device__ __forceinline__ void block_energy_add(long long* e, long long v) {
         long long t = 0;
         const int nw = (blockDim.x + 63) >> 6;
         for (int i = 0; i < nw; ++i) t += part[i];
-        energy_add_fixed(e, t);
+        energy_add_fixed(energy, s, term, t);
     }
     __syncthreads();
 }
 
-// Adds v of the valid lanes to energy[s * E_NTERMS + term] with one atomic per
+// Adds v of the valid lanes to system s's term with one atomic per
 // wavefront when all valid lanes belong to one system.  Every lane must call it.
 __device__ __forceinline__ void wave_energy_add(long long* energy, int s, int term, double v, bool valid) {
     const unsigned long long m = __ballot(valid);
@@ -265,9 +270,9 @@ __device__ __forceinline__ void wave_energy_add(long long* energy, int s, int te
     const int s0 = __shfl(s, lead, 64);
     if (__all(!valid || s == s0)) {
         const long long t = wave_sum(q);
-        if ((int)(threadIdx.x & 63) == lead) energy_add_fixed(&energy[s0 * E_NTERMS + term], t);
+        if ((int)(threadIdx.x & 63) == lead) energy_add_fixed(energy, s0, term, t);
     } else if (valid) {
-        energy_add_fixed(&energy[s * E_NTERMS + term], q);
+        energy_add_fixed(energy, s, term, q);
     }
 }
 

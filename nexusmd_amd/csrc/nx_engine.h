@@ -157,8 +157,8 @@ struct Batch {
     size_t fft_spread_lds = 0, fft_plane_lds = 0, fft_x_lds = 0;
     int pme_any = 0;
 
-    // energies [nsys][E_NTERMS] in 2^30 fixed point
-    long long* energy = nullptr;
+    // energies in 2^30 fixed point: the kernels' sums [nsys][kEnergySlots][E_NTERMS], their totals [nsys][E_NTERMS]
+    long long *energy = nullptr, *energy_total = nullptr;
 
     // flags
     int timing = 0;                 // NX_TIMING_* mode
@@ -184,6 +184,7 @@ template <class P> void launch_fft_forward(Batch<P>& B);
 template <class P> void launch_fft_convolve(Batch<P>& B, bool energy);
 template <class P> void launch_fft_inverse(Batch<P>& B);
 template <class P> void launch_pme_gather(Batch<P>& B);
+template <class P> void launch_energy_sum(Batch<P>& B);     // energy -> energy_total
 template <class P> void launch_kinetic(Batch<P>& B, double dt);
 template <class P> void launch_integrate(Batch<P>& B, double dt);
 template <class P> void launch_collect_forces(Batch<P>& B, double* FX, double* FY, double* FZ);

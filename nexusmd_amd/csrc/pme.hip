@@ -708,7 +708,7 @@ __global__ __launch_bounds__(256) void fft_x_conv(const SysDev* __restrict__ sd,
         const int x = qdiv(i, inv_nt), t = i - x * nt;
         c[x * sx + t] = res2[t * Kx + x];
     }
-    if constexpr (ENERGY) block_energy_add(&energy[s * E_NTERMS + E_RECIP], e);
+    if constexpr (ENERGY) block_energy_add(energy, s, E_RECIP, e);
 }
 
 // Plain X pass (no convolution) for the standalone transform.
@@ -953,7 +953,7 @@ __global__ __launch_bounds__(kPlaneThreads) void fft_x_block(const SysDev* __res
         }
         __syncthreads();
         R = fft_lines_lds<real, R2>(R, R == A ? Bf : A, Kx, nk, 1, nk, TW, +1);
-        if constexpr (MODE == 3) block_energy_add(&energy[s * E_NTERMS + E_RECIP], e);
+        if constexpr (MODE == 3) block_energy_add(energy, s, E_RECIP, e);
     }
     for (int i = threadIdx.x; i < Kx * nk; i += blockDim.x) {
         const int x = qdiv(i, inv_nk), t = i - x * nk;
