@@ -124,8 +124,20 @@ void copy_topology(nx::HostSystem& h, const nx_topology* t) {
 }
 
 void check_positions(int n, const double* p) {
-    for (int i = 0; i < 3 * n; ++i)
-        if (!std::isfinite(p[i])) throw ArgError("non-finite position or velocity component " + std::to_string(i));
+    // a block at a time by the exponents' bits, which the compiler can do several of at once
+    const size_t total = 3 * (size_t)n;
+    for (size_t b = 0; b < total; b += 4096) {
+        const size_t e = std::min(total, b + 4096);
+        uint64_t bad = 0;
+        for (size_t i = b; i < e; ++i) {
+            uint64_t u;
+            std::memcpy(&u, p + i, sizeof(u));
+            bad |= (u & 0x7ff0000000000000ull) == 0x7ff0000000000000ull;
+        }
+        if (!bad) continue;
+        for (size_t i = b; i < e; ++i)
+            if (!std::isfinite(p[i])) throw ArgError("non-finite position or velocity component " + std::to_string(i));
+    }
 }
 
 // After a list overflow inside a call the device froze the system at the last
@@ -164,6 +176,15 @@ void ensure(nx_ctx* c) {
 }
 
 }  // namespace
+
+std::string nx::topology_error(const nx_topology* t) {
+    try {
+        check_topology(t);
+        return std::string();
+    } catch (const ArgError& e) {
+        return e.what();
+    }
+}
 
 extern "C" {
 
@@ -314,15 +335,8 @@ nx_status nx_get_state(nx_ctx* c, double* pos, double* vel, double* forces) {
             return;
         }
         ensure(c);
-        std::vector<double> p, v;
-        c->eng->get_state(pos ? &p : nullptr, vel ? &v : nullptr);
-        if (pos) std::memcpy(pos, p.data(), p.size() * sizeof(double));
-        if (vel) std::memcpy(vel, v.data(), v.size() * sizeof(double));
-        if (forces) {
-            std::vector<double> F;
-            c->eng->compute(NX_FORCE_ALL, false, 0.0, false, &F, nullptr, nullptr, nullptr);
-            std::memcpy(forces, F.data(), F.size() * sizeof(double));
-        }
+        c->eng->get_state(pos, vel);
+        if (forces) c->eng->compute(NX_FORCE_ALL, false, 0.0, false, forces, nullptr, nullptr, nullptr);
     });
 }
 
@@ -330,10 +344,8 @@ nx_status nx_compute_forces(nx_ctx* c, int mask, double* forces, nx_energies* e)
     return guarded(c, [&] {
         if (mask & ~NX_FORCE_ALL) throw ArgError("unknown force bits");
         ensure(c);
-        std::vector<double> F;
         std::vector<nx_energies> E;
-        with_capacity_recovery(c, [&] { c->eng->compute(mask, true, 0.0, false, forces ? &F : nullptr, nullptr, nullptr, &E); });
-        if (forces) std::memcpy(forces, F.data(), F.size() * sizeof(double));
+        with_capacity_recovery(c, [&] { c->eng->compute(mask, true, 0.0, false, forces, nullptr, nullptr, &E); });
         if (e) *e = E[0];
         if (e && !std::isfinite(e->potential)) throw std::runtime_error("non-finite energy");
     });
@@ -353,14 +365,8 @@ nx_status nx_step_report(nx_ctx* c, double dt, int mask, double* pos, double* ve
         if (!(dt > 0) || !std::isfinite(dt)) throw ArgError("dt > 0 required");
         if (mask & ~NX_FORCE_ALL) throw ArgError("unknown force bits");
         ensure(c);
-        std::vector<double> F, p, v;
         std::vector<nx_energies> E;
-        with_capacity_recovery(c, [&] {
-            c->eng->compute(mask, true, dt, true, forces ? &F : nullptr, pos ? &p : nullptr, vel ? &v : nullptr, &E);
-        });
-        if (forces) std::memcpy(forces, F.data(), F.size() * sizeof(double));
-        if (pos) std::memcpy(pos, p.data(), p.size() * sizeof(double));
-        if (vel) std::memcpy(vel, v.data(), v.size() * sizeof(double));
+        with_capacity_recovery(c, [&] { c->eng->compute(mask, true, dt, true, forces, pos, vel, &E); });
         if (e) *e = E[0];
     });
 }

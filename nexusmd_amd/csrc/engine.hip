@@ -15,6 +15,7 @@
 #include <mutex>
 #include <stdexcept>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/nexusmd.h"
@@ -50,18 +51,47 @@ static void upload(T* d, const std::vector<T>& h, hipStream_t st) {
     if (!h.empty()) HIPCHK(hipMemcpyAsync(d, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice, st));
 }
 
+// Copy between caller memory and pinned staging.  Large copies go over several
+// threads: a caller's fresh array is touched for the first time here, and its
+// page faults are most of the time (72 MB into fresh memory: 15 ms on one thread,
+// 5 on four, 3.7 on eight; starting a thread costs ~20 us).
+static void copy_host(void* dst, const void* src, size_t bytes) {
+    const int nt = bytes >= (16u << 20) ? 8 : (bytes >= (1u << 20) ? 4 : 1);
+    std::vector<std::thread> pool;
+    size_t at = 0;
+    try {
+        for (int t = 0; t + 1 < nt; ++t) {
+            const size_t len = bytes / nt;
+            pool.emplace_back([=] { std::memcpy((char*)dst + at, (const char*)src + at, len); });
+            at += len;
+        }
+    } catch (const std::exception&) {      // no thread to be had: the rest is copied here
+    }
+    std::memcpy((char*)dst + at, (const char*)src + at, bytes - at);
+    for (auto& t : pool) t.join();
+}
+
 // ------------------------------------------------------------- host setup
 
 // 1-2, 1-3 and 1-4 partners (graph distance <= 3 over the bond graph), the
 // set Exclusions::createExclusions builds with bondCutoff = 3
 // (core/baseline/src/Forces/Exclusions.cpp:7-44).
 void exclusions_from_bonds(int n, const std::vector<nx_bond>& bonds, std::vector<int>& off, std::vector<int>& idx) {
-    std::vector<std::vector<int>> adj(n);
+    // partners of each atom, in the order of the bonds
+    std::vector<int> first(n + 1, 0), adj(2 * bonds.size());
     for (const auto& b : bonds) {
         if (b.p1 < 0 || b.p2 < 0 || b.p1 >= n || b.p2 >= n)
             throw HipError(NX_ERR_ARG, "createExclusions: Illegal particle index in list of bonds");
-        adj[b.p1].push_back(b.p2);
-        adj[b.p2].push_back(b.p1);
+        ++first[b.p1 + 1];
+        ++first[b.p2 + 1];
+    }
+    for (int i = 0; i < n; ++i) first[i + 1] += first[i];
+    {
+        std::vector<int> at(first.begin(), first.end() - 1);
+        for (const auto& b : bonds) {
+            adj[at[b.p1]++] = b.p2;
+            adj[at[b.p2]++] = b.p1;
+        }
     }
     off.assign(n + 1, 0);
     idx.clear();
@@ -73,12 +103,14 @@ void exclusions_from_bonds(int n, const std::vector<nx_bond>& bonds, std::vector
         for (int depth = 0; depth < 3; ++depth) {
             nxt.clear();
             for (int u : frontier)
-                for (int v : adj[u])
+                for (int e = first[u]; e < first[u + 1]; ++e) {
+                    const int v = adj[e];
                     if (mark[v] != i) {
                         mark[v] = i;
                         nxt.push_back(v);
                         found.push_back(v);
                     }
+                }
             frontier.swap(nxt);
         }
         std::sort(found.begin(), found.end());
@@ -251,14 +283,21 @@ class Engine : public EngineBase {
         for (auto& e : step_ev_) hipEventDestroy(e);
         if (copy_) hipStreamDestroy(copy_);
         if (packed_) hipEventDestroy(packed_);
+        if (staged_) hipEventDestroy(staged_);
     }
 
     void release() {
+        if (B.stream) hipStreamSynchronize(B.stream);      // a state may still be on its way in
         free_reports();
         destroy_graphs();
         destroy_segments();
         for (void* p : owned_) hipFree(p);
         owned_.clear();
+        for (Staging* b : {&in_, &out_}) {
+            if (b->host) hipHostFree(b->host);
+            if (b->dev) hipFree(b->dev);
+            *b = Staging{};
+        }
         Batch<P> fresh;
         fresh.stream = B.stream;
         fresh.timing = B.timing;
@@ -458,7 +497,6 @@ class Engine : public EngineBase {
         dalloc(&B.eta, (size_t)B.cgrid_total, o, B.stream);
         dalloc(&B.twiddle, (size_t)B.tw_total, o, B.stream);
         dalloc(&B.energy, (size_t)B.nsys * kEnergySlots * E_NTERMS, o, B.stream);
-        dalloc(&B.energy_total, (size_t)B.nsys * E_NTERMS, o, B.stream);
         dalloc(&d_count_, 1, o, B.stream);
         if (B.n_bonds) { dalloc(&B.bond_idx, B.n_bonds, o, B.stream); dalloc(&B.bond_par, B.n_bonds, o, B.stream); }
         if (B.n_angles) { dalloc(&B.angle_idx, B.n_angles, o, B.stream); dalloc(&B.angle_par, B.n_angles, o, B.stream); }
@@ -557,22 +595,25 @@ class Engine : public EngineBase {
             const double factor = kPi * kPi / (d.alpha * d.alpha);
             const double boxfactor = kPi * d.L[0] * d.L[1] * d.L[2];
             const int mkx = (Kx + 1) / 2, mky = (Ky + 1) / 2, mkz = (Kz + 1) / 2;
+            // exp(-factor m^2) as the product of its axes' factors: Kx + Ky + Kz
+            // exponentials instead of one per point
+            const int Kn[3] = {Kx, Ky, Kzh}, half[3] = {mkx, mky, mkz}, Kf[3] = {Kx, Ky, Kz};
+            std::vector<double> mh2[3], ex[3];
+            for (int c = 0; c < 3; ++c)
+                for (int k = 0; k < Kn[c]; ++k) {
+                    const double mh = ((k < half[c]) ? k : (k - Kf[c])) * d.invL[c];
+                    mh2[c].push_back(mh * mh);
+                    ex[c].push_back(exp(-factor * (mh * mh)));
+                }
             for (int kx = 0; kx < Kx; ++kx) {
-                const double mx = (kx < mkx) ? kx : (kx - Kx);
-                const double mhx = mx * d.invL[0];
                 const double bx = boxfactor * mod[0][kx];
                 for (int ky = 0; ky < Ky; ++ky) {
-                    const double my = (ky < mky) ? ky : (ky - Ky);
-                    const double mhy = my * d.invL[1];
                     const double by = mod[1][ky];
+                    const double m2xy = mh2[0][kx] + mh2[1][ky], exy = kOne4PiEps0 * (ex[0][kx] * ex[1][ky]);
                     for (int kz = 0; kz < Kzh; ++kz) {
                         if (kx == 0 && ky == 0 && kz == 0) { eta.push_back((real)0); continue; }
-                        const double mz = (kz < mkz) ? kz : (kz - Kz);
-                        const double mhz = mz * d.invL[2];
-                        const double m2 = mhx * mhx + mhy * mhy + mhz * mhz;
-                        const double bz = mod[2][kz];
-                        const double denom = m2 * bx * by * bz;
-                        eta.push_back((real)(kOne4PiEps0 * exp(-factor * m2) / denom));
+                        const double denom = (m2xy + mh2[2][kz]) * bx * by * mod[2][kz];
+                        eta.push_back((real)(exy * ex[2][kz] / denom));
                     }
                 }
             }
@@ -760,12 +801,33 @@ class Engine : public EngineBase {
         HIPCHK(hipStreamSynchronize(B.stream));
     }
 
+    // Pinned host memory and its device counterpart, for state in and results out
+    // (a copy from or to pageable memory costs 40 us at 75 KB and 800 at 2.4 MB,
+    // where a pinned one takes 10 and 50).  They grow to the largest use and go with
+    // the layout.
+    struct Staging {
+        char *host = nullptr, *dev = nullptr;
+        size_t cap = 0;
+    };
+    void stage(Staging& b, size_t bytes) {
+        if (bytes <= b.cap) return;
+        HIPCHK(hipStreamSynchronize(B.stream));
+        if (b.host) HIPCHK(hipHostFree(b.host));
+        if (b.dev) HIPCHK(hipFree(b.dev));
+        b = Staging{};
+        HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&b.host), bytes, hipHostMallocDefault));
+        HIPCHK(hipMalloc(reinterpret_cast<void**>(&b.dev), bytes));
+        b.cap = bytes;
+    }
+    // device -> host of the first `bytes` of the output staging, complete at return
+    void fetch(size_t bytes) {
+        HIPCHK(hipMemcpyAsync(out_.host, out_.dev, bytes, hipMemcpyDeviceToHost, B.stream));
+        HIPCHK(hipStreamSynchronize(B.stream));
+    }
+
     void request_rebuild() {
-        std::vector<SysCount> c(B.nsys);
-        copy_sync(c.data(), B.d_cnt, sizeof(SysCount) * B.nsys, hipMemcpyDeviceToHost);
-        for (auto& v : c) { v.rebuild = 1; v.overflow = 0; }
         force_full_ = true;
-        copy_sync(B.d_cnt, c.data(), sizeof(SysCount) * B.nsys, hipMemcpyHostToDevice);
+        launch_set_state<P>(B, nullptr, nullptr);
     }
 
     // ---------------------------------------------------------------- steps
@@ -928,6 +990,9 @@ class Engine : public EngineBase {
     void check_counters() {
         std::vector<SysCount> c(B.nsys);
         copy_sync(c.data(), B.d_cnt, sizeof(SysCount) * B.nsys, hipMemcpyDeviceToHost);
+        check_counts(std::move(c));
+    }
+    void check_counts(std::vector<SysCount> c) {
         counts_ = c;
         failed_sys_.clear();
         for (int s = 0; s < B.nsys; ++s)
@@ -1213,12 +1278,6 @@ class Engine : public EngineBase {
         }
     }
 
-    void energies_out(int s, int mask, nx_energies* e) {
-        std::vector<long long> h(E_NTERMS);
-        copy_sync(h.data(), B.energy_total + (size_t)s * E_NTERMS, sizeof(long long) * E_NTERMS, hipMemcpyDeviceToHost);
-        energies_from(h.data(), s, mask, e);
-    }
-
     // system s's energies from its E_NTERMS fixed-point sums h
     void energies_from(const long long* h, int s, int mask, nx_energies* e) {
         auto v = [&](int t) { return (double)h[t] / kEnergyScale; };
@@ -1241,28 +1300,51 @@ class Engine : public EngineBase {
         }
     }
 
-    // Forces + energies at the current positions; optionally kinetic energy and integrate.
-    void compute(int mask, bool kinetic, double dt, bool integrate, std::vector<double>* F,
-                 std::vector<double>* pos, std::vector<double>* vel, std::vector<nx_energies>* E) override {
+    // Forces + energies at the current positions; optionally kinetic energy and
+    // integrate.  Everything asked for comes back in one copy: the energy totals and
+    // counters, then the blocks [n][3].  Nothing is written on a failure.
+    void compute(int mask, bool kinetic, double dt, bool integrate, double* F, double* pos, double* vel,
+                 std::vector<nx_energies>* E) override {
         begin_call();
         zero_energy();
         forces(mask, true);
         if (kinetic) launch_kinetic<P>(B, dt);
-        launch_energy_sum<P>(B);
-        HIPCHK(hipStreamSynchronize(B.stream));
-        if (F) gather_forces(*F);
-        if (pos || vel) get_state(pos, vel);
-        if (E) {
-            E->resize(B.nsys);
-            for (int s = 0; s < B.nsys; ++s) energies_out(s, mask, &(*E)[s]);
-        }
+        const size_t block = 3 * (size_t)B.n_atoms * sizeof(double);
+        const size_t c_off = sizeof(long long) * B.nsys * E_NTERMS;
+        const size_t head = (c_off + sizeof(SysCount) * B.nsys + 255) & ~(size_t)255;
+        stage(out_, head + 3 * block);
+        double* dst[3] = {pos, vel, F};
+        double* dev[3] = {};
+        size_t bytes = head;
+        for (int b = 0; b < 3; ++b)
+            if (dst[b]) {
+                dev[b] = reinterpret_cast<double*>(out_.dev + bytes);
+                bytes += block;
+            }
+        if (bytes > head) launch_report_snapshot<P>(B, dev[0], dev[1], dev[2], 0, B.n_atoms);
         if (integrate) {
             timed("integrate", [&] { launch_integrate<P>(B, dt); });
             ++steps_;
         } else {
             pack_needed_ = true;          // the slot forces still hold this evaluation
         }
-        end_call();
+        launch_energy_sum<P>(B, reinterpret_cast<long long*>(out_.dev), reinterpret_cast<SysCount*>(out_.dev + c_off));
+        fetch(bytes);
+        HIPCHK(hipGetLastError());
+        harvest();
+        const SysCount* c = reinterpret_cast<const SysCount*>(out_.host + c_off);
+        check_counts(std::vector<SysCount>(c, c + B.nsys));
+        if (E) {
+            const long long* h = reinterpret_cast<const long long*>(out_.host);
+            E->resize(B.nsys);
+            for (int s = 0; s < B.nsys; ++s) energies_from(h + (size_t)s * E_NTERMS, s, mask, &(*E)[s]);
+        }
+        bytes = head;
+        for (int b = 0; b < 3; ++b)
+            if (dst[b]) {
+                copy_host(dst[b], out_.host + bytes, block);
+                bytes += block;
+            }
     }
 
     // ------------------------------------------------------ async reports
@@ -1303,10 +1385,8 @@ class Engine : public EngineBase {
         zero_energy();
         forces(mask, true);
         launch_kinetic<P>(B, dt);
-        launch_energy_sum<P>(B);
-        launch_report_snapshot<P>(B, r.d_stage);
-        HIPCHK(hipMemcpyAsync(r.d_energy, B.energy_total, ebytes, hipMemcpyDeviceToDevice, B.stream));
-        HIPCHK(hipMemcpyAsync(r.d_cnt, B.d_cnt, cbytes, hipMemcpyDeviceToDevice, B.stream));
+        launch_energy_sum<P>(B, r.d_energy, r.d_cnt);
+        launch_report_snapshot<P>(B, r.d_stage, r.d_stage + 3 * n, r.d_stage + 6 * n, 0, B.n_atoms);
         HIPCHK(hipEventRecord(packed_, B.stream));
         HIPCHK(hipStreamWaitEvent(copy_, packed_, 0));
         double* dst[3] = {pos, vel, F};
@@ -1369,56 +1449,32 @@ class Engine : public EngineBase {
         }
     }
 
-    void gather_forces(std::vector<double>& F) {
-        double* d;
-        HIPCHK(hipMallocAsync(reinterpret_cast<void**>(&d), sizeof(double) * 3 * (size_t)B.n_atoms, B.stream));
-        launch_collect_forces<P>(B, d, d + B.n_atoms, d + 2 * (size_t)B.n_atoms);
-        std::vector<double> h(3 * (size_t)B.n_atoms);
-        HIPCHK(hipMemcpyAsync(h.data(), d, h.size() * sizeof(double), hipMemcpyDeviceToHost, B.stream));
-        HIPCHK(hipFreeAsync(d, B.stream));
-        HIPCHK(hipStreamSynchronize(B.stream));
-        F.resize(3 * (size_t)B.n_atoms);
-        for (int a = 0; a < B.n_atoms; ++a)
-            for (int k = 0; k < 3; ++k) F[3 * (size_t)a + k] = h[(size_t)k * B.n_atoms + a];
+    // positions and velocities (each may be NULL) of n atoms from a0 on
+    void read_state(int a0, int n, double* pos, double* vel) {
+        const size_t block = 3 * (size_t)n * sizeof(double);
+        if (!pos && !vel) return;
+        stage(out_, 2 * block);
+        double* dv = reinterpret_cast<double*>(out_.dev + (pos ? block : 0));
+        launch_report_snapshot<P>(B, pos ? reinterpret_cast<double*>(out_.dev) : nullptr, vel ? dv : nullptr, nullptr, a0, n);
+        fetch((pos ? block : 0) + (vel ? block : 0));
+        if (pos) copy_host(pos, out_.host, block);
+        if (vel) copy_host(vel, out_.host + (pos ? block : 0), block);
     }
-
-    void get_state(std::vector<double>* pos, std::vector<double>* vel) override {
-        const size_t n = B.n_atoms;
-        std::vector<double> h(3 * n);
-        if (pos) {
-            HIPCHK(hipMemcpyAsync(h.data(), B.X, n * 8, hipMemcpyDeviceToHost, B.stream));
-            HIPCHK(hipMemcpyAsync(h.data() + n, B.Y, n * 8, hipMemcpyDeviceToHost, B.stream));
-            HIPCHK(hipMemcpyAsync(h.data() + 2 * n, B.Z, n * 8, hipMemcpyDeviceToHost, B.stream));
-            HIPCHK(hipStreamSynchronize(B.stream));
-            pos->resize(3 * n);
-            for (size_t a = 0; a < n; ++a)
-                for (int k = 0; k < 3; ++k) (*pos)[3 * a + k] = h[k * n + a];
-        }
-        if (vel) {
-            HIPCHK(hipMemcpyAsync(h.data(), B.VX, n * 8, hipMemcpyDeviceToHost, B.stream));
-            HIPCHK(hipMemcpyAsync(h.data() + n, B.VY, n * 8, hipMemcpyDeviceToHost, B.stream));
-            HIPCHK(hipMemcpyAsync(h.data() + 2 * n, B.VZ, n * 8, hipMemcpyDeviceToHost, B.stream));
-            HIPCHK(hipStreamSynchronize(B.stream));
-            vel->resize(3 * n);
-            for (size_t a = 0; a < n; ++a)
-                for (int k = 0; k < 3; ++k) (*vel)[3 * a + k] = h[k * n + a];
-        }
-    }
+    void get_state(double* pos, double* vel) override { read_state(0, B.n_atoms, pos, vel); }
 
     void set_state(const double* pos, const double* vel) override {
-        const size_t n = B.n_atoms;
-        std::vector<double> h(3 * n);
-        for (int k = 0; k < 3; ++k)
-            for (size_t a = 0; a < n; ++a) h[k * n + a] = pos[3 * a + k];
-        copy_sync(B.X, h.data(), n * 8, hipMemcpyHostToDevice);
-        copy_sync(B.Y, h.data() + n, n * 8, hipMemcpyHostToDevice);
-        copy_sync(B.Z, h.data() + 2 * n, n * 8, hipMemcpyHostToDevice);
-        for (int k = 0; k < 3; ++k)
-            for (size_t a = 0; a < n; ++a) h[k * n + a] = vel ? vel[3 * a + k] : 0.0;
-        copy_sync(B.VX, h.data(), n * 8, hipMemcpyHostToDevice);
-        copy_sync(B.VY, h.data() + n, n * 8, hipMemcpyHostToDevice);
-        copy_sync(B.VZ, h.data() + 2 * n, n * 8, hipMemcpyHostToDevice);
-        request_rebuild();
+        const size_t block = 3 * (size_t)B.n_atoms * sizeof(double);
+        // the staging may still feed the call before this one
+        if (!staged_) HIPCHK(hipEventCreateWithFlags(&staged_, hipEventDisableTiming));
+        else HIPCHK(hipEventSynchronize(staged_));
+        stage(in_, 2 * block);
+        copy_host(in_.host, pos, block);
+        if (vel) copy_host(in_.host + block, vel, block);
+        HIPCHK(hipMemcpyAsync(in_.dev, in_.host, vel ? 2 * block : block, hipMemcpyHostToDevice, B.stream));
+        HIPCHK(hipEventRecord(staged_, B.stream));
+        force_full_ = true;
+        launch_set_state<P>(B, reinterpret_cast<const double*>(in_.dev),
+                            vel ? reinterpret_cast<const double*>(in_.dev + block) : nullptr);
     }
 
     long long export_pairs(std::vector<int>* out) override {
@@ -1583,30 +1639,22 @@ class Engine : public EngineBase {
     const std::vector<SysCount>& counters() const override { return counts_; }
     hipStream_t stream() const override { return B.stream; }
     void device_state(int s, double* pos, double* vel) override {
-        const SysDev& d = B.sys[s];
-        const size_t n = d.n_atoms, o = d.atom_off;
-        std::vector<double> h(n);
-        double* dst[6] = {pos, pos, pos, vel, vel, vel};
-        double* src[6] = {B.X, B.Y, B.Z, B.VX, B.VY, B.VZ};
-        for (int k = 0; k < 6; ++k) {
-            if (!dst[k]) continue;
-            HIPCHK(hipMemcpyAsync(h.data(), src[k] + o, n * 8, hipMemcpyDeviceToHost, B.stream));
-            HIPCHK(hipStreamSynchronize(B.stream));
-            for (size_t a = 0; a < n; ++a) dst[k][3 * a + (k % 3)] = h[a];
-        }
+        read_state(B.sys[s].atom_off, B.sys[s].n_atoms, pos, vel);
     }
     void device_list_state(int s, double* build_pos, int* rebuild_due) override {
         const SysDev& d = B.sys[s];
         const size_t n = d.n_atoms, o = d.atom_off;
-        std::vector<double> h(n);
+        stage(out_, 3 * n * sizeof(double) + sizeof(SysCount));
         const double* src[3] = {B.XB, B.YB, B.ZB};
-        for (int k = 0; k < 3; ++k) {
-            copy_sync(h.data(), src[k] + o, n * 8, hipMemcpyDeviceToHost);
-            for (size_t a = 0; a < n; ++a) build_pos[3 * a + k] = h[a];
-        }
-        SysCount c;
-        copy_sync(&c, B.d_cnt + s, sizeof(SysCount), hipMemcpyDeviceToHost);
-        *rebuild_due = c.rebuild;
+        double* h = reinterpret_cast<double*>(out_.host);
+        SysCount* c = reinterpret_cast<SysCount*>(h + 3 * n);
+        for (int k = 0; k < 3; ++k)
+            HIPCHK(hipMemcpyAsync(h + k * n, src[k] + o, n * 8, hipMemcpyDeviceToHost, B.stream));
+        HIPCHK(hipMemcpyAsync(c, B.d_cnt + s, sizeof(SysCount), hipMemcpyDeviceToHost, B.stream));
+        HIPCHK(hipStreamSynchronize(B.stream));
+        for (int k = 0; k < 3; ++k)
+            for (size_t a = 0; a < n; ++a) build_pos[3 * a + k] = h[k * n + a];
+        *rebuild_due = c->rebuild;
     }
     size_t bytes() const override { return footprint_bytes(B); }
     static size_t footprint_bytes(const Batch<P>& b) {
@@ -1643,6 +1691,8 @@ class Engine : public EngineBase {
     ReportSlot rs_[kReportSlots];
     hipStream_t copy_ = nullptr;
     hipEvent_t packed_ = nullptr;
+    Staging in_, out_;
+    hipEvent_t staged_ = nullptr;           // the input staging has been read
     long long next_ticket_ = 1;
     size_t ev_used_ = 0;
     std::vector<Ev> evs_;

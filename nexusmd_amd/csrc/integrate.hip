@@ -7,6 +7,8 @@
 // (core/baseline/src/KineticEnergy.cpp:21-41).  Positions and velocities stay
 // FP64 in both precision paths; the mixed path converts its fixed-point
 // force sums to FP64 here.
+#include <algorithm>
+
 #include "nx_device.h"
 #include "nx_engine.h"
 
@@ -99,22 +101,25 @@ __global__ void kinetic_kernel(const int* __restrict__ atom_sys, const int* __re
     wave_energy_add(energy, s < 0 ? 0 : s, E_KIN, ke, s >= 0);
 }
 
-// A block per system: thread = (part of the slots, term).
-__global__ __launch_bounds__(64) void energy_sum_kernel(const long long* __restrict__ energy, long long* total) {
+// A block per system: thread = (part of the slots, term).  With `counts` given,
+// the system's counters go there too.
+__global__ __launch_bounds__(64) void energy_sum_kernel(const long long* __restrict__ energy, long long* total,
+                                                        const SysCount* sc, SysCount* counts) {
     const int s = blockIdx.x, term = threadIdx.x & (E_NTERMS - 1), part = threadIdx.x / E_NTERMS;
     static_assert(E_NTERMS == 8, "a wavefront holds 8 parts of 8 terms");
     long long t = 0;
     for (int k = part; k < kEnergySlots; k += 64 / E_NTERMS) t += energy[((size_t)s * kEnergySlots + k) * E_NTERMS + term];
     for (int o = E_NTERMS; o < 64; o <<= 1) t += __shfl_xor(t, o, 64);
     if (part == 0) total[s * E_NTERMS + term] = t;
+    if (counts && threadIdx.x == 0) counts[s] = sc[s];
 }
 
 template <class P>
-void launch_energy_sum(Batch<P>& B) {
-    energy_sum_kernel<<<B.nsys, 64, 0, B.stream>>>(B.energy, B.energy_total);
+void launch_energy_sum(Batch<P>& B, long long* total, SysCount* counts) {
+    energy_sum_kernel<<<B.nsys, 64, 0, B.stream>>>(B.energy, total, B.d_cnt, counts);
 }
-template void launch_energy_sum<PrecFP64>(Batch<PrecFP64>&);
-template void launch_energy_sum<PrecMixed>(Batch<PrecMixed>&);
+template void launch_energy_sum<PrecFP64>(Batch<PrecFP64>&, long long*, SysCount*);
+template void launch_energy_sum<PrecMixed>(Batch<PrecMixed>&, long long*, SysCount*);
 
 // The largest squared displacement of the block's atoms, into slot
 // blockIdx % kStepMaxSlots of step_max (one atomic per block, few blocks per
@@ -197,22 +202,9 @@ __global__ void integrate_kernel(const SysDev* __restrict__ sd, SysCount* sc, co
     if (step_max) block_max_displacement(step_max, dm2);
 }
 
-template <class P>
-__global__ void collect_kernel(const int* __restrict__ slot_of_atom, const typename P::facc* FAx,
-                               const typename P::facc* FAy, const typename P::facc* FAz, const typename P::facc* FSx,
-                               const typename P::facc* FSy, const typename P::facc* FSz, double* FX, double* FY,
-                               double* FZ, int n_atoms) {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= n_atoms) return;
-    double f[3];
-    total_force<P>(a, slot_of_atom[a], FAx, FAy, FAz, FSx, FSy, FSz, f);
-    FX[a] = f[0];
-    FY[a] = f[1];
-    FZ[a] = f[2];
-}
-
-// A report's snapshot in atom order, AoS, as three blocks [n][3]: positions,
-// velocities, total forces (the layout the reports and the caller take).
+// A snapshot of n atoms from a0 on in atom order, AoS [n][3], of what is asked
+// for (not NULL): positions, velocities, total forces (the layout the reports and
+// the caller take).
 template <class P>
 __global__ void report_snapshot_kernel(const int* __restrict__ slot_of_atom, const double* __restrict__ X,
                                        const double* __restrict__ Y, const double* __restrict__ Z,
@@ -220,31 +212,62 @@ __global__ void report_snapshot_kernel(const int* __restrict__ slot_of_atom, con
                                        const double* __restrict__ VZ, const typename P::facc* FAx,
                                        const typename P::facc* FAy, const typename P::facc* FAz,
                                        const typename P::facc* FSx, const typename P::facc* FSy,
-                                       const typename P::facc* FSz, double* out, int n_atoms) {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= n_atoms) return;
-    double f[3];
-    total_force<P>(a, slot_of_atom[a], FAx, FAy, FAz, FSx, FSy, FSz, f);
-    const size_t n = (size_t)n_atoms, i = 3 * (size_t)a;
-    out[i] = X[a];
-    out[i + 1] = Y[a];
-    out[i + 2] = Z[a];
-    out[3 * n + i] = VX[a];
-    out[3 * n + i + 1] = VY[a];
-    out[3 * n + i + 2] = VZ[a];
-    out[6 * n + i] = f[0];
-    out[6 * n + i + 1] = f[1];
-    out[6 * n + i + 2] = f[2];
+                                       const typename P::facc* FSz, double* pos, double* vel, double* force,
+                                       int a0, int n) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    const int a = a0 + k;
+    const size_t i = 3 * (size_t)k;
+    if (pos) {
+        pos[i] = X[a];
+        pos[i + 1] = Y[a];
+        pos[i + 2] = Z[a];
+    }
+    if (vel) {
+        vel[i] = VX[a];
+        vel[i + 1] = VY[a];
+        vel[i + 2] = VZ[a];
+    }
+    if (force) total_force<P>(a, slot_of_atom[a], FAx, FAy, FAz, FSx, FSy, FSz, force + i);
 }
 
 template <class P>
-void launch_report_snapshot(Batch<P>& B, double* out) {
+void launch_report_snapshot(Batch<P>& B, double* pos, double* vel, double* force, int a0, int n) {
     const int T = 256;
-    report_snapshot_kernel<P><<<(unsigned)((B.n_atoms + T - 1) / T), T, 0, B.stream>>>(
-        B.slot_of_atom, B.X, B.Y, B.Z, B.VX, B.VY, B.VZ, B.FAx, B.FAy, B.FAz, B.FSx, B.FSy, B.FSz, out, B.n_atoms);
+    report_snapshot_kernel<P><<<(unsigned)((n + T - 1) / T), T, 0, B.stream>>>(
+        B.slot_of_atom, B.X, B.Y, B.Z, B.VX, B.VY, B.VZ, B.FAx, B.FAy, B.FAz, B.FSx, B.FSy, B.FSz, pos, vel, force, a0,
+        n);
 }
-template void launch_report_snapshot<PrecFP64>(Batch<PrecFP64>&, double*);
-template void launch_report_snapshot<PrecMixed>(Batch<PrecMixed>&, double*);
+template void launch_report_snapshot<PrecFP64>(Batch<PrecFP64>&, double*, double*, double*, int, int);
+template void launch_report_snapshot<PrecMixed>(Batch<PrecMixed>&, double*, double*, double*, int, int);
+
+// The reverse, for every atom: AoS positions and velocities (NULL: zeros) into
+// the state; every system's list is due and none has overflowed.
+__global__ void set_state_kernel(const double* __restrict__ pos, const double* __restrict__ vel, double* X, double* Y,
+                                 double* Z, double* VX, double* VY, double* VZ, int n_atoms, SysCount* sc, int nsys) {
+    const int a = blockIdx.x * blockDim.x + threadIdx.x;
+    if (a < nsys) {
+        sc[a].rebuild = 1;
+        sc[a].overflow = 0;
+    }
+    if (a >= n_atoms || !pos) return;
+    const size_t i = 3 * (size_t)a;
+    X[a] = pos[i];
+    Y[a] = pos[i + 1];
+    Z[a] = pos[i + 2];
+    VX[a] = vel ? vel[i] : 0.0;
+    VY[a] = vel ? vel[i + 1] : 0.0;
+    VZ[a] = vel ? vel[i + 2] : 0.0;
+}
+// pos NULL: the flags alone
+template <class P>
+void launch_set_state(Batch<P>& B, const double* pos, const double* vel) {
+    const int T = 256, n = pos ? std::max(B.n_atoms, B.nsys) : B.nsys;
+    set_state_kernel<<<(unsigned)((n + T - 1) / T), T, 0, B.stream>>>(pos, vel, B.X, B.Y, B.Z, B.VX, B.VY, B.VZ,
+                                                                      B.n_atoms, B.d_cnt, B.nsys);
+}
+template void launch_set_state<PrecFP64>(Batch<PrecFP64>&, const double*, const double*);
+template void launch_set_state<PrecMixed>(Batch<PrecMixed>&, const double*, const double*);
 
 template <class P>
 void launch_pack(Batch<P>& B) {
@@ -270,20 +293,11 @@ void launch_integrate(Batch<P>& B, double dt) {
         B.FAx, B.FAy, B.FAz, B.FSx, B.FSy, B.FSz, B.pos, dt, B.n_atoms, B.step_max);
 }
 
-template <class P>
-void launch_collect_forces(Batch<P>& B, double* FX, double* FY, double* FZ) {
-    const int T = 256;
-    collect_kernel<P><<<(unsigned)((B.n_atoms + T - 1) / T), T, 0, B.stream>>>(
-        B.slot_of_atom, B.FAx, B.FAy, B.FAz, B.FSx, B.FSy, B.FSz, FX, FY, FZ, B.n_atoms);
-}
-
 template void launch_pack<PrecFP64>(Batch<PrecFP64>&);
 template void launch_pack<PrecMixed>(Batch<PrecMixed>&);
 template void launch_kinetic<PrecFP64>(Batch<PrecFP64>&, double);
 template void launch_kinetic<PrecMixed>(Batch<PrecMixed>&, double);
 template void launch_integrate<PrecFP64>(Batch<PrecFP64>&, double);
 template void launch_integrate<PrecMixed>(Batch<PrecMixed>&, double);
-template void launch_collect_forces<PrecFP64>(Batch<PrecFP64>&, double*, double*, double*);
-template void launch_collect_forces<PrecMixed>(Batch<PrecMixed>&, double*, double*, double*);
 
 }  // namespace nx

@@ -157,8 +157,8 @@ struct Batch {
     size_t fft_spread_lds = 0, fft_plane_lds = 0, fft_x_lds = 0;
     int pme_any = 0;
 
-    // energies in 2^30 fixed point: the kernels' sums [nsys][kEnergySlots][E_NTERMS], their totals [nsys][E_NTERMS]
-    long long *energy = nullptr, *energy_total = nullptr;
+    // energies [nsys][kEnergySlots][E_NTERMS] in 2^30 fixed point
+    long long* energy = nullptr;
 
     // flags
     int timing = 0;                 // NX_TIMING_* mode
@@ -184,12 +184,14 @@ template <class P> void launch_fft_forward(Batch<P>& B);
 template <class P> void launch_fft_convolve(Batch<P>& B, bool energy);
 template <class P> void launch_fft_inverse(Batch<P>& B);
 template <class P> void launch_pme_gather(Batch<P>& B);
-template <class P> void launch_energy_sum(Batch<P>& B);     // energy -> energy_total
+// the systems' energies [nsys][E_NTERMS] into total and their counters into counts (may be NULL)
+template <class P> void launch_energy_sum(Batch<P>& B, long long* total, SysCount* counts);
 template <class P> void launch_kinetic(Batch<P>& B, double dt);
 template <class P> void launch_integrate(Batch<P>& B, double dt);
-template <class P> void launch_collect_forces(Batch<P>& B, double* FX, double* FY, double* FZ);
-// positions, velocities and total forces in atom order into out[3][n][3]
-template <class P> void launch_report_snapshot(Batch<P>& B, double* out);
+// positions, velocities and total forces (each may be NULL) of n atoms from a0 on, [n][3] each
+template <class P> void launch_report_snapshot(Batch<P>& B, double* pos, double* vel, double* force, int a0, int n);
+// positions and velocities (NULL: zeros) [n][3] into the state (pos NULL: it stays), every list due
+template <class P> void launch_set_state(Batch<P>& B, const double* pos, const double* vel);
 // Writes up to cap pairs to out and their total count to *d_count, which must be zero before the launch.
 template <class P> void launch_export_pairs(Batch<P>& B, int2* out, long long cap, long long* d_count);
 // standalone FFT (verification)

@@ -40,6 +40,8 @@ struct HostSystem {
     bool rebuild_pending = false;
 };
 
+// what nx_set_topology would refuse it for; empty: nothing
+std::string topology_error(const nx_topology* t);
 void exclusions_from_bonds(int n, const std::vector<nx_bond>& bonds, std::vector<int>& off, std::vector<int>& idx);
 
 // Launch shapes the autotuner chooses among (0 = the built-in rule).  None of
@@ -59,9 +61,10 @@ class EngineBase {
     virtual void run(int nsteps, double dt, int mask) = 0;
     // as run, with the device time of every step (ms, from the end of the previous step)
     virtual void run_step_times(int nsteps, double dt, int mask, std::vector<double>& ms) = 0;
-    virtual void compute(int mask, bool kinetic, double dt, bool integrate, std::vector<double>* F,
-                         std::vector<double>* pos, std::vector<double>* vel, std::vector<nx_energies>* E) = 0;
-    virtual void get_state(std::vector<double>* pos, std::vector<double>* vel) = 0;
+    // F, pos, vel: [n][3] each, may be NULL
+    virtual void compute(int mask, bool kinetic, double dt, bool integrate, double* F, double* pos, double* vel,
+                         std::vector<nx_energies>* E) = 0;
+    virtual void get_state(double* pos, double* vel) = 0;
     // one report step enqueued without waiting (see nx_step_report_async); returns its ticket
     virtual long long report_async(int mask, double dt, double* pos, double* vel, double* F) = 0;
     // waits for a ticket's copies; energies per system

@@ -102,6 +102,7 @@ void sync_active_to_host(nx_server* s) {
     if (!s->eng || s->dirty) return;
     for (size_t i = 0; i < s->active.size(); ++i) {
         Request& r = *s->reqs[s->active[i]];
+        if (r.status == 2) continue;        // retired with its state in place
         s->eng->device_state((int)i, r.sys.pos.data(), r.sys.vel.data());
         r.sys.build_pos.resize(r.sys.pos.size());
         int due = 0;
@@ -217,14 +218,8 @@ nx_status nx_submit(nx_server* s, const nx_topology* t, const double lb[3], cons
                     const double* vel, int nsteps, double dt, int64_t* req) {
     return sguard(s, [&] {
         if (!t || !lb || !ub || !pos || nsteps < 0 || !(dt > 0)) throw std::invalid_argument("bad submit arguments");
-        // reuse the single-context validation through a scratch context
-        nx_ctx* c = nullptr;
-        nx_status st = nx_create(s->device, s->precision, &c);
-        if (st != NX_OK) throw nx::HipError(st, "cannot create a validation context");
-        st = nx_set_topology(c, t);
-        std::string msg = nx_last_error(c);
-        nx_destroy(c);
-        if (st != NX_OK) throw std::invalid_argument(msg);
+        const std::string msg = nx::topology_error(t);
+        if (!msg.empty()) throw std::invalid_argument(msg);
         auto r = std::make_unique<Request>();
         r->id = s->next_id++;
         nx::HostSystem& h = r->sys;

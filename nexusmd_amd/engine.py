@@ -17,6 +17,20 @@ def _d(a):
     return a.ctypes.data_as(L.D) if a is not None else None
 
 
+def _records(struct, count, *columns):
+    """ctypes array of `count` records (at least one) with the columns of the given
+    arrays in the order of the record's fields."""
+    out = (struct * max(1, count))()
+    if count:
+        view = np.frombuffer(out, np.dtype(struct))
+        fields = iter(view.dtype.names)
+        for c in columns:
+            c = np.asarray(c)
+            for k in range(1 if c.ndim == 1 else c.shape[1]):
+                view[next(fields)] = c if c.ndim == 1 else c[:, k]
+    return out
+
+
 class TopologyBuffers:
     """Keeps the ctypes arrays behind an nx_topology alive."""
 
@@ -27,19 +41,9 @@ class TopologyBuffers:
         self.sig = np.ascontiguousarray(sys.sig, np.float64)
         self.eps = np.ascontiguousarray(sys.eps, np.float64)
         nb, na, nt = len(sys.bond_idx), len(sys.angle_idx), len(sys.torsion_idx)
-        self.bonds = (L.Bond * max(1, nb))()
-        for t in range(nb):
-            i, j = sys.bond_idx[t]
-            self.bonds[t] = L.Bond(int(i), int(j), float(sys.bond_par[t, 0]), float(sys.bond_par[t, 1]))
-        self.angles = (L.Angle * max(1, na))()
-        for t in range(na):
-            i, j, k = sys.angle_idx[t]
-            self.angles[t] = L.Angle(int(i), int(j), int(k), float(sys.angle_par[t, 0]), float(sys.angle_par[t, 1]))
-        self.torsions = (L.Torsion * max(1, nt))()
-        for t in range(nt):
-            i, j, k, l = sys.torsion_idx[t]
-            self.torsions[t] = L.Torsion(int(i), int(j), int(k), int(l), float(sys.torsion_par[t, 0]),
-                                         float(sys.torsion_par[t, 1]), int(sys.torsion_per[t]))
+        self.bonds = _records(L.Bond, nb, sys.bond_idx, sys.bond_par)
+        self.angles = _records(L.Angle, na, sys.angle_idx, sys.angle_par)
+        self.torsions = _records(L.Torsion, nt, sys.torsion_idx, sys.torsion_par, sys.torsion_per)
         self.top = L.Topology()
         t = self.top
         t.n_atoms = n

@@ -132,3 +132,36 @@ def test_coincident_columns_sort_by_atom():
         f.append(ctx.compute_forces()[0])
         ctx.close()
     np.testing.assert_array_equal(f[0], f[1])
+
+
+@pytest.mark.parametrize("n", [7, 45000])       # one thread and several in the copies
+def test_state_and_results_round_trip(n):
+    """State in, report out: every buffer whole, in the caller's order, on a second
+    state in the same context too; what was not asked for is not written."""
+    s = _gas(n, (2.0, 2.0, 2.0) if n < 100 else (7.0, 7.4, 7.8), 2, grid=(20, 20, 20) if n < 100 else (64, 64, 64))
+    rng = np.random.default_rng(3)
+    ctx = E.Context(s, precision=L.FP64)
+    for k in range(2):
+        pos = (s.pos + 0.3 * k) % s.L
+        vel = rng.normal(size=(n, 3))
+        ctx.set_state(pos, vel)
+        p, v = ctx.get_state()
+        np.testing.assert_array_equal(p, pos)
+        np.testing.assert_array_equal(v, vel)
+        f0, e0 = ctx.compute_forces()
+        p, v, f, e = ctx.step_report(0.0005)
+        np.testing.assert_array_equal(p, pos)
+        np.testing.assert_array_equal(v, vel)
+        np.testing.assert_array_equal(f, f0)
+        assert e["potential"] == e0["potential"]
+        p, v = ctx.get_state()
+        np.testing.assert_allclose(v, vel + 0.0005 * f / s.mass[:, None], rtol=1e-14, atol=1e-13)
+        ctx.set_state(pos)
+        p, v = ctx.get_state()
+        assert not v.any()
+    bad = s.pos.copy()
+    bad[n // 2, 1] = np.nan
+    with pytest.raises(L.NexusError) as ex:
+        ctx.set_state(bad)
+    assert ex.value.status == L.NX_ERR_ARG and str(3 * (n // 2) + 1) in str(ex.value)
+    ctx.close()
