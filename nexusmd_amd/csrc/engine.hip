@@ -399,7 +399,7 @@ class Engine : public EngineBase {
                 fft_maxK_ = std::max(fft_maxK_, g[k]);
             }
             d.sp_margin = 0.5 * skin + 0.002;
-            rg_off += (long long)g[0] * g[1] * g[2];
+            rg_off += (long long)g[0] * g[1] * (g[2] + kPhiPad);
             cg_off += (long long)g[0] * g[1] * (g[2] / 2 + 1);
             d.bond_off = bond_off;
             d.n_bonds = (int)h.bonds.size();

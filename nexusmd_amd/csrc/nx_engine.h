@@ -25,6 +25,9 @@ constexpr int kSpreadPlaneThreads = 768;     // with the spread: three waves per
 // Most LDS of a plane pass with the spread: what the pair kernel's blocks leave of a CU's 160 KB.
 constexpr size_t kPlaneSpreadLds = 100 * 1024;
 constexpr int kXPassThreads = 512;
+// Points by which each row of the potential runs on past its end (its first
+// ones again): the gather reads five consecutive points from any of the row's.
+constexpr int kPhiPad = 4;
 constexpr size_t kMaxBlockLds = 160 * 1024 - 1024;   // less the kernels' static LDS
 
 // LDS bytes of the spread in a block of `threads`: its table of slot segments
