@@ -197,9 +197,9 @@ nx_status nx_kernel_time(nx_ctx* ctx, const char* name, double* ms_per_launch, i
  * built-in rule.  No shape changes what any kernel computes for an atom, a
  * pair or a grid line, so every choice gives the same bits in the mixed path:
  *   pair_per_cu    persistent pair-kernel workgroups per CU (capped by occupancy)
- *   spread_block   PME spread tile side, in neighbour-list columns
- *   fft_xblocks    plane FFT: number of workgroups the x pass is split into
- *   fft_lines      line FFT: lines per workgroup */
+ *   spread_block   no effect (the PME spread has no tiles any more)
+ *   fft_xblocks    workgroups that the FFT's x pass is split into, as nearly as whole or half cache lines allow
+ *   fft_lines      line FFT: columns of a y workgroup, pairs of rows of a z one, at most */
 typedef struct { int pair_per_cu, spread_block, fft_xblocks, fft_lines; } nx_tuning;
 /* Shapes for the next layout of the context (taken at its next call). */
 nx_status nx_set_tuning(nx_ctx* ctx, const nx_tuning* t);

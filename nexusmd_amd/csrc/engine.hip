@@ -395,6 +395,7 @@ class Engine : public EngineBase {
             d.cgrid_off = cg_off;
             for (int k = 0; k < 3; ++k) {
                 d.tw_off[k] = (int)tw_off;
+                d.fft_plan[k] = fft_plan(g[k]);
                 tw_off += g[k];
                 fft_maxK_ = std::max(fft_maxK_, g[k]);
             }
@@ -517,28 +518,32 @@ class Engine : public EngineBase {
         std::vector<real2> tw;
         std::vector<int4> zi, pi, li, yi, xi;
         const int maxK = fft_maxK_;
-        // LDS per FFT block: two buffers of T lines plus the twiddles, within 60 KiB
-        const int Tfit = std::max(1, std::min(8, (int)((61440 / (int)sizeof(real2) - maxK) / (2 * maxK))));
-        const int T = tuning_.fft_lines > 0 ? std::min(tuning_.fft_lines, Tfit) : Tfit;
-        B.fft_lines = T;
+        // y tiles of up to a cache line's columns, z passes over up to 8 pairs of rows
+        // (in an odd pitch), within 60 KiB of LDS
+        const int row = kPassRowBytes / (int)sizeof(real2);
+        const int Tfit = std::max(1, (int)((61440 / (int)sizeof(real2) - maxK) / (2 * maxK)));
+        const int most = tuning_.fft_lines > 0 ? tuning_.fft_lines : row;
+        const int T = std::min({most, row, Tfit}), pairs = std::min({most, 8, (Tfit - 1) | 1});
         B.fft_tile = T;
-        B.fft_maxK = maxK;
-        // plane passes when every system's planes fit one workgroup's LDS; the x
-        // pass splits the kz range so that the batch has about 512 x blocks
+        B.fft_y_lds = line_lds_bytes<real2>(maxK, T);
+        B.fft_z_lds = line_lds_bytes<real2>(maxK, pairs | 1);
+        // plane passes when every system's planes fit one workgroup's LDS
         bool plane = fft_plane_enabled(), plane_spread = true;
-        int sum_ky = 0;
-        long long rows = 0;
+        long long rows = 0, x_lines = 0;
         for (int s = 0; s < ns; ++s) {
             const SysDev& d = B.sys[s];
-            if (plane_lds_bytes<real2>(d.grid[1], d.grid[2]) > kMaxBlockLds ||
-                xpass_lds_bytes<real2>(d.grid[0], 1) > kMaxBlockLds)
-                plane = false;
+            if (plane_lds_bytes<real2>(d.grid[1], d.grid[2]) > kMaxBlockLds) plane = false;
             if (plane_spread_lds_bytes<real2>(d.grid[1], d.grid[2]) > kPlaneSpreadLds) plane_spread = false;
-            sum_ky += d.grid[1];
+            x_lines += (long long)d.grid[1] * (d.grid[2] / 2 + 1);
             rows += (long long)d.grid[0] * d.grid[1];
         }
-        const int xtarget = tuning_.fft_xblocks > 0 ? tuning_.fft_xblocks : 512;
-        const int xsplit = std::max(1, (xtarget + sum_ky - 1) / std::max(1, sum_ky));
+        // lines of a workgroup of the x pass: a cache line's width, half of one for more
+        // workgroups only on request (the passes after the spread, us alone, whole and
+        // half: 64^3 15.1, 15.4; 50 x 50 x 75 17.9, 18.1; unaligned widths between them
+        // are worse: 96^3 21.6 with 16 lines, 25.3 with 10)
+        const int xlines = x_lines > (long long)row * tuning_.fft_xblocks ? row : row / 2;
+        B.fft_x_threads = 64;
+        B.fft_plane_threads = 64;
         B.fft_plane = plane ? 1 : 0;
         // The spread goes into the plane pass where the plane's workgroup finds room
         // beside the pair kernel's on a CU: one launch and one trip of the spectrum
@@ -633,7 +638,7 @@ class Engine : public EngineBase {
                 for (int x = 0; x < Kx; ++x)
                     for (int y = 0; y < Ky; y += ny) zi.push_back(make_int4(s, x, y, std::min(ny, Ky - y)));
                 B.fft_spread_lds =
-                    std::max(B.fft_spread_lds, (size_t)(Kz + spread_points<real2>((ny + 1) / 2 * Kz, ny, Kz)) * sizeof(real2) +
+                    std::max(B.fft_spread_lds, (size_t)(Kz + spread_points<real2>(((ny + 1) / 2 | 1) * Kz, ny, Kz)) * sizeof(real2) +
                                                    spread_lds_bytes(kSpreadZThreads));
                 for (int x = 0; x < Kx; ++x)
                     for (int k = 0; k < Kzh; k += T) yi.push_back(make_int4(s, x, k, 0));
@@ -643,16 +648,20 @@ class Engine : public EngineBase {
             }
             if (B.fft_plane) {
                 for (int x = 0; x < Kx; ++x) pi.push_back(make_int4(s, x, 0, 0));
-                int nk = (Kzh + xsplit - 1) / xsplit;
-                while (nk > 1 && xpass_lds_bytes<real2>(Kx, nk) > kMaxBlockLds) nk = (nk + 1) / 2;
-                for (int y = 0; y < Ky; ++y)
-                    for (int k = 0; k < Kzh; k += nk) xi.push_back(make_int4(s, y, k, std::min(nk, Kzh - k)));
                 B.fft_plane_lds = std::max(B.fft_plane_lds, plane_lds_bytes<real2>(Ky, Kz));
-                B.fft_x_lds = std::max(B.fft_x_lds, xpass_lds_bytes<real2>(Kx, nk));
+                // a thread for every radix-5 butterfly of a stage
+                B.fft_plane_threads =
+                    std::max(B.fft_plane_threads, std::min(kPlaneThreads, (plane_cap(Ky, Kz) / 5 + 63) & ~63));
             } else {
-                for (int l = 0; l < Kx * Ky; l += T) li.push_back(make_int4(s, l, std::min(T, Kx * Ky - l), 0));
-                for (int y = 0; y < Ky; ++y)
-                    for (int k = 0; k < Kzh; k += T) xi.push_back(make_int4(s, y, k, 0));
+                for (int l = 0; l < Kx * Ky; l += 2 * pairs)
+                    li.push_back(make_int4(s, l, std::min(2 * pairs, Kx * Ky - l), 0));
+            }
+            {
+                int nr = xlines;
+                while (nr > 1 && line_lds_bytes<real2>(Kx, nr) > (size_t)61440) nr = (nr + 1) / 2;
+                for (int r = 0; r < Ky * Kzh; r += nr) xi.push_back(make_int4(s, r, std::min(nr, Ky * Kzh - r), 0));
+                B.fft_x_lds = std::max(B.fft_x_lds, line_lds_bytes<real2>(Kx, nr));
+                B.fft_x_threads = std::max(B.fft_x_threads, std::min(kXPassThreads, (nr * Kx / 5 + 63) & ~63));
             }
             self_energy_.resize(ns);
             double se = 0.0;

@@ -57,6 +57,7 @@ struct SysDev {
     int excl_off, n_excl;        // excluded pair list
     int bond_off, n_bonds, angle_off, n_angles, tors_off, n_tors;
     int tw_off[3];               // twiddle-table offsets per axis
+    unsigned fft_plan[3];        // radices of the axes' transforms (fft_plan)
     double sp_margin;            // distance an atom may move between rebuilds
 };
 
@@ -150,7 +151,7 @@ struct PrecMixed {
     static constexpr int pair_waves_per_simd = 4;
     // Three pair-kernel waves per SIMD (the persistent grid's three blocks per
     // CU) at 112 VGPRs leave 176 of a SIMD's 512 to the PME kernels beside
-    // them: a 1024-thread plane-FFT block (four waves per SIMD at 40 VGPRs)
+    // them: a 768-thread plane-FFT block (three waves per SIMD at 56 VGPRs)
     // then fits; at 120 it does not, and PME waits for the pair kernel.
     static constexpr int pair_max_vgpr = 112;
 };

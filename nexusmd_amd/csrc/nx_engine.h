@@ -20,11 +20,12 @@ namespace nx {
 struct HostSystem;   // engine.hip
 
 // Plane FFT passes: threads per block, LDS available to one workgroup on gfx950.
-constexpr int kPlaneThreads = 1024;
-constexpr int kSpreadPlaneThreads = 768;     // with the spread: three waves per SIMD of at most 56 VGPRs
+constexpr int kPlaneThreads = 768;           // three waves per SIMD, in the mixed path of at most 56 VGPRs
 // Most LDS of a plane pass with the spread: what the pair kernel's blocks leave of a CU's 160 KB.
 constexpr size_t kPlaneSpreadLds = 100 * 1024;
-constexpr int kXPassThreads = 512;
+constexpr int kXPassThreads = 256;
+// Bytes of a row that the y and x passes take at a time: a cache line.
+constexpr int kPassRowBytes = 128;
 // Points by which each row of the potential runs on past its end (its first
 // ones again): the gather reads five consecutive points from any of the row's.
 constexpr int kPhiPad = 4;
@@ -47,26 +48,46 @@ constexpr int kSpreadZThreads = 512;
 constexpr int kSpreadZPerThread = 6;
 constexpr int kSpreadZPoints = kSpreadZThreads * kSpreadZPerThread;
 
+// The radices of a transform of N = 2^a 3^b 5^c points, four bits each, the first
+// stage's lowest: as few stages as radices up to 8 allow.
+__host__ __device__ inline unsigned fft_plan(int N) {
+    int twos = 0, m = N;
+    for (; m % 2 == 0; m /= 2) ++twos;
+    unsigned plan = 0;
+    int at = 0;
+    auto add = [&](unsigned r) { plan |= r << at; at += 4; };
+    if (twos == 1) add(2);
+    else if (twos % 3 == 1) { add(4); add(4); twos -= 4; }
+    else if (twos % 3 == 2) { add(4); twos -= 2; }
+    for (; twos >= 3; twos -= 3) add(8);
+    for (; m % 3 == 0; m /= 3) add(3);
+    for (; m % 5 == 0; m /= 5) add(5);
+    return plan;
+}
+
+// Complex points of a line buffer of a plane pass: row pairs by z or, the other
+// way, wave numbers by y, the inner extent made odd.
+__host__ __device__ constexpr int plane_cap(int Ky, int Kz) {
+    const int z = Kz * (((Ky + 1) / 2) | 1), y = Ky * ((Kz / 2 + 1) | 1);
+    return z > y ? z : y;
+}
+
 // LDS bytes of a plane pass (two buffers, the y and z twiddles).
 template <typename R2>
 inline size_t plane_lds_bytes(int Ky, int Kz) {
-    const int np = (Ky + 1) / 2, Kzh = Kz / 2 + 1;
-    const int cap = np * Kz > Ky * Kzh ? np * Kz : Ky * Kzh;
-    return (size_t)(Ky + Kz + 2 * cap) * sizeof(R2);
+    return (size_t)(Ky + Kz + 2 * plane_cap(Ky, Kz)) * sizeof(R2);
 }
 
 // The same with the spread in it.
 template <typename R2>
 inline size_t plane_spread_lds_bytes(int Ky, int Kz) {
-    const int np = (Ky + 1) / 2, Kzh = Kz / 2 + 1;
-    const int cap = np * Kz > Ky * Kzh ? np * Kz : Ky * Kzh;
-    return (size_t)(Ky + Kz + spread_points<R2>(cap, Ky, Kz)) * sizeof(R2) + spread_lds_bytes(kSpreadPlaneThreads);
+    return (size_t)(Ky + Kz + spread_points<R2>(plane_cap(Ky, Kz), Ky, Kz)) * sizeof(R2) + spread_lds_bytes(kPlaneThreads);
 }
 
-// LDS bytes of an x pass over nk wave numbers kz (two buffers, the twiddles).
+// LDS bytes of `lines` lines of K points (two buffers, the twiddles).
 template <typename R2>
-inline size_t xpass_lds_bytes(int Kx, int nk) {
-    return (size_t)(Kx + 2 * nk * Kx) * sizeof(R2);
+inline size_t line_lds_bytes(int K, int lines) {
+    return (size_t)(K + 2 * lines * K) * sizeof(R2);
 }
 
 template <class P>
@@ -152,12 +173,13 @@ struct Batch {
     int4* fftp_items = nullptr;     // inverse plane pass: (sys, x)
     int4* fftl_items = nullptr;     // inverse z pass: (sys, first line, n lines, 0)
     int4* ffty_items = nullptr;     // (sys, x, kz0, 0)
-    int4* fftx_items = nullptr;     // (sys, y, kz0, 0)
+    int4* fftx_items = nullptr;     // (sys, first (y, kz) line, n lines, 0)
     int n_fftz = 0, n_fftp = 0, n_fftl = 0, n_ffty = 0, n_fftx = 0;
-    int fft_lines = 1, fft_tile = 1, fft_maxK = 0;
-    int fft_plane = 0;              // 1: plane passes (fftp_items, fftx_items = x blocks); 0: line passes
+    int fft_tile = 1;               // columns of a y pass's tile
+    int fft_plane_threads = 0, fft_x_threads = 0;
+    int fft_plane = 0;              // 1: plane passes (fftp_items); 0: y and z passes over lines
     int fft_split = 0;              // 1: spread and z pass over rows, then a y pass; 0: spread in the plane pass
-    size_t fft_spread_lds = 0, fft_plane_lds = 0, fft_x_lds = 0;
+    size_t fft_spread_lds = 0, fft_plane_lds = 0, fft_x_lds = 0, fft_y_lds = 0, fft_z_lds = 0;
     int pme_any = 0;
 
     // energies [nsys][kEnergySlots][E_NTERMS] in 2^30 fixed point

@@ -49,9 +49,9 @@ void exclusions_from_bonds(int n, const std::vector<nx_bond>& bonds, std::vector
 // every choice gives the same bits in the mixed path.
 struct Tuning {
     int pair_per_cu = 0;     // persistent pair-kernel blocks per CU (built-in: min(occupancy, 3))
-    int spread_block = 0;    // spread tile: columns per block side (built-in: the cost model's choice)
-    int fft_xblocks = 0;     // plane FFT: x-pass blocks the kz range is split into (built-in: ~512)
-    int fft_lines = 0;       // line FFT: lines per block (built-in: as many as fit 60 KiB of LDS, <= 8)
+    int spread_block = 0;    // no effect (the spread has no tiles any more)
+    int fft_xblocks = 0;     // x-pass blocks: more than a cache line's lines each would make (built-in: those)
+    int fft_lines = 0;       // line FFT: most y columns, or z row pairs, per block (built-in: what fits 60 KiB of LDS)
 };
 
 class EngineBase {

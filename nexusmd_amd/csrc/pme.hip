@@ -11,16 +11,17 @@
 // Here the spread grid is real, so the forward transform is real-to-complex
 // onto the half spectrum [Kx][Ky][Kz/2+1] and the backward one complex-to-
 // real; by Hermitian symmetry this is the same result (the reference keeps
-// only the real part after its backward transform).  Five passes, each one
-// read and one write of the grid:
-//   Z  : R2C along z (lines contiguous), fixed-point -> real on load;
+// only the real part after its backward transform).  Five passes:
+//   Z  : the charges spread to rows in LDS (there is no charge grid in memory),
+//        R2C along z;
 //   Y  : C2C along y on tiles of consecutive kz (coalesced rows);
 //   X  : C2C along x, multiply by the influence function eta(k) and sum the
 //        energy, inverse C2C along x -- fused so the spectrum makes one trip;
 //   Y' : inverse C2C along y;
 //   Z' : C2R along z into the real potential grid.
-// Each line FFT is a Stockham autosort radix-{4,2,3,5} transform in LDS with
-// twiddles from a per-axis table exp(-2 pi i t / K) computed on the host in FP64.
+// Z with Y, and Y' with Z', are one kernel each where planes fit in LDS.  Each
+// line FFT is a Stockham autosort transform in LDS (fft_lines) with twiddles from
+// a per-axis table exp(-2 pi i t / K) computed on the host in FP64.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -282,8 +283,8 @@ __device__ __forceinline__ void spread_rows(const SysDev& d, const SpreadArgs& a
 // The loads bound it: the lanes' stencils start anywhere, so a load costs by the
 // cache lines its lanes touch, not by the bytes.  A row of the stencil is
 // therefore read as four points and one instead of point by point, which the
-// rows' copied first points (kPhiPad) allow at any start: on 10^6 atoms, 128^3
-// points, 165 -> 92 us; on 10^5 atoms and 100^3, 24 -> 15 us (FP64 29 -> 26 us).
+// rows' copied first points (kPhiPad) allow at any start: on 10^6 atoms, 200^3
+// points, 165 -> 92 us; on 10^5 atoms and 96^3, 24 -> 15 us (FP64 29 -> 26 us).
 // Staging the points under a super-cluster in LDS first cost more than it saved.
 constexpr int kGatherSlots = 64;
 
@@ -386,58 +387,68 @@ __device__ __forceinline__ R2 cmul(R2 a, R2 b) {
     return r;
 }
 
-// Small DFT of radix r in registers; sign -1 forward, +1 backward.
-template <typename real, typename R2>
-__device__ __forceinline__ void dft_small(R2* v, int r, int sign) {
-    if (r == 2) {
-        R2 a = v[0], b = v[1];
+// DFT of R points in registers; SIGN -1 forward, +1 backward.
+template <int R, int SIGN, typename R2>
+__device__ __forceinline__ void dft(R2* v) {
+    using real = decltype(v->x);
+    constexpr real sg = (real)SIGN;
+    if constexpr (R == 2) {
+        const R2 a = v[0], b = v[1];
         v[0].x = a.x + b.x; v[0].y = a.y + b.y;
         v[1].x = a.x - b.x; v[1].y = a.y - b.y;
-    } else if (r == 4) {
-        R2 a0 = v[0], a1 = v[1], a2 = v[2], a3 = v[3];
-        R2 s02 = {a0.x + a2.x, a0.y + a2.y}, d02 = {a0.x - a2.x, a0.y - a2.y};
-        R2 s13 = {a1.x + a3.x, a1.y + a3.y}, d13 = {a1.x - a3.x, a1.y - a3.y};
-        // W = sign * i ; W * (x + iy) = sign * (-y + ix)
-        R2 wd = {(real)sign * -d13.y, (real)sign * d13.x};
-        v[0].x = s02.x + s13.x; v[0].y = s02.y + s13.y;
-        v[2].x = s02.x - s13.x; v[2].y = s02.y - s13.y;
-        v[1].x = d02.x + wd.x;  v[1].y = d02.y + wd.y;
-        v[3].x = d02.x - wd.x;  v[3].y = d02.y - wd.y;
-    } else if (r == 3) {
-        const real c1 = (real)-0.5, s1 = (real)sign * (real)0.86602540378443864676;
-        R2 a0 = v[0], a1 = v[1], a2 = v[2];
-        R2 sm = {a1.x + a2.x, a1.y + a2.y}, df = {a1.x - a2.x, a1.y - a2.y};
-        R2 t = {a0.x + c1 * sm.x, a0.y + c1 * sm.y};
+    } else if constexpr (R == 3) {
+        constexpr real c1 = (real)-0.5, s1 = sg * (real)0.86602540378443864676;
+        const R2 a0 = v[0], a1 = v[1], a2 = v[2];
+        const R2 sm = {a1.x + a2.x, a1.y + a2.y}, df = {a1.x - a2.x, a1.y - a2.y};
+        const R2 t = {a0.x + c1 * sm.x, a0.y + c1 * sm.y};
         // i * s1 * df = (-s1 df.y, s1 df.x)
         v[0].x = a0.x + sm.x; v[0].y = a0.y + sm.y;
         v[1].x = t.x - s1 * df.y; v[1].y = t.y + s1 * df.x;
         v[2].x = t.x + s1 * df.y; v[2].y = t.y - s1 * df.x;
-    } else {  // r == 5
-        const real c1 = (real)0.30901699437494742410, c2 = (real)-0.80901699437494742410;
-        const real s1 = (real)sign * (real)0.95105651629515357212, s2 = (real)sign * (real)0.58778525229247312917;
-        R2 a0 = v[0], a1 = v[1], a2 = v[2], a3 = v[3], a4 = v[4];
-        R2 b1 = {a1.x + a4.x, a1.y + a4.y}, b4 = {a1.x - a4.x, a1.y - a4.y};
-        R2 b2 = {a2.x + a3.x, a2.y + a3.y}, b3 = {a2.x - a3.x, a2.y - a3.y};
-        R2 t1 = {a0.x + c1 * b1.x + c2 * b2.x, a0.y + c1 * b1.y + c2 * b2.y};
-        R2 t2 = {a0.x + c2 * b1.x + c1 * b2.x, a0.y + c2 * b1.y + c1 * b2.y};
+    } else if constexpr (R == 4) {
+        const R2 s02 = {v[0].x + v[2].x, v[0].y + v[2].y}, d02 = {v[0].x - v[2].x, v[0].y - v[2].y};
+        const R2 s13 = {v[1].x + v[3].x, v[1].y + v[3].y}, d13 = {v[1].x - v[3].x, v[1].y - v[3].y};
+        const R2 wd = {-sg * d13.y, sg * d13.x};         // +-i (v1 - v3)
+        v[0].x = s02.x + s13.x; v[0].y = s02.y + s13.y;
+        v[2].x = s02.x - s13.x; v[2].y = s02.y - s13.y;
+        v[1].x = d02.x + wd.x;  v[1].y = d02.y + wd.y;
+        v[3].x = d02.x - wd.x;  v[3].y = d02.y - wd.y;
+    } else if constexpr (R == 5) {
+        constexpr real c1 = (real)0.30901699437494742410, c2 = (real)-0.80901699437494742410;
+        constexpr real s1 = sg * (real)0.95105651629515357212, s2 = sg * (real)0.58778525229247312917;
+        const R2 a0 = v[0], a1 = v[1], a2 = v[2], a3 = v[3], a4 = v[4];
+        const R2 b1 = {a1.x + a4.x, a1.y + a4.y}, b4 = {a1.x - a4.x, a1.y - a4.y};
+        const R2 b2 = {a2.x + a3.x, a2.y + a3.y}, b3 = {a2.x - a3.x, a2.y - a3.y};
+        const R2 t1 = {a0.x + c1 * b1.x + c2 * b2.x, a0.y + c1 * b1.y + c2 * b2.y};
+        const R2 t2 = {a0.x + c2 * b1.x + c1 * b2.x, a0.y + c2 * b1.y + c1 * b2.y};
         // u1 = s1 b4 + s2 b3, u2 = s2 b4 - s1 b3 ; X1 = t1 + i u1, X4 = t1 - i u1, X2 = t2 + i u2, X3 = t2 - i u2
-        R2 u1 = {s1 * b4.x + s2 * b3.x, s1 * b4.y + s2 * b3.y};
-        R2 u2 = {s2 * b4.x - s1 * b3.x, s2 * b4.y - s1 * b3.y};
+        const R2 u1 = {s1 * b4.x + s2 * b3.x, s1 * b4.y + s2 * b3.y};
+        const R2 u2 = {s2 * b4.x - s1 * b3.x, s2 * b4.y - s1 * b3.y};
         v[0].x = a0.x + b1.x + b2.x; v[0].y = a0.y + b1.y + b2.y;
         v[1].x = t1.x - u1.y; v[1].y = t1.y + u1.x;
         v[4].x = t1.x + u1.y; v[4].y = t1.y - u1.x;
         v[2].x = t2.x - u2.y; v[2].y = t2.y + u2.x;
         v[3].x = t2.x + u2.y; v[3].y = t2.y - u2.x;
+    } else {
+        static_assert(R == 8, "radix");
+        constexpr real h = (real)0.70710678118654752440;
+        R2 e[4] = {v[0], v[2], v[4], v[6]}, o[4] = {v[1], v[3], v[5], v[7]};
+        dft<4, SIGN>(e);
+        dft<4, SIGN>(o);
+        // o[k] times exp(SIGN i pi k / 4)
+        const R2 o1 = {h * (o[1].x - sg * o[1].y), h * (o[1].y + sg * o[1].x)};
+        const R2 o2 = {-sg * o[2].y, sg * o[2].x};
+        const R2 o3 = {-h * (o[3].x + sg * o[3].y), h * (sg * o[3].x - o[3].y)};
+        v[0].x = e[0].x + o[0].x; v[0].y = e[0].y + o[0].y;
+        v[4].x = e[0].x - o[0].x; v[4].y = e[0].y - o[0].y;
+        v[1].x = e[1].x + o1.x;   v[1].y = e[1].y + o1.y;
+        v[5].x = e[1].x - o1.x;   v[5].y = e[1].y - o1.y;
+        v[2].x = e[2].x + o2.x;   v[2].y = e[2].y + o2.y;
+        v[6].x = e[2].x - o2.x;   v[6].y = e[2].y - o2.y;
+        v[3].x = e[3].x + o3.x;   v[3].y = e[3].y + o3.y;
+        v[7].x = e[3].x - o3.x;   v[7].y = e[3].y - o3.y;
     }
 }
-
-__device__ __forceinline__ int next_radix(int m) {
-    if (m % 4 == 0) return 4;
-    if (m % 2 == 0) return 2;
-    if (m % 3 == 0) return 3;
-    return 5;
-}
-
 
 // Copies the N twiddles of an axis into LDS (all threads of the block).
 template <typename R2>
@@ -445,57 +456,105 @@ __device__ __forceinline__ void load_twiddles(R2* dst, const R2* __restrict__ sr
     for (int i = threadIdx.x; i < N; i += blockDim.x) dst[i] = src[i];
 }
 
-// FFT of `lines` lines of length N in LDS, point m of line l at a[l * ls + m * es];
-// `b` is scratch of the same layout; `tw` holds exp(-2 pi i m / N), m < N, in
-// LDS.  Stockham autosort, radix 4, 2, 3, 5; unnormalised; sign -1 forward, +1
-// backward.  Returns the buffer holding the result.  All threads of the block
-// call it; every stage ends with a barrier.
-template <typename real, typename R2>
-__device__ R2* fft_lines_lds(R2* a, R2* b, int N, int lines, int ls, int es, const R2* tw, int sign) {
-    int Ns = 1;
-    int rem = N;
-    R2* src = a;
-    R2* dst = b;
-    while (rem > 1) {
-        const int r = next_radix(rem);
-        const int nb = N / r;
-        const int step = N / (Ns * r);
-        const float inv_nb = 1.0f / (float)nb, inv_ns = 1.0f / (float)Ns;
-        const int total = lines * nb;
-        for (int w = threadIdx.x; w < total; w += blockDim.x) {
-            const int line = qdiv(w, inv_nb), j = w - line * nb;
-            const int jq = qdiv(j, inv_ns), k = j - jq * Ns;
-            const R2* sp = src + line * ls;
-            R2* dp = dst + line * ls;
-            R2 v[5];
+// FFTs of `lines` lines of N points by a block: Stockham autosort, unnormalised,
+// the radices in `plan` (fft_plan).  `tw` holds exp(-2 pi i m / N), m < N, in LDS.
+//
+// The passes are bound by their trips through LDS and by the barriers between
+// them, so the radices go up to 8 (64 points in two stages, 96 in three), the
+// first stage takes its points from load(m, l) -- global memory, mostly -- and the
+// last one gives them to store(buf, m, l, v), and between stages point m of line l
+// stands at [m * pitch + l] with the threads running over the lines: no bank
+// conflicts, and one twiddle read serves all lines.  (Radices up to 5, every line's
+// points side by side, and copies into and out of LDS before: the passes after the
+// spread's took 23.4 us alone at 64^3, 36.8 at 96^3, 209 at 200^3, FP64 57 at 96^3;
+// now 15.0, 21.7, 122 and 39.6.)  FAST_IN / FAST_OUT run the
+// threads of the first / last stage over the points instead, where those are
+// consecutive in memory; an odd pitch then keeps the LDS side free of conflicts.
+//
+// Buffers: stages alternate, the first into b0, the next into b1; store gets the
+// one that would be next.  With Ns > 1 (a power product of radices already done)
+// the points stand in b1 and `load` is not called.  Returns the buffer after the
+// last stage, without a barrier.
+template <int R, int SIGN, bool FAST_IN, bool FAST_OUT, typename R2, class Load, class Store>
+__device__ __forceinline__ void fft_stage(int Ns, int step, int lines, int pitch, bool first, bool last, const R2* tw,
+                                          const R2* src, R2* dst, Load& load, Store& store) {
+    const int nb = step * Ns, total = nb * lines;      // nb butterflies a line
+    const bool fast = (FAST_IN && first) || (FAST_OUT && last);
+    const int inner = fast ? nb : lines;
+    const float inv_inner = 1.0f / (float)inner, inv_ns = 1.0f / (float)Ns;
+    for (int w = threadIdx.x; w < total; w += blockDim.x) {
+        const int outer = qdiv(w, inv_inner), in = w - outer * inner;
+        const int j = fast ? in : outer, l = fast ? outer : in;
+        R2 v[R];
+        int k = 0, base = j * R;
+        if (first) {
 #pragma unroll
-            for (int q = 0; q < 5; ++q)
-                if (q < r) v[q] = sp[(j + q * nb) * es];
-            if (k != 0) {
+            for (int q = 0; q < R; ++q) v[q] = load(j + q * nb, l);
+        } else {
+            const int jq = qdiv(j, inv_ns);
+            k = j - jq * Ns;
+            base = jq * Ns * R + k;
 #pragma unroll
-                for (int q = 1; q < 5; ++q) {
-                    if (q < r) {
-                        R2 t = tw[k * q * step];     // k q step < N
-                        if (sign > 0) t.y = -t.y;
-                        v[q] = cmul(v[q], t);
-                    }
-                }
+            for (int q = 0; q < R; ++q) v[q] = src[(j + q * nb) * pitch + l];
+#pragma unroll
+            for (int q = 1; q < R; ++q) {
+                R2 t = tw[k * q * step];     // k q step < N
+                if (SIGN > 0) t.y = -t.y;
+                v[q] = cmul(v[q], t);
             }
-            dft_small<real, R2>(v, r, sign);
-            const int base = jq * Ns * r + k;
-#pragma unroll
-            for (int q = 0; q < 5; ++q)
-                if (q < r) dp[(base + q * Ns) * es] = v[q];
         }
-        __syncthreads();
+        dft<R, SIGN>(v);
+        if (last) {
+#pragma unroll
+            for (int q = 0; q < R; ++q) store(dst, base + q * Ns, l, v[q]);
+        } else {
+#pragma unroll
+            for (int q = 0; q < R; ++q) dst[(base + q * Ns) * pitch + l] = v[q];
+        }
+    }
+}
+
+// fn(radix) with the radix a compile-time constant.
+template <class Fn>
+__device__ __forceinline__ void with_radix(int r, Fn&& fn) {
+    if (r == 8) fn(std::integral_constant<int, 8>{});
+    else if (r == 4) fn(std::integral_constant<int, 4>{});
+    else if (r == 5) fn(std::integral_constant<int, 5>{});
+    else if (r == 3) fn(std::integral_constant<int, 3>{});
+    else fn(std::integral_constant<int, 2>{});
+}
+
+template <int SIGN, bool FAST_IN, bool FAST_OUT, typename R2, class Load, class Store>
+__device__ __forceinline__ R2* fft_lines(int N, unsigned plan, int lines, int pitch, const R2* tw, R2* b0, R2* b1, int Ns,
+                                         Load load, Store store) {
+    R2* src = b1;
+    R2* dst = b0;
+    int rem = N / Ns;
+    while (plan) {
+        const int r = plan & 15;
+        plan >>= 4;
+        const bool first = Ns == 1, last = plan == 0;
+        int step = 0;
+        with_radix(r, [&](auto R) {
+            step = rem / R.value;
+            fft_stage<R.value, SIGN, FAST_IN, FAST_OUT>(Ns, step, lines, pitch, first, last, tw, src, dst, load, store);
+        });
+        Ns *= r;
+        rem = step;
         R2* t = src;
         src = dst;
         dst = t;
-        Ns *= r;
-        rem /= r;
+        if (!last) __syncthreads();
     }
     return src;
 }
+
+// store() of a last stage whose result stays in LDS
+template <typename R2>
+struct KeepLine {
+    int pitch;
+    __device__ __forceinline__ void operator()(R2* buf, int m, int l, R2 v) const { buf[m * pitch + l] = v; }
+};
 
 __device__ __forceinline__ float fixed_to_real(long long v, float) { return (float)((double)v * (1.0 / PrecMixed::grid_scale)); }
 __device__ __forceinline__ double fixed_to_real(long long v, double) { return (double)v * (1.0 / PrecFP64::grid_scale); }
@@ -509,6 +568,84 @@ __device__ __forceinline__ long long grid_value(const long long* g, int y, int z
     return z < 4 ? row[z] + row[z + Kz] : row[z];
 }
 
+// Point m of the real rows at o and o + second, and the copies past their ends.
+template <typename real, typename R2>
+__device__ __forceinline__ void store_rows(real* o, int second, bool both, int m, int Kz, int pad, R2 v) {
+    o[m] = v.x;
+    if (m < pad) o[Kz + m] = v.x;
+    if (both) {
+        o[second + m] = v.y;
+        if (m < pad) o[second + Kz + m] = v.y;
+    }
+}
+
+// First z stage of `rows` rows of the spread's sums g, rows 2p and 2p + 1 as one
+// complex line: the sums take the room of the line buffers, so every thread holds
+// its butterflies over the barrier (at most `Points` points of all lines in
+// THREADS threads).
+template <int R, int THREADS, int Points, typename R2>
+__device__ __forceinline__ void fft_sums_stage(const long long* g, int rows, int np, int Kz, int pitch, R2* out) {
+    using real = decltype(out->x);
+    constexpr int U = (Points / R + THREADS - 1) / THREADS;
+    const int nb = Kz / R, total = nb * np;
+    const float inv_nb = 1.0f / (float)nb;
+    R2 v[U][R];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int w = threadIdx.x + u * THREADS;
+        if (w < total) {
+            const int p = qdiv(w, inv_nb), j = w - p * nb;
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                const int z = j + q * nb;
+                v[u][q].x = fixed_to_real(grid_value<true>(g, 2 * p, z, Kz), (real)0);
+                v[u][q].y = 2 * p + 1 < rows ? fixed_to_real(grid_value<true>(g, 2 * p + 1, z, Kz), (real)0) : (real)0;
+            }
+            dft<R, -1>(v[u]);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int w = threadIdx.x + u * THREADS;
+        if (w < total) {
+            const int p = qdiv(w, inv_nb), j = w - p * nb;
+#pragma unroll
+            for (int q = 0; q < R; ++q) out[(j * R + q) * pitch + p] = v[u][q];
+        }
+    }
+    __syncthreads();
+}
+
+// Wave number k of row y, from the transform Z of the complex lines that rows 2p
+// and 2p + 1 make:  A_k = (Z_k + conj Z_{N-k}) / 2,  B_k = (Z_k - conj Z_{N-k}) / 2i.
+template <typename R2>
+__device__ __forceinline__ R2 paired_row(const R2* Z, int pitch, int Kz, int y, int k) {
+    using real = decltype(Z->x);
+    const bool second = y & 1;
+    const int p = y >> 1;
+    const R2 zk = Z[k * pitch + p], zn = Z[(k == 0 ? 0 : Kz - k) * pitch + p];
+    R2 r;
+    r.x = (real)0.5 * (second ? zk.y + zn.y : zk.x + zn.x);
+    r.y = (real)0.5 * (second ? zn.x - zk.x : zk.y - zn.y);
+    return r;
+}
+
+// Point m of the complex line a + ib whose inverse transform holds two real rows,
+// from the half spectra: row(ks, 0) of the first, row(ks, 1) of the second.
+template <typename R2, class Row>
+__device__ __forceinline__ R2 paired_point(int m, int Kz, Row&& row) {
+    const bool hi = 2 * m > Kz;               // upper half from the Hermitian symmetry
+    const int ks = hi ? Kz - m : m;
+    R2 a = row(ks, 0), b = row(ks, 1);
+    if (ks == 0 || 2 * ks == Kz) { a.y = 0; b.y = 0; }      // DC and Nyquist terms are real
+    if (hi) { a.y = -a.y; b.y = -b.y; }
+    R2 z;
+    z.x = a.x - b.y;
+    z.y = a.y + b.x;
+    return z;
+}
+
 // Z pass forward with the spread: rows y0 .. y0 + ny - 1 of plane x, two rows as
 // one complex line (see fft_plane_fwd).  item = (sys, x, y0, ny)
 template <class P>
@@ -518,7 +655,6 @@ __global__ __launch_bounds__(kSpreadZThreads) void fft_z_spread(const SysDev* __
                                                                typename P::real2* cgrid,
                                                                const typename P::real2* __restrict__ tw) {
     side_priority();
-    using real = typename P::real;
     using R2 = typename P::real2;
     extern __shared__ unsigned char smem_raw[];
     const int4 it = items[blockIdx.x];
@@ -526,47 +662,24 @@ __global__ __launch_bounds__(kSpreadZThreads) void fft_z_spread(const SysDev* __
     const SysCount& sc = sp.sc[it.x];
     if (sc.n_slots == 0 || sc.overflow) return;      // overflowed build: the system is frozen
     const int x = it.y, y0 = it.z, ny = it.w;
-    const int Ky = d.grid[1], Kz = d.grid[2], Kzh = Kz / 2 + 1, np = (ny + 1) >> 1, cap = np * Kz;
+    const int Ky = d.grid[1], Kz = d.grid[2], Kzh = Kz / 2 + 1, np = (ny + 1) >> 1, pz = np | 1, cap = pz * Kz;
     R2* TW = reinterpret_cast<R2*>(smem_raw);
     R2* A = TW + Kz;
     R2* B = A + cap;
     load_twiddles(TW, tw + d.tw_off[2], Kz);
-    typename P::gacc* g = reinterpret_cast<typename P::gacc*>(A);
+    long long* g = reinterpret_cast<long long*>(A);
     spread_rows<P>(d, sp, pos, x, y0, ny, reinterpret_cast<int*>(A + spread_points<R2>(cap, ny, Kz)), g);
-    // through registers into place, as in fft_plane_fwd
-    const float inv_kz = 1.0f / (float)Kz;
-    R2 v[kSpreadZPerThread];
-#pragma unroll
-    for (int u = 0; u < kSpreadZPerThread; ++u) {
-        const int i = threadIdx.x + u * kSpreadZThreads;
-        if (i < cap) {
-            const int p = qdiv(i, inv_kz), z = i - p * Kz;
-            v[u].x = fixed_to_real(grid_value<true>(g, 2 * p, z, Kz), (real)0);
-            v[u].y = (2 * p + 1 < ny) ? fixed_to_real(grid_value<true>(g, 2 * p + 1, z, Kz), (real)0) : (real)0;
-        }
-    }
+    const unsigned plan = d.fft_plan[2];
+    const int r0 = plan & 15;
+    with_radix(r0, [&](auto R) { fft_sums_stage<R.value, kSpreadZThreads, kSpreadZPoints>(g, ny, np, Kz, pz, A); });
+    const R2* Z = fft_lines<-1, false, false>(Kz, plan >> 4, np, pz, TW, B, A, r0, [](int, int) { return R2{}; },
+                                              KeepLine<R2>{pz});
     __syncthreads();
-#pragma unroll
-    for (int u = 0; u < kSpreadZPerThread; ++u) {
-        const int i = threadIdx.x + u * kSpreadZThreads;
-        if (i < cap) A[i] = v[u];
-    }
-    __syncthreads();
-    R2* Z = fft_lines_lds<real, R2>(A, B, Kz, np, Kz, 1, TW, -1);
     R2* c = cgrid + d.cgrid_off + ((long long)x * Ky + y0) * Kzh;
     const float inv_kzh = 1.0f / (float)Kzh;
     for (int i = threadIdx.x; i < ny * Kzh; i += kSpreadZThreads) {
         const int y = qdiv(i, inv_kzh), k = i - y * Kzh;
-        const R2 zk = Z[(y >> 1) * Kz + k], zn = Z[(y >> 1) * Kz + (k == 0 ? 0 : Kz - k)];
-        R2 r;
-        if (y & 1) {
-            r.x = (real)0.5 * (zk.y + zn.y);
-            r.y = (real)0.5 * (zn.x - zk.x);
-        } else {
-            r.x = (real)0.5 * (zk.x + zn.x);
-            r.y = (real)0.5 * (zk.y - zn.y);
-        }
-        c[i] = r;
+        c[i] = paired_row(Z, pz, Kz, y, k);
     }
 }
 
@@ -579,33 +692,25 @@ __global__ __launch_bounds__(256) void fft_z_fwd(const SysDev* __restrict__ sd, 
     using real = typename P::real;
     using R2 = typename P::real2;
     extern __shared__ unsigned char smem_raw[];
-    R2* smem = reinterpret_cast<R2*>(smem_raw);
     const int4 it = items[blockIdx.x];
     const SysDev& d = sd[it.x];
     const int Kz = d.grid[2], Kzh = Kz / 2 + 1;
     const int line0 = it.y, nl = it.z;
-    R2* A = smem;
-    R2* B = smem + nl * Kz;
+    R2* A = reinterpret_cast<R2*>(smem_raw);
+    R2* B = A + nl * Kz;
     R2* TW = B + nl * Kz;
     load_twiddles(TW, tw + d.tw_off[2], Kz);
-    const typename P::gacc* g = rgrid + d.rgrid_off + (long long)line0 * Kz;
-    for (int i = threadIdx.x; i < nl * Kz; i += blockDim.x) {
-        R2 v;
-        v.x = fixed_to_real(g[i], (real)0);
-        v.y = 0;
-        A[i] = v;
-    }
     __syncthreads();
-    R2* res = fft_lines_lds<real, R2>(A, B, Kz, nl, Kz, 1, TW, -1);
+    const typename P::gacc* g = rgrid + d.rgrid_off + (long long)line0 * Kz;
     R2* c = cgrid + d.cgrid_off + (long long)line0 * Kzh;
-    const float inv_kzh = 1.0f / (float)Kzh;
-    for (int i = threadIdx.x; i < nl * Kzh; i += blockDim.x) {
-        const int t = qdiv(i, inv_kzh), kz = i - t * Kzh;
-        c[i] = res[t * Kz + kz];
-    }
+    fft_lines<-1, false, false>(
+        Kz, d.fft_plan[2], nl, nl, TW, A, B, 1,
+        [=](int m, int l) { return R2{fixed_to_real(g[l * Kz + m], (real)0), (real)0}; },
+        [=](R2*, int m, int l, R2 v) { if (m < Kzh) c[l * Kzh + m] = v; });
 }
 
-// Z pass inverse: C2R into the potential grid.
+// Z pass inverse: C2R into the potential grid, two rows as one complex line.
+// item = (sys, first row, n rows)
 template <class P>
 __global__ __launch_bounds__(256) void fft_z_inv(const SysDev* __restrict__ sd, const int4* __restrict__ items,
                                                  const typename P::real2* __restrict__ cgrid, typename P::real* phi,
@@ -614,154 +719,49 @@ __global__ __launch_bounds__(256) void fft_z_inv(const SysDev* __restrict__ sd, 
     using real = typename P::real;
     using R2 = typename P::real2;
     extern __shared__ unsigned char smem_raw[];
-    R2* smem = reinterpret_cast<R2*>(smem_raw);
     const int4 it = items[blockIdx.x];
     const SysDev& d = sd[it.x];
     const int Kz = d.grid[2], Kzh = Kz / 2 + 1;
-    const int line0 = it.y, nl = it.z;
-    R2* A = smem;
-    R2* B = smem + nl * Kz;
-    R2* TW = B + nl * Kz;
+    const int line0 = it.y, nl = it.z, np = (nl + 1) >> 1, pz = np | 1;
+    R2* A = reinterpret_cast<R2*>(smem_raw);
+    R2* B = A + pz * Kz;
+    R2* TW = B + pz * Kz;
     load_twiddles(TW, tw + d.tw_off[2], Kz);
-    const R2* c = cgrid + d.cgrid_off + (long long)line0 * Kzh;
-    const float inv_kz = 1.0f / (float)Kz;
-    for (int i = threadIdx.x; i < nl * Kz; i += blockDim.x) {
-        const int t = qdiv(i, inv_kz), z = i - t * Kz;
-        R2 v;
-        if (z < Kzh) v = c[t * Kzh + z];
-        else { v = c[t * Kzh + (Kz - z)]; v.y = -v.y; }
-        A[i] = v;
-    }
     __syncthreads();
-    R2* res = fft_lines_lds<real, R2>(A, B, Kz, nl, Kz, 1, TW, +1);
+    const R2* c = cgrid + d.cgrid_off + (long long)line0 * Kzh;
     const int pitch = Kz + pad;
     real* o = phi + d.rgrid_off + (long long)line0 * pitch;
-    for (int i = threadIdx.x; i < nl * pitch; i += blockDim.x) {
-        const int t = qdiv(i, 1.0f / (float)pitch), z = i - t * pitch;
-        o[i] = res[t * Kz + (z < Kz ? z : z - Kz)].x;
-    }
+    fft_lines<+1, true, true>(
+        Kz, d.fft_plan[2], np, pz, TW, A, B, 1,
+        [=](int m, int p) {
+            return paired_point<R2>(m, Kz, [=](int ks, int second) {
+                return !second || 2 * p + 1 < nl ? c[(2 * p + second) * Kzh + ks] : R2{};
+            });
+        },
+        [=](R2*, int m, int p, R2 v) { store_rows(o + 2 * p * pitch, pitch, 2 * p + 1 < nl, m, Kz, pad, v); });
 }
 
 // Y pass: tile (sys, x, kz0) of TZ consecutive kz columns, lines along y.
-template <class P>
+template <class P, int SIGN>
 __global__ __launch_bounds__(256) void fft_y(const SysDev* __restrict__ sd, const int4* __restrict__ items,
                                              typename P::real2* cgrid, const typename P::real2* __restrict__ tw,
-                                             int TZ, int sign) {
+                                             int TZ) {
     side_priority();
-    using real = typename P::real;
     using R2 = typename P::real2;
     extern __shared__ unsigned char smem_raw[];
-    R2* smem = reinterpret_cast<R2*>(smem_raw);
     const int4 it = items[blockIdx.x];
     const SysDev& d = sd[it.x];
     const int Ky = d.grid[1], Kzh = d.grid[2] / 2 + 1;
-    const int x = it.y, kz0 = it.z;
-    const int nt = min(TZ, Kzh - kz0);
-    R2* A = smem;
-    R2* B = smem + TZ * Ky;
-    R2* TW = B + TZ * Ky;
+    const int x = it.y, kz0 = it.z, nt = min(TZ, Kzh - kz0);
+    R2* A = reinterpret_cast<R2*>(smem_raw);
+    R2* B = A + nt * Ky;
+    R2* TW = B + nt * Ky;
     load_twiddles(TW, tw + d.tw_off[1], Ky);
+    __syncthreads();
     R2* c = cgrid + d.cgrid_off + (long long)x * Ky * Kzh + kz0;
-    const float inv_nt = 1.0f / (float)nt;
-    for (int i = threadIdx.x; i < nt * Ky; i += blockDim.x) {
-        const int y = qdiv(i, inv_nt), t = i - y * nt;
-        A[t * Ky + y] = c[(long long)y * Kzh + t];
-    }
-    __syncthreads();
-    R2* res = fft_lines_lds<real, R2>(A, B, Ky, nt, Ky, 1, TW, sign);
-    for (int i = threadIdx.x; i < nt * Ky; i += blockDim.x) {
-        const int y = qdiv(i, inv_nt), t = i - y * nt;
-        c[(long long)y * Kzh + t] = res[t * Ky + y];
-    }
-}
-
-// X pass: forward FFT along x, convolution with eta (and energy), inverse FFT.
-template <class P, bool ENERGY>
-__global__ __launch_bounds__(256) void fft_x_conv(const SysDev* __restrict__ sd, const int4* __restrict__ items,
-                                                  typename P::real2* cgrid, const typename P::real* __restrict__ eta,
-                                                  const typename P::real2* __restrict__ tw, int TZ,
-                                                  long long* energy) {
-    side_priority();
-    using real = typename P::real;
-    using R2 = typename P::real2;
-    extern __shared__ unsigned char smem_raw[];
-    R2* smem = reinterpret_cast<R2*>(smem_raw);
-    const int4 it = items[blockIdx.x];
-    const int s = it.x;
-    const SysDev& d = sd[s];
-    const int Kx = d.grid[0], Ky = d.grid[1], Kz = d.grid[2], Kzh = Kz / 2 + 1;
-    const int y = it.y, kz0 = it.z;
-    const int nt = min(TZ, Kzh - kz0);
-    R2* A = smem;
-    R2* B = smem + TZ * Kx;
-    const long long sx = (long long)Ky * Kzh;
-    R2* c = cgrid + d.cgrid_off + (long long)y * Kzh + kz0;
-    const real* et = eta + d.cgrid_off + (long long)y * Kzh + kz0;
-    R2* TW = B + TZ * Kx;
-    load_twiddles(TW, tw + d.tw_off[0], Kx);
-    const float inv_nt = 1.0f / (float)nt;
-    for (int i = threadIdx.x; i < nt * Kx; i += blockDim.x) {
-        const int x = qdiv(i, inv_nt), t = i - x * nt;
-        A[t * Kx + x] = c[x * sx + t];
-    }
-    __syncthreads();
-    R2* res = fft_lines_lds<real, R2>(A, B, Kx, nt, Kx, 1, TW, -1);
-    long long e = 0;   // fixed point per element: independent of the tile shape
-    for (int i = threadIdx.x; i < nt * Kx; i += blockDim.x) {
-        const int x = qdiv(i, inv_nt), t = i - x * nt;
-        const real w = eta ? et[x * sx + t] : (real)0;
-        R2 v = res[t * Kx + x];
-        if constexpr (ENERGY) {
-            const int kz = kz0 + t;
-            const double wt = (kz == 0 || (2 * kz == Kz)) ? 0.5 : 1.0;
-            e += energy_fixed(wt * (double)w * ((double)v.x * v.x + (double)v.y * v.y));
-        }
-        v.x *= w;
-        v.y *= w;
-        res[t * Kx + x] = v;
-    }
-    __syncthreads();
-    R2* other = (res == A) ? B : A;
-    R2* res2 = fft_lines_lds<real, R2>(res, other, Kx, nt, Kx, 1, TW, +1);
-    for (int i = threadIdx.x; i < nt * Kx; i += blockDim.x) {
-        const int x = qdiv(i, inv_nt), t = i - x * nt;
-        c[x * sx + t] = res2[t * Kx + x];
-    }
-    if constexpr (ENERGY) block_energy_add(energy, s, E_RECIP, e);
-}
-
-// Plain X pass (no convolution) for the standalone transform.
-template <class P>
-__global__ __launch_bounds__(256) void fft_x_plain(const SysDev* __restrict__ sd, const int4* __restrict__ items,
-                                                   typename P::real2* cgrid, const typename P::real2* __restrict__ tw,
-                                                   int TZ, int sign) {
-    side_priority();
-    using real = typename P::real;
-    using R2 = typename P::real2;
-    extern __shared__ unsigned char smem_raw[];
-    R2* smem = reinterpret_cast<R2*>(smem_raw);
-    const int4 it = items[blockIdx.x];
-    const SysDev& d = sd[it.x];
-    const int Kx = d.grid[0], Ky = d.grid[1], Kzh = d.grid[2] / 2 + 1;
-    const int y = it.y, kz0 = it.z;
-    const int nt = min(TZ, Kzh - kz0);
-    R2* A = smem;
-    R2* B = smem + TZ * Kx;
-    const long long sx = (long long)Ky * Kzh;
-    R2* c = cgrid + d.cgrid_off + (long long)y * Kzh + kz0;
-    R2* TW = B + TZ * Kx;
-    load_twiddles(TW, tw + d.tw_off[0], Kx);
-    const float inv_nt = 1.0f / (float)nt;
-    for (int i = threadIdx.x; i < nt * Kx; i += blockDim.x) {
-        const int x = qdiv(i, inv_nt), t = i - x * nt;
-        A[t * Kx + x] = c[x * sx + t];
-    }
-    __syncthreads();
-    R2* res = fft_lines_lds<real, R2>(A, B, Kx, nt, Kx, 1, TW, sign);
-    for (int i = threadIdx.x; i < nt * Kx; i += blockDim.x) {
-        const int x = qdiv(i, inv_nt), t = i - x * nt;
-        c[x * sx + t] = res[t * Kx + x];
-    }
+    fft_lines<SIGN, false, false>(
+        Ky, d.fft_plan[1], nt, nt, TW, A, B, 1, [=](int m, int l) { return c[m * Kzh + l]; },
+        [=](R2*, int m, int l, R2 v) { c[m * Kzh + l] = v; });
 }
 
 // ---------------------------------------------------------- plane FFT passes
@@ -770,17 +770,18 @@ __global__ __launch_bounds__(256) void fft_x_plain(const SysDev* __restrict__ sd
 // pass transforms along z and then y in one kernel, the x pass transforms
 // along x, multiplies by the influence function and transforms back, and the
 // inverse pass runs y and then z.  Three launches per step instead of five.
-// The real-to-complex z transform handles two real lines (y = 2p, 2p + 1) as
-// one complex line a + ib and separates them afterwards:
-//   A_k = (Z_k + conj Z_{N-k}) / 2,  B_k = (Z_k - conj Z_{N-k}) / 2i.
-// The complex-to-real inverse packs them the same way: Z_k = A_k + i B_k over
-// the Hermitian extension, then a = Re, b = Im of the inverse transform.
+// The real-to-complex z transform handles two real rows (2p and 2p + 1) as one
+// complex line a + ib and separates them as the y transform reads them
+// (paired_row); the complex-to-real inverse packs two rows (p and p + np: the
+// reads of neighbouring p then meet no bank twice) the same way, Z_k = A_k + i B_k
+// over the Hermitian extension (paired_point), then a = Re, b = Im.  Which rows
+// make a pair never depends on how the rows are dealt to workgroups.
 
 // Forward: plane x of the charge grid -> plane x of the half spectrum (z then y).
 // The grid's plane is spread here (SPREAD) or read from `rgrid`.
 // item = (sys, x)
 template <class P, bool SPREAD>
-__global__ __launch_bounds__(SPREAD ? kSpreadPlaneThreads : kPlaneThreads) void fft_plane_fwd(const SysDev* __restrict__ sd,
+__global__ __launch_bounds__(kPlaneThreads) void fft_plane_fwd(const SysDev* __restrict__ sd,
                                                               const int4* __restrict__ items,
                                                               const typename P::gacc* __restrict__ rgrid, SpreadArgs sp,
                                                               const typename P::real4* __restrict__ pos,
@@ -790,81 +791,49 @@ __global__ __launch_bounds__(SPREAD ? kSpreadPlaneThreads : kPlaneThreads) void 
     using real = typename P::real;
     using R2 = typename P::real2;
     extern __shared__ unsigned char smem_raw[];
-    R2* smem = reinterpret_cast<R2*>(smem_raw);
     const int4 it = items[blockIdx.x];
     const SysDev& d = sd[it.x];
     const int x = it.y;
     const int Ky = d.grid[1], Kz = d.grid[2], Kzh = Kz / 2 + 1, np = (Ky + 1) >> 1;
-    const int cap = max(np * Kz, Ky * Kzh);
-    R2* TWy = smem;
+    const int pz = np | 1, py = Kzh | 1, cap = plane_cap(Ky, Kz);
+    R2* TWy = reinterpret_cast<R2*>(smem_raw);
     R2* TWz = TWy + Ky;
     R2* A = TWz + Kz;
-    R2* Bf = A + cap;
-    load_twiddles(TWy, tw + d.tw_off[1], Ky);
-    load_twiddles(TWz, tw + d.tw_off[2], Kz);
-    const float inv_kz = 1.0f / (float)Kz;
-    // rows 2p and 2p + 1 as one complex line
-    auto line_pair = [&](const typename P::gacc* g, int i) {
-        const int p = qdiv(i, inv_kz), z = i - p * Kz;
-        R2 v;
-        v.x = fixed_to_real(grid_value<SPREAD>(g, 2 * p, z, Kz), (real)0);
-        v.y = (2 * p + 1 < Ky) ? fixed_to_real(grid_value<SPREAD>(g, 2 * p + 1, z, Kz), (real)0) : (real)0;
-        return v;
-    };
+    R2* B = A + cap;
+    const unsigned plan = d.fft_plan[2];
+    const R2* Z;
     if constexpr (SPREAD) {
-        // the sums take the room of the two line buffers: through registers into place
         const SysCount& sc = sp.sc[it.x];
         if (sc.n_slots == 0 || sc.overflow) return;      // overflowed build: the system is frozen
-        typename P::gacc* g = reinterpret_cast<typename P::gacc*>(A);
+        long long* g = reinterpret_cast<long long*>(A);
         spread_rows<P>(d, sp, pos, x, 0, Ky, reinterpret_cast<int*>(A + spread_points<R2>(cap, Ky, Kz)), g);
-        if constexpr (P::mixed) {
-            // a point of the line takes the room of the sum at its own index, and
-            // reads the sums at that index or past it
-            for (int b = 0; b < np * Kz; b += kSpreadPlaneThreads) {
-                const int i = b + threadIdx.x;
-                R2 v;
-                if (i < np * Kz) v = line_pair(g, i);
-                __syncthreads();
-                if (i < np * Kz) A[i] = v;
-            }
-        } else {
-            constexpr int kMax = (int)(kMaxBlockLds / (2 * sizeof(R2)) + kSpreadPlaneThreads - 1) / kSpreadPlaneThreads;
-            R2 v[kMax];
-#pragma unroll
-            for (int u = 0; u < kMax; ++u) {
-                const int i = threadIdx.x + u * kSpreadPlaneThreads;
-                if (i < np * Kz) v[u] = line_pair(g, i);
-            }
-            __syncthreads();
-#pragma unroll
-            for (int u = 0; u < kMax; ++u) {
-                const int i = threadIdx.x + u * kSpreadPlaneThreads;
-                if (i < np * Kz) A[i] = v[u];
-            }
-        }
+        load_twiddles(TWy, tw + d.tw_off[1], Ky);
+        load_twiddles(TWz, tw + d.tw_off[2], Kz);
+        const int r0 = plan & 15;
+        with_radix(r0, [&](auto R) {
+            fft_sums_stage<R.value, kPlaneThreads, (int)(kPlaneSpreadLds / (2 * sizeof(R2)))>(g, Ky, np, Kz, pz, A);
+        });
+        Z = fft_lines<-1, false, false>(Kz, plan >> 4, np, pz, TWz, B, A, r0, [](int, int) { return R2{}; },
+                                        KeepLine<R2>{pz});
     } else {
+        load_twiddles(TWy, tw + d.tw_off[1], Ky);
+        load_twiddles(TWz, tw + d.tw_off[2], Kz);
+        __syncthreads();
         const typename P::gacc* g = rgrid + d.rgrid_off + (long long)x * Ky * Kz;
-        for (int i = threadIdx.x; i < np * Kz; i += blockDim.x) A[i] = line_pair(g, i);
+        Z = fft_lines<-1, true, false>(
+            Kz, plan, np, pz, TWz, B, A, 1,
+            [=](int m, int p) {
+                return R2{fixed_to_real(g[2 * p * Kz + m], (real)0),
+                          2 * p + 1 < Ky ? fixed_to_real(g[(2 * p + 1) * Kz + m], (real)0) : (real)0};
+            },
+            KeepLine<R2>{pz});
     }
     __syncthreads();
-    R2* Z = fft_lines_lds<real, R2>(A, Bf, Kz, np, Kz, 1, TWz, -1);
-    R2* Q = (Z == A) ? Bf : A;
-    const float inv_kzh = 1.0f / (float)Kzh;
-    for (int i = threadIdx.x; i < np * Kzh; i += blockDim.x) {
-        const int p = qdiv(i, inv_kzh), k = i - p * Kzh;
-        const R2 zk = Z[p * Kz + k], zn = Z[p * Kz + (k == 0 ? 0 : Kz - k)];
-        R2 a, b;
-        a.x = (real)0.5 * (zk.x + zn.x);
-        a.y = (real)0.5 * (zk.y - zn.y);
-        b.x = (real)0.5 * (zk.y + zn.y);
-        b.y = (real)0.5 * (zn.x - zk.x);
-        Q[(2 * p) * Kzh + k] = a;
-        if (2 * p + 1 < Ky) Q[(2 * p + 1) * Kzh + k] = b;
-    }
-    __syncthreads();
-    R2* Y = fft_lines_lds<real, R2>(Q, Z, Ky, Kzh, 1, Kzh, TWy, -1);
-    R2* c = cgrid + d.cgrid_off + (long long)x * Ky * Kzh;       // the plane is contiguous
-    for (int i = threadIdx.x; i < Ky * Kzh; i += blockDim.x) c[i] = Y[i];
+    R2* c = cgrid + d.cgrid_off + (long long)x * Ky * Kzh;
+    fft_lines<-1, false, false>(
+        Ky, d.fft_plan[1], Kzh, py, TWy, Z == A ? B : A, Z == A ? A : B, 1,
+        [=](int m, int l) { return paired_row(Z, pz, Kz, m, l); },
+        [=](R2*, int m, int l, R2 v) { c[m * Kzh + l] = v; });
 }
 
 // Inverse: plane x of the half spectrum -> plane x of the potential (y then z).
@@ -878,114 +847,126 @@ __global__ __launch_bounds__(kPlaneThreads) void fft_plane_inv(const SysDev* __r
     using real = typename P::real;
     using R2 = typename P::real2;
     extern __shared__ unsigned char smem_raw[];
-    R2* smem = reinterpret_cast<R2*>(smem_raw);
     const int4 it = items[blockIdx.x];
     const SysDev& d = sd[it.x];
     const int x = it.y;
     const int Ky = d.grid[1], Kz = d.grid[2], Kzh = Kz / 2 + 1, np = (Ky + 1) >> 1;
-    const int cap = max(np * Kz, Ky * Kzh);
-    R2* TWy = smem;
+    const int pz = np | 1, py = Kzh | 1, cap = plane_cap(Ky, Kz);
+    R2* TWy = reinterpret_cast<R2*>(smem_raw);
     R2* TWz = TWy + Ky;
     R2* A = TWz + Kz;
-    R2* Bf = A + cap;
+    R2* B = A + cap;
     load_twiddles(TWy, tw + d.tw_off[1], Ky);
     load_twiddles(TWz, tw + d.tw_off[2], Kz);
+    __syncthreads();
     const R2* c = cgrid + d.cgrid_off + (long long)x * Ky * Kzh;
-    for (int i = threadIdx.x; i < Ky * Kzh; i += blockDim.x) A[i] = c[i];
+    R2* Y = fft_lines<+1, false, false>(Ky, d.fft_plan[1], Kzh, py, TWy, A, B, 1,
+                                        [=](int m, int l) { return c[m * Kzh + l]; }, KeepLine<R2>{py});
     __syncthreads();
-    R2* Y = fft_lines_lds<real, R2>(A, Bf, Ky, Kzh, 1, Kzh, TWy, +1);
-    R2* W = (Y == A) ? Bf : A;
-    const float inv_kz = 1.0f / (float)Kz;
-    for (int i = threadIdx.x; i < np * Kz; i += blockDim.x) {
-        const int p = qdiv(i, inv_kz), k = i - p * Kz;
-        const bool hi = k >= Kzh;                 // upper half from the Hermitian symmetry
-        const int ks = hi ? Kz - k : k;
-        R2 a = Y[(2 * p) * Kzh + ks];
-        R2 b;
-        if (2 * p + 1 < Ky) b = Y[(2 * p + 1) * Kzh + ks];
-        else { b.x = 0; b.y = 0; }
-        if (ks == 0 || 2 * ks == Kz) { a.y = 0; b.y = 0; }      // DC and Nyquist terms are real
-        if (hi) { a.y = -a.y; b.y = -b.y; }
-        R2 zv;
-        zv.x = a.x - b.y;
-        zv.y = a.y + b.x;
-        W[i] = zv;
-    }
-    __syncthreads();
-    R2* Z = fft_lines_lds<real, R2>(W, Y, Kz, np, Kz, 1, TWz, +1);
     const int pitch = Kz + pad;
-    const float inv_pitch = 1.0f / (float)pitch;
     real* o = phi + d.rgrid_off + (long long)x * Ky * pitch;
-    for (int i = threadIdx.x; i < np * pitch; i += blockDim.x) {
-        const int p = qdiv(i, inv_pitch), z = i - p * pitch;
-        const R2 v = Z[p * Kz + (z < Kz ? z : z - Kz)];
-        o[(2 * p) * pitch + z] = v.x;
-        if (2 * p + 1 < Ky) o[(2 * p + 1) * pitch + z] = v.y;
-    }
+    fft_lines<+1, false, true>(
+        Kz, d.fft_plan[2], np, pz, TWz, Y == A ? B : A, Y, 1,
+        [=](int m, int p) {
+            return paired_point<R2>(m, Kz, [=](int ks, int second) {
+                return !second || p + np < Ky ? Y[(p + second * np) * py + ks] : R2{};
+            });
+        },
+        [=](R2*, int m, int p, R2 v) { store_rows(o + p * pitch, np * pitch, p + np < Ky, m, Kz, pad, v); });
 }
 
-// X pass over the lines (y, k0 .. k0 + nk - 1): MODE 0 forward, 1 inverse,
-// 2 forward / influence function / inverse, 3 the same with the energy.
-// item = (sys, y, k0, nk)
+// X pass over nr consecutive (y, kz) lines from r0 = y Kzh + kz on (they stand
+// side by side in memory, whatever Kzh): MODE 0 forward, 1 inverse, 2 forward /
+// influence function / inverse, 3 the same with the energy.  The inverse takes
+// the radices in reverse, so its first stage needs the very points that the
+// forward's last one leaves in a thread's registers: the product and both stages
+// are one (64 points: two trips through LDS for both transforms).
+// item = (sys, r0, nr)
 template <class P, int MODE>
-__global__ __launch_bounds__(kPlaneThreads) void fft_x_block(const SysDev* __restrict__ sd,
-                                                            const int4* __restrict__ items,
-                                                            typename P::real2* cgrid,
-                                                            const typename P::real* __restrict__ eta,
-                                                            const typename P::real2* __restrict__ tw,
-                                                            long long* energy) {
+__global__ __launch_bounds__(kXPassThreads) void fft_x(const SysDev* __restrict__ sd, const int4* __restrict__ items,
+                                                      typename P::real2* cgrid,
+                                                      const typename P::real* __restrict__ eta,
+                                                      const typename P::real2* __restrict__ tw, long long* energy) {
     side_priority();
-    using real = typename P::real;
     using R2 = typename P::real2;
     extern __shared__ unsigned char smem_raw[];
-    R2* smem = reinterpret_cast<R2*>(smem_raw);
     const int4 it = items[blockIdx.x];
-    const int s = it.x, y = it.y, k0 = it.z, nk = it.w;
+    const int s = it.x, r0 = it.y, nr = it.z;
     const SysDev& d = sd[s];
     const int Kx = d.grid[0], Ky = d.grid[1], Kz = d.grid[2], Kzh = Kz / 2 + 1;
-    R2* TW = smem;
+    R2* TW = reinterpret_cast<R2*>(smem_raw);
     R2* A = TW + Kx;
-    R2* Bf = A + nk * Kx;
+    R2* B = A + nr * Kx;
     load_twiddles(TW, tw + d.tw_off[0], Kx);
-    const long long sx = (long long)Ky * Kzh;
-    R2* c = cgrid + d.cgrid_off + (long long)y * Kzh + k0;
-    const float inv_nk = 1.0f / (float)nk;
-    // A[x * nk + t]: one row of nk wave numbers per x
-    for (int i = threadIdx.x; i < Kx * nk; i += blockDim.x) {
-        const int x = qdiv(i, inv_nk), t = i - x * nk;
-        A[i] = c[x * sx + t];
-    }
     __syncthreads();
-    R2* R = fft_lines_lds<real, R2>(A, Bf, Kx, nk, 1, nk, TW, MODE == 1 ? +1 : -1);
-    if constexpr (MODE >= 2) {
-        const real* et = eta + d.cgrid_off + (long long)y * Kzh + k0;
-        long long e = 0;   // fixed point per element: independent of the tiling
-        for (int i = threadIdx.x; i < Kx * nk; i += blockDim.x) {
-            const int x = qdiv(i, inv_nk), t = i - x * nk;
-            const real w = et[x * sx + t];
-            R2 v = R[i];
-            if constexpr (MODE == 3) {
-                const int kz = k0 + t;
-                const double wt = (kz == 0 || (2 * kz == Kz)) ? 0.5 : 1.0;
-                e += energy_fixed(wt * (double)w * ((double)v.x * v.x + (double)v.y * v.y));
-            }
-            v.x *= w;
-            v.y *= w;
-            R[i] = v;
+    const int sx = Ky * Kzh;
+    R2* c = cgrid + d.cgrid_off + r0;
+    auto from_grid = [=](int m, int l) { return c[(long long)m * sx + l]; };
+    auto to_grid = [=](R2*, int m, int l, R2 v) { c[(long long)m * sx + l] = v; };
+    const unsigned plan = d.fft_plan[0];
+    if constexpr (MODE < 2) {
+        fft_lines<(MODE == 0 ? -1 : +1), false, false>(Kx, plan, nr, nr, TW, A, B, 1, from_grid, to_grid);
+    } else {
+        const auto* et = eta + d.cgrid_off + r0;
+        // the radices before the last, and the same in reverse
+        unsigned head = 0, back = 0, rest = plan;
+        int at = 0;
+        for (; rest >> 4; rest >>= 4, at += 4) {
+            head |= (rest & 15) << at;
+            back = back << 4 | (rest & 15);
         }
-        __syncthreads();
-        R = fft_lines_lds<real, R2>(R, R == A ? Bf : A, Kx, nk, 1, nk, TW, +1);
+        const R2* src = fft_lines<-1, false, false>(Kx, head, nr, nr, TW, A, B, 1, from_grid, KeepLine<R2>{nr});
+        if (head) __syncthreads();
+        R2* dst = src == A ? B : A;
+        long long e = 0;   // fixed point per element: independent of the tiling
+        with_radix((int)rest, [&](auto RC) {
+            constexpr int R = RC.value;
+            const int nb = Kx / R;
+            const float inv_nr = 1.0f / (float)nr, inv_kzh = 1.0f / (float)Kzh;
+            for (int w = threadIdx.x; w < nb * nr; w += blockDim.x) {
+                const int j = qdiv(w, inv_nr), l = w - j * nr;
+                typename P::real wt[R];
+#pragma unroll
+                for (int q = 0; q < R; ++q) wt[q] = et[(long long)(j + q * nb) * sx + l];
+                R2 v[R];
+                if (!head) {
+#pragma unroll
+                    for (int q = 0; q < R; ++q) v[q] = from_grid(j + q * nb, l);
+                } else {
+#pragma unroll
+                    for (int q = 0; q < R; ++q) v[q] = src[(j + q * nb) * nr + l];
+#pragma unroll
+                    for (int q = 1; q < R; ++q) v[q] = cmul(v[q], TW[j * q]);      // j q < Kx
+                }
+                dft<R, -1>(v);
+                if constexpr (MODE == 3) {
+                    const int kz = (r0 + l) - qdiv(r0 + l, inv_kzh) * Kzh;
+                    const double half = (kz == 0 || 2 * kz == Kz) ? 0.5 : 1.0;
+#pragma unroll
+                    for (int q = 0; q < R; ++q)
+                        e += energy_fixed(half * (double)wt[q] * ((double)v[q].x * v[q].x + (double)v[q].y * v[q].y));
+                }
+#pragma unroll
+                for (int q = 0; q < R; ++q) {
+                    v[q].x *= wt[q];
+                    v[q].y *= wt[q];
+                }
+                dft<R, +1>(v);
+                if (!head) {
+#pragma unroll
+                    for (int q = 0; q < R; ++q) to_grid(nullptr, j * R + q, l, v[q]);
+                } else {
+#pragma unroll
+                    for (int q = 0; q < R; ++q) dst[(j * R + q) * nr + l] = v[q];
+                }
+            }
+        });
+        if (head) {
+            __syncthreads();
+            fft_lines<+1, false, false>(Kx, back, nr, nr, TW, dst == A ? B : A, dst, (int)rest, from_grid, to_grid);
+        }
         if constexpr (MODE == 3) block_energy_add(energy, s, E_RECIP, e);
     }
-    for (int i = threadIdx.x; i < Kx * nk; i += blockDim.x) {
-        const int x = qdiv(i, inv_nk), t = i - x * nk;
-        c[x * sx + t] = R[i];
-    }
-}
-
-template <class P>
-static size_t fft_smem(const Batch<P>& B, int lines, int N) {
-    return (size_t)(2 * lines + 1) * N * sizeof(typename P::real2);   // two line buffers + twiddles
 }
 
 // NEXUSMD_FFT_PLANE=0 selects the five line passes even where planes fit.
@@ -1001,10 +982,9 @@ hipError_t prepare_fft(Batch<P>& B) {
     const hipFuncAttribute a = hipFuncAttributeMaxDynamicSharedMemorySize;
     hipError_t e = hipFuncSetAttribute(
         B.fft_split ? (const void*)fft_z_spread<P> : (const void*)fft_plane_fwd<P, true>, a, sl);
-    if (!B.fft_plane) return e;
-    if (e == hipSuccess) e = hipFuncSetAttribute((const void*)fft_plane_inv<P>, a, pl);
-    if (e == hipSuccess) e = hipFuncSetAttribute((const void*)fft_x_block<P, 2>, a, xl);
-    if (e == hipSuccess) e = hipFuncSetAttribute((const void*)fft_x_block<P, 3>, a, xl);
+    if (e == hipSuccess) e = hipFuncSetAttribute((const void*)fft_x<P, 2>, a, xl);
+    if (e == hipSuccess) e = hipFuncSetAttribute((const void*)fft_x<P, 3>, a, xl);
+    if (e == hipSuccess && B.fft_plane) e = hipFuncSetAttribute((const void*)fft_plane_inv<P>, a, pl);
     return e;
 }
 
@@ -1013,7 +993,7 @@ void launch_pme_spread(Batch<P>& B) {
     if (!B.pme_any) return;
     const SpreadArgs sp{B.d_cnt, B.col_count, B.col_slot};
     if (!B.fft_split)
-        fft_plane_fwd<P, true><<<B.n_fftz, kSpreadPlaneThreads, B.fft_spread_lds, B.stream>>>(
+        fft_plane_fwd<P, true><<<B.n_fftz, kPlaneThreads, B.fft_spread_lds, B.stream>>>(
             B.d_sys, B.fftz_items, nullptr, sp, B.pos, B.cgrid, B.twiddle);
     else
         fft_z_spread<P><<<B.n_fftz, kSpreadZThreads, B.fft_spread_lds, B.stream>>>(B.d_sys, B.fftz_items, sp, B.pos,
@@ -1023,42 +1003,30 @@ void launch_pme_spread(Batch<P>& B) {
 template <class P>
 void launch_fft_forward(Batch<P>& B) {
     if (!B.pme_any || !B.fft_split) return;      // the spread's launch ran the plane pass
-    fft_y<P><<<B.n_ffty, 256, fft_smem(B, B.fft_tile, B.fft_maxK), B.stream>>>(B.d_sys, B.ffty_items, B.cgrid,
-                                                                              B.twiddle, B.fft_tile, -1);
+    fft_y<P, -1><<<B.n_ffty, 256, B.fft_y_lds, B.stream>>>(B.d_sys, B.ffty_items, B.cgrid, B.twiddle, B.fft_tile);
 }
 
 template <class P>
 void launch_fft_convolve(Batch<P>& B, bool energy) {
     if (!B.pme_any) return;
-    if (B.fft_plane) {
-        if (energy)
-            fft_x_block<P, 3><<<B.n_fftx, kXPassThreads, B.fft_x_lds, B.stream>>>(B.d_sys, B.fftx_items, B.cgrid,
-                                                                                B.eta, B.twiddle, B.energy);
-        else
-            fft_x_block<P, 2><<<B.n_fftx, kXPassThreads, B.fft_x_lds, B.stream>>>(B.d_sys, B.fftx_items, B.cgrid,
-                                                                                B.eta, B.twiddle, B.energy);
-        return;
-    }
     if (energy)
-        fft_x_conv<P, true><<<B.n_fftx, 256, fft_smem(B, B.fft_tile, B.fft_maxK), B.stream>>>(
-            B.d_sys, B.fftx_items, B.cgrid, B.eta, B.twiddle, B.fft_tile, B.energy);
+        fft_x<P, 3><<<B.n_fftx, B.fft_x_threads, B.fft_x_lds, B.stream>>>(B.d_sys, B.fftx_items, B.cgrid, B.eta,
+                                                                         B.twiddle, B.energy);
     else
-        fft_x_conv<P, false><<<B.n_fftx, 256, fft_smem(B, B.fft_tile, B.fft_maxK), B.stream>>>(
-            B.d_sys, B.fftx_items, B.cgrid, B.eta, B.twiddle, B.fft_tile, B.energy);
+        fft_x<P, 2><<<B.n_fftx, B.fft_x_threads, B.fft_x_lds, B.stream>>>(B.d_sys, B.fftx_items, B.cgrid, B.eta,
+                                                                         B.twiddle, B.energy);
 }
 
 template <class P>
 void launch_fft_inverse(Batch<P>& B) {
     if (!B.pme_any) return;
     if (B.fft_plane) {
-        fft_plane_inv<P><<<B.n_fftp, kPlaneThreads, B.fft_plane_lds, B.stream>>>(B.d_sys, B.fftp_items, B.cgrid,
-                                                                               B.phi, B.twiddle, kPhiPad);
+        fft_plane_inv<P><<<B.n_fftp, B.fft_plane_threads, B.fft_plane_lds, B.stream>>>(B.d_sys, B.fftp_items, B.cgrid,
+                                                                                      B.phi, B.twiddle, kPhiPad);
         return;
     }
-    fft_y<P><<<B.n_ffty, 256, fft_smem(B, B.fft_tile, B.fft_maxK), B.stream>>>(B.d_sys, B.ffty_items, B.cgrid,
-                                                                              B.twiddle, B.fft_tile, +1);
-    fft_z_inv<P><<<B.n_fftl, 256, fft_smem(B, B.fft_lines, B.fft_maxK), B.stream>>>(B.d_sys, B.fftl_items, B.cgrid,
-                                                                                   B.phi, B.twiddle, kPhiPad);
+    fft_y<P, +1><<<B.n_ffty, 256, B.fft_y_lds, B.stream>>>(B.d_sys, B.ffty_items, B.cgrid, B.twiddle, B.fft_tile);
+    fft_z_inv<P><<<B.n_fftl, 256, B.fft_z_lds, B.stream>>>(B.d_sys, B.fftl_items, B.cgrid, B.phi, B.twiddle, kPhiPad);
 }
 
 template <class P>
@@ -1092,6 +1060,7 @@ void fft3d_roundtrip(int nx, int ny, int nz, const double* in, double* out, bool
     d.grid[0] = nx; d.grid[1] = ny; d.grid[2] = nz;
     d.rgrid_off = 0; d.cgrid_off = 0;
     d.tw_off[0] = 0; d.tw_off[1] = nx; d.tw_off[2] = nx + ny;
+    for (int a = 0; a < 3; ++a) d.fft_plan[a] = fft_plan(d.grid[a]);
     std::vector<R2> tw(nx + ny + nz);
     const int K[3] = {nx, ny, nz};
     for (int a = 0, o = 0; a < 3; o += K[a], ++a)
@@ -1107,7 +1076,7 @@ void fft3d_roundtrip(int nx, int ny, int nz, const double* in, double* out, bool
     for (int x = 0; x < nx; ++x)
         for (int k = 0; k < nzh; k += T) yi.push_back(make_int4(0, x, k, 0));
     for (int y = 0; y < ny; ++y)
-        for (int k = 0; k < nzh; k += T) xi.push_back(make_int4(0, y, k, 0));
+        for (int k = 0; k < nzh; k += T) xi.push_back(make_int4(0, y * nzh + k, std::min(T, nzh - k), 0));
     SysDev* dd; R2* dtw; int4 *dz, *dy, *dx; typename P::gacc* rg; R2* cg; real* ph;
     const size_t G = (size_t)nx * ny * nz, Gh = (size_t)nx * ny * nzh;
     hipMalloc(&dd, sizeof(SysDev));
@@ -1126,21 +1095,21 @@ void fft3d_roundtrip(int nx, int ny, int nz, const double* in, double* out, bool
     const size_t sm = (size_t)(2 * T + 1) * maxK * sizeof(R2);
     // plane passes (as the engine uses them) when the planes fit
     const bool plane = fft_plane_enabled() && plane_lds_bytes<R2>(ny, nz) <= kMaxBlockLds &&
-                       xpass_lds_bytes<R2>(nx, nzh) <= kMaxBlockLds;
+                       line_lds_bytes<R2>(nx, nzh) <= kMaxBlockLds;
     std::vector<int4> pi, bi;
     int4 *dp = nullptr, *db = nullptr;
-    const size_t pl = plane_lds_bytes<R2>(ny, nz), xl = xpass_lds_bytes<R2>(nx, nzh);
+    const size_t pl = plane_lds_bytes<R2>(ny, nz), xl = line_lds_bytes<R2>(nx, nzh);
     if (plane) {
         for (int x = 0; x < nx; ++x) pi.push_back(make_int4(0, x, 0, 0));
-        for (int y = 0; y < ny; ++y) bi.push_back(make_int4(0, y, 0, nzh));
+        for (int y = 0; y < ny; ++y) bi.push_back(make_int4(0, y * nzh, nzh, 0));
         hipMalloc(&dp, pi.size() * sizeof(int4));
         hipMalloc(&db, bi.size() * sizeof(int4));
         hipMemcpyAsync(dp, pi.data(), pi.size() * sizeof(int4), hipMemcpyHostToDevice, st);
         hipMemcpyAsync(db, bi.data(), bi.size() * sizeof(int4), hipMemcpyHostToDevice, st);
         hipFuncSetAttribute((const void*)fft_plane_fwd<P, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl);
         hipFuncSetAttribute((const void*)fft_plane_inv<P>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pl);
-        hipFuncSetAttribute((const void*)fft_x_block<P, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)xl);
-        hipFuncSetAttribute((const void*)fft_x_block<P, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)xl);
+        hipFuncSetAttribute((const void*)fft_x<P, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)xl);
+        hipFuncSetAttribute((const void*)fft_x<P, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)xl);
     }
     if (forward) {
         std::vector<typename P::gacc> h(G);
@@ -1150,11 +1119,11 @@ void fft3d_roundtrip(int nx, int ny, int nz, const double* in, double* out, bool
         hipMemcpyAsync(rg, h.data(), G * sizeof(typename P::gacc), hipMemcpyHostToDevice, st);
         if (plane) {
             fft_plane_fwd<P, false><<<(unsigned)pi.size(), kPlaneThreads, pl, st>>>(dd, dp, rg, {}, nullptr, cg, dtw);
-            fft_x_block<P, 0><<<(unsigned)bi.size(), kXPassThreads, xl, st>>>(dd, db, cg, nullptr, dtw, nullptr);
+            fft_x<P, 0><<<(unsigned)bi.size(), kXPassThreads, xl, st>>>(dd, db, cg, nullptr, dtw, nullptr);
         } else {
             fft_z_fwd<P><<<(unsigned)zi.size(), 256, sm, st>>>(dd, dz, rg, cg, dtw);
-            fft_y<P><<<(unsigned)yi.size(), 256, sm, st>>>(dd, dy, cg, dtw, T, -1);
-            fft_x_plain<P><<<(unsigned)xi.size(), 256, sm, st>>>(dd, dx, cg, dtw, T, -1);
+            fft_y<P, -1><<<(unsigned)yi.size(), 256, sm, st>>>(dd, dy, cg, dtw, T);
+            fft_x<P, 0><<<(unsigned)xi.size(), 256, sm, st>>>(dd, dx, cg, nullptr, dtw, nullptr);
         }
         std::vector<R2> hc(Gh);
         hipMemcpyAsync(hc.data(), cg, Gh * sizeof(R2), hipMemcpyDeviceToHost, st);
@@ -1165,11 +1134,11 @@ void fft3d_roundtrip(int nx, int ny, int nz, const double* in, double* out, bool
         for (size_t i = 0; i < Gh; ++i) { hc[i].x = (real)in[2 * i]; hc[i].y = (real)in[2 * i + 1]; }
         hipMemcpyAsync(cg, hc.data(), Gh * sizeof(R2), hipMemcpyHostToDevice, st);
         if (plane) {
-            fft_x_block<P, 1><<<(unsigned)bi.size(), kXPassThreads, xl, st>>>(dd, db, cg, nullptr, dtw, nullptr);
+            fft_x<P, 1><<<(unsigned)bi.size(), kXPassThreads, xl, st>>>(dd, db, cg, nullptr, dtw, nullptr);
             fft_plane_inv<P><<<(unsigned)pi.size(), kPlaneThreads, pl, st>>>(dd, dp, cg, ph, dtw, 0);
         } else {
-            fft_x_plain<P><<<(unsigned)xi.size(), 256, sm, st>>>(dd, dx, cg, dtw, T, +1);
-            fft_y<P><<<(unsigned)yi.size(), 256, sm, st>>>(dd, dy, cg, dtw, T, +1);
+            fft_x<P, 1><<<(unsigned)xi.size(), 256, sm, st>>>(dd, dx, cg, nullptr, dtw, nullptr);
+            fft_y<P, +1><<<(unsigned)yi.size(), 256, sm, st>>>(dd, dy, cg, dtw, T);
             fft_z_inv<P><<<(unsigned)zi.size(), 256, sm, st>>>(dd, dz, cg, ph, dtw, 0);
         }
         std::vector<real> hr(G);
@@ -1215,14 +1184,14 @@ void* g_noalloc_ptr[kNoAllocMaxDevices] = {};    // device address of each devic
 constexpr size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 // Work items of the forward passes, in fft3d_roundtrip's order.  Plane passes:
-// x planes, then y rows of the x pass over every kz.  Line passes: groups of
-// T z lines, then (x, kz block) and (y, kz block) items.
+// x planes, then the x pass's lines of one y.  Line passes: groups of T z
+// lines, then (x, kz block) items and the x pass's lines of a (y, kz block).
 __global__ void noalloc_items_kernel(int4* it, int nx, int ny, int nzh, int T, int plane, int n0, int n1, int n2) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n0 + n1 + n2) return;
     if (plane) {
         if (i < n0) it[i] = make_int4(0, i, 0, 0);
-        else it[i] = make_int4(0, i - n0, 0, nzh);
+        else it[i] = make_int4(0, (i - n0) * nzh, nzh, 0);
         return;
     }
     const int nkb = (nzh + T - 1) / T;
@@ -1233,8 +1202,8 @@ __global__ void noalloc_items_kernel(int4* it, int nx, int ny, int nzh, int T, i
         const int j = i - n0;
         it[i] = make_int4(0, j / nkb, (j % nkb) * T, 0);
     } else {
-        const int j = i - n0 - n1;
-        it[i] = make_int4(0, j / nkb, (j % nkb) * T, 0);
+        const int j = i - n0 - n1, k = (j % nkb) * T;
+        it[i] = make_int4(0, j / nkb * nzh + k, min(T, nzh - k), 0);
     }
 }
 
@@ -1265,7 +1234,7 @@ nx_status fft3d_r2c_noalloc(int device, int nx, int ny, int nz, const double* in
     const int maxK = std::max(nx, std::max(ny, nz));
     const int T = std::max(1, std::min(8, (int)((61440 / (int)sizeof(R2) - maxK) / (2 * maxK))));
     const bool plane = fft_plane_enabled() && plane_lds_bytes<R2>(ny, nz) <= kMaxBlockLds &&
-                       xpass_lds_bytes<R2>(nx, nzh) <= kMaxBlockLds;
+                       line_lds_bytes<R2>(nx, nzh) <= kMaxBlockLds;
     const int nkb = (nzh + T - 1) / T;
     const int n0 = plane ? nx : (nx * ny + T - 1) / T;
     const int n1 = plane ? ny : nx * nkb;
@@ -1305,6 +1274,7 @@ nx_status fft3d_r2c_noalloc(int device, int nx, int ny, int nz, const double* in
     SysDev d{};
     d.grid[0] = nx; d.grid[1] = ny; d.grid[2] = nz;
     d.tw_off[0] = 0; d.tw_off[1] = nx; d.tw_off[2] = nx + ny;
+    for (int a = 0; a < 3; ++a) d.fft_plan[a] = fft_plan(d.grid[a]);
     R2 tw[3 * kNoAllocMaxK];
     const int K[3] = {nx, ny, nz};
     for (int a = 0, o = 0; a < 3; o += K[a], ++a)
@@ -1321,19 +1291,19 @@ nx_status fft3d_r2c_noalloc(int device, int nx, int ny, int nz, const double* in
         return fail(e, "copy");
     noalloc_to_fixed_kernel<<<(unsigned)((G + 255) / 256), 256, 0, st>>>(rg, G, P::grid_scale);
     if (plane) {
-        const size_t pl = plane_lds_bytes<R2>(ny, nz), xl = xpass_lds_bytes<R2>(nx, nzh);
+        const size_t pl = plane_lds_bytes<R2>(ny, nz), xl = line_lds_bytes<R2>(nx, nzh);
         if ((e = hipFuncSetAttribute((const void*)fft_plane_fwd<P, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int)pl)) != hipSuccess ||
-            (e = hipFuncSetAttribute((const void*)fft_x_block<P, 0>, hipFuncAttributeMaxDynamicSharedMemorySize,
+            (e = hipFuncSetAttribute((const void*)fft_x<P, 0>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int)xl)) != hipSuccess)
             return fail(e, "hipFuncSetAttribute");
         fft_plane_fwd<P, false><<<(unsigned)n0, kPlaneThreads, pl, st>>>(dd, items, rg, {}, nullptr, cg, dtw);
-        fft_x_block<P, 0><<<(unsigned)n1, kXPassThreads, xl, st>>>(dd, items + n0, cg, nullptr, dtw, nullptr);
+        fft_x<P, 0><<<(unsigned)n1, kXPassThreads, xl, st>>>(dd, items + n0, cg, nullptr, dtw, nullptr);
     } else {
         const size_t sm = (size_t)(2 * T + 1) * maxK * sizeof(R2);
         fft_z_fwd<P><<<(unsigned)n0, 256, sm, st>>>(dd, items, rg, cg, dtw);
-        fft_y<P><<<(unsigned)n1, 256, sm, st>>>(dd, items + n0, cg, dtw, T, -1);
-        fft_x_plain<P><<<(unsigned)n2, 256, sm, st>>>(dd, items + n0 + n1, cg, dtw, T, -1);
+        fft_y<P, -1><<<(unsigned)n1, 256, sm, st>>>(dd, items + n0, cg, dtw, T);
+        fft_x<P, 0><<<(unsigned)n2, 256, sm, st>>>(dd, items + n0 + n1, cg, nullptr, dtw, nullptr);
     }
     if ((e = hipGetLastError()) != hipSuccess) return fail(e, "kernel launch");
     if ((e = hipMemcpyAsync(out, cg, (size_t)Gh * sizeof(R2), hipMemcpyDeviceToHost, st)) != hipSuccess)

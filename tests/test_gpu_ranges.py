@@ -165,3 +165,14 @@ def test_state_and_results_round_trip(n):
         ctx.set_state(bad)
     assert ex.value.status == L.NX_ERR_ARG and str(3 * (n // 2) + 1) in str(ex.value)
     ctx.close()
+
+
+@pytest.mark.parametrize("prec", [L.FP64, L.MIXED])
+@pytest.mark.parametrize("passes", ["plane", "lines"])
+@pytest.mark.parametrize("grid", [(8, 8, 8),        # one stage an axis
+                                  (6, 15, 10),      # odd rows, lines past the last full tile
+                                  (16, 27, 32),     # 4 4, 3 3 3, 4 8
+                                  (128, 25, 64)])   # three stages along x, 8 8 along z
+def test_transform_stages(grid, passes, prec, monkeypatch):
+    monkeypatch.setenv("NEXUSMD_FFT_PLANE", "1" if passes == "plane" else "0")
+    _check(_gas(411, (2.0, 2.3, 2.1), 5, grid=grid), prec, "stages %s %s" % (grid, passes))
