@@ -400,10 +400,11 @@ __device__ __forceinline__ int window_col(int k, int c0, int D, int nc, int nwin
     return st + k;
 }
 
-constexpr int kPlThreads = 256;       // threads per super-cluster in nl_pairlist
+constexpr int kPlThreads = 256;       // threads of nl_waves
 
-// Exclusive prefix sum over the kPlThreads threads of a block (thread order);
-// `total` receives the block sum.  Every thread must call it.
+// Exclusive prefix sum over the T threads of a block (thread order); `total`
+// receives the block sum.  Every thread must call it.
+template <int T>
 __device__ __forceinline__ int block_excl_scan(int v, int* wsum, int& total) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     int incl = v;
@@ -416,7 +417,7 @@ __device__ __forceinline__ int block_excl_scan(int v, int* wsum, int& total) {
     __syncthreads();
     int off = 0, tot = 0;
 #pragma unroll
-    for (int w = 0; w < kPlThreads / 64; ++w) {
+    for (int w = 0; w < T / 64; ++w) {
         const int x = wsum[w];
         off += (w < wv) ? x : 0;
         tot += x;
@@ -426,7 +427,15 @@ __device__ __forceinline__ int block_excl_scan(int v, int* wsum, int& total) {
     return off + incl - v;
 }
 
-// One block of kPlThreads per super-cluster item:
+// Super-clusters per CU up to which nl_pairlist takes 512 threads each instead of
+// 256.  Up to a few blocks per CU a build lasts as long as one block, and twice the
+// threads shorten its stages; past that the blocks fill the device, and half of
+// 512 threads would idle in the stages over a few hundred candidates.  A build's
+// launch, us, 512 and 256 threads: 48 super-clusters 40, 64; 2,000 121, 134; 20,000
+// 950, 903.  (1,024 threads: no gain over 512 at any size.)
+constexpr int kPlWide = 16;
+
+// One block of T threads per super-cluster item:
 //   1. the columns of the xy window whose rectangle comes within rlist of the
 //      super-cluster's box, in increasing column order; of their super-clusters,
 //      those whose box does (one thread each, ordered compaction);
@@ -434,12 +443,13 @@ __device__ __forceinline__ int block_excl_scan(int v, int* wsum, int& total) {
 //      i-cluster box, ordered compaction; the entry's periodic image
 //      (tile_image), when one image holds for all of its tiles, else the
 //      per-pair marker;
-//   3. per entry and i-cluster, the 64 atom pairs at build positions, one
-//      wavefront per entry: a tile is kept only if one of its pairs is within
+//   3. per entry and i-cluster, the 64 atom pairs at build positions and the
+//      entry's image, one wavefront per entry: a tile is kept only if one of its pairs is within
 //      rlist (both atoms move at most skin/2 before the next build, so every
 //      pair that can come within rc is in a kept tile); ordered compaction;
 //   4. exclusion masks for the kept tiles.
-__global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysCount* sc, const int* super_sys,
+template <int T>
+__global__ __launch_bounds__(T) void nl_pairlist(const SysDev* sd, SysCount* sc, const int* super_sys,
                                                           int4* super_item, const int* col_count,
                                                           const float4* cl_ctr,
                                                           const float4* cl_half, const float4* sup_ctr,
@@ -465,11 +475,11 @@ __global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysC
     __shared__ int l_eid[kListCap];
     __shared__ unsigned char l_img[kListCap];     // periodic image code of the entry's j cluster
     __shared__ unsigned int x_rec[kExclCap];      // (entry * 8 + i-cluster) << 6 | pair bit
-    __shared__ int n_x, id_base, lbase, cbase;
+    __shared__ int n_x, room[3];
     __shared__ float4 ic[8], ih[8];
     __shared__ float4 ip[64];                     // i-atom build positions (NaN for padding)
-    __shared__ int w_first[kPlThreads], w_pre[kPlThreads], near_s[kPlThreads];
-    __shared__ int wsum[kPlThreads / 64];
+    __shared__ int w_first[T], w_pre[T], near_s[T];
+    __shared__ int wsum[T / 64];
     if (tid == 0) n_x = 0;
     if (tid < 8) {
         if (tid < ncl) { ic[tid] = cl_ctr[fc + tid]; ih[tid] = cl_half[fc + tid]; }
@@ -479,6 +489,12 @@ __global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysC
         const float nan = __int_as_float(0x7fc00000);
         ip[tid] = ((tid >> 3) < ncl) ? slot_wpos[fc * 8 + tid] : make_float4(nan, nan, nan, 0.f);
     }
+    // the exclusions of stage 4, T / 64 threads per atom: the first one's slot is
+    // three loads away, which pass during the stages before
+    const int il = tid & 63, xsi = fc * 8 + il;
+    const int xai = (il >> 3) < ncl ? atom_of_slot[xsi] : -1;
+    const int x0 = xai >= 0 ? excl_off[xai] + (tid >> 6) : 0, x1 = xai >= 0 ? excl_off[xai + 1] : 0;
+    const int xsp = x0 < x1 ? slot_of_atom[excl_idx[x0]] : 0;
     __syncthreads();
     const float Lx = (float)d.L[0], Ly = (float)d.L[1], Lz = (float)d.L[2];
     const float iLx = (float)d.invL[0], iLy = (float)d.invL[1], iLz = (float)d.invL[2];
@@ -503,7 +519,7 @@ __global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysC
 
     // 1-2: candidates by cluster boxes
     int ne = 0;                                   // entries so far (the same in every thread)
-    for (int w0 = 0; w0 < nwin; w0 += kPlThreads) {
+    for (int w0 = 0; w0 < nwin; w0 += T) {
         const int w = w0 + tid;
         int nsu = 0, sfirst = 0;
         if (w < nwin) {
@@ -521,17 +537,17 @@ __global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysC
             }
         }
         int total;
-        const int pre = block_excl_scan(nsu, wsum, total);
+        const int pre = block_excl_scan<T>(nsu, wsum, total);
         w_pre[tid] = pre;
         w_first[tid] = sfirst;
         __syncthreads();
-        for (int b = 0; b < total; b += kPlThreads) {
+        for (int b = 0; b < total; b += T) {
             // a super-cluster each, from its own index on (the half list)
             const int t = b + tid;
             int sj = 0;
             bool near = false;
             if (t < total) {
-                int lo = 0, hi = kPlThreads - 1;      // last column whose range starts at or before t
+                int lo = 0, hi = T - 1;      // last column whose range starts at or before t
                 while (lo < hi) {
                     const int m = (lo + hi + 1) >> 1;
                     if (w_pre[m] <= t) lo = m; else hi = m - 1;
@@ -540,10 +556,10 @@ __global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysC
                 near = sj >= item && bbox_gap2(scc, sch, sup_ctr[sj], sup_half[sj], Lx, Ly, Lz) < rl2;
             }
             int nnear;
-            const int at = block_excl_scan(near, wsum, nnear);
+            const int at = block_excl_scan<T>(near, wsum, nnear);
             if (near) near_s[at] = sj;
             __syncthreads();
-            for (int c = 0; c < nnear * 8; c += kPlThreads) {
+            for (int c = 0; c < nnear * 8; c += T) {
                 const int u = c + tid;
                 unsigned int im = 0, img = kImgPerPair;
                 int cj = 0;
@@ -560,11 +576,11 @@ __global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysC
                                 const int ck = tile_image(ic[k], ih[k], jc, jh, Lx, Ly, Lz, iLx, iLy, iLz, img_slack);
                                 code = (ck < 0 || (code >= 0 && ck != code) || code == kImgMixed) ? kImgMixed : ck;
                             }
-                        img = (d.pair_image && code >= 0 && code != kImgMixed) ? image_bits(code) : kImgPerPair;
+                        img = (code >= 0 && code != kImgMixed) ? image_bits(code) : kImgPerPair;
                     }
                 }
                 int cnt;
-                const int pos = ne + block_excl_scan(im != 0, wsum, cnt);
+                const int pos = ne + block_excl_scan<T>(im != 0, wsum, cnt);
                 if (im && pos < kListCap) {
                     l_ent[pos] = (unsigned)cj | (im << 24);
                     l_img[pos] = (unsigned char)img;
@@ -578,18 +594,22 @@ __global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysC
     if (ne > kListCap) { overflow = true; ne = kListCap; }
 
     // 3: atom pairs, one wavefront per entry, batches of eight entries per
-    // wavefront so that their j loads overlap; the kept mask is written in place
+    // wavefront so that their j loads overlap; the kept mask is written in place.
+    // At the entry's image, which holds for every pair of its tiles, a pair costs
+    // 7 instructions, with the nearest image taken pair by pair 16.
     {
         const int ia = lane >> 3, ja = lane & 7;
         float4 pi[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) pi[k] = ip[k * 8 + ia];
-        for (int e0 = wv * 8; e0 < ne; e0 += kPlThreads / 8) {
-            unsigned int ent[8];
+        for (int e0 = wv * 8; e0 < ne; e0 += T / 8) {
+            unsigned int ent[8], img[8];
             float4 pj[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
-                ent[u] = (e0 + u < ne) ? l_ent[e0 + u] : 0u;
+                const bool have = e0 + u < ne;
+                ent[u] = __builtin_amdgcn_readfirstlane(have ? l_ent[e0 + u] : 0u);
+                img[u] = __builtin_amdgcn_readfirstlane(have ? l_img[e0 + u] : 0u);
                 pj[u] = slot_wpos[(ent[u] & 0xffffffu) * 8 + ja];
             }
 #pragma unroll
@@ -597,13 +617,21 @@ __global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysC
                 const int cj = (int)(ent[u] & 0xffffffu);
                 const unsigned int im = ent[u] >> 24;
                 unsigned int keep = 0;
+                const bool per_pair = img[u] == kImgPerPair;
+                if (!per_pair) {
+                    pj[u].x += (img[u] & 3u) == 1u ? Lx : ((img[u] & 3u) == 2u ? -Lx : 0.0f);
+                    pj[u].y += (img[u] & 12u) == 4u ? Ly : ((img[u] & 12u) == 8u ? -Ly : 0.0f);
+                    pj[u].z += (img[u] & 48u) == 16u ? Lz : ((img[u] & 48u) == 32u ? -Lz : 0.0f);
+                }
 #pragma unroll
                 for (int k = 0; k < 8; ++k) {
                     if (im & (1u << k)) {
                         float dx = pi[k].x - pj[u].x, dy = pi[k].y - pj[u].y, dz = pi[k].z - pj[u].z;
-                        dx -= Lx * rintf(dx * iLx);
-                        dy -= Ly * rintf(dy * iLy);
-                        dz -= Lz * rintf(dz * iLz);
+                        if (per_pair) {
+                            dx -= Lx * rintf(dx * iLx);
+                            dy -= Ly * rintf(dy * iLy);
+                            dz -= Lz * rintf(dz * iLz);
+                        }
                         // NaN (padding) compares false
                         bool ok = dx * dx + dy * dy + dz * dz < rl2;
                         if (cj == fc + k) ok = ok && ja > ia;
@@ -617,104 +645,90 @@ __global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysC
     __syncthreads();
     {
         int nk = 0;
-        for (int b = 0; b < ne; b += kPlThreads) {
+        for (int b = 0; b < ne; b += T) {
             const int e = b + tid;
             const unsigned int v = (e < ne) ? l_ent[e] : 0u;
             const unsigned char vi = (e < ne) ? l_img[e] : (unsigned char)0;
             const bool kept = (v >> 24) != 0u;
             int cnt;
-            const int pos = nk + block_excl_scan(kept, wsum, cnt);   // every read precedes every write
+            const int pos = nk + block_excl_scan<T>(kept, wsum, cnt);   // every read precedes every write
             if (kept) { l_ent[pos] = v; l_img[pos] = vi; }
             nk += cnt;
             __syncthreads();
         }
         ne = nk;
     }
-    for (int e = tid; e < ne; e += kPlThreads) l_eid[e] = -1;
+    for (int e = tid; e < ne; e += T) l_eid[e] = -1;
     __syncthreads();
 
-    // 4: exclusions of the 64 i-atoms that fall in kept tiles, four threads per atom
+    // 4: exclusions of the 64 i-atoms that fall in kept tiles
     {
-        const int il = tid & 63, part = tid >> 6;
         const int k = il >> 3, iat = il & 7;
-        if (k < ncl) {
-            const int si = (fc + k) * 8 + iat;
-            const int ai = atom_of_slot[si];
-            if (ai >= 0) {
-                for (int e = excl_off[ai] + part; e < excl_off[ai + 1]; e += kPlThreads / 64) {
-                    const int p = excl_idx[e];
-                    const int sp = slot_of_atom[p];
-                    const int cj = sp >> 3;
-                    if (cj < fc + k) continue;
-                    if (cj == fc + k && sp <= si) continue;
-                    int lo = 0, hi = ne;              // entries are sorted by cluster
-                    while (lo < hi) {
-                        const int m = (lo + hi) >> 1;
-                        if ((int)(l_ent[m] & 0xffffffu) < cj) lo = m + 1; else hi = m;
-                    }
-                    if (lo < ne && (int)(l_ent[lo] & 0xffffffu) == cj && ((l_ent[lo] >> 24) >> k & 1u)) {
-                        const int t = atomicAdd(&n_x, 1);
-                        if (t < kExclCap) x_rec[t] = ((unsigned)(lo * 8 + k) << 6) | (unsigned)(iat * 8 + (sp & 7));
-                        l_eid[lo] = 0;      // mark
-                    }
-                }
+        for (int e = x0; e < x1; e += T / 64) {
+            const int sp = e == x0 ? xsp : slot_of_atom[excl_idx[e]];
+            const int cj = sp >> 3;
+            if (cj < fc + k) continue;
+            if (cj == fc + k && sp <= xsi) continue;
+            int lo = 0, hi = ne;              // entries are sorted by cluster
+            while (lo < hi) {
+                const int m = (lo + hi) >> 1;
+                if ((int)(l_ent[m] & 0xffffffu) < cj) lo = m + 1; else hi = m;
+            }
+            if (lo < ne && (int)(l_ent[lo] & 0xffffffu) == cj && ((l_ent[lo] >> 24) >> k & 1u)) {
+                const int t = atomicAdd(&n_x, 1);
+                if (t < kExclCap) x_rec[t] = ((unsigned)(lo * 8 + k) << 6) | (unsigned)(iat * 8 + (sp & 7));
+                l_eid[lo] = 0;      // mark
             }
         }
     }
     __syncthreads();
     int nx_ = n_x;
     if (nx_ > kExclCap) { overflow = true; nx_ = kExclCap; }
-    // mask ids for the entries with exclusions, in entry order
+    // chunks of at most chunk_entries entries, as equal as they come
+    const int nch = (ne + d.chunk_entries - 1) / d.chunk_entries, ce = nch > 0 ? (ne + nch - 1) / nch : 1;
+    // mask ids for the entries with exclusions, in entry order; the room for them,
+    // for the entries and for the chunks in one atomic instruction
     {
         int nm = 0;
-        for (int b = 0; b < ne; b += kPlThreads) {
+        for (int b = 0; b < ne; b += T) {
             const int e = b + tid;
             const bool has = e < ne && l_eid[e] == 0;
             int cnt;
-            const int r = block_excl_scan(has, wsum, cnt);
+            const int r = block_excl_scan<T>(has, wsum, cnt);
             if (has) l_eid[e] = nm + r;
             nm += cnt;
         }
-        if (tid == 0) {
-            const int b = atomicAdd(&sc[s].emask_count, nm);
-            id_base = (b + nm > d.emask_cap) ? -1 : b;
+        if (tid < 3) {
+            const int n = tid == 0 ? nm : tid == 1 ? ne : nch;
+            const int cap = tid == 0 ? d.emask_cap : tid == 1 ? d.list_cap : d.chunk_cap;
+            const int b = atomicAdd(tid == 0 ? &sc[s].emask_count : tid == 1 ? &sc[s].list_count : &sc[s].n_chunks, n);
+            room[tid] = (b + n > cap) ? -1 : b;
         }
     }
     __syncthreads();
-    if (id_base < 0) overflow = true;
-    if (!overflow) {
-        for (int e = tid; e < ne; e += kPlThreads) {
-            if (l_eid[e] >= 0) {
-                const int g = d.emask_off + id_base + l_eid[e];
-                for (int k = 0; k < 8; ++k) emask[(size_t)g * 8 + k] = 0ull;
-            }
-        }
-        __syncthreads();
-        for (int t = tid; t < nx_; t += kPlThreads) {
-            const int ek = (int)(x_rec[t] >> 6), e = ek >> 3, k = ek & 7;
-            const int g = d.emask_off + id_base + l_eid[e];
-            atomicOr(&emask[(size_t)g * 8 + k], 1ull << (x_rec[t] & 63u));
-        }
-    }
-    // chunks of at most chunk_entries entries, as equal as they come
-    const int nch = (ne + d.chunk_entries - 1) / d.chunk_entries, ce = nch > 0 ? (ne + nch - 1) / nch : 1;
-    if (tid == 0) {
-        const int b = atomicAdd(&sc[s].list_count, ne);
-        lbase = (b + ne > d.list_cap) ? -1 : b;
-        const int c = atomicAdd(&sc[s].n_chunks, nch);
-        cbase = (c + nch > d.chunk_cap) ? -1 : c;
-    }
-    __syncthreads();
-    if (lbase < 0 || cbase < 0) overflow = true;
+    const int id_base = room[0], lbase = room[1], cbase = room[2];
+    if (id_base < 0 || lbase < 0 || cbase < 0) overflow = true;
     if (overflow) {
         if (tid == 0) atomicOr(&sc[s].overflow, 4);
         return;
     }
-    for (int e = tid; e < ne; e += kPlThreads) {
+    for (int e = tid; e < ne; e += T) {
+        if (l_eid[e] >= 0) {
+            const int g = d.emask_off + id_base + l_eid[e];
+            for (int k = 0; k < 8; ++k) emask[(size_t)g * 8 + k] = 0ull;
+        }
+    }
+    __syncthreads();
+    for (int t = tid; t < nx_; t += T) {
+        const int ek = (int)(x_rec[t] >> 6), e = ek >> 3, k = ek & 7;
+        const int g = d.emask_off + id_base + l_eid[e];
+        atomicOr(&emask[(size_t)g * 8 + k], 1ull << (x_rec[t] & 63u));
+    }
+    for (int e = tid; e < ne; e += T) {
         uint2 v;
         v.x = l_ent[e];
         v.y = ((l_eid[e] >= 0) ? (unsigned)(d.emask_off + id_base + l_eid[e]) : kNoMask) |
-              ((unsigned)l_img[e] << kImgShift);
+              ((d.pair_image ? (unsigned)l_img[e] : kImgPerPair) << kImgShift);
         list[d.list_off + lbase + e] = v;
     }
     if (tid == 0) {
@@ -722,7 +736,7 @@ __global__ __launch_bounds__(kPlThreads) void nl_pairlist(const SysDev* sd, SysC
         it.w = ne;
         super_item[item] = it;
     }
-    for (int c = tid; c < nch; c += kPlThreads) {
+    for (int c = tid; c < nch; c += T) {
         const int e0 = d.list_off + lbase + c * ce;
         const int e1 = d.list_off + lbase + min(ne, (c + 1) * ce);
         chunks[d.chunk_off + cbase + c] = make_int4(fc, ncl, e0, e1);
@@ -801,7 +815,7 @@ __global__ __launch_bounds__(kPlThreads) void nl_waves(const SysDev* sd, SysCoun
         // overflowed reserved chunk slots it did not write): no pair work
         const int n = (s < nsys && !sc[s].overflow) ? min(sc[s].n_chunks, sd[s].chunk_cap) : 0;
         int total;
-        const int pre = block_excl_scan(n, wsum, total);
+        const int pre = block_excl_scan<kPlThreads>(n, wsum, total);
         if (s < nsys) prefix[s] = carry + pre;
         carry += total;
     }
@@ -841,7 +855,8 @@ void launch_nlist(Batch<P>& B, bool clear_flags, int part) {
                                             B.col_super, B.slot_tmp, B.X, B.Y, B.Z, B.q, B.sig, B.eps,
                                             B.atom_of_slot, B.slot_of_atom, B.cl_ctr, B.cl_half, B.sup_ctr, B.sup_half,
                                             B.super_item, B.slot_wpos, B.pos, B.lj, B.XB, B.YB, B.ZB);
-    nl_pairlist<<<B.n_super_cap, kPlThreads, 0, st>>>(B.d_sys, B.d_cnt, B.super_sys, B.super_item, B.col_count,
+    const bool wide = B.n_super_cap <= kPlWide * B.n_cu;
+    (wide ? nl_pairlist<512> : nl_pairlist<256>)<<<B.n_super_cap, wide ? 512 : 256, 0, st>>>(B.d_sys, B.d_cnt, B.super_sys, B.super_item, B.col_count,
                                               B.cl_ctr, B.cl_half, B.sup_ctr, B.sup_half, B.col_super, B.slot_wpos, B.atom_of_slot, B.slot_of_atom, B.excl_off,
                                               B.excl_idx, B.list, B.emask, B.chunks, B.n_super_cap);
     if (part == 1) return;  // all but the last kernel

@@ -176,3 +176,9 @@ def test_state_and_results_round_trip(n):
 def test_transform_stages(grid, passes, prec, monkeypatch):
     monkeypatch.setenv("NEXUSMD_FFT_PLANE", "1" if passes == "plane" else "0")
     _check(_gas(411, (2.0, 2.3, 2.1), 5, grid=grid), prec, "stages %s %s" % (grid, passes))
+
+
+@pytest.mark.parametrize("prec", [L.FP64, L.MIXED])
+def test_list_of_a_system_that_fills_the_device(prec):
+    """More than 16 super-clusters per CU: the pair-list kernel's narrow blocks."""
+    _check(_gas(290000, (14.2, 14.4, 14.6), 6, grid=(80, 80, 80), cutoff=0.5), prec, "full device", skin=0.05)
