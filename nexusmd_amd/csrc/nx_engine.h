@@ -206,9 +206,11 @@ template <class P> void launch_pme_spread(Batch<P>& B);
 bool fft_plane_enabled();
 template <class P> hipError_t prepare_fft(Batch<P>& B);
 template <class P> void launch_fft_forward(Batch<P>& B);
-template <class P> void launch_fft_convolve(Batch<P>& B, bool energy);
+// without energies also the bonded terms of the kinds in term_mask
+template <class P> void launch_fft_convolve(Batch<P>& B, bool energy, int term_mask = 0);
 template <class P> void launch_fft_inverse(Batch<P>& B);
-template <class P> void launch_pme_gather(Batch<P>& B);
+// also the atom forces of a step with force mask atom_mask (launch_atom_forces), unless it is negative
+template <class P> void launch_pme_gather(Batch<P>& B, int atom_mask = -1);
 // the systems' energies [nsys][E_NTERMS] into total and their counters into counts (may be NULL)
 template <class P> void launch_energy_sum(Batch<P>& B, long long* total, SysCount* counts);
 template <class P> void launch_kinetic(Batch<P>& B, double dt);

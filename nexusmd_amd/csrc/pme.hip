@@ -30,8 +30,7 @@
 #include <string>
 #include <vector>
 
-#include "nx_device.h"
-#include "nx_engine.h"
+#include "nx_terms.h"
 
 namespace nx {
 
@@ -298,19 +297,27 @@ struct Row5 {
 };
 
 template <class P>
-__global__ __launch_bounds__(5 * kGatherSlots) void pme_gather_kernel(const SysDev* __restrict__ sd,
+__global__ __launch_bounds__(5 * kGatherSlots, 5) void pme_gather_kernel(const SysDev* __restrict__ sd,
                                                                      const SysCount* __restrict__ sc,
                                                                      const int* __restrict__ slot_sys,
                                                                      const int* __restrict__ atom_of_slot,
                                                                      const typename P::real4* __restrict__ pos,
                                                                      const typename P::real* __restrict__ phi,
                                                                      typename P::facc* FX, typename P::facc* FY,
-                                                                     typename P::facc* FZ, int n_slots_total) {
+                                                                     typename P::facc* FZ, int n_slots_total,
+                                                                     int atom_blocks, TermArgs<P> terms) {
     side_priority();
+    // the atom forces' blocks first: theirs is the longer chain of loads (the last
+    // ones, FP64, 100,000 atoms: a step of 368 us instead of 363)
+    if ((int)blockIdx.x < atom_blocks) {
+        const int a = (int)blockIdx.x * (5 * kGatherSlots) + (int)threadIdx.x;
+        atom_force<P, false>(terms, a, nullptr);
+        return;
+    }
     using real = typename P::real;
     __shared__ real part[3][5][kGatherSlots];
     const int ix = threadIdx.x / kGatherSlots, l = threadIdx.x - ix * kGatherSlots;
-    const int slot = blockIdx.x * kGatherSlots + l;
+    const int slot = ((int)blockIdx.x - atom_blocks) * kGatherSlots + l;
     bool on = slot < n_slots_total;
     int s = 0;
     if (on) {
@@ -875,6 +882,11 @@ __global__ __launch_bounds__(kPlaneThreads) void fft_plane_inv(const SysDev* __r
         [=](R2*, int m, int p, R2 v) { store_rows(o + p * pitch, np * pitch, p + np < Ky, m, Kz, pad, v); });
 }
 
+// fft_x's terms: in MODE 2 alone
+struct NoTerms {};
+template <class P, int MODE>
+using XTerms = typename std::conditional<MODE == 2, TermArgs<P>, NoTerms>::type;
+
 // X pass over nr consecutive (y, kz) lines from r0 = y Kzh + kz on (they stand
 // side by side in memory, whatever Kzh): MODE 0 forward, 1 inverse, 2 forward /
 // influence function / inverse, 3 the same with the energy.  The inverse takes
@@ -882,12 +894,26 @@ __global__ __launch_bounds__(kPlaneThreads) void fft_plane_inv(const SysDev* __r
 // forward's last one leaves in a thread's registers: the product and both stages
 // are one (64 points: two trips through LDS for both transforms).
 // item = (sys, r0, nr)
+//
+// A step's bonded terms ride along (MODE 2): the blocks past the items' are a
+// thread a term, and the forces per atom follow in the gather's launch.  On a small
+// system a launch costs the step about as much as its kernel, on the device and on
+// the host, which needs 5 us for a node of the two-branch step graph (as kernels of
+// their own, before the spread, the two made the 1,500-bead chain's step 64.6 us
+// instead of 51.2).
 template <class P, int MODE>
 __global__ __launch_bounds__(kXPassThreads) void fft_x(const SysDev* __restrict__ sd, const int4* __restrict__ items,
-                                                      typename P::real2* cgrid,
+                                                      int n_items, typename P::real2* cgrid,
                                                       const typename P::real* __restrict__ eta,
-                                                      const typename P::real2* __restrict__ tw, long long* energy) {
+                                                      const typename P::real2* __restrict__ tw, long long* energy,
+                                                      XTerms<P, MODE> terms) {
     side_priority();
+    if constexpr (MODE == 2) {
+        if ((int)blockIdx.x >= n_items) {
+            bonded_term<P, false>(terms, ((int)blockIdx.x - n_items) * (int)blockDim.x + (int)threadIdx.x, nullptr);
+            return;
+        }
+    }
     using R2 = typename P::real2;
     extern __shared__ unsigned char smem_raw[];
     const int4 it = items[blockIdx.x];
@@ -1007,14 +1033,17 @@ void launch_fft_forward(Batch<P>& B) {
 }
 
 template <class P>
-void launch_fft_convolve(Batch<P>& B, bool energy) {
+void launch_fft_convolve(Batch<P>& B, bool energy, int term_mask) {
     if (!B.pme_any) return;
-    if (energy)
-        fft_x<P, 3><<<B.n_fftx, B.fft_x_threads, B.fft_x_lds, B.stream>>>(B.d_sys, B.fftx_items, B.cgrid, B.eta,
-                                                                         B.twiddle, B.energy);
-    else
-        fft_x<P, 2><<<B.n_fftx, B.fft_x_threads, B.fft_x_lds, B.stream>>>(B.d_sys, B.fftx_items, B.cgrid, B.eta,
-                                                                         B.twiddle, B.energy);
+    const int T = B.fft_x_threads;
+    if (energy) {
+        fft_x<P, 3><<<B.n_fftx, T, B.fft_x_lds, B.stream>>>(B.d_sys, B.fftx_items, B.n_fftx, B.cgrid, B.eta, B.twiddle,
+                                                           B.energy, {});
+    } else {
+        const int blocks = (bonded_count(B, term_mask) + T - 1) / T;
+        fft_x<P, 2><<<B.n_fftx + blocks, T, B.fft_x_lds, B.stream>>>(B.d_sys, B.fftx_items, B.n_fftx, B.cgrid, B.eta,
+                                                                    B.twiddle, B.energy, term_args(B, term_mask));
+    }
 }
 
 template <class P>
@@ -1030,11 +1059,12 @@ void launch_fft_inverse(Batch<P>& B) {
 }
 
 template <class P>
-void launch_pme_gather(Batch<P>& B) {
+void launch_pme_gather(Batch<P>& B, int atom_mask) {
     if (!B.pme_any) return;
-    pme_gather_kernel<P><<<(unsigned)((B.n_slots_cap + kGatherSlots - 1) / kGatherSlots), 5 * kGatherSlots, 0,
-                           B.stream>>>(B.d_sys, B.d_cnt, B.slot_sys, B.atom_of_slot, B.pos, B.phi, B.FSx, B.FSy,
-                                       B.FSz, B.n_slots_cap);
+    const int T = 5 * kGatherSlots, atom_blocks = atom_mask >= 0 ? (B.n_atoms + T - 1) / T : 0;
+    pme_gather_kernel<P><<<(unsigned)(atom_blocks + (B.n_slots_cap + kGatherSlots - 1) / kGatherSlots), T, 0, B.stream>>>(
+        B.d_sys, B.d_cnt, B.slot_sys, B.atom_of_slot, B.pos, B.phi, B.FSx, B.FSy, B.FSz, B.n_slots_cap, atom_blocks,
+        term_args(B, atom_force_mask(B, std::max(0, atom_mask))));
 }
 
 template void launch_pme_spread<PrecFP64>(Batch<PrecFP64>&);
@@ -1043,12 +1073,12 @@ template hipError_t prepare_fft<PrecFP64>(Batch<PrecFP64>&);
 template hipError_t prepare_fft<PrecMixed>(Batch<PrecMixed>&);
 template void launch_fft_forward<PrecFP64>(Batch<PrecFP64>&);
 template void launch_fft_forward<PrecMixed>(Batch<PrecMixed>&);
-template void launch_fft_convolve<PrecFP64>(Batch<PrecFP64>&, bool);
-template void launch_fft_convolve<PrecMixed>(Batch<PrecMixed>&, bool);
+template void launch_fft_convolve<PrecFP64>(Batch<PrecFP64>&, bool, int);
+template void launch_fft_convolve<PrecMixed>(Batch<PrecMixed>&, bool, int);
 template void launch_fft_inverse<PrecFP64>(Batch<PrecFP64>&);
 template void launch_fft_inverse<PrecMixed>(Batch<PrecMixed>&);
-template void launch_pme_gather<PrecFP64>(Batch<PrecFP64>&);
-template void launch_pme_gather<PrecMixed>(Batch<PrecMixed>&);
+template void launch_pme_gather<PrecFP64>(Batch<PrecFP64>&, int);
+template void launch_pme_gather<PrecMixed>(Batch<PrecMixed>&, int);
 
 // Standalone 3D transform of one real grid through the same pass kernels.
 template <class P>
@@ -1119,11 +1149,11 @@ void fft3d_roundtrip(int nx, int ny, int nz, const double* in, double* out, bool
         hipMemcpyAsync(rg, h.data(), G * sizeof(typename P::gacc), hipMemcpyHostToDevice, st);
         if (plane) {
             fft_plane_fwd<P, false><<<(unsigned)pi.size(), kPlaneThreads, pl, st>>>(dd, dp, rg, {}, nullptr, cg, dtw);
-            fft_x<P, 0><<<(unsigned)bi.size(), kXPassThreads, xl, st>>>(dd, db, cg, nullptr, dtw, nullptr);
+            fft_x<P, 0><<<(unsigned)bi.size(), kXPassThreads, xl, st>>>(dd, db, (int)bi.size(), cg, nullptr, dtw, nullptr, {});
         } else {
             fft_z_fwd<P><<<(unsigned)zi.size(), 256, sm, st>>>(dd, dz, rg, cg, dtw);
             fft_y<P, -1><<<(unsigned)yi.size(), 256, sm, st>>>(dd, dy, cg, dtw, T);
-            fft_x<P, 0><<<(unsigned)xi.size(), 256, sm, st>>>(dd, dx, cg, nullptr, dtw, nullptr);
+            fft_x<P, 0><<<(unsigned)xi.size(), 256, sm, st>>>(dd, dx, (int)xi.size(), cg, nullptr, dtw, nullptr, {});
         }
         std::vector<R2> hc(Gh);
         hipMemcpyAsync(hc.data(), cg, Gh * sizeof(R2), hipMemcpyDeviceToHost, st);
@@ -1134,10 +1164,10 @@ void fft3d_roundtrip(int nx, int ny, int nz, const double* in, double* out, bool
         for (size_t i = 0; i < Gh; ++i) { hc[i].x = (real)in[2 * i]; hc[i].y = (real)in[2 * i + 1]; }
         hipMemcpyAsync(cg, hc.data(), Gh * sizeof(R2), hipMemcpyHostToDevice, st);
         if (plane) {
-            fft_x<P, 1><<<(unsigned)bi.size(), kXPassThreads, xl, st>>>(dd, db, cg, nullptr, dtw, nullptr);
+            fft_x<P, 1><<<(unsigned)bi.size(), kXPassThreads, xl, st>>>(dd, db, (int)bi.size(), cg, nullptr, dtw, nullptr, {});
             fft_plane_inv<P><<<(unsigned)pi.size(), kPlaneThreads, pl, st>>>(dd, dp, cg, ph, dtw, 0);
         } else {
-            fft_x<P, 1><<<(unsigned)xi.size(), 256, sm, st>>>(dd, dx, cg, nullptr, dtw, nullptr);
+            fft_x<P, 1><<<(unsigned)xi.size(), 256, sm, st>>>(dd, dx, (int)xi.size(), cg, nullptr, dtw, nullptr, {});
             fft_y<P, +1><<<(unsigned)yi.size(), 256, sm, st>>>(dd, dy, cg, dtw, T);
             fft_z_inv<P><<<(unsigned)zi.size(), 256, sm, st>>>(dd, dz, cg, ph, dtw, 0);
         }
@@ -1298,12 +1328,12 @@ nx_status fft3d_r2c_noalloc(int device, int nx, int ny, int nz, const double* in
                                      (int)xl)) != hipSuccess)
             return fail(e, "hipFuncSetAttribute");
         fft_plane_fwd<P, false><<<(unsigned)n0, kPlaneThreads, pl, st>>>(dd, items, rg, {}, nullptr, cg, dtw);
-        fft_x<P, 0><<<(unsigned)n1, kXPassThreads, xl, st>>>(dd, items + n0, cg, nullptr, dtw, nullptr);
+        fft_x<P, 0><<<(unsigned)n1, kXPassThreads, xl, st>>>(dd, items + n0, n1, cg, nullptr, dtw, nullptr, {});
     } else {
         const size_t sm = (size_t)(2 * T + 1) * maxK * sizeof(R2);
         fft_z_fwd<P><<<(unsigned)n0, 256, sm, st>>>(dd, items, rg, cg, dtw);
         fft_y<P, -1><<<(unsigned)n1, 256, sm, st>>>(dd, items + n0, cg, dtw, T);
-        fft_x<P, 0><<<(unsigned)n2, 256, sm, st>>>(dd, items + n0 + n1, cg, nullptr, dtw, nullptr);
+        fft_x<P, 0><<<(unsigned)n2, 256, sm, st>>>(dd, items + n0 + n1, n2, cg, nullptr, dtw, nullptr, {});
     }
     if ((e = hipGetLastError()) != hipSuccess) return fail(e, "kernel launch");
     if ((e = hipMemcpyAsync(out, cg, (size_t)Gh * sizeof(R2), hipMemcpyDeviceToHost, st)) != hipSuccess)

@@ -182,3 +182,22 @@ def test_transform_stages(grid, passes, prec, monkeypatch):
 def test_list_of_a_system_that_fills_the_device(prec):
     """More than 16 super-clusters per CU: the pair-list kernel's narrow blocks."""
     _check(_gas(290000, (14.2, 14.4, 14.6), 6, grid=(80, 80, 80), cutoff=0.5), prec, "full device", skin=0.05)
+
+
+@pytest.mark.parametrize("prec,tol", [(L.FP64, 1e-12), (L.MIXED, 1e-6)])
+@pytest.mark.parametrize("mask", [L.ALL, L.NONBONDED, L.NONBONDED | L.ANGLE, L.BOND | L.TORSION])
+@pytest.mark.parametrize("n", [7, 400])
+def test_terms_in_pme_launches(n, mask, prec, tol, monkeypatch):
+    """Six steps with the terms in PME's launches (beside the pair kernel) and in their
+    own: the same terms, so positions (nm) apart by rounding at most -- forces of
+    1e4 kJ/mol/nm off by 1e-16 or 6e-8 of themselves, dt^2 / m = 4e-7."""
+    s = S.bead_chain(n=n, L=2.6, grid=(24, 24, 24), seed=11)
+    out = []
+    for overlap in ("1", "0"):
+        monkeypatch.setenv("NEXUSMD_OVERLAP", overlap)
+        ctx = E.Context(s, precision=prec, skin=0.1)
+        ctx.step(6, 0.0005, mask)
+        out.append(np.asarray(ctx.get_state()[0]))
+        ctx.close()
+    print("[gpu] terms n=%d mask=%d: %.2e apart" % (n, mask, np.abs(out[0] - out[1]).max()), flush=True)
+    assert np.abs(out[0] - out[1]).max() <= tol
