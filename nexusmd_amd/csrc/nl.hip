@@ -25,7 +25,7 @@
 // Columns are about as wide as 64 atoms are tall, so a super-cluster is about a
 // cube and a j cluster near it meets most of its clusters: 5 tiles an entry on
 // liquids, where super-clusters of one 8-atom-wide column (3.5 nm tall) had 2.9.
-// The pair kernel pays ~45 instructions per entry besides its tiles.
+// The pair kernel pays ~35 instructions per entry besides its tiles (~49 each).
 // The pair kernel applies r^2 < rc^2 exactly per pair, so the evaluated pair
 // set is the reference's set whatever the buffer (skin) is.
 //

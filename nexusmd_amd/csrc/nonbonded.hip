@@ -190,6 +190,7 @@ __device__ __forceinline__ void pair_body(const SysDev* __restrict__ sd, const i
     real4* ipos = ipos_s[w];
     real2* ilj = ilj_s[w];
     real* jf = jf_s[w];
+    const bool j_out = lane < 48 && (lane & 8) == 0;     // lanes that hold a j force (sum3_stride8)
     uint2* jw = jw_s[w];
 
     // Each XCD's wavefronts (blocks b with b % 8 equal, as the hardware hands
@@ -204,10 +205,12 @@ __device__ __forceinline__ void pair_body(const SysDev* __restrict__ sd, const i
     // does not depend on who does it or when.
     int* counter = pool + (blockIdx.x & 7) * kPoolStride;
     const int hi = __builtin_amdgcn_readfirstlane(counter[kPoolEnd]);
-    // lane 0 claims the next chunk; the result is read (and waited for) later
+    // lane 0 claims the next chunk; the result is read (and waited for) later.  An
+    // increment, not an addition of 1: the compiler aggregates additions over the
+    // wavefront, and the code it makes for that waits for the result at once.
     auto claim = [&]() {
         int t = 0;
-        if (lane == 0) t = atomicAdd(counter, 1);
+        if (lane == 0) t = (int)atomicInc(reinterpret_cast<unsigned*>(counter), 0xffffffffu);
         return t;
     };
     auto claimed = [&](int t) { return __builtin_amdgcn_readfirstlane(t); };
@@ -342,12 +345,22 @@ __device__ __forceinline__ void pair_body(const SysDev* __restrict__ sd, const i
             const bool per_pair = !P::mixed || img == kImgPerPair;
             real4 pjs;
             {
-                const real sx = per_pair ? (real)0 : ((img & 3u) == 1u ? Lx : ((img & 3u) == 2u ? -Lx : (real)0));
-                const real sy = per_pair ? (real)0 : ((img & 12u) == 4u ? Ly : ((img & 12u) == 8u ? -Ly : (real)0));
-                const real sz = per_pair ? (real)0 : ((img & 48u) == 16u ? Lz : ((img & 48u) == 32u ? -Lz : (real)0));
-                pjs.x = (pj.x > (real)(0.5 * kPadPos)) ? (real)(-kPadPos) : pj.x + sx;
-                pjs.y = pj.y + sy;
-                pjs.z = pj.z + sz;
+                // +1, -1 or 0 boxes, selected in scalar registers (the pair-by-pair
+                // marker has both bits of an axis: 0)
+                auto boxes = [&](unsigned both, unsigned plus) {
+                    const unsigned b = img & both;
+                    const unsigned one = b == plus ? 0x3f800000u : (b == 2u * plus ? 0xbf800000u : 0u);
+                    return __uint_as_float(one);
+                };
+                real x = pj.x;
+                pjs.y = pj.y;
+                pjs.z = pj.z;
+                if constexpr (P::mixed) {
+                    x = fmaf(boxes(3u, 1u), Lx, x);
+                    pjs.y = fmaf(boxes(12u, 4u), Ly, pjs.y);
+                    pjs.z = fmaf(boxes(48u, 16u), Lz, pjs.z);
+                }
+                pjs.x = (pj.x > (real)(0.5 * kPadPos)) ? (real)(-kPadPos) : x;
                 pjs.w = pj.w;
             }
             real4 pj_n = pj;
@@ -431,17 +444,11 @@ __device__ __forceinline__ void pair_body(const SysDev* __restrict__ sd, const i
                     }
                 }
             }
-            fxj = sum_stride8(fxj);
-            fyj = sum_stride8(fyj);
-            fzj = sum_stride8(fzj);
+            const real fj = sum3_stride8(fxj, fyj, fzj);
             // staged in LDS: no global atomics inside the loop, so waiting for the
             // prefetched loads never waits behind atomics
             const int el = e - e0;
-            if (ia == 0) {
-                jf[(el * 3 + 0) * 8 + ja] = fxj;
-                jf[(el * 3 + 1) * 8 + ja] = fyj;
-                jf[(el * 3 + 2) * 8 + ja] = fzj;
-            }
+            if (j_out) jf[el * 24 + (lane >> 4) * 8 + ja] = fj;
             if (e + 2 < e1) wv = jw[el + 2];
             pj = pj_n;
             lj_j = lj_n;

@@ -388,6 +388,56 @@ __device__ __forceinline__ double sum_stride8(double v) {
     auto qh = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
     return __hiloint2double(qh[0], ql[0]) + __hiloint2double(qh[1], ql[1]);
 }
+// v[0], v[1], v[2] summed over the lanes with the same l & 7, each as sum_stride8
+// does: the sum of v[0] on lanes 0-15, of v[1] on 16-31, of v[2] on 32-63 (each at
+// every lane of its l & 7).  Two of them share a swap and an addition where one
+// alone wastes half: 10 instructions instead of 21.
+template <typename real>
+__device__ __forceinline__ void swap16(real& a, real& b);      // odd rows of 16 lanes of a with even ones of b
+template <typename real>
+__device__ __forceinline__ void swap32(real& a, real& b);      // upper half of a with the lower one of b
+template <>
+__device__ __forceinline__ void swap16(float& a, float& b) {
+    auto p = __builtin_amdgcn_permlane16_swap(__float_as_int(a), __float_as_int(b), false, false);
+    a = __int_as_float(p[0]);
+    b = __int_as_float(p[1]);
+}
+template <>
+__device__ __forceinline__ void swap32(float& a, float& b) {
+    auto p = __builtin_amdgcn_permlane32_swap(__float_as_int(a), __float_as_int(b), false, false);
+    a = __int_as_float(p[0]);
+    b = __int_as_float(p[1]);
+}
+template <>
+__device__ __forceinline__ void swap16(double& a, double& b) {
+    auto l = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+    auto h = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+    a = __hiloint2double(h[0], l[0]);
+    b = __hiloint2double(h[1], l[1]);
+}
+template <>
+__device__ __forceinline__ void swap32(double& a, double& b) {
+    auto l = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+    auto h = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+    a = __hiloint2double(h[0], l[0]);
+    b = __hiloint2double(h[1], l[1]);
+}
+__device__ __forceinline__ float add_ror8(float v) { return v + __int_as_float(dpp_ror8(__float_as_int(v))); }
+__device__ __forceinline__ double add_ror8(double v) {
+    return v + __hiloint2double(dpp_ror8(__double2hiint(v)), dpp_ror8(__double2loint(v)));
+}
+template <typename real>
+__device__ __forceinline__ real sum3_stride8(real x, real y, real z) {
+    x = add_ror8(x);
+    y = add_ror8(y);
+    z = add_ror8(z);
+    swap16(x, y);           // x: rows 0, 2 of x in rows 0, 2, of y in 1, 3; y: rows 1, 3
+    real xy = x + y, z2 = z;
+    swap16(z, z2);
+    z += z2;
+    swap32(xy, z);          // xy: rows 0, 1 of both; z: rows 2, 3
+    return xy + z;
+}
 // sum over the 8 lanes l & ~7 .. l | 7
 __device__ __forceinline__ float sum_group8(float v) {
     v += __int_as_float(dpp_xor1(__float_as_int(v)));
