@@ -527,13 +527,11 @@ class Engine : public EngineBase {
         B.fft_tile = T;
         B.fft_y_lds = line_lds_bytes<real2>(maxK, T);
         B.fft_z_lds = line_lds_bytes<real2>(maxK, pairs | 1);
-        // plane passes when every system's planes fit one workgroup's LDS
-        bool plane = fft_plane_enabled(), plane_spread = true;
+        bool plane = fft_plane_enabled();
         long long rows = 0, x_lines = 0;
         for (int s = 0; s < ns; ++s) {
             const SysDev& d = B.sys[s];
-            if (plane_lds_bytes<real2>(d.grid[1], d.grid[2]) > kMaxBlockLds) plane = false;
-            if (plane_spread_lds_bytes<real2>(d.grid[1], d.grid[2]) > kPlaneSpreadLds) plane_spread = false;
+            if (plane_spread_lds_bytes<real2>(d.grid[1], d.grid[2]) > kPlaneSpreadLds<real2>) plane = false;
             x_lines += (long long)d.grid[1] * (d.grid[2] / 2 + 1);
             rows += (long long)d.grid[0] * d.grid[1];
         }
@@ -545,13 +543,12 @@ class Engine : public EngineBase {
         B.fft_x_threads = 64;
         B.fft_plane_threads = 64;
         B.fft_plane = plane ? 1 : 0;
-        // The spread goes into the plane pass where the plane's workgroup finds room
-        // beside the pair kernel's on a CU: one launch and one trip of the spectrum
-        // less (us a step, together against apart: 100,000 atoms at 96^3 mixed 214,
-        // 220; the 1,500-bead chain 71, 72).  A larger one would wait for the pair
-        // kernel to end, and the spread then goes over rows (100,000 atoms FP64, 155
-        // KB a plane: 463 together, 412 apart).
-        B.fft_split = !plane || !plane_spread;
+        // Plane passes where the workgroup of every system's plane, the spread with it,
+        // finds room beside the pair kernel's on a CU: two launches and two trips of
+        // the spectrum less (us a step, planes against lines: the 1,500-bead chain 51,
+        // 64; 24,000 atoms at 64^3 74.9, 76.0; 100,000 at 96^3 165.1, 167.3).  A larger
+        // one waits for the pair kernel to end (100,000 atoms FP64, 150 KB a plane:
+        // planes for the inverse alone 341.5, lines 338).
         // rows per workgroup of the spread: three workgroups per CU, at least 8 rows
         // (each sees the atoms of four more)
         const int want_rows = (int)std::max<long long>(8, rows / (3 * B.n_cu));
@@ -632,7 +629,7 @@ class Engine : public EngineBase {
                     tw.push_back(v);
                 }
             // the spread: whole planes, or rows of them, an even count as equal as they come
-            if (B.fft_split) {
+            if (!B.fft_plane) {
                 const int most = std::max(2, std::min(kSpreadZPoints / Kz * 2, want_rows)), blocks = (Ky + most - 1) / most;
                 const int ny = std::min(Ky, ((Ky + blocks - 1) / blocks + 1) & ~1);
                 for (int x = 0; x < Kx; ++x)
@@ -651,7 +648,7 @@ class Engine : public EngineBase {
                 B.fft_plane_lds = std::max(B.fft_plane_lds, plane_lds_bytes<real2>(Ky, Kz));
                 // a thread for every radix-5 butterfly of a stage
                 B.fft_plane_threads =
-                    std::max(B.fft_plane_threads, std::min(kPlaneThreads, (plane_cap(Ky, Kz) / 5 + 63) & ~63));
+                    std::max(B.fft_plane_threads, std::min(kPlaneThreads<real2>, (plane_cap(Ky, Kz) / 5 + 63) & ~63));
             } else {
                 for (int l = 0; l < Kx * Ky; l += 2 * pairs)
                     li.push_back(make_int4(s, l, std::min(2 * pairs, Kx * Ky - l), 0));
@@ -916,8 +913,8 @@ class Engine : public EngineBase {
     // on the 1,500-bead chain (FP64 64.6 -> 56.6), 78.9 -> 77.8 on 24,000 atoms (FP64
     // 141 -> 136.4), 176 -> 174.4 on 100,000.  FP64 systems past kRideAtomsFP64 keep
     // their own launches: the FP64 exclusions take 96 registers a thread, so their
-    // blocks in the gather's launch wait for the pair kernel's registers (359 -> 363
-    // on 100,000 atoms).
+    // blocks in the gather's launch wait for the pair kernel's registers (100,000
+    // atoms: 337 apart, 344 riding).
     static constexpr int kRideAtomsFP64 = 50000;
     void side_work(int mask, bool energy) {
         const bool ride = P::mixed || B.n_atoms <= kRideAtomsFP64;

@@ -20,9 +20,15 @@ namespace nx {
 struct HostSystem;   // engine.hip
 
 // Plane FFT passes: threads per block, LDS available to one workgroup on gfx950.
-constexpr int kPlaneThreads = 768;           // three waves per SIMD, in the mixed path of at most 56 VGPRs
+// Threads of a plane pass: what the pair kernel's blocks leave of a SIMD's 512 VGPRs
+// holds three waves of 56 VGPRs in the mixed path (R2 float2), two of 96 in FP64
+// (with three the pass waited for the pair kernel: 24,000 atoms at 64^3 130.3 us a
+// step, with two 125.1).
+template <typename R2>
+constexpr int kPlaneThreads = sizeof(R2) == 8 ? 768 : 512;
 // Most LDS of a plane pass with the spread: what the pair kernel's blocks leave of a CU's 160 KB.
-constexpr size_t kPlaneSpreadLds = 100 * 1024;
+template <typename R2>
+constexpr size_t kPlaneSpreadLds = (sizeof(R2) == 8 ? 100 : 82) * 1024;
 constexpr int kXPassThreads = 256;
 // Bytes of a row that the y and x passes take at a time: a cache line.
 constexpr int kPassRowBytes = 128;
@@ -81,7 +87,7 @@ inline size_t plane_lds_bytes(int Ky, int Kz) {
 // The same with the spread in it.
 template <typename R2>
 inline size_t plane_spread_lds_bytes(int Ky, int Kz) {
-    return (size_t)(Ky + Kz + spread_points<R2>(plane_cap(Ky, Kz), Ky, Kz)) * sizeof(R2) + spread_lds_bytes(kPlaneThreads);
+    return (size_t)(Ky + Kz + spread_points<R2>(plane_cap(Ky, Kz), Ky, Kz)) * sizeof(R2) + spread_lds_bytes(kPlaneThreads<R2>);
 }
 
 // LDS bytes of `lines` lines of K points (two buffers, the twiddles).
@@ -178,7 +184,6 @@ struct Batch {
     int fft_tile = 1;               // columns of a y pass's tile
     int fft_plane_threads = 0, fft_x_threads = 0;
     int fft_plane = 0;              // 1: plane passes (fftp_items); 0: y and z passes over lines
-    int fft_split = 0;              // 1: spread and z pass over rows, then a y pass; 0: spread in the plane pass
     size_t fft_spread_lds = 0, fft_plane_lds = 0, fft_x_lds = 0, fft_y_lds = 0, fft_z_lds = 0;
     int pme_any = 0;
 

@@ -308,7 +308,7 @@ __global__ __launch_bounds__(5 * kGatherSlots, 5) void pme_gather_kernel(const S
                                                                      int atom_blocks, TermArgs<P> terms) {
     side_priority();
     // the atom forces' blocks first: theirs is the longer chain of loads (the last
-    // ones, FP64, 100,000 atoms: a step of 368 us instead of 363)
+    // ones, FP64, 100,000 atoms: a step 5 us longer)
     if ((int)blockIdx.x < atom_blocks) {
         const int a = (int)blockIdx.x * (5 * kGatherSlots) + (int)threadIdx.x;
         atom_force<P, false>(terms, a, nullptr);
@@ -788,7 +788,7 @@ __global__ __launch_bounds__(256) void fft_y(const SysDev* __restrict__ sd, cons
 // The grid's plane is spread here (SPREAD) or read from `rgrid`.
 // item = (sys, x)
 template <class P, bool SPREAD>
-__global__ __launch_bounds__(kPlaneThreads) void fft_plane_fwd(const SysDev* __restrict__ sd,
+__global__ __launch_bounds__(kPlaneThreads<typename P::real2>) void fft_plane_fwd(const SysDev* __restrict__ sd,
                                                               const int4* __restrict__ items,
                                                               const typename P::gacc* __restrict__ rgrid, SpreadArgs sp,
                                                               const typename P::real4* __restrict__ pos,
@@ -818,7 +818,7 @@ __global__ __launch_bounds__(kPlaneThreads) void fft_plane_fwd(const SysDev* __r
         load_twiddles(TWz, tw + d.tw_off[2], Kz);
         const int r0 = plan & 15;
         with_radix(r0, [&](auto R) {
-            fft_sums_stage<R.value, kPlaneThreads, (int)(kPlaneSpreadLds / (2 * sizeof(R2)))>(g, Ky, np, Kz, pz, A);
+            fft_sums_stage<R.value, kPlaneThreads<R2>, (int)(kPlaneSpreadLds<R2> / (2 * sizeof(R2)))>(g, Ky, np, Kz, pz, A);
         });
         Z = fft_lines<-1, false, false>(Kz, plan >> 4, np, pz, TWz, B, A, r0, [](int, int) { return R2{}; },
                                         KeepLine<R2>{pz});
@@ -845,7 +845,7 @@ __global__ __launch_bounds__(kPlaneThreads) void fft_plane_fwd(const SysDev* __r
 
 // Inverse: plane x of the half spectrum -> plane x of the potential (y then z).
 template <class P>
-__global__ __launch_bounds__(kPlaneThreads) void fft_plane_inv(const SysDev* __restrict__ sd,
+__global__ __launch_bounds__(kPlaneThreads<typename P::real2>) void fft_plane_inv(const SysDev* __restrict__ sd,
                                                               const int4* __restrict__ items,
                                                               const typename P::real2* __restrict__ cgrid,
                                                               typename P::real* phi,
@@ -1007,7 +1007,7 @@ hipError_t prepare_fft(Batch<P>& B) {
     const int sl = (int)B.fft_spread_lds, pl = (int)B.fft_plane_lds, xl = (int)B.fft_x_lds;
     const hipFuncAttribute a = hipFuncAttributeMaxDynamicSharedMemorySize;
     hipError_t e = hipFuncSetAttribute(
-        B.fft_split ? (const void*)fft_z_spread<P> : (const void*)fft_plane_fwd<P, true>, a, sl);
+        !B.fft_plane ? (const void*)fft_z_spread<P> : (const void*)fft_plane_fwd<P, true>, a, sl);
     if (e == hipSuccess) e = hipFuncSetAttribute((const void*)fft_x<P, 2>, a, xl);
     if (e == hipSuccess) e = hipFuncSetAttribute((const void*)fft_x<P, 3>, a, xl);
     if (e == hipSuccess && B.fft_plane) e = hipFuncSetAttribute((const void*)fft_plane_inv<P>, a, pl);
@@ -1018,8 +1018,8 @@ template <class P>
 void launch_pme_spread(Batch<P>& B) {
     if (!B.pme_any) return;
     const SpreadArgs sp{B.d_cnt, B.col_count, B.col_slot};
-    if (!B.fft_split)
-        fft_plane_fwd<P, true><<<B.n_fftz, kPlaneThreads, B.fft_spread_lds, B.stream>>>(
+    if (B.fft_plane)
+        fft_plane_fwd<P, true><<<B.n_fftz, kPlaneThreads<typename P::real2>, B.fft_spread_lds, B.stream>>>(
             B.d_sys, B.fftz_items, nullptr, sp, B.pos, B.cgrid, B.twiddle);
     else
         fft_z_spread<P><<<B.n_fftz, kSpreadZThreads, B.fft_spread_lds, B.stream>>>(B.d_sys, B.fftz_items, sp, B.pos,
@@ -1028,7 +1028,7 @@ void launch_pme_spread(Batch<P>& B) {
 
 template <class P>
 void launch_fft_forward(Batch<P>& B) {
-    if (!B.pme_any || !B.fft_split) return;      // the spread's launch ran the plane pass
+    if (!B.pme_any || B.fft_plane) return;      // the spread's launch ran the plane pass
     fft_y<P, -1><<<B.n_ffty, 256, B.fft_y_lds, B.stream>>>(B.d_sys, B.ffty_items, B.cgrid, B.twiddle, B.fft_tile);
 }
 
@@ -1148,7 +1148,7 @@ void fft3d_roundtrip(int nx, int ny, int nz, const double* in, double* out, bool
         }
         hipMemcpyAsync(rg, h.data(), G * sizeof(typename P::gacc), hipMemcpyHostToDevice, st);
         if (plane) {
-            fft_plane_fwd<P, false><<<(unsigned)pi.size(), kPlaneThreads, pl, st>>>(dd, dp, rg, {}, nullptr, cg, dtw);
+            fft_plane_fwd<P, false><<<(unsigned)pi.size(), kPlaneThreads<R2>, pl, st>>>(dd, dp, rg, {}, nullptr, cg, dtw);
             fft_x<P, 0><<<(unsigned)bi.size(), kXPassThreads, xl, st>>>(dd, db, (int)bi.size(), cg, nullptr, dtw, nullptr, {});
         } else {
             fft_z_fwd<P><<<(unsigned)zi.size(), 256, sm, st>>>(dd, dz, rg, cg, dtw);
@@ -1165,7 +1165,7 @@ void fft3d_roundtrip(int nx, int ny, int nz, const double* in, double* out, bool
         hipMemcpyAsync(cg, hc.data(), Gh * sizeof(R2), hipMemcpyHostToDevice, st);
         if (plane) {
             fft_x<P, 1><<<(unsigned)bi.size(), kXPassThreads, xl, st>>>(dd, db, (int)bi.size(), cg, nullptr, dtw, nullptr, {});
-            fft_plane_inv<P><<<(unsigned)pi.size(), kPlaneThreads, pl, st>>>(dd, dp, cg, ph, dtw, 0);
+            fft_plane_inv<P><<<(unsigned)pi.size(), kPlaneThreads<R2>, pl, st>>>(dd, dp, cg, ph, dtw, 0);
         } else {
             fft_x<P, 1><<<(unsigned)xi.size(), 256, sm, st>>>(dd, dx, (int)xi.size(), cg, nullptr, dtw, nullptr, {});
             fft_y<P, +1><<<(unsigned)yi.size(), 256, sm, st>>>(dd, dy, cg, dtw, T);
@@ -1327,7 +1327,7 @@ nx_status fft3d_r2c_noalloc(int device, int nx, int ny, int nz, const double* in
             (e = hipFuncSetAttribute((const void*)fft_x<P, 0>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int)xl)) != hipSuccess)
             return fail(e, "hipFuncSetAttribute");
-        fft_plane_fwd<P, false><<<(unsigned)n0, kPlaneThreads, pl, st>>>(dd, items, rg, {}, nullptr, cg, dtw);
+        fft_plane_fwd<P, false><<<(unsigned)n0, kPlaneThreads<R2>, pl, st>>>(dd, items, rg, {}, nullptr, cg, dtw);
         fft_x<P, 0><<<(unsigned)n1, kXPassThreads, xl, st>>>(dd, items + n0, n1, cg, nullptr, dtw, nullptr, {});
     } else {
         const size_t sm = (size_t)(2 * T + 1) * maxK * sizeof(R2);
