@@ -475,7 +475,7 @@ class Engine : public EngineBase {
         dalloc(&B.slot_wpos, S, o, B.stream);
         dalloc(&B.chunks, B.n_chunk_cap, o, B.stream);
         dalloc(&B.chunk_prefix, B.nsys + 1, o, B.stream);
-        B.pair_blocks = pair_grid_blocks<P>(B.n_cu, B.n_chunk_cap, tuning_.pair_per_cu);
+        B.pair_blocks = pair_grid_blocks<P>(B.n_cu, B.n_chunk_cap, B.n_atoms, tuning_.pair_per_cu);
         dalloc(&B.pair_pool, (size_t)kPoolInts, o, B.stream);
         if (B.nsys == 1 && lite_mode_) {
             // the update's report to the host, for the choice of step graph

@@ -588,17 +588,19 @@ static int pair_blocks_per_cu() {
 }
 
 // Persistent grid of the pair kernel, all blocks resident at once, at most
-// three per CU (FP64: two): the rest of a CU's wave slots go to the bonded and
+// three per CU: the rest of a CU's wave slots go to the bonded and
 // PME kernels running beside it.  Measured on the 100k-atom step (mixed, five
 // resident blocks possible): 3 per CU 261 us, 4 per CU 303 us, 2 per CU 268 us.
-// FP64 (three possible): 2 per CU 459 us, 3 per CU 461, 1 per CU 636; the
-// 24,000-atom water box 164, 177, 198.
+// FP64 takes two, which leave PME room, and three (all it can have) up to 30,000
+// atoms, where two waves per SIMD's worth of chunks end too unevenly: us a step with
+// 2 and 3 per CU on water of 3,000 to 12,000 atoms the same, 18,000 112.4 103.2,
+// 24,000 126.2 120.2, 30,000 140.4 137.8, 36,000 157.8 161.8, 81,000 295 344.
 // Fixed per batch layout: the claim counters are set for it.
 template <class P>
-int pair_grid_blocks(int n_cu, int n_chunk_cap, int per_cu_request) {
+int pair_grid_blocks(int n_cu, int n_chunk_cap, int n_atoms, int per_cu_request) {
     // a requested count (the autotuner's) is capped by what a CU can hold at once
     const int occ = pair_blocks_per_cu<P>();
-    const int per_cu = per_cu_request > 0 ? std::min(per_cu_request, occ) : std::min(occ, P::mixed ? 3 : 2);
+    const int per_cu = per_cu_request > 0 ? std::min(per_cu_request, occ) : std::min(occ, P::mixed || n_atoms <= 30000 ? 3 : 2);
     return std::max(1, std::min((n_chunk_cap + kPairWaves - 1) / kPairWaves, per_cu * std::max(1, n_cu)));
 }
 
@@ -651,8 +653,8 @@ void launch_export_pairs(Batch<P>& B, int2* out, long long cap, long long* d_cou
                                                                B.n_super_cap);
 }
 
-template int pair_grid_blocks<PrecFP64>(int, int, int);
-template int pair_grid_blocks<PrecMixed>(int, int, int);
+template int pair_grid_blocks<PrecFP64>(int, int, int, int);
+template int pair_grid_blocks<PrecMixed>(int, int, int, int);
 
 template <class P>
 int pair_blocks_occupancy() {
