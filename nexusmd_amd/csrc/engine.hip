@@ -650,8 +650,9 @@ class Engine : public EngineBase {
                 B.fft_plane_threads =
                     std::max(B.fft_plane_threads, std::min(kPlaneThreads<real2>, (plane_cap(Ky, Kz) / 5 + 63) & ~63));
             } else {
-                for (int l = 0; l < Kx * Ky; l += 2 * pairs)
-                    li.push_back(make_int4(s, l, std::min(2 * pairs, Kx * Ky - l), 0));
+                for (int x = 0; x < Kx; ++x)
+                    for (int y = 0; y < Ky; y += 2 * pairs)
+                        li.push_back(make_int4(s, x * Ky + y, std::min(2 * pairs, Ky - y), 0));
             }
             {
                 int nr = xlines;

@@ -717,7 +717,7 @@ __global__ __launch_bounds__(256) void fft_z_fwd(const SysDev* __restrict__ sd, 
 }
 
 // Z pass inverse: C2R into the potential grid, two rows as one complex line.
-// item = (sys, first row, n rows)
+// item = (sys, first row, n rows), the rows of one plane, the first an even one
 template <class P>
 __global__ __launch_bounds__(256) void fft_z_inv(const SysDev* __restrict__ sd, const int4* __restrict__ items,
                                                  const typename P::real2* __restrict__ cgrid, typename P::real* phi,
@@ -779,10 +779,10 @@ __global__ __launch_bounds__(256) void fft_y(const SysDev* __restrict__ sd, cons
 // inverse pass runs y and then z.  Three launches per step instead of five.
 // The real-to-complex z transform handles two real rows (2p and 2p + 1) as one
 // complex line a + ib and separates them as the y transform reads them
-// (paired_row); the complex-to-real inverse packs two rows (p and p + np: the
-// reads of neighbouring p then meet no bank twice) the same way, Z_k = A_k + i B_k
-// over the Hermitian extension (paired_point), then a = Re, b = Im.  Which rows
-// make a pair never depends on how the rows are dealt to workgroups.
+// (paired_row); the complex-to-real inverse packs two rows the same way, Z_k = A_k
+// + i B_k over the Hermitian extension (paired_point), then a = Re, b = Im.  The
+// pairs are the same ones in the line passes, however those deal the rows to
+// workgroups: a system's numbers do not depend on which passes its batch takes.
 
 // Forward: plane x of the charge grid -> plane x of the half spectrum (z then y).
 // The grid's plane is spread here (SPREAD) or read from `rgrid`.
@@ -876,10 +876,10 @@ __global__ __launch_bounds__(kPlaneThreads<typename P::real2>) void fft_plane_in
         Kz, d.fft_plan[2], np, pz, TWz, Y == A ? B : A, Y, 1,
         [=](int m, int p) {
             return paired_point<R2>(m, Kz, [=](int ks, int second) {
-                return !second || p + np < Ky ? Y[(p + second * np) * py + ks] : R2{};
+                return !second || 2 * p + 1 < Ky ? Y[(2 * p + second) * py + ks] : R2{};
             });
         },
-        [=](R2*, int m, int p, R2 v) { store_rows(o + p * pitch, np * pitch, p + np < Ky, m, Kz, pad, v); });
+        [=](R2*, int m, int p, R2 v) { store_rows(o + 2 * p * pitch, pitch, 2 * p + 1 < Ky, m, Kz, pad, v); });
 }
 
 // fft_x's terms: in MODE 2 alone

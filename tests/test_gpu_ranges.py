@@ -201,3 +201,19 @@ def test_terms_in_pme_launches(n, mask, prec, tol, monkeypatch):
         ctx.close()
     print("[gpu] terms n=%d mask=%d: %.2e apart" % (n, mask, np.abs(out[0] - out[1]).max()), flush=True)
     assert np.abs(out[0] - out[1]).max() <= tol
+
+
+@pytest.mark.parametrize("prec", [L.FP64, L.MIXED])
+@pytest.mark.parametrize("grid", [(24, 24, 24), (20, 27, 25), (9, 15, 64)])
+def test_planes_and_lines_give_the_same_bits(grid, prec, monkeypatch):
+    """A batch takes plane or line passes by its largest system; a system's own
+    numbers are the same on both."""
+    s = _gas(900, (2.1, 2.3, 2.0), 3, grid=grid)
+    out = []
+    for passes in ("1", "0"):
+        monkeypatch.setenv("NEXUSMD_FFT_PLANE", passes)
+        ctx = E.Context(s, precision=prec, skin=0.1)
+        ctx.step(5, 0.0005)
+        out.append(np.asarray(ctx.get_state()[0]))
+        ctx.close()
+    np.testing.assert_array_equal(out[0], out[1])
