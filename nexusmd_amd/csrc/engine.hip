@@ -2,9 +2,9 @@
 //
 // Replaces BaseLine::Engine (core/baseline/src/Engine.cpp:19-188): topology
 // and box set-up once, then per step  [neighbour-list rebuild if flagged] ->
-// pack -> bonded -> exclusion correction -> pair -> PME -> (report-step
-// kinetic energy) -> leapfrog, all enqueued on one HIP stream; the
-// report-free step is captured once into a hipGraph and replayed.
+// pair kernel, and beside it on a second stream the bonded and exclusion terms
+// and PME -> (report-step kinetic energy) -> leapfrog; the report-free step is
+// captured once into a hipGraph and replayed.
 #include <algorithm>
 #include <cmath>
 #include <cstdio>

@@ -4,18 +4,17 @@
 //   atom order  : FP64 master state x/y/z, vx/vy/vz, 1/m (SoA), per-atom
 //                 force accumulators F_atom (bonded terms, exclusion
 //                 correction), atom_sys, slot_of_atom.
-//   slot order  : atoms binned into xy columns, sorted by z inside a column
-//                 and padded to 8-atom clusters; 8 consecutive clusters of a
-//                 column form a super-cluster (one wavefront of the pair
-//                 kernel).  Per slot: packed (x,y,z,q), (sig/2, 2*sqrt(eps)),
+//   slot order  : atoms binned into xy columns, sorted by z inside a column and
+//                 cut into super-clusters of 64, each split into 8 clusters of
+//                 8 (padded).  Per slot: packed (x,y,z,q), (sig/2, 2*sqrt(eps)),
 //                 atom_of_slot (-1 = padding), force accumulators F_slot
 //                 (pair, PME).
-//   PME         : per system a real grid [Kx][Ky][Kz] (fixed-point int64 in
-//                 the mixed path, FP64 otherwise), a half-spectrum complex
-//                 grid [Kx][Ky][Kz/2+1] and a real potential grid.
-// Forces: FP64 path adds doubles with hardware atomics; mixed path converts
-// each contribution to 64-bit fixed point (2^32 units per kJ/mol/nm), so sums
-// are exact integers and independent of order.
+//   PME         : per system a half-spectrum complex grid [Kx][Ky][Kz/2+1] and
+//                 a real potential grid (rows of Kz + kPhiPad points); the
+//                 charge grid stands in LDS only.
+// Forces: each contribution is converted to fixed point (mixed: 64 bits, 2^32
+// units per kJ/mol/nm; FP64: two parts, Fix2), so sums are exact integers and
+// independent of order.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -48,7 +48,7 @@ void exclusions_from_bonds(int n, const std::vector<nx_bond>& bonds, std::vector
 // them changes what a kernel computes for a given atom, pair or grid line, so
 // every choice gives the same bits in the mixed path.
 struct Tuning {
-    int pair_per_cu = 0;     // persistent pair-kernel blocks per CU (built-in: min(occupancy, 3))
+    int pair_per_cu = 0;     // persistent pair-kernel blocks per CU (built-in: pair_grid_blocks)
     int spread_block = 0;    // no effect (the spread has no tiles any more)
     int fft_xblocks = 0;     // x-pass blocks: more than a cache line's lines each would make (built-in: those)
     int fft_lines = 0;       // line FFT: most y columns, or z row pairs, per block (built-in: what fits 60 KiB of LDS)
