@@ -650,9 +650,10 @@ class Engine : public EngineBase {
                 B.fft_plane_threads =
                     std::max(B.fft_plane_threads, std::min(kPlaneThreads<real2>, (plane_cap(Ky, Kz) / 5 + 63) & ~63));
             } else {
+                const int half = (Ky + 1) / 2;
                 for (int x = 0; x < Kx; ++x)
-                    for (int y = 0; y < Ky; y += 2 * pairs)
-                        li.push_back(make_int4(s, x * Ky + y, std::min(2 * pairs, Ky - y), 0));
+                    for (int p = 0; p < half; p += pairs)
+                        li.push_back(make_int4(s, x, p, std::min(pairs, half - p)));
             }
             {
                 int nr = xlines;

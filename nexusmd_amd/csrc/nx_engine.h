@@ -177,7 +177,7 @@ struct Batch {
     long long rgrid_total = 0, cgrid_total = 0, tw_total = 0;
     int4* fftz_items = nullptr;     // spread: (sys, x, y0, ny), or whole planes (sys, x)
     int4* fftp_items = nullptr;     // inverse plane pass: (sys, x)
-    int4* fftl_items = nullptr;     // inverse z pass: (sys, first line, n lines, 0)
+    int4* fftl_items = nullptr;     // inverse z pass: (sys, x, first pair of rows, n pairs)
     int4* ffty_items = nullptr;     // (sys, x, kz0, 0)
     int4* fftx_items = nullptr;     // (sys, first (y, kz) line, n lines, 0)
     int n_fftz = 0, n_fftp = 0, n_fftl = 0, n_ffty = 0, n_fftx = 0;

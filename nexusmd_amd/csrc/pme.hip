@@ -717,7 +717,8 @@ __global__ __launch_bounds__(256) void fft_z_fwd(const SysDev* __restrict__ sd, 
 }
 
 // Z pass inverse: C2R into the potential grid, two rows as one complex line.
-// item = (sys, first row, n rows), the rows of one plane, the first an even one
+// item = (sys, x, p0, n): rows p0 .. p0 + n - 1 of the plane and their partners half a
+// plane on, as in fft_plane_inv
 template <class P>
 __global__ __launch_bounds__(256) void fft_z_inv(const SysDev* __restrict__ sd, const int4* __restrict__ items,
                                                  const typename P::real2* __restrict__ cgrid, typename P::real* phi,
@@ -728,24 +729,26 @@ __global__ __launch_bounds__(256) void fft_z_inv(const SysDev* __restrict__ sd, 
     extern __shared__ unsigned char smem_raw[];
     const int4 it = items[blockIdx.x];
     const SysDev& d = sd[it.x];
-    const int Kz = d.grid[2], Kzh = Kz / 2 + 1;
-    const int line0 = it.y, nl = it.z, np = (nl + 1) >> 1, pz = np | 1;
+    const int Ky = d.grid[1], Kz = d.grid[2], Kzh = Kz / 2 + 1;
+    const int np = it.w, pz = np | 1, half = (Ky + 1) >> 1;
     R2* A = reinterpret_cast<R2*>(smem_raw);
     R2* B = A + pz * Kz;
     R2* TW = B + pz * Kz;
     load_twiddles(TW, tw + d.tw_off[2], Kz);
     __syncthreads();
-    const R2* c = cgrid + d.cgrid_off + (long long)line0 * Kzh;
+    const long long line0 = (long long)it.y * Ky + it.z;
+    const int past = Ky - it.z - half;      // pairs of the item with a second row
+    const R2* c = cgrid + d.cgrid_off + line0 * Kzh;
     const int pitch = Kz + pad;
-    real* o = phi + d.rgrid_off + (long long)line0 * pitch;
+    real* o = phi + d.rgrid_off + line0 * pitch;
     fft_lines<+1, true, true>(
         Kz, d.fft_plan[2], np, pz, TW, A, B, 1,
         [=](int m, int p) {
             return paired_point<R2>(m, Kz, [=](int ks, int second) {
-                return !second || 2 * p + 1 < nl ? c[(2 * p + second) * Kzh + ks] : R2{};
+                return !second || p < past ? c[(p + second * half) * Kzh + ks] : R2{};
             });
         },
-        [=](R2*, int m, int p, R2 v) { store_rows(o + 2 * p * pitch, pitch, 2 * p + 1 < nl, m, Kz, pad, v); });
+        [=](R2*, int m, int p, R2 v) { store_rows(o + p * pitch, half * pitch, p < past, m, Kz, pad, v); });
 }
 
 // Y pass: tile (sys, x, kz0) of TZ consecutive kz columns, lines along y.
@@ -779,10 +782,11 @@ __global__ __launch_bounds__(256) void fft_y(const SysDev* __restrict__ sd, cons
 // inverse pass runs y and then z.  Three launches per step instead of five.
 // The real-to-complex z transform handles two real rows (2p and 2p + 1) as one
 // complex line a + ib and separates them as the y transform reads them
-// (paired_row); the complex-to-real inverse packs two rows the same way, Z_k = A_k
-// + i B_k over the Hermitian extension (paired_point), then a = Re, b = Im.  The
-// pairs are the same ones in the line passes, however those deal the rows to
-// workgroups: a system's numbers do not depend on which passes its batch takes.
+// (paired_row); the complex-to-real inverse packs two rows (p and p + np: the
+// reads of neighbouring p then meet no bank twice) the same way, Z_k = A_k + i B_k
+// over the Hermitian extension (paired_point), then a = Re, b = Im.  The pairs are
+// the same ones in the line passes, however those deal the rows to workgroups: a
+// system's numbers do not depend on which passes its batch takes.
 
 // Forward: plane x of the charge grid -> plane x of the half spectrum (z then y).
 // The grid's plane is spread here (SPREAD) or read from `rgrid`.
@@ -876,10 +880,10 @@ __global__ __launch_bounds__(kPlaneThreads<typename P::real2>) void fft_plane_in
         Kz, d.fft_plan[2], np, pz, TWz, Y == A ? B : A, Y, 1,
         [=](int m, int p) {
             return paired_point<R2>(m, Kz, [=](int ks, int second) {
-                return !second || 2 * p + 1 < Ky ? Y[(2 * p + second) * py + ks] : R2{};
+                return !second || p + np < Ky ? Y[(p + second * np) * py + ks] : R2{};
             });
         },
-        [=](R2*, int m, int p, R2 v) { store_rows(o + 2 * p * pitch, pitch, 2 * p + 1 < Ky, m, Kz, pad, v); });
+        [=](R2*, int m, int p, R2 v) { store_rows(o + p * pitch, np * pitch, p + np < Ky, m, Kz, pad, v); });
 }
 
 // fft_x's terms: in MODE 2 alone
@@ -1102,7 +1106,13 @@ void fft3d_roundtrip(int nx, int ny, int nz, const double* in, double* out, bool
     const int maxK = std::max(nx, std::max(ny, nz));
     const int T = std::max(1, std::min(8, (int)((61440 / (int)sizeof(R2) - maxK) / (2 * maxK))));
     std::vector<int4> zi, yi, xi;
-    for (int l = 0; l < nx * ny; l += T) zi.push_back(make_int4(0, l, std::min(T, nx * ny - l), 0));
+    if (forward) {
+        for (int l = 0; l < nx * ny; l += T) zi.push_back(make_int4(0, l, std::min(T, nx * ny - l), 0));
+    } else {
+        const int half = (ny + 1) / 2, pairs = (T - 1) | 1;
+        for (int x = 0; x < nx; ++x)
+            for (int p = 0; p < half; p += pairs) zi.push_back(make_int4(0, x, p, std::min(pairs, half - p)));
+    }
     for (int x = 0; x < nx; ++x)
         for (int k = 0; k < nzh; k += T) yi.push_back(make_int4(0, x, k, 0));
     for (int y = 0; y < ny; ++y)
