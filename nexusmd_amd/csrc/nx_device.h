@@ -367,30 +367,10 @@ __device__ __forceinline__ int dpp_xor1(int v) { return __builtin_amdgcn_update_
 __device__ __forceinline__ int dpp_xor2(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false); }
 __device__ __forceinline__ int dpp_hmirror(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, false); }
 
-// sum over lanes {l, l^8, l^16, ..., l^56} (lanes sharing l & 7)
-__device__ __forceinline__ float sum_stride8(float v) {
-    v += __int_as_float(dpp_ror8(__float_as_int(v)));
-    auto p = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
-    v = __int_as_float(p[0]) + __int_as_float(p[1]);
-    auto q = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
-    return __int_as_float(q[0]) + __int_as_float(q[1]);
-}
-__device__ __forceinline__ double sum_stride8(double v) {
-    int lo = __double2loint(v), hi = __double2hiint(v);
-    v += __hiloint2double(dpp_ror8(hi), dpp_ror8(lo));
-    lo = __double2loint(v); hi = __double2hiint(v);
-    auto pl = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
-    auto ph = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
-    v = __hiloint2double(ph[0], pl[0]) + __hiloint2double(ph[1], pl[1]);
-    lo = __double2loint(v); hi = __double2hiint(v);
-    auto ql = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
-    auto qh = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
-    return __hiloint2double(qh[0], ql[0]) + __hiloint2double(qh[1], ql[1]);
-}
-// v[0], v[1], v[2] summed over the lanes with the same l & 7, each as sum_stride8
-// does: the sum of v[0] on lanes 0-15, of v[1] on 16-31, of v[2] on 32-63 (each at
-// every lane of its l & 7).  Two of them share a swap and an addition where one
-// alone wastes half: 10 instructions instead of 21.
+// x, y and z summed over the lanes with the same l & 7 (by 8, 16, then 32 lanes
+// apart): the sum of x on lanes 0-15, of y on 16-31, of z on 32-63 (each at every
+// lane of its l & 7).  Two of them share a swap and an addition where one alone
+// wastes half: 10 instructions, where three sums of their own take 21.
 template <typename real>
 __device__ __forceinline__ void swap16(real& a, real& b);      // odd rows of 16 lanes of a with even ones of b
 template <typename real>
