@@ -70,6 +70,14 @@ struct SysCount {
 // its list was due for a build: the update froze it for that step (the host
 // runs the step again with the list kernels; not a failure)
 constexpr int kStaleList = 8;
+// No list to work on: the system is empty or its last build failed.  Every bit of
+// this was written before the work that asks for it was queued, so all wavefronts
+// of a workgroup see the same answer and may leave it on it, barriers or not.  Not
+// so kStaleList: nl_waves sets it while the kernels of the side stream run.  They
+// go through such a step on the last build's list (the update drops what they sum).
+__device__ __forceinline__ bool no_list(const SysCount& sc) {
+    return sc.n_slots == 0 || (sc.overflow & ~kStaleList) != 0;
+}
 
 // What nl_waves of a one-system batch reports to host memory early in every
 // step, for the host's choice between the step graphs with and without the

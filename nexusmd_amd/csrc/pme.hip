@@ -666,8 +666,7 @@ __global__ __launch_bounds__(kSpreadZThreads) void fft_z_spread(const SysDev* __
     extern __shared__ unsigned char smem_raw[];
     const int4 it = items[blockIdx.x];
     const SysDev& d = sd[it.x];
-    const SysCount& sc = sp.sc[it.x];
-    if (sc.n_slots == 0 || sc.overflow) return;      // overflowed build: the system is frozen
+    if (no_list(sp.sc[it.x])) return;      // the system is frozen
     const int x = it.y, y0 = it.z, ny = it.w;
     const int Ky = d.grid[1], Kz = d.grid[2], Kzh = Kz / 2 + 1, np = (ny + 1) >> 1, pz = np | 1, cap = pz * Kz;
     R2* TW = reinterpret_cast<R2*>(smem_raw);
@@ -814,8 +813,7 @@ __global__ __launch_bounds__(kPlaneThreads<typename P::real2>) void fft_plane_fw
     const unsigned plan = d.fft_plan[2];
     const R2* Z;
     if constexpr (SPREAD) {
-        const SysCount& sc = sp.sc[it.x];
-        if (sc.n_slots == 0 || sc.overflow) return;      // overflowed build: the system is frozen
+        if (no_list(sp.sc[it.x])) return;      // the system is frozen
         long long* g = reinterpret_cast<long long*>(A);
         spread_rows<P>(d, sp, pos, x, 0, Ky, reinterpret_cast<int*>(A + spread_points<R2>(cap, Ky, Kz)), g);
         load_twiddles(TWy, tw + d.tw_off[1], Ky);
