@@ -350,14 +350,17 @@ class Engine : public EngineBase {
             d.n_atoms = n;
             d.atom_off = (int)atom_off;
             d.pair_image = pair_image_ ? 1 : 0;
-            // columns as wide as 64 atoms are tall, so that a super-cluster is about a
-            // cube; their quarters hold at most 2048 atoms, 700 on average
+            // Columns about as wide as 64 atoms are tall, so that a super-cluster is about
+            // a cube, each of 2 x 2 quarters of at most 2,048 atoms (kQuarterCap).  A
+            // quarter is never wider than a column 8 atoms wide would be (cells x cells of
+            // them, 700 atoms on average at most): what fits such columns fits these.
             const double V = d.L[0] * d.L[1] * d.L[2];
             const double rho = std::max(1e-3, n / V);
-            double cw = 2.0 * cbrt(8.0 / rho);
-            int ncx = std::max(1, (int)floor(d.L[0] / cw));
-            int ncy = std::max(1, (int)floor(d.L[1] / cw));
-            while ((double)n / (4.0 * ncx * ncy) > 700.0) { ncx += 1; ncy += 1; }
+            const double cw = cbrt(8.0 / rho);
+            int cells[2];
+            for (int k = 0; k < 2; ++k) cells[k] = std::max(1, (int)floor(d.L[k] / cw));
+            while ((double)n / ((double)cells[0] * cells[1]) > 700.0) { cells[0] += 1; cells[1] += 1; }
+            const int ncx = (cells[0] + 1) / 2, ncy = (cells[1] + 1) / 2;
             d.ncx = ncx;
             d.ncy = ncy;
             d.colw[0] = d.L[0] / ncx;

@@ -1,0 +1,65 @@
+"""Systems at the room that a layout leaves them: crowded columns.
+
+Forces against the FP64 oracle, relative RMS: FP64 <= 1e-9, mixed <= 5e-4 (the
+bounds of the other parity tests).
+"""
+import numpy as np
+import pytest
+
+from nexusmd_amd import _lib as L
+from nexusmd_amd import engine as E
+from oracle import pyoracle as O
+
+from _util import bare_system, rel_rms
+
+pytestmark = pytest.mark.gpu
+
+TOL = {L.FP64: 1e-9, L.MIXED: 5e-4}
+
+
+def _lattice(n, box, rng):
+    """n jittered lattice points in [0, box)."""
+    box = np.asarray(box, float)
+    k = np.ceil(box * (n / box.prod()) ** (1 / 3)).astype(int)
+    while k.prod() < n:
+        k[np.argmin(k / box)] += 1
+    g = np.stack(np.meshgrid(*[np.arange(m) + 0.5 for m in k], indexing="ij"), -1).reshape(-1, 3) * (box / k)
+    return g[rng.permutation(len(g))[:n]] + rng.normal(0.0, 0.01, (n, 3))
+
+
+def _gas(n, box, rng, grid, cutoff=0.8):
+    q = rng.normal(0.0, 0.4, n)
+    return bare_system(_lattice(n, box, rng) % box, np.zeros(3), box, q=q - q.mean(), sig=np.full(n, 0.12),
+                       eps=rng.uniform(0.1, 0.4, n), cutoff=cutoff, grid=grid)
+
+
+def _same(sys, prec, f, pos, excl=None):
+    sys.pos = pos
+    ref, _ = O.compute_forces(O.Prepared(sys, excl=excl))
+    assert rel_rms(f, ref) <= TOL[prec]
+
+
+@pytest.mark.parametrize("prec", [L.FP64, L.MIXED])
+@pytest.mark.parametrize("layout", ["spread out", "clumped"])
+def test_a_clump_across_columns(layout, prec):
+    """2,100 of 2,800 atoms in one quarter of the xy plane, under 1,000 in every cell
+    of the 3 x 3 that a column of 8-atom clusters would have here: as the first
+    state, and as a later state of a context laid out for an even one."""
+    rng = np.random.default_rng(1)
+    box = np.array([1.95, 1.95, 11.5])
+    s = _gas(2800, box, rng, (24, 24, 128))
+    even = s.pos.copy()
+    dense = np.vstack([_lattice(2100, box * [0.5, 0.5, 1.0], rng), _lattice(700, box * [0.5, 1.0, 1.0], rng) + box * [0.5, 0, 0]])
+    dense %= box
+    cell = (dense[:, :2] / box[:2] * 3).astype(int)
+    assert np.bincount(cell[:, 0] * 3 + cell[:, 1]).max() < 2048
+    print("[gpu] clump, first %s, precision %d" % (layout, prec), flush=True)
+    if layout == "clumped":
+        s.pos = dense
+    ctx = E.Context(s, precision=prec, skin=0.1)
+    ctx.compute_forces()
+    ctx.set_state(dense)
+    f, _ = ctx.compute_forces()
+    ctx.close()
+    s.pos = even
+    _same(s, prec, f, dense)
