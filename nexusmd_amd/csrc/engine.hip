@@ -371,16 +371,21 @@ class Engine : public EngineBase {
             d.slot_cap = ((n + 8 * ncx * ncy + 63) / 64) * 64;
             d.super_off = (int)sup_off;
             d.super_cap = (n + 63) / 64 + ncx * ncy;
-            // pair-list capacity from density: clusters within the column neighbourhood
-            const double w = std::max(d.colw[0], d.colw[1]);
-            const double hz = std::min(d.L[2], 64.0 / (rho * d.colw[0] * d.colw[1]));
+            // Pair-list room: half as much again as the clusters at the mean density in
+            // reach of 64 atoms of an 8-atom-wide column, for as many groups of 64 as
+            // those columns make.  The super-clusters here, cubes, have two thirds of the
+            // entries; the rest is for systems that grow denser after the layout (water
+            // fills a tenth).
+            const double w = std::max(d.L[0] / cells[0], d.L[1] / cells[1]);
+            const double hz = std::min(d.L[2], 64.0 * cells[0] * cells[1] / (rho * d.L[0] * d.L[1]));
             const double r = d.rlist;
-            double ext = std::min(d.L[0], w + 2 * r) * std::min(d.L[1], w + 2 * r) * std::min(d.L[2], hz + 2 * r);
+            const double ext = std::min(d.L[0], 3 * w + 2 * r) * std::min(d.L[1], 3 * w + 2 * r) *
+                               std::min(d.L[2], hz + 2 * r + 0.5);
             double per_super = 1.5 * (rho / 8.0) * ext * h.list_scale;
             per_super = std::min(per_super, (double)kSuperListCap);
             per_super = std::max(per_super, 16.0);
             d.list_off = (int)list_off;
-            d.list_cap = (int)std::min<double>(2.0e9, per_super * d.super_cap + 64);
+            d.list_cap = (int)std::min<double>(2.0e9, per_super * ((n + 63) / 64 + (double)cells[0] * cells[1]) + 64);
             d.chunk_off = (int)chunk_off;
             d.chunk_entries = chunk_entries_for(n, P::mixed);
             d.chunk_cap = d.list_cap / d.chunk_entries + d.super_cap;

@@ -1,4 +1,5 @@
-"""Systems at the room that a layout leaves them: crowded columns.
+"""Systems at the room that a layout leaves them: crowded columns, lists that grow
+after the layout.
 
 Forces against the FP64 oracle, relative RMS: FP64 <= 1e-9, mixed <= 5e-4 (the
 bounds of the other parity tests).
@@ -63,3 +64,20 @@ def test_a_clump_across_columns(layout, prec):
     ctx.close()
     s.pos = even
     _same(s, prec, f, dense)
+
+
+@pytest.mark.parametrize("prec", [L.FP64, L.MIXED])
+def test_a_gas_that_condenses(prec):
+    """4,000 atoms at 1 in 2 nm^3, then as a drop of 60 per nm^3 in the same context:
+    the pair list has room for it."""
+    rng = np.random.default_rng(2)
+    box = np.array([20.0, 20.0, 20.0])
+    s = _gas(4000, box, rng, (64, 64, 64), cutoff=1.0)
+    print("[gpu] condensing gas, precision %d" % prec, flush=True)
+    ctx = E.Context(s, precision=prec, skin=0.1)
+    ctx.compute_forces()
+    drop = _lattice(4000, (4.05, 4.05, 4.05), rng) + 7.9
+    ctx.set_state(drop)
+    f, _ = ctx.compute_forces()
+    ctx.close()
+    _same(s, prec, f, drop)
