@@ -44,7 +44,7 @@ constexpr int kQuarterCap = 2048;     // most atoms in a quarter of a column (2 
 constexpr int kColSortCap = 4 * kQuarterCap;     // atoms per column sorted in LDS
 constexpr int kColThreads = 512;      // threads per column in nl_columns
 constexpr int kListCap = kSuperListCap;   // pair-list entries per super-cluster (LDS)
-constexpr int kExclCap = 2048;        // exclusion triples per super-cluster (LDS)
+constexpr int kExclCap = 2048;        // exclusion records per super-cluster (LDS)
 
 // Column of an atom from its wrapped position.
 __device__ __forceinline__ void wrapped(const SysDev& d, double x, double y, double z, double* w) {
@@ -661,8 +661,9 @@ __global__ __launch_bounds__(T) void nl_pairlist(const SysDev* sd, SysCount* sc,
     for (int e = tid; e < ne; e += T) l_eid[e] = -1;
     __syncthreads();
 
-    // 4: exclusions of the 64 i-atoms that fall in kept tiles
-    {
+    // 4: exclusions of the 64 i-atoms that fall in kept tiles: fn(entry, i-cluster,
+    // pair bit) for each
+    auto each_exclusion = [&](auto&& fn) {
         const int k = il >> 3, iat = il & 7;
         for (int e = x0; e < x1; e += T / 64) {
             const int sp = e == x0 ? xsp : slot_of_atom[excl_idx[e]];
@@ -674,16 +675,17 @@ __global__ __launch_bounds__(T) void nl_pairlist(const SysDev* sd, SysCount* sc,
                 const int m = (lo + hi) >> 1;
                 if ((int)(l_ent[m] & 0xffffffu) < cj) lo = m + 1; else hi = m;
             }
-            if (lo < ne && (int)(l_ent[lo] & 0xffffffu) == cj && ((l_ent[lo] >> 24) >> k & 1u)) {
-                const int t = atomicAdd(&n_x, 1);
-                if (t < kExclCap) x_rec[t] = ((unsigned)(lo * 8 + k) << 6) | (unsigned)(iat * 8 + (sp & 7));
-                l_eid[lo] = 0;      // mark
-            }
+            if (lo < ne && (int)(l_ent[lo] & 0xffffffu) == cj && ((l_ent[lo] >> 24) >> k & 1u))
+                fn(lo, k, (unsigned)(iat * 8 + (sp & 7)));
         }
-    }
+    };
+    each_exclusion([&](int e, int k, unsigned bit) {
+        const int t = atomicAdd(&n_x, 1);
+        if (t < kExclCap) x_rec[t] = ((unsigned)(e * 8 + k) << 6) | bit;
+        l_eid[e] = 0;      // mark
+    });
     __syncthreads();
-    int nx_ = n_x;
-    if (nx_ > kExclCap) { overflow = true; nx_ = kExclCap; }
+    const int nx_ = n_x;
     // chunks of at most chunk_entries entries, as equal as they come
     const int nch = (ne + d.chunk_entries - 1) / d.chunk_entries, ce = nch > 0 ? (ne + nch - 1) / nch : 1;
     // mask ids for the entries with exclusions, in entry order; the room for them,
@@ -719,10 +721,14 @@ __global__ __launch_bounds__(T) void nl_pairlist(const SysDev* sd, SysCount* sc,
         }
     }
     __syncthreads();
-    for (int t = tid; t < nx_; t += T) {
-        const int ek = (int)(x_rec[t] >> 6), e = ek >> 3, k = ek & 7;
+    auto exclude = [&](int e, int k, unsigned bit) {
         const int g = d.emask_off + id_base + l_eid[e];
-        atomicOr(&emask[(size_t)g * 8 + k], 1ull << (x_rec[t] & 63u));
+        atomicOr(&emask[(size_t)g * 8 + k], 1ull << bit);
+    };
+    if (nx_ <= kExclCap) {
+        for (int t = tid; t < nx_; t += T) exclude((int)(x_rec[t] >> 9), (int)(x_rec[t] >> 6) & 7, x_rec[t] & 63u);
+    } else {
+        each_exclusion(exclude);              // more than the records hold: found once more
     }
     for (int e = tid; e < ne; e += T) {
         uint2 v;

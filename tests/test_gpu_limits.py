@@ -1,5 +1,5 @@
 """Systems at the room that a layout leaves them: crowded columns, lists that grow
-after the layout.
+after the layout, exclusions by the hundred in one super-cluster.
 
 Forces against the FP64 oracle, relative RMS: FP64 <= 1e-9, mixed <= 5e-4 (the
 bounds of the other parity tests).
@@ -81,3 +81,30 @@ def test_a_gas_that_condenses(prec):
     f, _ = ctx.compute_forces()
     ctx.close()
     _same(s, prec, f, drop)
+
+
+@pytest.mark.parametrize("prec", [L.FP64, L.MIXED])
+@pytest.mark.parametrize("group", [60, 80])
+def test_a_group_without_interactions_inside(group, prec):
+    """`group` neighbouring atoms around the middle of a column, every pair of them
+    excluded, in a box of 900: with 80, some 2,700 excluded pairs in one
+    super-cluster."""
+    rng = np.random.default_rng(3)
+    box = np.array([2.4, 2.3, 2.2])
+    s = _gas(900, box, rng, (24, 24, 24))
+    d = s.pos - box * [0.25, 0.25, 0.5]
+    order = np.argsort((d * d).sum(1))
+    s.pos = s.pos[order]
+    s.q = s.q[order]
+    s.eps = s.eps[order]
+    off = np.concatenate([np.arange(group + 1) * (group - 1), np.full(900 - group, group * (group - 1))]).astype(np.int32)
+    idx = np.concatenate([[j for j in range(group) if j != i] for i in range(group)]).astype(np.int32)
+    print("[gpu] %d atoms excluded from each other, precision %d" % (group, prec), flush=True)
+    ctx = E.Context(s, precision=prec, skin=0.1, excl=(off, idx))
+    f, _ = ctx.compute_forces()
+    pairs = ctx.neighbor_pairs() if prec == L.FP64 else None
+    ctx.close()
+    _same(s, prec, f, s.pos, excl=(off, idx))
+    if pairs is not None:
+        want = O.pairs(s, (off, idx), method="brute")
+        assert set(map(tuple, pairs.tolist())) == set(map(tuple, want.tolist()))
