@@ -340,6 +340,11 @@ class Engine : public EngineBase {
             d.skin_half2 = skin > 0 ? 0.25 * skin * skin : -1.0;
             d.alpha = (1.0 / rc) * sqrt(-log(2.0 * h.nb.ewald_tolerance));
             if (!(d.alpha * d.alpha * d.rc2 <= kErfSeriesMax)) B.all_series = false;
+            const long double a = d.alpha, ex = a * a / 0.693147180559945309417L;
+            d.ew_exp = (double)ex;
+            d.ew_exp_lo = (double)(ex - (long double)d.ew_exp);
+            d.ew_u = (double)(a / 1.41421356237309504880L);
+            d.ew_q = (double)(a * 1.12837916709551257390L);
             if (h.nb.use_switch && h.nb.switch_distance < rc) {
                 d.sw_on = h.nb.switch_distance;
                 d.sw_inv = 1.0 / (rc - h.nb.switch_distance);

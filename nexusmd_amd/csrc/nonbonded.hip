@@ -91,23 +91,38 @@ __device__ __forceinline__ float pair_mixed(float r2, float qq, float sig, float
     return fmaf(qq, cy, dl) * inv_r2;
 }
 
-// FP64 path inside the range of the series: 1/r^3 - alpha^3 B(alpha^2 r^2) in
-// place of (erfc + 2 alpha r exp / sqrt(pi)) / r^3, and 1/r from the hardware's
-// reciprocal square root with one third-order step (its first error, 2^-26 or
-// less, goes to the third power).  The kernel is bound by its vector
-// instructions (82% of its time issuing them, 111 a tile): with library erfc,
-// exp, sqrt and division the 100,000-atom system's launch took 512 us, with the
-// series 328.  The forces' error against 64 bits stays what it was (6e-14 of
-// their norm, from the fixed-point sums).
+// FP64 path inside the range of kErfcx: the direct-space term as exp(-(alpha r)^2)
+// times a polynomial (nx_device.h), without a library function or a division.  1/r
+// is the hardware's reciprocal square root with one third-order step (its first
+// error, 2^-26 or less, goes to the third power), 1/r^2 its square with one
+// second-order step.  The kernel is bound by its vector instructions.  Its launch on
+// 100,000 atoms alone: 307 us; with library erfc, exp, sqrt and division 469; with
+// the difference 1/r^3 - alpha^3 B, which loses two digits near the cutoff, 260
+// (24,000 atoms: 98, 165, 84; a step 133, 199, 118).
+struct EwaldFit {
+    double ex, ex_lo, u, q;      // as SysDev::ew_*
+};
 template <bool ENERGY>
-__device__ __forceinline__ double pair_fp64_series(double r2, double qq, double sig, double epsij, double alpha,
+__device__ __forceinline__ double pair_fp64_series(double r2, double qq, double sig, double epsij, const EwaldFit& w,
                                                    double sw_on, double sw_inv, double& ecoul, double& elj) {
 #pragma clang fp contract(off)      // the same operations in both kernels below
     double y = __builtin_amdgcn_rsq(r2);
     const double err = fma(-(r2 * y), y, 1.0);
     y = fma(y * err, fma(0.375, err, 0.5), y);
-    const double y2 = y * y, s = alpha * alpha * r2;
-    const double cf = qq * fma(-(alpha * alpha * alpha), erf_series(kErfB, s), y2 * y);
+    double y2 = y * y;
+    y2 = fma(y2, fma(-r2, y2, 1.0), y2);
+    const double r = r2 * y;
+    // exp(-(alpha r)^2) = 2^k (1 + fp): k the integer nearest to the exponent in base
+    // two, in the low bits of the sum with 1.5 2^52; the rest of it, rounded once
+    const double big = fma(r2, -w.ex, 6755399441055744.0);
+    const double f = fma(r2, -w.ex_lo, fma(r2, -w.ex, -(big - 6755399441055744.0)));
+    double fp, e;
+    direct_space_series(f, fma(r, w.u, -1.0), fp, e);
+    const double q = fma(r, w.q, e);
+    auto scaled = [&](double v) {      // v of 0.1 to 6 times 2^k, k of -12 to 0
+        return __hiloint2double(__double2hiint(v) + (__double2loint(big) << 20), __double2loint(v));
+    };
+    const double cf = qq * (scaled(fma(fp, q, q)) * (y2 * y));
     double s2 = sig * y;
     s2 *= s2;
     const double s6 = s2 * s2 * s2;
@@ -115,14 +130,13 @@ __device__ __forceinline__ double pair_fp64_series(double r2, double qq, double 
     double lf = es * fma(12.0, s6, -6.0) * y2;
     double le = es * (s6 - 1.0);
     if (sw_on >= 0.0) {
-        const double r = r2 * y;
         const double t = r > sw_on ? (r - sw_on) * sw_inv : 0.0;
         const double sv = fma(t * t * t, fma(t, fma(-6.0, t, 15.0), -10.0), 1.0);
         const double sd = t * t * fma(t, fma(-30.0, t, 60.0), -30.0) * sw_inv;
         lf = fma(sv, lf, -(le * sd * y));
         le *= sv;
     }
-    if constexpr (ENERGY) ecoul = qq * fma(-alpha, erf_series(kErfA, s), y);
+    if constexpr (ENERGY) ecoul = qq * (scaled(fma(fp, e, e)) * y);
     elj = le;
     return cf + lf;
 }
@@ -294,6 +308,10 @@ __device__ __forceinline__ void pair_body(const SysDev* __restrict__ sd, const i
         const real alpha = (real)sd[s].alpha;
         const real sw_on = (real)sd[s].sw_on, sw_inv = (real)sd[s].sw_inv;
         const bool series = (double)alpha * (double)alpha * (double)rc2 <= kErfSeriesMax;   // FP64 path only
+        EwaldFit ew = {sd[s].ew_exp, sd[s].ew_exp_lo, sd[s].ew_u, sd[s].ew_q};
+        // in a vector register: an instruction takes one scalar operand, and the first
+        // one that reads it adds a constant
+        if constexpr (!P::mixed) asm("" : "+v"(ew.ex));
         const MixedPair mpc = mixed_pair_const(sd[s]);   // mixed path only
         {
             real4 p = cur.p;
@@ -430,7 +448,7 @@ __device__ __forceinline__ void pair_body(const SysDev* __restrict__ sd, const i
                         ecv = elv = 0;
                         if (on) {
                             const real qq = pi.w * pjs.w, sg = li.x + lj_j.x, ep = li.y * lj_j.y;
-                            if (ALL_SERIES || series) dEdR = pair_fp64_series<ENERGY>(r2, qq, sg, ep, alpha, sw_on, sw_inv, ecv, elv);
+                            if (ALL_SERIES || series) dEdR = pair_fp64_series<ENERGY>(r2, qq, sg, ep, ew, sw_on, sw_inv, ecv, elv);
                             else dEdR = pair_fp64(r2, qq, sg, ep, alpha, sw_on, sw_inv, ecv, elv);
                         }
                     }
@@ -520,8 +538,8 @@ pair_kernel_mixed(NX_PAIR_PARAMS(PrecMixed)) {
     pair_body<PrecMixed, ENERGY, true>(NX_PAIR_ARGS);
 }
 // The FP64 kernel with the series alone, for batches whose every system is in
-// its range, needs 147 VGPRs; with the library functions beside it (chosen per
-// system) 219.
+// its range, needs 156 VGPRs; with the library functions beside it (chosen per
+// system) 226.
 template <bool ENERGY, bool ALL_SERIES>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PrecFP64::pair_waves_per_simd))) void
 pair_kernel_fp64(NX_PAIR_PARAMS(PrecFP64)) {

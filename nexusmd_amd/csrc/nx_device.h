@@ -41,6 +41,8 @@ struct SysDev {
     double L[3], invL[3], lb[3], ub[3];
     double rc, rc2, rlist, alpha, skin_half2;
     double sw_on, sw_inv;        // switching: r_switch, 1/(rc - r_switch); sw_on < 0 = off
+    double ew_exp, ew_exp_lo;    // FP64 direct space: alpha^2 / ln 2 in two parts,
+    double ew_u, ew_q;           // alpha / sqrt(2), 2 alpha / sqrt(pi) (pair_fp64_series)
     int n_atoms, atom_off;
     int slot_off, slot_cap;
     int col_off, ncx, ncy, col_cap;   // columns: ncx*ncy, each of 2 x 2 quarters
@@ -318,14 +320,37 @@ __device__ __forceinline__ void continuous_position(const SysDev& d, double x, d
     p[2] = zb + min_image1(z - zb, d.L[2]);
 }
 
-// erf(x) / x and (erf(x) - 2 x exp(-x^2) / sqrt(pi)) / x^3 as functions of
-// s = x^2.  Both are entire, so a polynomial over a bounded range converges like
-// a Taylor series: Chebyshev interpolants over s in [0, 8] (computed with 60
-// digits), written in powers of u = s / 4 - 1.  Truncation < 2e-17 of 1/x and
-// 1/x^3, evaluation error < 1e-16.  With them the Ewald direct-space term is
-// 1/r - alpha A and 1/r^3 - alpha^3 B, and its exclusion correction alpha A and
-// alpha^3 B, without an exponential, an error function or a division.
+// The FP64 direct-space term, x = alpha r: erfc(x) / r and its force factor
+// (erfc(x) + 2 x exp(-x^2) / sqrt(pi)) / r^3 with
+//     erfc(x) = exp(-x^2) E(x),  E(x) = exp(x^2) erfc(x),
+// so that the force's bracket is exp(-x^2) (E(x) + 2 x / sqrt(pi)): positive terms
+// throughout, as accurate at the cutoff, where the bracket is 1e-3, as near it.
+// kErfcx: E over x^2 <= kErfSeriesMax in powers of u = x / sqrt(2) - 1; kExp2m1:
+// (2^f - 1) / f over |f| <= 1/2 in powers of f; both Chebyshev interpolants computed
+// with 60 digits, off by 7e-17 of E + 2 x / sqrt(pi) and 2e-17 of 2^f.  RMS error on
+// the device by ranges of r from 0.1 to 1 nm at alpha = 2.63 and 2.82 / nm, of the
+// force factor 1.3e-16 to 1.7e-16 of itself, of the energy 1.2e-16 to 2.9e-16.  The
+// library's erfc, exp, sqrt and division: 2.0e-16 to 7.5e-16 and 1.2e-16 to 7.9e-16.
+// The difference 1 / r^3 - alpha^3 B(x^2) (B below) takes 17 instructions less, and
+// near the cutoff it is off by 5e-14 to 2.5e-13 of itself, its energy by 1e-12.
 constexpr double kErfSeriesMax = 8.0;
+constexpr double kErfcx[25] = {
+    3.36204002446341188e-01, -2.50953111820364894e-01, 1.70501781251950396e-01, -1.07268440757989941e-01,
+    6.32333404940961935e-02, -3.52280802078909563e-02, 1.86701735210091091e-02, -9.46166101025903983e-03,
+    4.60425629257135618e-03, -2.15884616869028599e-03, 9.78163787719972793e-04, -4.29340898122935783e-04,
+    1.82942140905975538e-04, -7.58089997705473317e-05, 3.06059328780922143e-05, -1.20672317082442645e-05,
+    4.64191805310459557e-06, -1.72783460106342884e-06, 6.37418316159805450e-07, -2.48576005282112033e-07,
+    8.73588365632618443e-08, -1.87243078346221425e-08, 6.64889187949806792e-09, -6.46832001623310008e-09,
+    2.09039891445411742e-09,
+};
+constexpr double kExp2m1[11] = {
+    6.93147180559945286e-01, 2.40226506959100972e-01, 5.55041086648215970e-02, 9.61812910760688825e-03,
+    1.33335581464169356e-03, 1.54035304417360499e-04, 1.52527338298361192e-05, 1.32154425879216893e-06,
+    1.01780624458457737e-07, 7.07258594926922339e-09, 4.45496059818651856e-10,
+};
+// erf(x) / x and (erf(x) - 2 x exp(-x^2) / sqrt(pi)) / x^3, entire functions of x^2,
+// in powers of x^2 / 4 - 1: the same two quantities by another route, which the
+// coefficients above are checked against as this header is compiled.
 constexpr double kErfA[22] = {
     4.97661132509476356e-01, -2.38497073577692176e-01, 1.58205819829175892e-01, -1.04282202718857353e-01,
     6.36909469069244089e-02, -3.52770678385127892e-02, 1.76407892660984562e-02, -7.98271979410423126e-03,
@@ -342,6 +367,25 @@ constexpr double kErfB[23] = {
     3.08155303970224502e-07, -6.77366262557539614e-08, 1.41082605777249840e-08, -2.74907686745350267e-09,
     5.19796833377220498e-10, -1.12077170695342987e-10, 1.92301651041994177e-11,
 };
+constexpr double poly(const double* c, int n, double u) {
+    double r = 0.0;
+    for (int k = n - 1; k >= 0; --k) r = r * u + c[k];
+    return r;
+}
+constexpr double poly_difference(double x) {       // of 1 - x A and 1 - x^3 B from exp(-x^2) times E and E + 2 x / sqrt(pi)
+    const double s = x * x, t = -s / 0.69314718055994530942;
+    const int k = (int)(t - 0.5);
+    double ex = 1.0 + (t - k) * poly(kExp2m1, 11, t - k);
+    for (int i = 0; i > k; --i) ex *= 0.5;
+    const double e = poly(kErfcx, 25, x / 1.41421356237309504880 - 1.0), u = 0.25 * s - 1.0;
+    const double energy = 1.0 - x * poly(kErfA, 22, u) - ex * e;
+    const double force = 1.0 - x * s * poly(kErfB, 23, u) - ex * (e + kTwoOverSqrtPi * x);
+    const double a = energy < 0 ? -energy : energy, b = force < 0 ? -force : force;
+    return a > b ? a : b;
+}
+static_assert(poly_difference(0.01) < 4e-15 && poly_difference(0.6) < 4e-15 && poly_difference(1.3) < 4e-15 &&
+                  poly_difference(2.0) < 4e-15 && poly_difference(2.8) < 4e-15,
+              "the two routes to the direct-space term differ");
 // a b + c with the constant c in scalar registers.  Written out because the
 // compiler otherwise picks the two-address form, whose addend is its result: a
 // copy of the constant, kept in vector registers, before every step.
@@ -350,16 +394,20 @@ __device__ __forceinline__ double fma_const(double a, double b, double c) {
     asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "s"(c));
     return r;
 }
-template <int N>
-__device__ __forceinline__ double erf_series(const double (&c)[N], double s) {
-    // even and odd powers as two chains: half the depth
-    const double u = fma(s, 0.25, -1.0), u2 = u * u;
-    double e = c[(N - 1) & ~1], o = c[(N - 2) | 1];
+// 2^f - 1 and E at u: three chains of multiply-adds (E's even and odd powers), a step
+// of each in turn
+__device__ __forceinline__ void direct_space_series(double f, double u, double& fp, double& e) {
+    const double u2 = u * u;
+    double p = kExp2m1[10], o = kErfcx[23];
+    e = kErfcx[24];
 #pragma unroll
-    for (int k = ((N - 1) & ~1) - 2; k >= 0; k -= 2) e = fma_const(e, u2, c[k]);
-#pragma unroll
-    for (int k = ((N - 2) | 1) - 2; k >= 1; k -= 2) o = fma_const(o, u2, c[k]);
-    return fma(o, u, e);
+    for (int k = 11; k >= 0; --k) {
+        e = fma_const(e, u2, kErfcx[2 * k]);
+        if (k > 0) o = fma_const(o, u2, kErfcx[2 * k - 1]);
+        if (k < 10) p = fma_const(p, f, kExp2m1[k]);
+    }
+    e = fma(o, u, e);
+    fp = p * f;
 }
 
 // r^2 without contraction, left-to-right as Coords3D::dot (Coords3D.h:116-124).
