@@ -338,8 +338,8 @@ class Engine : public EngineBase {
             const double skin = std::max(0.0, h.nb.skin);
             d.rlist = rc + skin;
             d.skin_half2 = skin > 0 ? 0.25 * skin * skin : -1.0;
-            d.alpha = (1.0 / rc) * sqrt(-log(2.0 * h.nb.ewald_tolerance));
-            if (!(d.alpha * d.alpha * d.rc2 <= kErfSeriesMax)) B.all_series = false;
+            d.alpha = ewald_alpha(h);
+            if (!in_series(h)) B.all_series = false;
             const long double a = d.alpha, ex = a * a / 0.693147180559945309417L;
             d.ew_exp = (double)ex;
             d.ew_exp_lo = (double)(ex - (long double)d.ew_exp);
@@ -488,7 +488,7 @@ class Engine : public EngineBase {
         dalloc(&B.slot_wpos, S, o, B.stream);
         dalloc(&B.chunks, B.n_chunk_cap, o, B.stream);
         dalloc(&B.chunk_prefix, B.nsys + 1, o, B.stream);
-        B.pair_blocks = pair_grid_blocks<P>(B.n_cu, B.n_chunk_cap, B.n_atoms, tuning_.pair_per_cu);
+        B.pair_blocks = pair_grid_blocks<P>(B.n_cu, B.n_chunk_cap, B.n_atoms, B.all_series, tuning_.pair_per_cu);
         dalloc(&B.pair_pool, (size_t)kPoolInts, o, B.stream);
         if (B.nsys == 1 && lite_mode_) {
             // the update's report to the host, for the choice of step graph
@@ -1589,6 +1589,13 @@ class Engine : public EngineBase {
     }
     Tuning tuning() const override { return tuning_; }
 
+    static double ewald_alpha(const HostSystem& h) { return (1.0 / h.nb.cutoff) * sqrt(-log(2.0 * h.nb.ewald_tolerance)); }
+    // within the range of the FP64 pair kernel without library functions
+    static bool in_series(const HostSystem& h) {
+        const double a = ewald_alpha(h);
+        return a * a * (h.nb.cutoff * h.nb.cutoff) <= kErfSeriesMax;
+    }
+
     // What the launch shapes depend on: precision, the device's CU count and, per
     // system, its atom count, box (to 0.05 nm), PME grid and cutoff.  Batches of
     // more than four systems are not cached.
@@ -1641,7 +1648,7 @@ class Engine : public EngineBase {
             const double ms = trial(t);
             if (ms < 0.99 * best_ms) { best_ms = ms; best = t; }
         };
-        const int occ = std::min(5, pair_blocks_occupancy<P>());
+        const int occ = std::min(5, pair_blocks_occupancy<P>(B.all_series));
         {
             const Tuning base = best;
             for (int c = 1; c <= occ; ++c) { Tuning t = base; t.pair_per_cu = c; consider(t); }

@@ -593,16 +593,21 @@ __global__ __launch_bounds__(64) void export_pairs_kernel(const SysDev* sd, cons
     }
 }
 
-// Blocks of the pair kernel one CU holds at once (its occupancy limit).
-template <class P>
+// Blocks of the pair kernel one CU holds at once (its occupancy limit), for the
+// kernel that a batch takes.
+template <class P, bool ALL_SERIES>
 static int pair_blocks_per_cu() {
     static const int v = [] {
         int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, pair_kernel_of<P, false>(true), 256, 0) != hipSuccess || n <= 0)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, pair_kernel_of<P, false>(ALL_SERIES), 256, 0) != hipSuccess || n <= 0)
             n = 2;
         return n;
     }();
     return v;
+}
+template <class P>
+int pair_blocks_occupancy(bool all_series) {
+    return all_series ? pair_blocks_per_cu<P, true>() : pair_blocks_per_cu<P, false>();
 }
 
 // Persistent grid of the pair kernel, all blocks resident at once, at most
@@ -612,12 +617,15 @@ static int pair_blocks_per_cu() {
 // FP64 takes two, which leave PME room, and three (all it can have) up to 30,000
 // atoms, where two waves per SIMD's worth of chunks end too unevenly: us a step with
 // 2 and 3 per CU on water of 3,000 to 12,000 atoms the same, 18,000 112.4 103.2,
-// 24,000 126.2 120.2, 30,000 140.4 137.8, 36,000 157.8 161.8, 81,000 295 344.
+// 24,000 126.2 120.2, 30,000 140.4 137.8, 36,000 157.8 161.8, 81,000 295 344.  The
+// FP64 kernel with library functions in it has room for two only: a third would
+// start its first chunks when another ends (24,000 atoms 222 us a step, with two
+// 199).
 // Fixed per batch layout: the claim counters are set for it.
 template <class P>
-int pair_grid_blocks(int n_cu, int n_chunk_cap, int n_atoms, int per_cu_request) {
+int pair_grid_blocks(int n_cu, int n_chunk_cap, int n_atoms, bool all_series, int per_cu_request) {
     // a requested count (the autotuner's) is capped by what a CU can hold at once
-    const int occ = pair_blocks_per_cu<P>();
+    const int occ = pair_blocks_occupancy<P>(all_series);
     const int per_cu = per_cu_request > 0 ? std::min(per_cu_request, occ) : std::min(occ, P::mixed || n_atoms <= 30000 ? 3 : 2);
     return std::max(1, std::min((n_chunk_cap + kPairWaves - 1) / kPairWaves, per_cu * std::max(1, n_cu)));
 }
@@ -671,15 +679,10 @@ void launch_export_pairs(Batch<P>& B, int2* out, long long cap, long long* d_cou
                                                                B.n_super_cap);
 }
 
-template int pair_grid_blocks<PrecFP64>(int, int, int, int);
-template int pair_grid_blocks<PrecMixed>(int, int, int, int);
-
-template <class P>
-int pair_blocks_occupancy() {
-    return pair_blocks_per_cu<P>();
-}
-template int pair_blocks_occupancy<PrecFP64>();
-template int pair_blocks_occupancy<PrecMixed>();
+template int pair_grid_blocks<PrecFP64>(int, int, int, bool, int);
+template int pair_grid_blocks<PrecMixed>(int, int, int, bool, int);
+template int pair_blocks_occupancy<PrecFP64>(bool);
+template int pair_blocks_occupancy<PrecMixed>(bool);
 template void launch_pair<PrecFP64>(Batch<PrecFP64>&, bool);
 template void launch_pair<PrecMixed>(Batch<PrecMixed>&, bool);
 template void launch_pair_begin<PrecFP64>(Batch<PrecFP64>&);

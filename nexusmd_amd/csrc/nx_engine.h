@@ -198,8 +198,8 @@ struct Batch {
 // alone, which then also does the pair kernel's set-up (launch_pair_begin)
 template <class P> void launch_nlist(Batch<P>& B, bool clear_flags, int part = 0);
 // persistent pair-kernel grid: per_cu_request blocks per CU (0: the built-in count), capped by occupancy
-template <class P> int pair_grid_blocks(int n_cu, int n_chunk_cap, int n_atoms, int per_cu_request);
-template <class P> int pair_blocks_occupancy();     // pair-kernel blocks one CU holds at once
+template <class P> int pair_grid_blocks(int n_cu, int n_chunk_cap, int n_atoms, bool all_series, int per_cu_request);
+template <class P> int pair_blocks_occupancy(bool all_series);     // pair-kernel blocks one CU holds at once
 template <class P> void launch_pack(Batch<P>& B);
 template <class P> void launch_pair(Batch<P>& B, bool energy);
 // the two launches of launch_pair: the per-system set-up kernel, then the pair kernel
