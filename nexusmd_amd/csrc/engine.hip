@@ -1597,8 +1597,9 @@ class Engine : public EngineBase {
     }
 
     // What the launch shapes depend on: precision, the device's CU count and, per
-    // system, its atom count, box (to 0.05 nm), PME grid and cutoff.  Batches of
-    // more than four systems are not cached.
+    // system, its atom count, box (to 0.05 nm), PME grid and cutoff, in FP64 also
+    // whether its pair kernel needs library functions.  Batches of more than four
+    // systems are not cached.
     std::string tune_key() const {
         if (hs_.empty() || hs_.size() > 4) return std::string();
         char buf[160];
@@ -1612,6 +1613,7 @@ class Engine : public EngineBase {
                           20.0 * fabs(h->ub[0] - h->lb[0]), 20.0 * fabs(h->ub[1] - h->lb[1]),
                           20.0 * fabs(h->ub[2] - h->lb[2]), g[0], g[1], g[2], h->nb.cutoff, h->nb.skin);
             k += buf;
+            if (!P::mixed && !in_series(*h)) k += ",erfc";
         }
         return k;
     }
