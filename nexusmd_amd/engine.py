@@ -17,17 +17,28 @@ def _d(a):
     return a.ctypes.data_as(L.D) if a is not None else None
 
 
-def _records(struct, count, *columns):
-    """ctypes array of `count` records (at least one) with the columns of the given
-    arrays in the order of the record's fields."""
+def _records(struct, count, index, *params):
+    """ctypes array of `count` records (at least one) from a row of `index` each, the
+    particles, and of `params`, pairs of an array and how many of its columns count.
+    Rows and parameter columns past those are not read; a missing one raises."""
     out = (struct * max(1, count))()
     if count:
         view = np.frombuffer(out, np.dtype(struct))
         fields = iter(view.dtype.names)
-        for c in columns:
-            c = np.asarray(c)
-            for k in range(1 if c.ndim == 1 else c.shape[1]):
-                view[next(fields)] = c if c.ndim == 1 else c[:, k]
+        index = np.asarray(index)
+        particles = len(view.dtype.names) - sum(width for _, width in params)
+        if index.shape[1] != particles:
+            raise ValueError("%d particles in a record of %d" % (index.shape[1], particles))
+        for c, width in ((index, particles), *params):
+            c = np.asarray(c)[:count]
+            if len(c) < count:
+                raise IndexError("%d rows of parameters for %d records" % (len(c), count))
+            c = c.reshape(count, -1)
+            for k in range(width):
+                name = next(fields)
+                if view.dtype[name].kind == "i" and not np.isfinite(c[:, k]).all():
+                    raise ValueError("%s is not a number" % name)
+                view[name] = c[:, k]
     return out
 
 
@@ -41,9 +52,9 @@ class TopologyBuffers:
         self.sig = np.ascontiguousarray(sys.sig, np.float64)
         self.eps = np.ascontiguousarray(sys.eps, np.float64)
         nb, na, nt = len(sys.bond_idx), len(sys.angle_idx), len(sys.torsion_idx)
-        self.bonds = _records(L.Bond, nb, sys.bond_idx, sys.bond_par)
-        self.angles = _records(L.Angle, na, sys.angle_idx, sys.angle_par)
-        self.torsions = _records(L.Torsion, nt, sys.torsion_idx, sys.torsion_par, sys.torsion_per)
+        self.bonds = _records(L.Bond, nb, sys.bond_idx, (sys.bond_par, 2))
+        self.angles = _records(L.Angle, na, sys.angle_idx, (sys.angle_par, 2))
+        self.torsions = _records(L.Torsion, nt, sys.torsion_idx, (sys.torsion_par, 2), (sys.torsion_per, 1))
         self.top = L.Topology()
         t = self.top
         t.n_atoms = n
