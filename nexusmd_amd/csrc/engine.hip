@@ -548,11 +548,7 @@ class Engine : public EngineBase {
             x_lines += (long long)d.grid[1] * (d.grid[2] / 2 + 1);
             rows += (long long)d.grid[0] * d.grid[1];
         }
-        // lines of a workgroup of the x pass: a cache line's width, half of one for more
-        // workgroups only on request (the passes after the spread, us alone, whole and
-        // half: 64^3 15.1, 15.4; 50 x 50 x 75 17.9, 18.1; unaligned widths between them
-        // are worse: 96^3 21.6 with 16 lines, 25.3 with 10)
-        const int xlines = x_lines > (long long)row * tuning_.fft_xblocks ? row : row / 2;
+        const int xlines = x_pass_lines(x_lines, row, tuning_.fft_xblocks);
         B.fft_x_threads = 64;
         B.fft_plane_threads = 64;
         B.fft_plane = plane ? 1 : 0;
@@ -1657,11 +1653,9 @@ class Engine : public EngineBase {
         }
         {
             const Tuning base = best;
-            if (B.fft_plane) {
-                for (int x : {128, 256, 1024, 2048}) { Tuning t = base; t.fft_xblocks = x; consider(t); }
-            } else {
+            { Tuning t = base; t.fft_xblocks = kXPassHalfLines; consider(t); }
+            if (!B.fft_plane)
                 for (int l : {1, 2, 4}) { Tuning t = base; t.fft_lines = l; consider(t); }
-            }
         }
         // the two finalists measured once more, side by side
         const double d_ms = trial(Tuning{});

@@ -90,6 +90,18 @@ inline size_t plane_spread_lds_bytes(int Ky, int Kz) {
     return (size_t)(Ky + Kz + spread_points<R2>(plane_cap(Ky, Kz), Ky, Kz)) * sizeof(R2) + spread_lds_bytes(kPlaneThreads<R2>);
 }
 
+// Lines of a workgroup of the x pass: a cache line's width (`row` of them), half of
+// one for more workgroups only on request (the passes after the spread, us alone,
+// whole and half: 64^3 15.1, 15.4; 50 x 50 x 75 17.9, 18.1; unaligned widths between
+// them are worse: 96^3 21.6 with 16 lines, 25.3 with 10).
+constexpr int kXPassHalfLines = 65536;      // as the request: half lines on any grid, the one other shape to try
+constexpr int x_pass_lines(long long x_lines, int row, int workgroups) {
+    return workgroups < kXPassHalfLines && x_lines > (long long)row * workgroups ? row : row / 2;
+}
+static_assert(x_pass_lines(1, 8, 0) == 8 && x_pass_lines(1024 * 513, 8, 0) == 8 &&
+                  x_pass_lines(1, 8, kXPassHalfLines) == 4 && x_pass_lines(1024 * 513, 8, kXPassHalfLines) == 4,
+              "two shapes on the smallest grid and on the largest");
+
 // LDS bytes of `lines` lines of K points (two buffers, the twiddles).
 template <typename R2>
 inline size_t line_lds_bytes(int K, int lines) {
