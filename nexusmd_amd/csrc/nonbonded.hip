@@ -9,13 +9,13 @@
 //
 // Work decomposition: the list is cut into chunks of up to kChunkEntries
 // entries of one super-cluster (up to 8 clusters of 8 atoms); wavefronts claim
-// chunks one at a time, their XCD's first.  Lane
-// l = 8*ia + ja holds i-atom ia of the current i-cluster and j-atom ja of the
-// current j-cluster, so one (i-cluster, j-cluster) tile is 64 pairs in one
-// VALU pass.  i-forces stay in registers over the chunk; j-forces are reduced
-// across the 8 lanes sharing ja and added once per entry.  The FP64 path tests r^2 < rc^2 with the reference's
-// minimum image and an uncontracted left-to-right dot product, so its pair
-// set is bit-identical to the reference's.
+// chunks one at a time from their XCD's range.  Lane l = 8*ia + ja holds i-atom
+// ia of the current i-cluster and j-atom ja of the current j-cluster, so one
+// (i-cluster, j-cluster) tile is 64 pairs in one VALU pass.  i-forces stay in
+// registers over the chunk; j-forces are reduced across the 8 lanes sharing ja
+// and added once per entry.  The FP64 path tests r^2 < rc^2 with the
+// reference's minimum image and an uncontracted left-to-right dot product, so
+// its pair set is bit-identical to the reference's.
 #include <algorithm>
 
 #include "nx_device.h"
@@ -611,22 +611,22 @@ int pair_blocks_occupancy(bool all_series) {
 }
 
 // Persistent grid of the pair kernel, all blocks resident at once, at most
-// three per CU: the rest of a CU's wave slots go to the bonded and
-// PME kernels running beside it.  Measured on the 100k-atom step (mixed, five
+// three per CU: the rest of a CU's wave slots go to the bonded and PME kernels
+// running beside it.  Measured on the 100k-atom step (mixed, five
 // resident blocks possible): 3 per CU 261 us, 4 per CU 303 us, 2 per CU 268 us.
-// FP64 takes two, which leave PME room, and three (all it can have) up to 30,000
+// FP64 takes two, which leave PME room, and three (all it can have) up to 50,000
 // atoms, where two waves per SIMD's worth of chunks end too unevenly: us a step with
-// 2 and 3 per CU on water of 3,000 to 12,000 atoms the same, 18,000 112.4 103.2,
-// 24,000 126.2 120.2, 30,000 140.4 137.8, 36,000 157.8 161.8, 81,000 295 344.  The
-// FP64 kernel with library functions in it has room for two only: a third would
-// start its first chunks when another ends (24,000 atoms 222 us a step, with two
-// 199).
+// 2 and 3 per CU on water of 3,000 to 12,000 atoms the same, 18,000 125 117, 24,000
+// 143 133, 30,000 161 149, 36,000 179 168, 48,000 215 198, 54,000 245 250, 81,000 331
+// 334; solvated chains of 100,000 386 387.  The FP64 kernel with library functions in
+// it has room for two only: a third would start its first chunks when another ends
+// (24,000 atoms 222 us a step, with two 199).
 // Fixed per batch layout: the claim counters are set for it.
 template <class P>
 int pair_grid_blocks(int n_cu, int n_chunk_cap, int n_atoms, bool all_series, int per_cu_request) {
     // a requested count (the autotuner's) is capped by what a CU can hold at once
     const int occ = pair_blocks_occupancy<P>(all_series);
-    const int per_cu = per_cu_request > 0 ? std::min(per_cu_request, occ) : std::min(occ, P::mixed || n_atoms <= 30000 ? 3 : 2);
+    const int per_cu = per_cu_request > 0 ? std::min(per_cu_request, occ) : std::min(occ, P::mixed || n_atoms <= 50000 ? 3 : 2);
     return std::max(1, std::min((n_chunk_cap + kPairWaves - 1) / kPairWaves, per_cu * std::max(1, n_cu)));
 }
 

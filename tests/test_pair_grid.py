@@ -34,7 +34,7 @@ def _vgprs(name, tmp):
 
 def test_fp64_pair_grid_is_resident(tmp_path):
     """The kernel without library functions leaves room for three blocks a CU (batches
-    up to 30,000 atoms) and, at two, for two 96-register wavefronts beside them (the
+    up to 50,000 atoms) and, at two, for two 96-register wavefronts beside them (the
     gather, the plane passes); the one with them holds two."""
     v = _vgprs("nonbonded", tmp_path)
     series, chooses = v("pair_kernel_fp64", "ILb0ELb1E"), v("pair_kernel_fp64", "ILb0ELb0E")
