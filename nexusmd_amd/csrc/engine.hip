@@ -173,15 +173,23 @@ static int grid_rule(double L) {
 // the batch's: a request's arithmetic is the same alone and in any batch).  A
 // chunk costs its wavefront a claim, the i data and a force flush besides its
 // entries, so large systems take the longest; with fewer chunks than a few per
-// wavefront the last ones to end leave the chip idle.  us a step with 8, 12, 16,
-// 24, 32 entries (mixed): 1,500-bead chain 66.8 66.0 66.3 68.2 73.5; water of
-// 24,000 atoms 87.6 86.9 87.2 93.6 97.5, of 36,000 95.5 96.2 98.6 101 109, of a
-// million 1598 1524 1470 1439 1426; solvated chains of 100,000 196 190 188 190
-// 193.  FP64: chain 69.0 69.2 75.6 90.4 100; 24,000 171 158 155 155 157; 100,000
-// 454 389 376 375 377.
+// wavefront the last ones to end leave the chip idle.  us a step on water boxes
+// (thousands of atoms: 8, 12, 16, 24, 32 entries), mixed:
+//   3: 58-63 60 61 69 80      6: 59-63 61 62 69 80     12: 60-63 62 62 72 79
+//   18: 66 69 65 73 83       24: 74 75 77 79 83       36: 89 89 91 97 91
+//   48: 106 104 105 110 116  60: 120 118 119 122 126  81: 149 145 145 148 151
+//   192: 301 287 283 283 285   300: 445 418 408 404 404   375: 556 519 507 499 496
+// FP64 (8, 12, 16; then 16, 24, 32):
+//   3: 64 76 63     6: 72 87 86     9: 83 90 100    12: 92 101 98   15: 106 109 116
+//   18: 118 114 118   21: 130 128 130   24: 137 129 133   30: 161 148 150
+//   36: 182 166 168   48: 225 201 199   60: 281 253 255
+//   192: 697 692 --   300: 1035 1030 1035   375: 1403 1329 1371   540: 1966 1942 1936
+// Solvated chains of 100,000, FP64: 439 389 386 (24: 391); the 1,500-bead chain 57 64
+// 76 (24: 85), mixed 58 58 58 60 67.
 static int chunk_entries_for(int n_atoms, bool mixed) {
     if (n_atoms >= 300000) return kChunkEntries;
-    return mixed ? (n_atoms < 60000 ? 12 : 16) : (n_atoms < 6000 ? 8 : 16);
+    if (mixed) return n_atoms < 60000 ? 12 : 16;
+    return n_atoms < 16500 ? 8 : (n_atoms < 42000 ? 12 : 16);
 }
 
 // ----------------------------------------------------------- tuning cache
@@ -925,7 +933,7 @@ class Engine : public EngineBase {
     // 141 -> 136.4), 176 -> 174.4 on 100,000.  FP64 systems past kRideAtomsFP64 keep
     // their own launches: the FP64 exclusions take 96 registers a thread, so their
     // blocks in the gather's launch wait for the pair kernel's registers (100,000
-    // atoms: 337 apart, 344 riding).
+    // atoms: 386 apart, 400 riding).
     static constexpr int kRideAtomsFP64 = 50000;
     void side_work(int mask, bool energy) {
         const bool ride = P::mixed || B.n_atoms <= kRideAtomsFP64;

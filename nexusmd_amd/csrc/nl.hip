@@ -444,9 +444,9 @@ constexpr int kPlWide = 16;
 //      (tile_image), when one image holds for all of its tiles, else the
 //      per-pair marker;
 //   3. per entry and i-cluster, the 64 atom pairs at build positions and the
-//      entry's image, one wavefront per entry: a tile is kept only if one of its pairs is within
-//      rlist (both atoms move at most skin/2 before the next build, so every
-//      pair that can come within rc is in a kept tile); ordered compaction;
+//      entry's image, one wavefront per entry: a tile is kept only if one of its
+//      pairs is within rlist (both atoms move at most skin/2 before the next build,
+//      so every pair that can come within rc is in a kept tile); ordered compaction;
 //   4. exclusion masks for the kept tiles.
 template <int T>
 __global__ __launch_bounds__(T) void nl_pairlist(const SysDev* sd, SysCount* sc, const int* super_sys,

@@ -19,14 +19,17 @@ namespace nx {
 
 struct HostSystem;   // engine.hip
 
-// Plane FFT passes: threads per block, LDS available to one workgroup on gfx950.
 // Threads of a plane pass: what the pair kernel's blocks leave of a SIMD's 512 VGPRs
-// holds three waves of 56 VGPRs in the mixed path (R2 float2), two of 96 in FP64
-// (with three the pass waited for the pair kernel: 24,000 atoms at 64^3 130.3 us a
-// step, with two 125.1).
+// holds three waves of 56 VGPRs in the mixed path (R2 float2; three blocks a CU of
+// 112), two of 96 in FP64 (two blocks of 160; with three waves the pass waited for the
+// pair kernel: 24,000 atoms at 64^3 130.3 us a step, with two 125.1).
 template <typename R2>
 constexpr int kPlaneThreads = sizeof(R2) == 8 ? 768 : 512;
-// Most LDS of a plane pass with the spread: what the pair kernel's blocks leave of a CU's 160 KB.
+// Most LDS of a plane pass with the spread: what those blocks leave of a CU's 160 KB.
+// Beside the three blocks that FP64 takes up to 50,000 atoms (pair_grid_blocks) a
+// plane pass finds neither the registers nor the LDS and waits for one of them to
+// end.  So would the line passes, and planes are still the faster ones: us a step,
+// planes and lines, 12,000 atoms 98.2, 100.7; 24,000 132.8, 136.9.
 template <typename R2>
 constexpr size_t kPlaneSpreadLds = (sizeof(R2) == 8 ? 100 : 82) * 1024;
 constexpr int kXPassThreads = 256;
@@ -35,7 +38,8 @@ constexpr int kPassRowBytes = 128;
 // Points by which each row of the potential runs on past its end (its first
 // ones again): the gather reads five consecutive points from any of the row's.
 constexpr int kPhiPad = 4;
-constexpr size_t kMaxBlockLds = 160 * 1024 - 1024;   // less the kernels' static LDS
+// LDS of one workgroup on gfx950, less the kernels' static LDS.
+constexpr size_t kMaxBlockLds = 160 * 1024 - 1024;
 
 // LDS bytes of the spread in a block of `threads`: its table of slot segments
 // and 128 queued slots per wavefront.
@@ -183,7 +187,7 @@ struct Batch {
     // PME
     using gacc = typename P::gacc;
     real2* cgrid = nullptr;         // half spectrum [sum Kx*Ky*(Kz/2+1)]
-    real* phi = nullptr;            // potential grid [sum Kx*Ky*Kz]
+    real* phi = nullptr;            // potential grid [sum Kx*Ky*(Kz + kPhiPad)]
     real* eta = nullptr;            // influence function on the half spectrum
     real2* twiddle = nullptr;       // per system, per axis exp(-2 pi i t / K)
     long long rgrid_total = 0, cgrid_total = 0, tw_total = 0;
@@ -207,7 +211,8 @@ struct Batch {
 };
 
 // part 0: the whole list work; 1: all but its last kernel; 2: the last kernel
-// alone, which then also does the pair kernel's set-up (launch_pair_begin)
+// alone, which then also does the pair kernel's set-up (launch_pair_begin); 3: the
+// same in a step without the other list kernels (a due list is marked stale)
 template <class P> void launch_nlist(Batch<P>& B, bool clear_flags, int part = 0);
 // persistent pair-kernel grid: per_cu_request blocks per CU (0: the built-in count), capped by occupancy
 template <class P> int pair_grid_blocks(int n_cu, int n_chunk_cap, int n_atoms, bool all_series, int per_cu_request);
